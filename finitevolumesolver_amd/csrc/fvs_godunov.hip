@@ -52,14 +52,22 @@ __device__ __forceinline__ unsigned long long WaveMaxU(unsigned long long k) {
   return k;
 }
 
-// Block reduction of (min dt key, sum iterations, max iterations,
-// non-converged faces, faces) to partials[block * 5 + i].
-__device__ void BlockReduceGodunov(unsigned long long key, unsigned long long iters,
+// Key of the stable dt dx / speed of a largest signal speed (+inf for 0): a
+// rounded quotient falls monotonically with its denominator, so the smallest
+// face dt is the quotient by the largest speed.
+__device__ __forceinline__ unsigned long long SpeedKey(double dx, double speed) {
+  return speed > 0.0 ? DtKey(DivRn(dx, speed)) : kInfKey;
+}
+
+// Block reduction of (largest speed, sum iterations, max iterations,
+// non-converged faces, faces) to partials[block * 5 + i], the speed as the
+// key of its stable dt.
+__device__ void BlockReduceGodunov(double speed, double dx, unsigned long long iters,
                                    unsigned long long maxit, unsigned long long fails,
                                    unsigned long long faces, unsigned long long* out) {
   __shared__ unsigned long long s[5][kBlock / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  key = WaveMinKey(key);
+  unsigned long long key = WaveMinKey(SpeedKey(dx, speed));
   iters = WaveSum(iters);
   maxit = WaveMaxU(maxit);
   fails = WaveSum(fails);
@@ -122,48 +130,24 @@ __device__ __forceinline__ void ShflUpState(const double* q, double* r) {
   for (int k = 0; k < D + 4; ++k) r[k] = __shfl_up(q[k], 1, 64);
 }
 
-// Mixed form of the flux: the sampled state and its physical flux in float.
-template <int D, int DIR>
-__device__ __forceinline__ void GodunovFluxMixed(double* flux, const double* L, const double* R,
-                                                 const MiddleState& ms, const Gas<double>& g) {
-  constexpr int NQ = D + 4;
-  float lf[NQ], rf[NQ], sol[NQ], ff[D + 2];
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    lf[k] = static_cast<float>(L[k]);
-    rf[k] = static_cast<float>(R[k]);
-    sol[k] = 0.0f;
-  }
-  Gas<float> gf;
-  gf.gamma = static_cast<float>(g.gamma);
-  gf.gm1inv = static_cast<float>(g.gm1inv);
-  gf.gm1 = static_cast<float>(g.gm1);
-  if (0.0 < L[0] && 0.0 < R[0])
-    SampleRiemannT<D, DIR, float>(sol, lf, rf, static_cast<float>(ms.pM),
-                                  static_cast<float>(ms.uM), gf);
-  PhysFlux<D, DIR, float>(ff, sol);
-#pragma unroll
-  for (int k = 0; k < D + 2; ++k) flux[k] = static_cast<double>(ff[k]);
-}
-
 // Newton from a caller's seed (learned or given), with the reference's
 // initial guess, the mean pressure, as the fallback.  A seed that is not a
 // finite positive pressure (an overflowed or underflowed network output) is
 // not tried; a run from the seed that does not converge, or ends on a
 // pressure that is not finite and non-negative, is redone from the mean.
 // Both count as a fallback.
-template <int D, int DIR, bool MIXED>
+template <int D, int DIR>
 __device__ __forceinline__ MiddleState SeededMiddleState(const double* L, const double* R,
                                                          const Gas<double>& g,
                                                          const NewtonParams& np, bool seeded,
                                                          double seed, double mean, int* iters,
                                                          int* fallback) {
   const bool usable = seeded && seed > 0.0 && seed <= 1.7976931348623157e308;
-  MiddleState ms = ComputeMiddleState<D, DIR, MIXED>(L, R, g, np, usable ? seed : mean);
+  MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, usable ? seed : mean);
   int it = ms.iterations;
   int fb = seeded && !usable;
   if (usable && !(ms.converged && ms.pM >= 0.0 && ms.pM <= 1.7976931348623157e308)) {
-    ms = ComputeMiddleState<D, DIR, MIXED>(L, R, g, np, mean);
+    ms = ComputeMiddleState<D, DIR>(L, R, g, np, mean);
     it += ms.iterations;
     fb = 1;
   }
@@ -172,9 +156,33 @@ __device__ __forceinline__ MiddleState SeededMiddleState(const double* L, const 
   return ms;
 }
 
-// One face: Newton (shared by flux and CFL), flux, dt.  MIXED: the Newton
-// iteration stays FP64 (with exp/log powers) and the sample and flux are
-// float.
+// Largest signal speed of a face from its middle state.
+template <int D, int DIR>
+__device__ __forceinline__ double FaceSpeed(const double* L, const double* R,
+                                            const MiddleState& ms) {
+  using I = Idx<D>;
+  double wL, wR;
+  return GodunovSpeed(L[I::kRho], NearArith::quot(L[I::kMom + DIR], L[I::kRho]), L[I::kP],
+                      L[I::kA], R[I::kRho], NearArith::quot(R[I::kMom + DIR], R[I::kRho]),
+                      R[I::kP], R[I::kA], ms, &wL, &wR);
+}
+
+// Flux and largest signal speed of a face from its middle state.
+template <int D, int DIR, bool MIXED>
+__device__ __forceinline__ void FaceFluxSpeed(const double* L, const double* R,
+                                              const MiddleState& ms, const Gas<double>& g,
+                                              double* F, double* speed) {
+  using I = Idx<D>;
+  const double yL = NearArith::inv(L[I::kRho]), yR = NearArith::inv(R[I::kRho]);
+  double wL, wR;
+  *speed = GodunovSpeed(L[I::kRho], NearArith::div(L[I::kMom + DIR], L[I::kRho], yL), L[I::kP],
+                        L[I::kA], R[I::kRho], NearArith::div(R[I::kMom + DIR], R[I::kRho], yR),
+                        R[I::kP], R[I::kA], ms, &wL, &wR);
+  GodunovFlux<D, DIR, MIXED>(F, L, yL, R, yR, ms, wL, wR, g);
+}
+
+// One face: Newton (shared by flux and CFL), flux, largest signal speed.
+// MIXED: the sampled star density's power in single precision.
 //
 // With a.reuse the seed is the converged iterate of the step-start CFL pass
 // for the same face and state: Newton from it evaluates the side functions
@@ -185,7 +193,7 @@ __device__ __forceinline__ MiddleState SeededMiddleState(const double* L, const 
 template <int D, int DIR, bool MIXED>
 __device__ __forceinline__ void GodunovFace(const double* L, const double* R, double guess,
                                             bool has_guess, const GodunovArgs& a,
-                                            const Gas<double>& g, double* F, double* dt_face,
+                                            const Gas<double>& g, double* F, double* speed,
                                             int* iters, int* conv) {
   NewtonParams np;
   np.tol = a.tol;
@@ -196,17 +204,12 @@ __device__ __forceinline__ void GodunovFace(const double* L, const double* R, do
   MiddleState ms;
   if (a.reuse) {
     reused = guess > 0.0 && guess <= 1.7976931348623157e308;
-    ms = ComputeMiddleState<D, DIR, MIXED>(L, R, g, np, reused ? guess : mean);
+    ms = ComputeMiddleState<D, DIR>(L, R, g, np, reused ? guess : mean);
     it = ms.iterations;
   } else {
-    ms = SeededMiddleState<D, DIR, MIXED>(L, R, g, np, has_guess, guess, mean, &it, &fallback);
+    ms = SeededMiddleState<D, DIR>(L, R, g, np, has_guess, guess, mean, &it, &fallback);
   }
-  if constexpr (MIXED) {
-    GodunovFluxMixed<D, DIR>(F, L, R, ms, g);
-  } else {
-    GodunovFluxFromMiddle<D, DIR>(F, L, R, ms, g);
-  }
-  *dt_face = GodunovDtFromMiddle<D, DIR>(L, R, ms.pM, g, a.dx);
+  FaceFluxSpeed<D, DIR, MIXED>(L, R, ms, g, F, speed);
   *iters = it;
   *conv = ms.converged | (fallback << 1) | (reused << 2);
 }
@@ -246,7 +249,8 @@ __global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
   const bool face_lane = valid && lane >= 1 && sl >= 1;
   const bool owned = lane >= 1 && lane <= kXOwned;
   double F[NC];
-  unsigned long long key = kInfKey, it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
+  double smax = 0.0;
+  unsigned long long it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
   // Inline learned guess: every lane takes part in the wave's matrix-core step.
   double inline_guess = 0.0;
   if constexpr (LEARNED) inline_guess = mlp::LearnedGuess<D, 0>(L, u, a.tiles, a.bias);
@@ -255,12 +259,12 @@ __global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
     const double guess = LEARNED   ? inline_guess
                          : a.guess ? a.guess[static_cast<int64_t>(row) * (nx + 1) + f]
                                    : 0.0;
-    double dtf;
+    double speed;
     int it, conv;
-    GodunovFace<D, 0, MIXED>(L, u, guess, LEARNED || a.guess != nullptr, a, g, F, &dtf, &it,
+    GodunovFace<D, 0, MIXED>(L, u, guess, LEARNED || a.guess != nullptr, a, g, F, &speed, &it,
                              &conv);
     if (owned) {
-      key = DtKey(dtf);
+      smax = speed;
       it_sum = it;
       it_max = it;
       nfail = (conv & 1) ? 0 : 1;
@@ -278,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
 #pragma unroll
     for (int k = 0; k < NC; ++k) a.out[k][off] = u[k] + dt_dx * (F[k] - Fnext[k]);
   }
-  BlockReduceGodunov(key, it_sum, it_max, nfail, nfaces, a.partials + 5 * blockIdx.x);
+  BlockReduceGodunov(smax, a.dx, it_sum, it_max, nfail, nfaces, a.partials + 5 * blockIdx.x);
 }
 
 template <int D, int DIR, bool MIXED, bool LEARNED>
@@ -305,7 +309,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const double dt_dx = DivRn(dt, a.dx);
   (void)nz;
 
-  unsigned long long key = kInfKey, it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
+  double smax = 0.0;
+  unsigned long long it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
   {
     auto load = [&](double* q, int64_t j) {
       const int64_t off = base + Clamp(j, nd) * stride;
@@ -318,7 +323,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     double Fprev[NC];
     for (int64_t j = j0; j <= j1; ++j) {
       load(q0, j);
-      double F[NC], dtf;
+      double F[NC], speed;
       int it, conv;
       double guess = 0.0;
       if constexpr (LEARNED) {
@@ -326,10 +331,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       } else if (a.guess) {
         guess = a.guess[fbase + j * fstride];
       }
-      GodunovFace<D, DIR, MIXED>(qm, q0, guess, LEARNED || a.guess != nullptr, a, g, F, &dtf,
+      GodunovFace<D, DIR, MIXED>(qm, q0, guess, LEARNED || a.guess != nullptr, a, g, F, &speed,
                                  &it, &conv);
       if (active && (j < j1 || j1 == nd)) {
-        key = KMin(key, DtKey(dtf));
+        smax = __builtin_fmax(smax, speed);
         it_sum += it;
         it_max = (unsigned long long)it > it_max ? it : it_max;
         nfail += (conv & 1) ? 0 : 1;
@@ -347,7 +352,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       for (int k = 0; k < NC; ++k) Fprev[k] = F[k];
     }
   }
-  BlockReduceGodunov(key, it_sum, it_max, nfail, nfaces,
+  BlockReduceGodunov(smax, a.dx, it_sum, it_max, nfail, nfaces,
                      a.partials + 5 * (blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x));
 }
 
@@ -476,8 +481,8 @@ __global__ __launch_bounds__(kBlock) void GodunovViewFlux(DevView fl, DevView st
   np.max_it = max_it;
   const MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, 0.5 * (L[D + 2] + R[D + 2]));
   if (!ms.converged) atomicAdd(nfail, 1ull);
-  double F[NC];
-  GodunovFluxFromMiddle<D, DIR>(F, L, R, ms, g);
+  double F[NC], speed;
+  FaceFluxSpeed<D, DIR, false>(L, R, ms, g, F, &speed);
   for (int k = 0; k < NC; ++k) *fl.at(f, k) = F[k];
 }
 
@@ -503,7 +508,7 @@ __global__ __launch_bounds__(kBlock) void GodunovViewStableDt(DevView st, DevVie
     np.tol = tol;
     np.max_it = max_it;
     const MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, 0.5 * (L[D + 2] + R[D + 2]));
-    key = DtKey(GodunovDtFromMiddle<D, DIR>(L, R, ms.pM, g, dx));
+    key = SpeedKey(dx, FaceSpeed<D, DIR>(L, R, ms));
   }
   __shared__ unsigned long long s[kBlock / 64];
   key = WaveMinKey(key);
@@ -547,7 +552,7 @@ struct GodunovCflArgs {
 // where the reference's would be.
 
 // Certified upper bound of the exact solver's signal speeds max(|s0|, |s1|)
-// (GodunovDtFromMiddle) of a face, without Newton, for the faces of the
+// (GodunovSpeed) of a face, without Newton, for the faces of the
 // class on which Newton from the mean pressure converges quickly: positive
 // densities and pressures, pressure ratio at most 4, sound speeds at most
 // 1e6 and |uR - uL| at most the smaller sound speed (no vacuum).  Toro's f(p)
@@ -597,7 +602,7 @@ __device__ __forceinline__ bool GodunovSpeedBound(const double* L, const double*
 
 // Newton seed of a face: the inline learned guess (lg, computed by the whole
 // wave), else the face's guess array entry, else the mean pressure.
-template <int D, int DIR, bool MIXED, bool LEARNED>
+template <int D, int DIR, bool LEARNED>
 __device__ __forceinline__ double CflFace(const double* L, const double* R,
                                           const GodunovCflArgs& a, const Gas<double>& g,
                                           int64_t fidx, double lg, unsigned long long* acc) {
@@ -609,20 +614,18 @@ __device__ __forceinline__ double CflFace(const double* L, const double* R,
   const double x0 = LEARNED ? lg : a.guess[DIR] ? a.guess[DIR][fidx] : mean;
   int iters, fallback;
   const MiddleState ms =
-      SeededMiddleState<D, DIR, MIXED>(L, R, g, np, seeded, x0, mean, &iters, &fallback);
+      SeededMiddleState<D, DIR>(L, R, g, np, seeded, x0, mean, &iters, &fallback);
   const unsigned long long it = static_cast<unsigned long long>(iters);
   const unsigned long long fb = static_cast<unsigned long long>(fallback);
   if (a.pm_out && DIR == a.pm_dir) a.pm_out[fidx] = ms.converged ? ms.pM : __builtin_nan("");
-  const double dt = GodunovDtFromMiddle<D, DIR>(L, R, ms.pM, g, a.dx[DIR]);
-  acc[0] = KMin(acc[0], DtKey(dt));
-  acc[1] += it;
-  acc[2] = it > acc[2] ? it : acc[2];
-  acc[3] += ms.converged ? 0 : 1;
-  acc[4] += 1 + (fb << 32);
-  return dt;
+  acc[0] += it;
+  acc[1] = it > acc[1] ? it : acc[1];
+  acc[2] += ms.converged ? 0 : 1;
+  acc[3] += 1 + (fb << 32);
+  return FaceSpeed<D, DIR>(L, R, ms);
 }
 
-template <int D, bool MIXED, bool LEARNED>
+template <int D, bool LEARNED>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovCflKernel(GodunovCflArgs a) {
   constexpr int NC = D + 2, NQ = D + 4;
   constexpr int M = D - 1;
@@ -645,16 +648,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int64_t m1 = (m0 + kCflSeg < nm) ? m0 + kCflSeg : nm;
   const int64_t rowoff = (D == 3) ? y * nx : 0;
   // Speed floor of the directions other than pm_dir (0: every face solved).
-  double F[3] = {0.0, 0.0, 0.0}, dtF[3] = {0.0, 0.0, 0.0};
+  double F[3] = {0.0, 0.0, 0.0};
   if (a.floor) {
     for (int d = 0; d < D; ++d) {
-      if (d != a.pm_dir && a.floor[d] > 0.0) {
-        F[d] = a.floor[d];
-        dtF[d] = a.dx[d] / F[d];
-      }
+      if (d != a.pm_dir && a.floor[d] > 0.0) F[d] = a.floor[d];
     }
   }
-  bool hit[3] = {false, false, false};
   // A face skips its Newton solve when its certified speed bound stays below
   // the floor by a relative 2^-30 (far above the rounding of either side).
   auto skipped = [&](auto dir_tag, const double* l, const double* r) -> bool {
@@ -664,11 +663,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     return GodunovSpeedBound<D, DD>(l, r, g, a.tol, &sb) && sb * (1.0 + 0x1p-30) < F[DD];
   };
   __shared__ double s_q[NQ][kTX];
-  unsigned long long acc[3][5];
-  for (int d = 0; d < 3; ++d) {
-    acc[d][0] = kInfKey;
-    acc[d][1] = acc[d][2] = acc[d][3] = acc[d][4] = 0;
-  }
+  double smax[3] = {0.0, 0.0, 0.0};
+  unsigned long long acc[3][4] = {};
   auto load = [&](int64_t off, double* q) {
 #pragma unroll
     for (int k = 0; k < NC; ++k) q[k] = a.in[k][off];
@@ -704,15 +700,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       const bool skip = active && skipped(XM{}, l, qc);
       const double lg = __all(skip || !active) ? 0.0 : learned(XM{}, l, qc);
       if (active && !skip) {
-        const double dt = CflFace<D, M, MIXED, LEARNED>(
+        const double sp = CflFace<D, M, LEARNED>(
             l, qc, a, g, (M == 1) ? fidx(1, xs, m, 0) : fidx(2, xs, cy, m), lg, acc[M]);
-        hit[M] = hit[M] || dt <= dtF[M];
+        smax[M] = __builtin_fmax(smax[M], sp);
       }
       if (active && m == nm - 1 && !skipped(XM{}, qc, qc)) {
-        const double dt = CflFace<D, M, MIXED, LEARNED>(
+        const double sp = CflFace<D, M, LEARNED>(
             qc, qc, a, g, (M == 1) ? fidx(1, xs, m + 1, 0) : fidx(2, xs, cy, m + 1),
             0.5 * (qc[D + 2] + qc[D + 2]), acc[M]);
-        hit[M] = hit[M] || dt <= dtF[M];
+        smax[M] = __builtin_fmax(smax[M], sp);
       }
     }
     if constexpr (D == 3) {
@@ -725,13 +721,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       const bool skip = active && skipped(X1{}, qy, qc);
       const double lg = __all(skip || !active) ? 0.0 : learned(X1{}, qy, qc);
       if (active && !skip) {
-        const double dt = CflFace<D, 1, MIXED, LEARNED>(qy, qc, a, g, fidx(1, xs, y, cz), lg, acc[1]);
-        hit[1] = hit[1] || dt <= dtF[1];
+        const double sp = CflFace<D, 1, LEARNED>(qy, qc, a, g, fidx(1, xs, y, cz), lg, acc[1]);
+        smax[1] = __builtin_fmax(smax[1], sp);
       }
       if (active && y == ny - 1 && !skipped(X1{}, qc, qc)) {
-        const double dt = CflFace<D, 1, MIXED, LEARNED>(qc, qc, a, g, fidx(1, xs, y + 1, cz),
+        const double sp = CflFace<D, 1, LEARNED>(qc, qc, a, g, fidx(1, xs, y + 1, cz),
                                                         0.5 * (qc[D + 2] + qc[D + 2]), acc[1]);
-        hit[1] = hit[1] || dt <= dtF[1];
+        smax[1] = __builtin_fmax(smax[1], sp);
       }
     }
 #pragma unroll
@@ -749,13 +745,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       const bool skip = active && skipped(X0{}, ql, qc);
       const double lg = __all(skip || !active) ? 0.0 : learned(X0{}, ql, qc);
       if (active && !skip) {
-        const double dt = CflFace<D, 0, MIXED, LEARNED>(ql, qc, a, g, fidx(0, xs, cy, cz), lg, acc[0]);
-        hit[0] = hit[0] || dt <= dtF[0];
+        const double sp = CflFace<D, 0, LEARNED>(ql, qc, a, g, fidx(0, xs, cy, cz), lg, acc[0]);
+        smax[0] = __builtin_fmax(smax[0], sp);
       }
       if (active && x == nx - 1 && !skipped(X0{}, qc, qc)) {
-        const double dt = CflFace<D, 0, MIXED, LEARNED>(qc, qc, a, g, fidx(0, xs + 1, cy, cz),
+        const double sp = CflFace<D, 0, LEARNED>(qc, qc, a, g, fidx(0, xs + 1, cy, cz),
                                                         0.5 * (qc[D + 2] + qc[D + 2]), acc[0]);
-        hit[0] = hit[0] || dt <= dtF[0];
+        smax[0] = __builtin_fmax(smax[0], sp);
       }
     }
     __syncthreads();
@@ -765,10 +761,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int64_t nblocks = static_cast<int64_t>(gridDim.x) * gridDim.y;
   const int64_t bid = blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x;
   for (int d = 0; d < D; ++d)
-    BlockReduceGodunov(acc[d][0], acc[d][1], acc[d][2], acc[d][3], acc[d][4],
+    BlockReduceGodunov(smax[d], a.dx[d], acc[d][0], acc[d][1], acc[d][2], acc[d][3],
                        a.partials + 5 * (d * nblocks + bid));
   for (int d = 0; d < D; ++d) {
-    if (__syncthreads_or(hit[d] ? 1 : 0) && threadIdx.x == 0 && a.hit) a.hit[d] = 1;
+    const bool hit = F[d] > 0.0 && smax[d] >= F[d];
+    if (__syncthreads_or(hit ? 1 : 0) && threadIdx.x == 0 && a.hit) a.hit[d] = 1;
   }
 }
 
@@ -938,18 +935,15 @@ int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* c
     a.floor = floor_ctl->cfl_floor;
     a.hit = floor_ctl->floor_hit;
   }
-  const bool mixed = desc.precision == FVS_FP32_FLUX;
   const int64_t tiles = (a.n[0] + kTX - 1) / kTX;
   const int64_t gx = tiles * (D == 3 ? a.n[1] : 1);
   const int64_t gy = ((D == 3 ? a.n[2] : a.n[1]) + kCflSeg - 1) / kCflSeg;
   if (gx > 0x7fffffff || gy > 65535) return FVS_BAD_ARGUMENT;
   using K = void (*)(GodunovCflArgs);
-  const K ks[2][2][2] = {{{GodunovCflKernel<2, false, false>, GodunovCflKernel<2, false, true>},
-                          {GodunovCflKernel<2, true, false>, GodunovCflKernel<2, true, true>}},
-                         {{GodunovCflKernel<3, false, false>, GodunovCflKernel<3, false, true>},
-                          {GodunovCflKernel<3, true, false>, GodunovCflKernel<3, true, true>}}};
+  const K ks[2][2] = {{GodunovCflKernel<2, false>, GodunovCflKernel<2, true>},
+                      {GodunovCflKernel<3, false>, GodunovCflKernel<3, true>}};
   const bool learned = a.tiles != nullptr;
-  hipLaunchKernelGGL(ks[D == 3][mixed][learned], dim3(unsigned(gx), unsigned(gy)), dim3(kBlock),
+  hipLaunchKernelGGL(ks[D == 3][learned], dim3(unsigned(gx), unsigned(gy)), dim3(kBlock),
                      0, s, a);
   FVS_LAUNCH_CHECK();
   return FVS_OK;

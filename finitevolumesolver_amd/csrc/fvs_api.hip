@@ -1,6 +1,7 @@
 // C ABI of libfvs_hip.so: handles, the reference's patch-level operators on
 // strided views, and the single-patch level driver built on the fused
 // sweeps.
+#include "fvs_godunov_bound.hpp"
 #include "fvs_internal.hpp"
 #include "fvs_physics.hpp"
 #include "fvs_views.hpp"
@@ -714,7 +715,7 @@ static int PatchStableDt(fvs_handle* h, const double* const* cons, const int64_t
     partials = h->partials;
   }
   if (godunov) {
-    if (int rc = LaunchGodunovCfl(h->desc, h->stream, cons, nn, dx, nullptr, partials, nullptr))
+    if (int rc = LaunchGodunovCfl(h->desc, h->stream, cons, nn, dx, partials, nullptr))
       return rc;
     for (int d = 0; d < D; ++d) {
       if (int rc = LaunchGodunovFinalize(h->stream, partials + 5 * d * nb, nb,
@@ -906,8 +907,6 @@ struct fvs_level {
   Ctl* ctl;               // device control block
   unsigned long long* partials;  // per-workgroup minima
   int64_t cfl_redos = 0;  // steps repeated because a speed floor was wrong
-  double* pm = nullptr;   // exact Godunov: the step-start CFL pass's star
-                          // pressures of the first sweep's faces
   int cur;                // buffer holding the current state
   // Kernel timing (off by default): HIP events recorded on the level's stream
   // around every launch, reduced per kernel class when read.
@@ -1059,18 +1058,6 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch, fvs_level** out
     SetError("hipMalloc of the reduction partials failed");
     return FVS_HIP_ERROR;
   }
-  if (godunov) {
-    int64_t nf = 0;
-    for (int d = 0; d < D; ++d) nf = std::max<int64_t>(nf, L->ncell / n[d] * (n[d] + 1));
-    if (hipMalloc(&L->pm, nf * sizeof(double)) != hipSuccess) {
-      (void)hipFree(L->block);
-      (void)hipFree(L->ctl);
-      (void)hipFree(L->partials);
-      delete L;
-      SetError("hipMalloc of the star-pressure faces failed");
-      return FVS_HIP_ERROR;
-    }
-  }
   for (int b = 0; b < 3; ++b)
     for (int c = 0; c < D + 2; ++c) L->buf[b][c] = L->block + (static_cast<int64_t>(b) * (D + 2) + c) * L->ncell;
   L->cur = 0;
@@ -1097,7 +1084,6 @@ int fvs_level_destroy(fvs_level* L) {
   (void)hipFree(L->block);
   (void)hipFree(L->ctl);
   (void)hipFree(L->partials);
-  if (L->pm) (void)hipFree(L->pm);
   for (const auto& m : L->marks) {
     (void)hipEventDestroy(m.a);
     (void)hipEventDestroy(m.b);
@@ -1271,8 +1257,8 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
   if (godunov) {
     const int64_t nb = GodunovCflBlocks(D, L->n);
     rc = Timed(L, s, FVS_TIMER_CFL, [&] {
-      return LaunchGodunovCfl(h->desc, s, cin, L->n, L->patch.dx, nullptr, L->partials,
-                              &L->ctl->halt, net, L->pm, seq[0], L->ctl);
+      return LaunchGodunovCfl(h->desc, s, cin, L->n, L->patch.dx, L->partials, &L->ctl->halt,
+                              L->ctl);
     });
     for (int d = 0; d < D && rc == FVS_OK; ++d) {
       rc = LaunchGodunovFinalize(s, L->partials + 5 * d * nb, nb, &L->ctl->dt_dir[d],
@@ -1301,13 +1287,10 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
     for (int q = 0; q < D + 2; ++q) inp[q] = L->buf[src][q];
     if (godunov) {
       const int64_t nb = GodunovSweepBlocks(D, seq[w], L->n, PencilSeg(D, seq[w], L->n));
-      // The first sweep runs on the step-start state, whose star pressures
-      // in its direction the CFL pass kept: its faces are not solved again.
       rc = Timed(L, s, FVS_TIMER_SWEEP_X + seq[w], [&] {
         return LaunchGodunovSweep(h->desc, s, seq[w], inp, outp, L->n, L->patch.dx[seq[w]],
-                                  &L->ctl->split_dt, 0.0, w == 0 ? L->pm : nullptr,
-                                  L->partials, &L->ctl->halt, 1, w == 0 ? nullptr : net,
-                                  w == 0 ? 1 : 0);
+                                  &L->ctl->split_dt, 0.0, nullptr, L->partials, &L->ctl->halt, 1,
+                                  net);
       });
       if (rc == FVS_OK)
         rc = LaunchGodunovFinalize(s, L->partials, nb, &L->ctl->last_check, h->newton_stats,

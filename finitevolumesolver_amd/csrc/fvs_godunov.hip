@@ -9,7 +9,9 @@
 // guess (the learned star pressure) replaces 0.5 (pL + pR); Newton itself,
 // its tolerance and its safeguards are unchanged.  Newton statistics
 // (iterations, non-converged faces) are accumulated per workgroup.
+#include "fvs_godunov_bound.hpp"
 #include "fvs_internal.hpp"
+#include "fvs_lanes.hpp"
 #include "fvs_mlp_infer.hpp"
 #include "fvs_riemann.hpp"
 #include "fvs_views.hpp"
@@ -62,10 +64,11 @@ __device__ __forceinline__ unsigned long long SpeedKey(double dx, double speed) 
 // Block reduction of (largest speed, sum iterations, max iterations,
 // non-converged faces, faces) to partials[block * 5 + i], the speed as the
 // key of its stable dt.
+template <int WAVES>
 __device__ void BlockReduceGodunov(double speed, double dx, unsigned long long iters,
                                    unsigned long long maxit, unsigned long long fails,
                                    unsigned long long faces, unsigned long long* out) {
-  __shared__ unsigned long long s[5][kBlock / 64];
+  __shared__ unsigned long long s[5][WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned long long key = WaveMinKey(SpeedKey(dx, speed));
   iters = WaveSum(iters);
@@ -82,7 +85,7 @@ __device__ void BlockReduceGodunov(double speed, double dx, unsigned long long i
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long r[5] = {s[0][0], s[1][0], s[2][0], s[3][0], s[4][0]};
-    for (int w = 1; w < kBlock / 64; ++w) {
+    for (int w = 1; w < WAVES; ++w) {
       r[0] = KMin(r[0], s[0][w]);
       r[1] += s[1][w];
       r[2] = s[2][w] > r[2] ? s[2][w] : r[2];
@@ -91,6 +94,7 @@ __device__ void BlockReduceGodunov(double speed, double dx, unsigned long long i
     }
     for (int i = 0; i < 5; ++i) out[i] = r[i];
   }
+  __syncthreads();
 }
 
 struct GodunovArgs {
@@ -111,9 +115,6 @@ struct GodunovArgs {
   int* halt;
   int seg;
   int update;            // 0: only fluxes' Newton + CFL (no state write)
-  int reuse;             // guess holds the star pressures the step-start CFL
-                         // pass found for these faces on the same state
-                         // (NaN where its Newton did not converge)
 };
 
 __device__ __forceinline__ Gas<double> GasOf(const GodunovArgs& a) {
@@ -183,13 +184,6 @@ __device__ __forceinline__ void FaceFluxSpeed(const double* L, const double* R,
 
 // One face: Newton (shared by flux and CFL), flux, largest signal speed.
 // MIXED: the sampled star density's power in single precision.
-//
-// With a.reuse the seed is the converged iterate of the step-start CFL pass
-// for the same face and state: Newton from it evaluates the side functions
-// at that pressure, finds the residual within the tolerance and stops at
-// once with the same star pressure and velocity, so the face is not solved
-// again (and not counted as a solved face, bit 2 of *conv).  A NaN seed (no
-// converged iterate) solves the face from the mean pressure.
 template <int D, int DIR, bool MIXED>
 __device__ __forceinline__ void GodunovFace(const double* L, const double* R, double guess,
                                             bool has_guess, const GodunovArgs& a,
@@ -200,18 +194,12 @@ __device__ __forceinline__ void GodunovFace(const double* L, const double* R, do
   np.max_it = a.max_it;
   using I = Idx<D>;
   const double mean = 0.5 * (L[I::kP] + R[I::kP]);
-  int it, fallback = 0, reused = 0;
-  MiddleState ms;
-  if (a.reuse) {
-    reused = guess > 0.0 && guess <= 1.7976931348623157e308;
-    ms = ComputeMiddleState<D, DIR>(L, R, g, np, reused ? guess : mean);
-    it = ms.iterations;
-  } else {
-    ms = SeededMiddleState<D, DIR>(L, R, g, np, has_guess, guess, mean, &it, &fallback);
-  }
+  int it, fallback;
+  const MiddleState ms =
+      SeededMiddleState<D, DIR>(L, R, g, np, has_guess, guess, mean, &it, &fallback);
   FaceFluxSpeed<D, DIR, MIXED>(L, R, ms, g, F, speed);
   *iters = it;
-  *conv = ms.converged | (fallback << 1) | (reused << 2);
+  *conv = ms.converged | (fallback << 1);
 }
 
 // LEARNED: the network's guess is inferred inline (a.tiles set); without it
@@ -268,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
       it_sum = it;
       it_max = it;
       nfail = (conv & 1) ? 0 : 1;
-      nfaces = ((conv >> 2) & 1) ? 0 : 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
+      nfaces = 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
     }
   } else {
 #pragma unroll
@@ -282,7 +270,7 @@ __global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
 #pragma unroll
     for (int k = 0; k < NC; ++k) a.out[k][off] = u[k] + dt_dx * (F[k] - Fnext[k]);
   }
-  BlockReduceGodunov(smax, a.dx, it_sum, it_max, nfail, nfaces, a.partials + 5 * blockIdx.x);
+  BlockReduceGodunov<kBlock / 64>(smax, a.dx, it_sum, it_max, nfail, nfaces, a.partials + 5 * blockIdx.x);
 }
 
 template <int D, int DIR, bool MIXED, bool LEARNED>
@@ -338,8 +326,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         it_sum += it;
         it_max = (unsigned long long)it > it_max ? it : it_max;
         nfail += (conv & 1) ? 0 : 1;
-        nfaces += ((conv >> 2) & 1) ? 0
-                                    : 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
+        nfaces += 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
       }
       if (a.update && active && j > j0) {
         const int64_t off = base + (j - 1) * stride;
@@ -352,7 +339,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       for (int k = 0; k < NC; ++k) Fprev[k] = F[k];
     }
   }
-  BlockReduceGodunov(smax, a.dx, it_sum, it_max, nfail, nfaces,
+  BlockReduceGodunov<kBlock / 64>(smax, a.dx, it_sum, it_max, nfail, nfaces,
                      a.partials + 5 * (blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x));
 }
 
@@ -521,251 +508,271 @@ __global__ __launch_bounds__(kBlock) void GodunovViewStableDt(DevView st, DevVie
   }
 }
 
-// Step-start CFL of all directions for the exact solver (one Newton per
-// face; faces as in the HLLEM pass: x through LDS, y recomputed in 3D,
-// march along the last dimension).  guess[d] (nullable) holds per-face
-// initial guesses in direction d's face box (n with n[d] + 1).
+// Step-start CFL of all directions for the exact solver: the largest signal
+// speed a direction, from the faces that can hold it.
+//
+// With a speed floor (floor[d] > 0, a lower bound of direction d's largest
+// speed) a face is solved only when its certified bounds (QuickSpeedBelow for
+// every face, SpeedBelow for those it leaves) reach the floor; blocks whose solved faces reach it set hit[d], which proves that
+// the skipped ones are slower than the maximum.  Without a floor every face is
+// solved, by the same instructions, so dt does not depend on the floor.
+//
+// 3D: a workgroup's eight waves are eight x rows of 64 cells marching along
+// z; lanes 1..62 own their cells and lane 0 and row 0 are halos.  2D: each
+// wave marches along y by itself.  A cell's six floats reach the x neighbour
+// by DPP, the y neighbour through LDS (3D), the marching neighbour in
+// registers; faces to be solved reload their cells.  Bound by instruction
+// issue (about 350 a cell) next to one read of the state.  The kernel it
+// replaces solved every face of the first sweep's direction, for that sweep's
+// reuse, and every face outside a narrow class; solving them in the sweep
+// alone costs less.  First-order step, 384^3 strong-wave blocks: 19.7 -> 11.0
+// ms, mixed learned form at 203 x 149 x 121: 1.72 -> 1.06 ms.
+constexpr int kCflRows = 8;
+constexpr int kCflOwnX = 62;
+constexpr int kCflBlocks = 4096;
+
 struct GodunovCflArgs {
   const double* in[5];
   int64_t n[3];
   double dx[3];
   double gamma, gm1inv, tol;
   int max_it;
-  const double* guess[3];
-  const short* tiles;  // learned guess computed inline (nullable)
-  const float* bias;
+  SpeedBound bound;
+  int64_t items;                 // tiles x segments
   unsigned long long* partials;  // 5 per workgroup and direction
   int* halt;
-  double* pm_out;  // star pressures of direction pm_dir's faces (nullable;
-  int pm_dir;      // NaN where Newton did not converge), for the first sweep
-  // Speed floor (nullable: none; the level driver's ctl->cfl_floor): faces of
-  // directions other than pm_dir whose certified speed bound stays below it
-  // skip the Newton solve; blocks whose evaluated faces reach it set hit[d].
-  const double* floor;
+  const double* floor;  // speed floor per direction (nullable: none)
   int* hit;
 };
 
-// kGodunovFloorCap: Newton iterations within which Newton from the mean
-// pressure converges on every face that GodunovSpeedBound certifies (at most
-// 6 were observed over millions of sampled pairs of that class); with a
-// smaller iteration cap the pass solves every face, so the cap is reported
-// where the reference's would be.
-
-// Certified upper bound of the exact solver's signal speeds max(|s0|, |s1|)
-// (GodunovSpeed) of a face, without Newton, for the faces of the
-// class on which Newton from the mean pressure converges quickly: positive
-// densities and pressures, pressure ratio at most 4, sound speeds at most
-// 1e6 and |uR - uL| at most the smaller sound speed (no vacuum).  Toro's f(p)
-// = fL(p) + fR(p) + (uR - uL) increases, so any P with f(P) >= 0 bounds the
-// star pressure p*: P = max(pL, pR) when uR >= uL (fK(max p) >= 0 on both
-// sides), else P = max(pL, pR) + 2 (uL - uR) / S with S the two shock
-// slopes sqrt(AK / (max p + BK)), checked on the shock branches.  Newton
-// stops at |f(pM)| <= tol, so pM <= P + tol / Dlo with Dlo the smaller of the
-// two branches' slopes on [0, 2P] summed over the sides (valid when that stays
-// below 2P).  The signal speeds grow with the star pressure, so |uK| + aK
-// w(P_eff / pK), w(r) = sqrt(1 + (g + 1) / (2 g) (r - 1)) for r > 1 and 1
-// otherwise, bounds them.  Returns false (no bound) outside the class.
-template <int D, int DIR>
-__device__ __forceinline__ bool GodunovSpeedBound(const double* L, const double* R,
-                                                  const Gas<double>& eq, double tol,
-                                                  double* bound) {
+// The face of direction d between the cells at off_l and off_r: its largest
+// signal speed, from Newton.
+template <int D>
+__device__ __forceinline__ double CflFace(const GodunovCflArgs& a, const Gas<double>& g, int d,
+                                          int64_t off_l, int64_t off_r,
+                                          unsigned long long* acc) {
   using I = Idx<D>;
-  const double rhoL = L[I::kRho], rhoR = R[I::kRho];
-  const double pL = L[I::kP], pR = R[I::kP], aL = L[I::kA], aR = R[I::kA];
-  const double uL = L[I::kMom + DIR] / rhoL, uR = R[I::kMom + DIR] / rhoR;
-  const double pmin = fmin(pL, pR), pmax = fmax(pL, pR);
-  const double amin = fmin(aL, aR), amax = fmax(aL, aR);
-  const double du = uR - uL;
-  if (!(rhoL > 0.0 && rhoR > 0.0 && pmin > 0.0 && pmax <= 4.0 * pmin && amax <= 1e6 &&
-        fabs(du) <= amin))
-    return false;  // NaN fails too
-  const double g = eq.gamma, gp1 = g + 1.0, gm1 = g - 1.0;
-  const double AL = 2.0 / (gp1 * rhoL), AR = 2.0 / (gp1 * rhoR);
-  const double BL = gm1 / gp1 * pL, BR = gm1 / gp1 * pR;
-  double P = pmax;
-  if (du < 0.0) {
-    const double S = sqrt(AL / (pmax + BL)) + sqrt(AR / (pmax + BR));
-    P = pmax + 2.0 * (-du) / S;
-    const double fP = (P - pL) * sqrt(AL / (P + BL)) + (P - pR) * sqrt(AR / (P + BR));
-    if (!(fP >= -du * (1.0 + 0x1p-30))) return false;
+  double L[D + 4], R[D + 4];
+#pragma unroll
+  for (int k = 0; k < D + 2; ++k) {
+    L[k] = a.in[k][off_l];
+    R[k] = a.in[k][off_r];
   }
-  const double Dlo = fmin(1.0 / (rhoL * aL), 0.5 * sqrt(AL / (2.0 * P + BL))) +
-                     fmin(1.0 / (rhoR * aR), 0.5 * sqrt(AR / (2.0 * P + BR)));
-  const double Peff = P + tol / Dlo;
-  if (!(Peff <= 2.0 * P)) return false;
-  const double c = gp1 / (2.0 * g);
-  const double wL = Peff > pL ? sqrt(1.0 + c * (Peff / pL - 1.0)) : 1.0;
-  const double wR = Peff > pR ? sqrt(1.0 + c * (Peff / pR - 1.0)) : 1.0;
-  *bound = fmax(fabs(uL) + aL * wL, fabs(uR) + aR * wR);
-  return true;
-}
-
-// Newton seed of a face: the inline learned guess (lg, computed by the whole
-// wave), else the face's guess array entry, else the mean pressure.
-template <int D, int DIR, bool LEARNED>
-__device__ __forceinline__ double CflFace(const double* L, const double* R,
-                                          const GodunovCflArgs& a, const Gas<double>& g,
-                                          int64_t fidx, double lg, unsigned long long* acc) {
+  CompleteFromCons<D>(L, g);
+  CompleteFromCons<D>(R, g);
+  const double mL = d == 0 ? L[1] : (D == 2 || d == 1) ? L[2] : L[D];
+  const double mR = d == 0 ? R[1] : (D == 2 || d == 1) ? R[2] : R[D];
+  const double uL = NearArith::quot(mL, L[0]), uR = NearArith::quot(mR, R[0]);
   NewtonParams np;
   np.tol = a.tol;
   np.max_it = a.max_it;
-  const double mean = 0.5 * (L[D + 2] + R[D + 2]);
-  const bool seeded = LEARNED || a.guess[DIR] != nullptr;
-  const double x0 = LEARNED ? lg : a.guess[DIR] ? a.guess[DIR][fidx] : mean;
-  int iters, fallback;
-  const MiddleState ms =
-      SeededMiddleState<D, DIR>(L, R, g, np, seeded, x0, mean, &iters, &fallback);
-  const unsigned long long it = static_cast<unsigned long long>(iters);
-  const unsigned long long fb = static_cast<unsigned long long>(fallback);
-  if (a.pm_out && DIR == a.pm_dir) a.pm_out[fidx] = ms.converged ? ms.pM : __builtin_nan("");
+  const MiddleState ms = SolveMiddleState(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP],
+                                          R[I::kA], g, np, 0.5 * (L[I::kP] + R[I::kP]));
+  const unsigned long long it = static_cast<unsigned long long>(ms.iterations);
   acc[0] += it;
   acc[1] = it > acc[1] ? it : acc[1];
   acc[2] += ms.converged ? 0 : 1;
-  acc[3] += 1 + (fb << 32);
-  return FaceSpeed<D, DIR>(L, R, ms);
+  double wL, wR;
+  return GodunovSpeed(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP], R[I::kA], ms, &wL, &wR);
 }
 
-template <int D, bool LEARNED>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovCflKernel(GodunovCflArgs a) {
-  constexpr int NC = D + 2, NQ = D + 4;
-  constexpr int M = D - 1;
+template <int D> __device__ __forceinline__ SpeedCell<D> ShiftUpCell(const SpeedCell<D>& c) {
+  SpeedCell<D> r;
+  r.ir = ShiftUp(c.ir);
+  r.p = ShiftUp(c.p);
+  r.a2 = ShiftUp(c.a2);
+#pragma unroll
+  for (int d = 0; d < D; ++d) r.u[d] = ShiftUp(c.u[d]);
+  return r;
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kCflRows) __attribute__((amdgpu_waves_per_eu(4))) void GodunovCflKernel(GodunovCflArgs a) {
+  constexpr int NC = D + 2;
+  constexpr int M = D - 1;  // marching direction
   if (a.halt && *a.halt) return;
   Gas<double> g;
   g.gamma = a.gamma;
   g.gm1inv = a.gm1inv;
   g.gm1 = a.gamma - 1.0;
   const int64_t nx = a.n[0], ny = a.n[1];
-  const int64_t tiles = (nx + kTX - 1) / kTX;
-  const int64_t x0 = (blockIdx.x % tiles) * kTX;
-  const int64_t y = (D == 3) ? static_cast<int64_t>(blockIdx.x / tiles) : 0;
-  const int tx = threadIdx.x;
-  const int64_t x = x0 + tx;
-  const bool active = x < nx;
-  const int64_t xs = active ? x : nx - 1;
-  const int64_t nm = (D == 3) ? a.n[2] : ny;
+  const int64_t nm = a.n[M];
   const int64_t ms = (D == 3) ? nx * ny : nx;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kCflSeg;
-  const int64_t m1 = (m0 + kCflSeg < nm) ? m0 + kCflSeg : nm;
-  const int64_t rowoff = (D == 3) ? y * nx : 0;
-  // Speed floor of the directions other than pm_dir (0: every face solved).
-  double F[3] = {0.0, 0.0, 0.0};
+  const int lane = threadIdx.x & 63;
+  const int row = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  float F[3] = {0.0f, 0.0f, 0.0f};
   if (a.floor) {
-    for (int d = 0; d < D; ++d) {
-      if (d != a.pm_dir && a.floor[d] > 0.0) F[d] = a.floor[d];
-    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) F[d] = static_cast<float>(a.floor[d] * (1.0 - 0x1p-20));
   }
-  // A face skips its Newton solve when its certified speed bound stays below
-  // the floor by a relative 2^-30 (far above the rounding of either side).
-  auto skipped = [&](auto dir_tag, const double* l, const double* r) -> bool {
-    constexpr int DD = decltype(dir_tag)::value;
-    if (!(F[DD] > 0.0)) return false;
-    double sb;
-    return GodunovSpeedBound<D, DD>(l, r, g, a.tol, &sb) && sb * (1.0 + 0x1p-30) < F[DD];
-  };
-  __shared__ double s_q[NQ][kTX];
+  __shared__ SpeedCell<D> s_c[D == 3 ? 2 * kCflRows * 64 : 1];
+  const int64_t tiles_x = (nx + kCflOwnX - 1) / kCflOwnX;
+  const int64_t tiles_y = (D == 3) ? (ny + kCflRows - 2) / (kCflRows - 1) : 1;
   double smax[3] = {0.0, 0.0, 0.0};
-  unsigned long long acc[3][4] = {};
-  auto load = [&](int64_t off, double* q) {
-#pragma unroll
-    for (int k = 0; k < NC; ++k) q[k] = a.in[k][off];
-    CompleteFromCons<D>(q, g);
+  unsigned long long acc[3] = {0, 0, 0};  // iterations, largest, not converged
+  unsigned faces[3] = {0, 0, 0};
+  // Faces to solve wait in a list of the wave's until 64 of them fill it: the
+  // few of a step (0.3% of the faces of strong-wave blocks) would each cost the
+  // whole wave a Newton solve.  An entry is a cell and the face of it: d its
+  // lower face of direction d, 4 + d a face that joins it with its own copy.
+  // A step adds at most six entries a lane.
+  __shared__ int64_t s_list[kCflRows][64 + 6 * 64];
+  int64_t* list = s_list[row];
+  int count = 0;  // wave-uniform
+  auto solve = [&]() {
+    const int n = count < 64 ? count : 64;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < n) {
+      const int64_t entry = list[count - n + lane];
+      const int d = static_cast<int>(entry & 3);
+      const int64_t off = entry >> 3;
+      const int64_t back = d == 0 ? 1 : d == M ? ms : nx;
+      const double v = CflFace<D>(a, g, d, (entry & 4) ? off : off - back, off, acc);
+      faces[0] += d == 0;
+      faces[1] += d == 1;
+      faces[2] += d == 2;
+      if (d == 0) smax[0] = __builtin_fmax(smax[0], v);
+      if (d == 1) smax[1] = __builtin_fmax(smax[1], v);
+      if (d == 2) smax[2] = __builtin_fmax(smax[2], v);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    count -= n;
   };
-  // Index in direction d's face box of the face at cell coordinates (cx, cy, cz).
-  auto fidx = [&](int d, int64_t cx, int64_t cy, int64_t cz) -> int64_t {
-    const int64_t fx = nx + (d == 0), fy = ny + (d == 1);
-    return cx + fx * (cy + fy * cz);
-  };
-  // Waves with an active lane run the inline learned guess with all lanes.
-  const bool wave_live = __ballot(active) != 0;
-  auto learned = [&](auto dir_tag, const double* l, const double* r) -> double {
-    constexpr int DD = decltype(dir_tag)::value;
-    if constexpr (LEARNED) {
-      if (wave_live) return mlp::LearnedGuess<D, DD>(l, r, a.tiles, a.bias);
-    }
-    return 0.0;
-  };
-  using X0 = std::integral_constant<int, 0>;
-  using X1 = std::integral_constant<int, 1>;
-  using XM = std::integral_constant<int, M>;
-  double qprev[NQ];
-  load(xs + rowoff + Clamp(m0 - 1, nm) * ms, qprev);
-  for (int64_t m = m0; m < m1; ++m) {
-    const int64_t off = xs + rowoff + m * ms;
-    const int64_t cy = (D == 3) ? y : m, cz = (D == 3) ? m : 0;
-    double qc[NQ];
-    load(off, qc);
-    // March direction.
-    {
-      const double* l = (m == 0) ? qc : qprev;
-      const bool skip = active && skipped(XM{}, l, qc);
-      const double lg = __all(skip || !active) ? 0.0 : learned(XM{}, l, qc);
-      if (active && !skip) {
-        const double sp = CflFace<D, M, LEARNED>(
-            l, qc, a, g, (M == 1) ? fidx(1, xs, m, 0) : fidx(2, xs, cy, m), lg, acc[M]);
-        smax[M] = __builtin_fmax(smax[M], sp);
-      }
-      if (active && m == nm - 1 && !skipped(XM{}, qc, qc)) {
-        const double sp = CflFace<D, M, LEARNED>(
-            qc, qc, a, g, (M == 1) ? fidx(1, xs, m + 1, 0) : fidx(2, xs, cy, m + 1),
-            0.5 * (qc[D + 2] + qc[D + 2]), acc[M]);
-        smax[M] = __builtin_fmax(smax[M], sp);
-      }
-    }
-    if constexpr (D == 3) {
-      double qy[NQ];
-      if (y == 0) {
-        for (int k = 0; k < NQ; ++k) qy[k] = qc[k];
-      } else {
-        load(off - nx, qy);
-      }
-      const bool skip = active && skipped(X1{}, qy, qc);
-      const double lg = __all(skip || !active) ? 0.0 : learned(X1{}, qy, qc);
-      if (active && !skip) {
-        const double sp = CflFace<D, 1, LEARNED>(qy, qc, a, g, fidx(1, xs, y, cz), lg, acc[1]);
-        smax[1] = __builtin_fmax(smax[1], sp);
-      }
-      if (active && y == ny - 1 && !skipped(X1{}, qc, qc)) {
-        const double sp = CflFace<D, 1, LEARNED>(qc, qc, a, g, fidx(1, xs, y + 1, cz),
-                                                        0.5 * (qc[D + 2] + qc[D + 2]), acc[1]);
-        smax[1] = __builtin_fmax(smax[1], sp);
-      }
-    }
+  // 3D: a block per item; 2D: a wave per item (uniform loops either way)
+  const int64_t first = D == 3 ? blockIdx.x : static_cast<int64_t>(blockIdx.x) * kCflRows + row;
+  const int64_t step = D == 3 ? gridDim.x : static_cast<int64_t>(gridDim.x) * kCflRows;
+  int buf = 0;
+  for (int64_t item = first; item < a.items; item += step) {
+    const int64_t tx = item % tiles_x, ty = (item / tiles_x) % tiles_y;
+    const int64_t seg = item / (tiles_x * tiles_y);
+    const int64_t x = tx * kCflOwnX + lane - 1;
+    const int64_t y = (D == 3) ? ty * (kCflRows - 1) + row - 1 : 0;
+    const bool own = lane >= 1 && lane <= kCflOwnX && x < nx && (D == 2 || (row >= 1 && y < ny));
+    const int64_t xs = Clamp(x, nx), ys = (D == 3) ? Clamp(y, ny) : 0;
+    const int64_t col = xs + (D == 3 ? ys * nx : 0);
+    const int64_t m0 = seg * kCflSeg;
+    const int64_t m1 = (m0 + kCflSeg < nm) ? m0 + kCflSeg : nm;
+    auto load = [&](double* u, int64_t m) {
+      const int64_t off = col + Clamp(m, nm) * ms;
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) s_q[k][tx] = qc[k];
-    __syncthreads();
-    {
-      double ql[NQ];
-      if (x == 0) {
-        for (int k = 0; k < NQ; ++k) ql[k] = qc[k];
-      } else if (tx > 0) {
-        for (int k = 0; k < NQ; ++k) ql[k] = s_q[k][tx - 1];
-      } else {
-        load(off - 1, ql);
+      for (int k = 0; k < NC; ++k) u[k] = a.in[k][off];
+    };
+    double ucur[NC], unext[NC];
+    load(ucur, m0 - 1);
+    SpeedCell<D> cprev = MakeSpeedCell<D>(ucur, g);
+    load(ucur, m0);
+    for (int64_t m = m0; m < m1; ++m) {
+      if (m + 1 < m1) load(unext, m + 1);
+      const SpeedCell<D> c = MakeSpeedCell<D>(ucur, g);
+      const SpeedCell<D> cl = ShiftUpCell<D>(c);
+      // Faces to solve: bit d the cell's lower face of direction d, bit 4 + d
+      // the patch's upper face, which joins a cell with its own copy.
+      unsigned todo = 0;
+      if constexpr (D == 3) {
+        s_c[(buf * kCflRows + row) * 64 + lane] = c;
+        __syncthreads();
       }
-      const bool skip = active && skipped(X0{}, ql, qc);
-      const double lg = __all(skip || !active) ? 0.0 : learned(X0{}, ql, qc);
-      if (active && !skip) {
-        const double sp = CflFace<D, 0, LEARNED>(ql, qc, a, g, fidx(0, xs, cy, cz), lg, acc[0]);
-        smax[0] = __builtin_fmax(smax[0], sp);
+      // Every face takes the quick test; a wave with a face that does not pass
+      // it (strong waves) takes the tight one.
+      auto below = [&](const SpeedCell<D>& l, float ul, float ur, float f) {
+        bool pass = !own || QuickSpeedBelow<D>(l, ul, c, ur, a.bound, f);
+        if (__any(!pass)) pass = !own || SpeedBelow<D>(l, ul, c, ur, a.bound, f);
+        return pass;
+      };
+      if (!below(cl, cl.u[0], c.u[0], F[0])) todo |= 1u;
+      if constexpr (D == 3) {
+        const SpeedCell<D> cb = s_c[(buf * kCflRows + (row > 0 ? row - 1 : 0)) * 64 + lane];
+        if (!below(cb, cb.u[1], c.u[1], F[1])) todo |= 2u;
+        if (own && y == ny - 1 && !QuickSpeedBelow<D>(c, c.u[1], c, c.u[1], a.bound, F[1]))
+          todo |= 32u;
       }
-      if (active && x == nx - 1 && !skipped(X0{}, qc, qc)) {
-        const double sp = CflFace<D, 0, LEARNED>(qc, qc, a, g, fidx(0, xs + 1, cy, cz),
-                                                        0.5 * (qc[D + 2] + qc[D + 2]), acc[0]);
-        smax[0] = __builtin_fmax(smax[0], sp);
+      if (!below(cprev, cprev.u[M], c.u[M], F[M])) todo |= 1u << M;
+      if (own) {
+        if (x == nx - 1 && !QuickSpeedBelow<D>(c, c.u[0], c, c.u[0], a.bound, F[0])) todo |= 16u;
+        if (m == nm - 1 && !QuickSpeedBelow<D>(c, c.u[M], c, c.u[M], a.bound, F[M]))
+          todo |= 16u << M;
       }
-    }
-    __syncthreads();
+      buf ^= 1;
+      if (__builtin_expect(__any(todo != 0), 0)) {
+        const int64_t off = col + m * ms;
+        // the patch's lower faces join a cell with its own copy, too
+        const unsigned edge = (x <= 0 ? 1u : 0u) | (D == 3 && y <= 0 ? 2u : 0u) |
+                              (m == 0 ? 1u << M : 0u);
+        todo = (todo & ~edge) | ((todo & edge) << 4);
+        for (int f = 0; f < 7; ++f) {
+          const bool mine = (todo >> f) & 1u;
+          const unsigned long long who = __ballot(mine);
+          if (mine)
+            list[count + __builtin_popcountll(who & ((1ull << lane) - 1ull))] = (off << 3) | f;
+          count += static_cast<int>(__builtin_popcountll(who));
+        }
+        while (count >= 64) solve();
+      }
+      cprev = c;
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) qprev[k] = qc[k];
+      for (int k = 0; k < NC; ++k) ucur[k] = unext[k];
+    }
   }
-  const int64_t nblocks = static_cast<int64_t>(gridDim.x) * gridDim.y;
-  const int64_t bid = blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x;
-  for (int d = 0; d < D; ++d)
-    BlockReduceGodunov(smax[d], a.dx[d], acc[d][0], acc[d][1], acc[d][2], acc[d][3],
-                       a.partials + 5 * (d * nblocks + bid));
+  while (count > 0) solve();
+  // The iteration counters of all directions go with direction 0's partials.
+  const int64_t nblocks = gridDim.x;
+#pragma unroll
   for (int d = 0; d < D; ++d) {
-    const bool hit = F[d] > 0.0 && smax[d] >= F[d];
+    const bool first_dir = d == 0;
+    BlockReduceGodunov<kCflRows>(smax[d], a.dx[d], first_dir ? acc[0] : 0, first_dir ? acc[1] : 0,
+                                 first_dir ? acc[2] : 0, faces[d],
+                                 a.partials + 5 * (d * nblocks + blockIdx.x));
+    const bool hit = a.floor && a.floor[d] > 0.0 && smax[d] >= a.floor[d];
     if (__syncthreads_or(hit ? 1 : 0) && threadIdx.x == 0 && a.hit) a.hit[d] = 1;
+  }
+}
+
+// Speed floor of a state the level knows nothing about yet (its first step):
+// the largest |u| + a of the cells, a lower bound of the largest signal speed
+// of direction d because each cell is the right state of one face and the left
+// state of the next (uR + aR or more where u >= 0, |uL| + aL or more where u <
+// 0).  Reads the state once; without it the first pass solves every face
+// (three Newton solves a cell).  cfl_floor[d] grows by an atomic maximum (non-
+// negative doubles order like their bits), on top of a caller's hint.
+template <int D>
+__global__ __launch_bounds__(kBlock) void GodunovFloorKernel(GodunovCflArgs a, int64_t ncell,
+                                                             Ctl* ctl) {
+  if (ctl->halt || ctl->floor_known) return;
+  Gas<double> g;
+  g.gamma = a.gamma;
+  g.gm1inv = a.gm1inv;
+  g.gm1 = a.gamma - 1.0;
+  double s[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) s[d] = 0.0;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kBlock;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < ncell; i += step) {
+    double q[D + 4];
+#pragma unroll
+    for (int k = 0; k < D + 2; ++k) q[k] = a.in[k][i];
+    const double y = NearArith::inv(q[0]);
+    const double p = (q[D + 1] - 0.5 * SqNormArray<D>(q + 1) * y) * g.gm1;
+    if (q[0] > 0.0 && p > 0.0) {
+      const double c = NearArith::sqrt(g.gamma * p * y);
+#pragma unroll
+      for (int d = 0; d < D; ++d) s[d] = __builtin_fmax(s[d], rabs(q[1 + d] * y) + c);
+    }
+  }
+  __shared__ double sh[D][kBlock / 64];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s[d] = __builtin_fmax(s[d], __shfl_xor(s[d], off, 64));
+    if ((threadIdx.x & 63) == 0) sh[d][threadIdx.x >> 6] = s[d];
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    double v = sh[threadIdx.x][0];
+    for (int w = 1; w < kBlock / 64; ++w) v = __builtin_fmax(v, sh[threadIdx.x][w]);
+    v *= 1.0 - 0x1p-20;
+    if (v > 0.0 && v < 1.7976931348623157e308)
+      atomicMax(reinterpret_cast<unsigned long long*>(&ctl->cfl_floor[threadIdx.x]),
+                static_cast<unsigned long long>(__double_as_longlong(v)));
   }
 }
 
@@ -831,18 +838,24 @@ int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3], int seg) {
   return ((npencil + kBlock - 1) / kBlock) * ((n[dir] + seg - 1) / seg);
 }
 
-int64_t GodunovCflBlocks(int dim, const int64_t n[3]) {
-  const int64_t tiles = (n[0] + kTX - 1) / kTX;
-  const int64_t rows = dim == 3 ? n[1] : 1;
+static int64_t GodunovCflItems(int dim, const int64_t n[3]) {
+  const int64_t tx = (n[0] + kCflOwnX - 1) / kCflOwnX;
+  const int64_t ty = dim == 3 ? (n[1] + kCflRows - 2) / (kCflRows - 1) : 1;
   const int64_t nm = dim == 3 ? n[2] : n[1];
-  return tiles * rows * ((nm + kCflSeg - 1) / kCflSeg);
+  return tx * ty * ((nm + kCflSeg - 1) / kCflSeg);
+}
+
+int64_t GodunovCflBlocks(int dim, const int64_t n[3]) {
+  const int64_t items = GodunovCflItems(dim, n);
+  const int64_t blocks = dim == 3 ? items : (items + kCflRows - 1) / kCflRows;
+  return blocks < kCflBlocks ? blocks : kCflBlocks;
 }
 
 int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
                        const double* const* in, double* const* out, const int64_t n[3],
                        double dx, const double* dt_ptr, double dt_val, const double* guess,
                        unsigned long long* partials, int* halt, int update,
-                       const fvs_mlp* net, int reuse) {
+                       const fvs_mlp* net) {
   GodunovArgs a;
   std::memset(&a, 0, sizeof a);
   const int D = desc.dim;
@@ -864,7 +877,6 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
   a.halt = halt;
   a.seg = PencilSeg(D, dir, a.n);
   a.update = update;
-  a.reuse = reuse && guess != nullptr;
   const bool mixed = desc.precision == FVS_FP32_FLUX;
   const bool learned = a.tiles != nullptr;
   const int64_t blocks = GodunovSweepBlocks(D, dir, a.n, a.seg);
@@ -910,41 +922,43 @@ int LaunchGodunovFinalize(hipStream_t s, const unsigned long long* partials, int
 }
 
 int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* const* cons,
-                     const int64_t n[3], const double dx[3], const double* const* guess,
-                     unsigned long long* partials, int* halt, const fvs_mlp* net,
-                     double* pm_out, int pm_dir, Ctl* floor_ctl) {
+                     const int64_t n[3], const double dx[3], unsigned long long* partials,
+                     int* halt, Ctl* floor_ctl) {
   GodunovCflArgs a;
   std::memset(&a, 0, sizeof a);
   const int D = desc.dim;
   for (int c = 0; c < D + 2; ++c) a.in[c] = cons[c];
+  int64_t ncell = 1;
   for (int d = 0; d < 3; ++d) {
     a.n[d] = (d < D) ? n[d] : 1;
     a.dx[d] = (d < D) ? dx[d] : 1.0;
-    a.guess[d] = (guess && d < D) ? guess[d] : nullptr;
+    ncell *= a.n[d];
   }
   a.gamma = desc.gamma;
   a.gm1inv = 1.0 / (desc.gamma - 1.0);
   a.tol = desc.newton_tolerance;
   a.max_it = desc.max_newton_iterations;
-  if (net) MlpOperands(net, &a.tiles, &a.bias);
+  a.bound = MakeSpeedBound(desc.gamma, desc.newton_tolerance, desc.max_newton_iterations);
+  a.items = GodunovCflItems(D, a.n);
   a.partials = partials;
   a.halt = halt;
-  a.pm_out = pm_out;
-  a.pm_dir = pm_dir;
+  const dim3 grid(static_cast<unsigned>(GodunovCflBlocks(D, a.n)));
+  const dim3 block(64 * kCflRows);
   if (floor_ctl && desc.max_newton_iterations >= kGodunovFloorCap) {
     a.floor = floor_ctl->cfl_floor;
     a.hit = floor_ctl->floor_hit;
+    const int64_t fb = (ncell + kBlock - 1) / kBlock;
+    const dim3 fgrid(static_cast<unsigned>(fb < 2048 ? fb : 2048));
+    if (D == 3)
+      hipLaunchKernelGGL(GodunovFloorKernel<3>, fgrid, dim3(kBlock), 0, s, a, ncell, floor_ctl);
+    else
+      hipLaunchKernelGGL(GodunovFloorKernel<2>, fgrid, dim3(kBlock), 0, s, a, ncell, floor_ctl);
+    FVS_LAUNCH_CHECK();
   }
-  const int64_t tiles = (a.n[0] + kTX - 1) / kTX;
-  const int64_t gx = tiles * (D == 3 ? a.n[1] : 1);
-  const int64_t gy = ((D == 3 ? a.n[2] : a.n[1]) + kCflSeg - 1) / kCflSeg;
-  if (gx > 0x7fffffff || gy > 65535) return FVS_BAD_ARGUMENT;
-  using K = void (*)(GodunovCflArgs);
-  const K ks[2][2] = {{GodunovCflKernel<2, false>, GodunovCflKernel<2, true>},
-                      {GodunovCflKernel<3, false>, GodunovCflKernel<3, true>}};
-  const bool learned = a.tiles != nullptr;
-  hipLaunchKernelGGL(ks[D == 3][learned], dim3(unsigned(gx), unsigned(gy)), dim3(kBlock),
-                     0, s, a);
+  if (D == 3)
+    hipLaunchKernelGGL(GodunovCflKernel<3>, grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL(GodunovCflKernel<2>, grid, block, 0, s, a);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }

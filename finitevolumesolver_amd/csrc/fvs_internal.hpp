@@ -111,6 +111,11 @@ struct Ctl {
   // proves that the skipped faces are below the maximum.
   double cfl_floor[3];
   int floor_hit[3];
+  int floor_known;        // exact Godunov: 0 the next pass takes its floor from
+                          // the cells (no pass yet, or the last pass's floor
+                          // was not reached), 1 from the last pass, 2 none (a
+                          // floor from the cells, or a caller's, was not
+                          // reached: every face is solved)
   double floor_margin;    // relative margin of the last floor (0: none yet)
   double floor_speed[3];  // largest speeds of the last pass (0: none yet)
   double* dt_log;       // optional log of the steps' dt (set per advance call)
@@ -164,20 +169,15 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
                        const double* const* in, double* const* out, const int64_t n[3],
                        double dx, const double* dt_ptr, double dt_val, const double* guess,
                        unsigned long long* partials, int* halt, int update,
-                       const fvs_mlp* net = nullptr, int reuse = 0);
+                       const fvs_mlp* net = nullptr);
 int LaunchGodunovFinalize(hipStream_t s, const unsigned long long* partials, int64_t nblocks,
                           double* out, unsigned long long* stats, Ctl* ctl = nullptr);
-// Newton iteration cap from which the exact-Godunov CFL pass uses the speed
-// floor (below it every face is solved, so a small cap is reported as the
-// reference's would be).
-constexpr int kGodunovFloorCap = 16;
-// With floor_ctl (the level driver) and an iteration cap of at least 16, the
-// faces of directions other than pm_dir that a certified speed bound keeps
-// below ctl->cfl_floor skip their Newton solve.
+// With floor_ctl (the level driver) and an iteration cap of at least
+// kGodunovFloorCap, the faces that a certified speed bound keeps below
+// ctl->cfl_floor skip their Newton solve.
 int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* const* cons,
-                     const int64_t n[3], const double dx[3], const double* const* guess,
-                     unsigned long long* partials, int* halt, const fvs_mlp* net = nullptr,
-                     double* pm_out = nullptr, int pm_dir = -1, Ctl* floor_ctl = nullptr);
+                     const int64_t n[3], const double dx[3], unsigned long long* partials,
+                     int* halt, Ctl* floor_ctl = nullptr);
 int LaunchGodunovViewFlux(const fvs_method_desc& desc, hipStream_t s, const fvs_view* fluxes,
                           const fvs_view* states, double dt, double dx, int dir,
                           unsigned long long* nfail);

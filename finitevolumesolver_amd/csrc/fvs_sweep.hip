@@ -856,22 +856,23 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
 // reached may have hidden the fastest face, so the step is repeated without
 // a floor (halt 3) and the margin quadruples; otherwise the next floor is
 // this pass's largest speed per direction (dx / dt) less a margin that
-// follows how fast that speed falls.  Directions equal to solved_dir had
-// every face evaluated.  Returns false after setting halt 3.
-__device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, int dim,
-                                int solved_dir) {
+// follows how fast that speed falls.  Returns false after setting halt 3.
+__device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, int dim) {
   bool floor_ok = true;
   for (int d = 0; d < 3; ++d) {
-    if (d != solved_dir && ctl->cfl_floor[d] > 0.0 && !ctl->floor_hit[d]) floor_ok = false;
+    if (ctl->cfl_floor[d] > 0.0 && !ctl->floor_hit[d]) floor_ok = false;
     ctl->floor_hit[d] = 0;
   }
   const double old_margin = ctl->floor_margin > 0.0 ? ctl->floor_margin : kFloorMarginFirst;
   if (!floor_ok) {
     for (int d = 0; d < 3; ++d) ctl->cfl_floor[d] = 0.0;
     ctl->floor_margin = fmin(4.0 * old_margin, kFloorMarginMax);
+    // the last pass's floor: the next one comes from the cells; that too: none
+    ctl->floor_known = ctl->floor_known == 1 ? 0 : 2;
     ctl->halt = 3;
     return false;
   }
+  ctl->floor_known = 1;
   double speed[3] = {0.0, 0.0, 0.0}, drop = 0.0;
   for (int d = 0; d < dim; ++d) {
     speed[d] = fdx[d] / v[d];
@@ -911,7 +912,7 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCflKernel(
   if (!ctl) return;
   if (use_floor) {
     const double fdx[3] = {fdx0, fdx1, fdx2};
-    if (!RenewSpeedFloor(ctl, v, fdx, dim, -1)) return;
+    if (!RenewSpeedFloor(ctl, v, fdx, dim)) return;
   }
   // DimensionalSplitLevelIntegrator::ComputeStableDt (:204-219) starts from
   // DBL_MAX; RunSimulation's limited_dt (RunSimulation.hpp:121-131).
@@ -947,7 +948,7 @@ __global__ void StepDtKernel(Ctl* ctl, int dim, int first_dir, int strang, doubl
   if (ctl->halt) return;
   if (use_floor) {
     const double fdx[3] = {fdx0, fdx1, fdx2};
-    if (!RenewSpeedFloor(ctl, ctl->dt_dir, fdx, dim, first_dir)) return;
+    if (!RenewSpeedFloor(ctl, ctl->dt_dir, fdx, dim)) return;
   }
   double stable = 1.7976931348623157e308;
   for (int d = 0; d < dim; ++d) stable = (ctl->dt_dir[d] < stable) ? ctl->dt_dir[d] : stable;

@@ -717,12 +717,7 @@ static int PatchStableDt(fvs_handle* h, const double* const* cons, const int64_t
   if (godunov) {
     if (int rc = LaunchGodunovCfl(h->desc, h->stream, cons, nn, dx, partials, nullptr))
       return rc;
-    for (int d = 0; d < D; ++d) {
-      if (int rc = LaunchGodunovFinalize(h->stream, partials + 5 * d * nb, nb,
-                                         dt_dir_device + d, h->newton_stats))
-        return rc;
-    }
-    return FVS_OK;
+    return LaunchGodunovFinalize(h->stream, partials, nb, D, dt_dir_device, h->newton_stats);
   }
   return LaunchPatchCfl(h->desc, h->stream, cons, nn, dx, partials, dt_dir_device, nullptr,
                         nullptr, 0, 0);
@@ -840,12 +835,12 @@ int fvs_godunov_sweep(fvs_handle* h, const double* const* cons_in, double* const
       return FVS_BAD_ARGUMENT;
     }
   }
-  const int64_t nb = GodunovSweepBlocks(D, dir, nn, PencilSeg(D, dir, nn));
+  const int64_t nb = GodunovSweepBlocks(D, dir, nn);
   if (int rc = EnsurePartials(h, 5 * nb)) return rc;
   if (int rc = LaunchGodunovSweep(h->desc, h->stream, dir, cons_in, cons_out, nn, dx, nullptr, dt,
                                   guess_device, h->partials, nullptr, cons_out != nullptr))
     return rc;
-  return LaunchGodunovFinalize(h->stream, h->partials, nb, stable_dt_device, h->newton_stats);
+  return LaunchGodunovFinalize(h->stream, h->partials, nb, 1, stable_dt_device, h->newton_stats);
 }
 
 int fvs_exact_middle_state(fvs_handle* h, int dir, const double* left, const double* right,
@@ -1012,8 +1007,8 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch, fvs_level** out
   L->h = h;
   L->patch = *patch;
   if (ComposedLevelNeeded(h->desc)) {
-    // MUSCL-Hancock over exact Godunov, HLL, MusclHancockPrim and
-    // MusclHancockCharacteristic: the level composed from the patch operators
+    // HLL, MusclHancockPrim and MusclHancockCharacteristic: the level
+    // composed from the patch operators
     for (int d = 0; d < 3; ++d) L->n[d] = n[d];
     L->ncell = n[0] * n[1] * n[2];
     if (int rc = ComposedCreate(h, patch, &L->composed)) {
@@ -1049,7 +1044,7 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch, fvs_level** out
   np = std::max<int64_t>(np, (2 * D - 1) * sweep_blocks);
   if (godunov) {
     np = std::max<int64_t>(np, 5 * D * GodunovCflBlocks(D, n));
-    for (int d = 0; d < D; ++d) np = std::max<int64_t>(np, 5 * GodunovSweepBlocks(D, d, n, PencilSeg(D, d, n)));
+    for (int d = 0; d < D; ++d) np = std::max<int64_t>(np, 5 * GodunovSweepBlocks(D, d, n));
   }
   if (hipMalloc(&L->partials, np * sizeof(unsigned long long)) != hipSuccess) {
     (void)hipFree(L->block);
@@ -1132,6 +1127,10 @@ double* fvs_level_state(fvs_level* L, int c) {
   if (!L || c < 0 || c >= L->h->desc.dim + 2) return nullptr;
   if (L->composed) {
     SetError("a composed level keeps its state inside a ghosted scratch (fvs_level_get_state)");
+    return nullptr;
+  }
+  if (L->h->desc.base == FVS_BASE_GODUNOV_EXACT && L->h->desc.reconstruction != FVS_RECON_NONE) {
+    SetError("no state pointer for MUSCL-Hancock over exact Godunov (fvs_level_get_state)");
     return nullptr;
   }
   return L->buf[L->cur][c];
@@ -1260,10 +1259,8 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
       return LaunchGodunovCfl(h->desc, s, cin, L->n, L->patch.dx, L->partials, &L->ctl->halt,
                               L->ctl);
     });
-    for (int d = 0; d < D && rc == FVS_OK; ++d) {
-      rc = LaunchGodunovFinalize(s, L->partials + 5 * d * nb, nb, &L->ctl->dt_dir[d],
-                                 h->newton_stats, L->ctl);
-    }
+    if (rc == FVS_OK)
+      rc = LaunchGodunovFinalize(s, L->partials, nb, D, L->ctl->dt_dir, h->newton_stats, L->ctl);
     const int use_floor = h->desc.max_newton_iterations >= kGodunovFloorCap;
     if (rc == FVS_OK) rc = LaunchStepDt(s, L->ctl, D, seq[0], strang, L->patch.dx, use_floor);
   } else {
@@ -1286,16 +1283,16 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
     const double* inp[5];
     for (int q = 0; q < D + 2; ++q) inp[q] = L->buf[src][q];
     if (godunov) {
-      const int64_t nb = GodunovSweepBlocks(D, seq[w], L->n, PencilSeg(D, seq[w], L->n));
+      const int64_t nb = GodunovSweepBlocks(D, seq[w], L->n);
       rc = Timed(L, s, FVS_TIMER_SWEEP_X + seq[w], [&] {
         return LaunchGodunovSweep(h->desc, s, seq[w], inp, outp, L->n, L->patch.dx[seq[w]],
                                   &L->ctl->split_dt, 0.0, nullptr, L->partials, &L->ctl->halt, 1,
-                                  net);
+                                  net, w > 0);
       });
+      // The first sweep's check is the step-start value of its direction.
       if (rc == FVS_OK)
-        rc = LaunchGodunovFinalize(s, L->partials, nb, &L->ctl->last_check, h->newton_stats,
-                                   L->ctl);
-      if (rc == FVS_OK && w > 0) rc = LaunchCheckValue(s, L->ctl, &L->ctl->last_check);
+        rc = LaunchGodunovFinalize(s, L->partials, nb, 1, w > 0 ? &L->ctl->last_check : nullptr,
+                                   h->newton_stats, L->ctl, w > 0);
       if (rc) break;
       src = dst;
       dst = (dst == b1) ? b2 : b1;

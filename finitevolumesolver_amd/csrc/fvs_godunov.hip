@@ -15,6 +15,7 @@
 #include "fvs_mlp_infer.hpp"
 #include "fvs_riemann.hpp"
 #include "fvs_views.hpp"
+#include "fvs_xslots.hpp"
 
 #include <cstring>
 #include <type_traits>
@@ -24,7 +25,6 @@ namespace fvs {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kXOwned = 62;
 constexpr int kTX = 256;
 constexpr int kCflSeg = 32;
 constexpr unsigned long long kInfKey = 0x7ff0000000000000ull;
@@ -115,6 +115,9 @@ struct GodunovArgs {
   int* halt;
   int seg;
   int update;            // 0: only fluxes' Newton + CFL (no state write)
+  int limiter;           // MUSCL-Hancock sweeps
+  int check;             // MUSCL-Hancock: the cells' CFL check against dt
+  SpeedBound bound;
 };
 
 __device__ __forceinline__ Gas<double> GasOf(const GodunovArgs& a) {
@@ -125,11 +128,11 @@ __device__ __forceinline__ Gas<double> GasOf(const GodunovArgs& a) {
   return g;
 }
 
-template <int D>
-__device__ __forceinline__ void ShflUpState(const double* q, double* r) {
-#pragma unroll
-  for (int k = 0; k < D + 4; ++k) r[k] = __shfl_up(q[k], 1, 64);
-}
+// A complete state in registers with the refined reciprocal of its density.
+template <int D> struct CellState {
+  double q[D + 4];
+  double y;
+};
 
 // Newton from a caller's seed (learned or given), with the reference's
 // initial guess, the mean pressure, as the fallback.  A seed that is not a
@@ -137,19 +140,24 @@ __device__ __forceinline__ void ShflUpState(const double* q, double* r) {
 // not tried; a run from the seed that does not converge, or ends on a
 // pressure that is not finite and non-negative, is redone from the mean.
 // Both count as a fallback.
-template <int D, int DIR>
-__device__ __forceinline__ MiddleState SeededMiddleState(const double* L, const double* R,
+template <int D>
+__device__ __forceinline__ MiddleState SeededMiddleState(const CellState<D>& L, double uL,
+                                                         const CellState<D>& R, double uR,
                                                          const Gas<double>& g,
                                                          const NewtonParams& np, bool seeded,
                                                          double seed, double mean, int* iters,
                                                          int* fallback) {
+  using I = Idx<D>;
   const bool usable = seeded && seed > 0.0 && seed <= 1.7976931348623157e308;
-  MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, usable ? seed : mean);
-  int it = ms.iterations;
-  int fb = seeded && !usable;
-  if (usable && !(ms.converged && ms.pM >= 0.0 && ms.pM <= 1.7976931348623157e308)) {
-    ms = ComputeMiddleState<D, DIR>(L, R, g, np, mean);
+  double x0 = usable ? seed : mean;
+  int it = 0, fb = seeded && !usable;
+  MiddleState ms;
+  while (true) {  // one Newton site for the seed and the mean
+    ms = SolveMiddleState(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA],
+                          g, np, x0);
     it += ms.iterations;
+    if (!usable || fb || (ms.converged && ms.pM >= 0.0 && ms.pM <= 1.7976931348623157e308)) break;
+    x0 = mean;
     fb = 1;
   }
   *iters = it;
@@ -157,129 +165,297 @@ __device__ __forceinline__ MiddleState SeededMiddleState(const double* L, const 
   return ms;
 }
 
-// Largest signal speed of a face from its middle state.
+// Largest signal speed of the face between complete states L and R (normal
+// momenta mL, mR), from Newton; acc (nullable): iterations, their maximum,
+// solves that hit the cap.
+template <int D>
+__device__ __forceinline__ double CellFaceSpeed(const double* L, double mL, const double* R,
+                                                double mR, const Gas<double>& g, double tol,
+                                                int max_it, unsigned long long* acc) {
+  using I = Idx<D>;
+  const double uL = NearArith::quot(mL, L[0]), uR = NearArith::quot(mR, R[0]);
+  NewtonParams np;
+  np.tol = tol;
+  np.max_it = max_it;
+  const MiddleState ms = SolveMiddleState(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP],
+                                          R[I::kA], g, np, 0.5 * (L[I::kP] + R[I::kP]));
+  if (acc) {
+    const unsigned long long it = static_cast<unsigned long long>(ms.iterations);
+    acc[0] += it;
+    acc[1] = it > acc[1] ? it : acc[1];
+    acc[2] += ms.converged ? 0 : 1;
+  }
+  double wL, wR;
+  return GodunovSpeed(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP], R[I::kA], ms, &wL, &wR);
+}
+
+// Pressure and speed of sound of a conservative state; SCALAR: kinetic energy
+// in the order of the scalar path (fvs_riemann.hpp).  y_g = inv(gm1inv).
+template <int D, bool SCALAR>
+__device__ __forceinline__ void Complete(CellState<D>& c, const Gas<double>& g, double y_g) {
+  using I = Idx<D>;
+  c.y = NearArith::inv(c.q[0]);
+  const double sq = SCALAR ? SqNormScalar<D>(c.q + 1) : SqNormArray<D>(c.q + 1);
+  const double e_int = c.q[I::kE] - NearArith::div(0.5 * sq, c.q[0], c.y);
+  c.q[I::kP] = NearArith::div(e_int, g.gm1inv, y_g);
+  c.q[I::kA] = NearArith::sqrt(NearArith::div(g.gamma * c.q[I::kP], c.q[0], c.y));
+}
+
+// MUSCL-Hancock half-step states of one cell at its left and right face
+// (MusclHancockMethod.hpp:419-485) in the sequential driver's arithmetic.
+template <int D, int DIR, int LIM>
+__device__ __forceinline__ void ReconNear(const double* um, const double* u0, const double* up,
+                                          double lh, const Gas<double>& g, double y_g,
+                                          CellState<D>& recL, CellState<D>& recR) {
+  using I = Idx<D>;
+  constexpr int NC = D + 2;
+  double f[2][NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const double s = LimitedSlope<LIM>(um[k], u0[k], up[k]);
+    recL.q[k] = u0[k] - 0.5 * s;
+    recR.q[k] = u0[k] + 0.5 * s;
+  }
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const double* q = side == 0 ? recL.q : recR.q;
+    const double y = NearArith::inv(q[0]);
+    const double e_kin = NearArith::div(0.5 * SqNormScalar<D>(q + 1), q[0], y);
+    const double p = NearArith::div(q[I::kE] - e_kin, g.gm1inv, y_g);
+    const double v = NearArith::div(q[1 + DIR], q[0], y);
+    f[side][0] = q[1 + DIR];
+#pragma unroll
+    for (int d = 0; d < D; ++d) f[side][1 + d] = v * q[1 + d];
+    f[side][1 + DIR] += p;
+    f[side][I::kE] = v * (q[I::kE] + p);
+  }
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const double dq = lh * (f[0][k] - f[1][k]);
+    recR.q[k] += dq;
+    recL.q[k] += dq;
+  }
+  Complete<D, true>(recR, g, y_g);
+  Complete<D, true>(recL, g, y_g);
+}
+
 template <int D, int DIR>
-__device__ __forceinline__ double FaceSpeed(const double* L, const double* R,
-                                            const MiddleState& ms) {
-  using I = Idx<D>;
-  double wL, wR;
-  return GodunovSpeed(L[I::kRho], NearArith::quot(L[I::kMom + DIR], L[I::kRho]), L[I::kP],
-                      L[I::kA], R[I::kRho], NearArith::quot(R[I::kMom + DIR], R[I::kRho]),
-                      R[I::kP], R[I::kA], ms, &wL, &wR);
+__device__ __forceinline__ void ReconAnyNear(int limiter, const double* um, const double* u0,
+                                             const double* up, double lh, const Gas<double>& g,
+                                             double y_g, CellState<D>& recL, CellState<D>& recR) {
+  switch (limiter) {
+  case kMinMod: ReconNear<D, DIR, kMinMod>(um, u0, up, lh, g, y_g, recL, recR); break;
+  case kVanLeer: ReconNear<D, DIR, kVanLeer>(um, u0, up, lh, g, y_g, recL, recR); break;
+  case kNoLimiter: ReconNear<D, DIR, kNoLimiter>(um, u0, up, lh, g, y_g, recL, recR); break;
+  default: ReconNear<D, DIR, kNoGradient>(um, u0, up, lh, g, y_g, recL, recR); break;
+  }
 }
 
-// Flux and largest signal speed of a face from its middle state.
-template <int D, int DIR, bool MIXED>
-__device__ __forceinline__ void FaceFluxSpeed(const double* L, const double* R,
-                                              const MiddleState& ms, const Gas<double>& g,
-                                              double* F, double* speed) {
-  using I = Idx<D>;
-  const double yL = NearArith::inv(L[I::kRho]), yR = NearArith::inv(R[I::kRho]);
-  double wL, wR;
-  *speed = GodunovSpeed(L[I::kRho], NearArith::div(L[I::kMom + DIR], L[I::kRho], yL), L[I::kP],
-                        L[I::kA], R[I::kRho], NearArith::div(R[I::kMom + DIR], R[I::kRho], yR),
-                        R[I::kP], R[I::kA], ms, &wL, &wR);
-  GodunovFlux<D, DIR, MIXED>(F, L, yL, R, yR, ms, wL, wR, g);
-}
+// Per-thread sums of a sweep: largest signal speed, Newton iterations (sum
+// and maximum), faces that hit the cap, faces and (high bits) fallbacks.
+struct FaceSums {
+  double smax = 0.0;
+  unsigned iters = 0, max_it = 0, fails = 0, faces = 0, fallbacks = 0;
+  __device__ __forceinline__ unsigned long long packed_faces() const {
+    return faces + (static_cast<unsigned long long>(fallbacks) << 32);
+  }
+};
 
-// One face: Newton (shared by flux and CFL), flux, largest signal speed.
-// MIXED: the sampled star density's power in single precision.
+// One face: Newton (shared by flux and CFL), flux and, from the same middle
+// state, the largest signal speed of a first-order face.  MIXED: the sampled
+// star density's power in single precision.
 template <int D, int DIR, bool MIXED>
-__device__ __forceinline__ void GodunovFace(const double* L, const double* R, double guess,
-                                            bool has_guess, const GodunovArgs& a,
-                                            const Gas<double>& g, double* F, double* speed,
-                                            int* iters, int* conv) {
+__device__ __forceinline__ void GodunovFace(const CellState<D>& L, const CellState<D>& R,
+                                            double guess, bool has_guess, const GodunovArgs& a,
+                                            const Gas<double>& g, double* F, bool count,
+                                            bool speeds, FaceSums& sums) {
+  using I = Idx<D>;
   NewtonParams np;
   np.tol = a.tol;
   np.max_it = a.max_it;
-  using I = Idx<D>;
-  const double mean = 0.5 * (L[I::kP] + R[I::kP]);
+  const double uL = NearArith::div(L.q[1 + DIR], L.q[0], L.y);
+  const double uR = NearArith::div(R.q[1 + DIR], R.q[0], R.y);
+  const double mean = 0.5 * (L.q[I::kP] + R.q[I::kP]);
   int it, fallback;
-  const MiddleState ms =
-      SeededMiddleState<D, DIR>(L, R, g, np, has_guess, guess, mean, &it, &fallback);
-  FaceFluxSpeed<D, DIR, MIXED>(L, R, ms, g, F, speed);
-  *iters = it;
-  *conv = ms.converged | (fallback << 1);
+  const MiddleState ms = SeededMiddleState<D>(L, uL, R, uR, g, np, has_guess, guess, mean, &it,
+                                              &fallback);
+  double wL, wR;
+  const double speed = GodunovSpeed(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP],
+                                    R.q[I::kA], ms, &wL, &wR);
+  GodunovFlux<D, DIR, MIXED>(F, L.q, L.y, R.q, R.y, ms, wL, wR, g);
+  if (count) {
+    const unsigned n = static_cast<unsigned>(it);
+    sums.iters += n;
+    sums.max_it = n > sums.max_it ? n : sums.max_it;
+    sums.fails += ms.converged ? 0 : 1;
+    sums.faces += 1;
+    sums.fallbacks += fallback;
+    if (speeds) sums.smax = __builtin_fmax(sums.smax, speed);
+  }
 }
 
-// LEARNED: the network's guess is inferred inline (a.tiles set); without it
-// the kernel carries none of the matrix-core code or its registers.
-template <int D, bool MIXED, bool LEARNED>
-__global__ __launch_bounds__(kBlock) void GodunovSweepX(GodunovArgs a) {
+// CFL check of a MUSCL-Hancock sweep's face, whose signal speeds are those of
+// the two cells and not of the half-step states the flux solves: the check
+// only decides pass or fail, so a face certified to stay below dx / dt
+// (`crit`, less a margin) needs no solve; the others are solved, and the
+// reported minimum is exact wherever the check fails.  Called by the whole
+// wave.
+template <int D, int DIR>
+__device__ __forceinline__ void CheckFace(const double* uL, const double* uR, bool face,
+                                          const GodunovArgs& a, const Gas<double>& g, float crit,
+                                          FaceSums& sums) {
+  using I = Idx<D>;
+  const SpeedCell<D> l = MakeSpeedCell<D>(uL, g), r = MakeSpeedCell<D>(uR, g);
+  bool pass = !face || QuickSpeedBelow<D>(l, l.u[DIR], r, r.u[DIR], a.bound, crit);
+  if (__builtin_expect(__any(!pass), 0)) {
+    pass = !face || SpeedBelow<D>(l, l.u[DIR], r, r.u[DIR], a.bound, crit);
+    if (!pass) {
+      double L[D + 4], R[D + 4];
+#pragma unroll
+      for (int k = 0; k < D + 2; ++k) {
+        L[k] = uL[k];
+        R[k] = uR[k];
+      }
+      CompleteFromCons<D>(L, g);
+      CompleteFromCons<D>(R, g);
+      sums.smax = __builtin_fmax(sums.smax, CellFaceSpeed<D>(L, L[1 + DIR], R, R[1 + DIR], g,
+                                                             a.tol, a.max_it, nullptr));
+    }
+  }
+}
+
+// X sweep: the slot walk of the HLLEM X sweep (fvs_xslots.hpp): persistent
+// waves over 64-slot chunks of the rows' cells and ghosts, neighbours by DPP,
+// the next chunk's load in flight behind Newton.  LEARNED: the network's guess
+// is inferred inline (a.tiles set); without it the kernel carries none of the
+// matrix-core code or its registers.  MUSCL: half-step states (FP64, mean
+// guess) and, with a.check, the cells' CFL check; a ghost slot's slopes vanish
+// (its clamped value equals its inner neighbour's; NoLimiter's outer neighbour
+// is replaced).  Bound by Newton's FP64 issue at two waves per SIMD (180 to 230
+// registers; held to 168 or 128 it spills and runs 1.5 to 3 times slower).
+// 384^3 strong-wave blocks: 3.9 -> 2.9 ms a sweep against one wave per 62
+// slots with LDS shuffles; MUSCL over 256^3: 8.6 -> 2.8 ms a step against the
+// patch operators' passes (fluxes, stable dt, update, completion).
+template <int D, bool MIXED, bool LEARNED, bool MUSCL>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovSweepX(GodunovArgs a) {
   constexpr int NC = D + 2, NQ = D + 4;
   if (a.halt && *a.halt) return;
   const int64_t nx = a.n[0];
-  const uint32_t S = static_cast<uint32_t>(nx + 2);
-  const uint32_t Q = static_cast<uint32_t>(a.n[1] * a.n[2]) * S;
+  const uint32_t Q = static_cast<uint32_t>(a.n[1] * a.n[2]) * static_cast<uint32_t>(nx + 2);
+  const int64_t nchunks = (static_cast<int64_t>(Q) + kXOwned - 1) / kXOwned;
   const int lane = threadIdx.x & 63;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-  const int64_t q64 = wave * kXOwned + lane - 1;
-  const bool valid = q64 >= 0 && q64 < static_cast<int64_t>(Q);
-  const uint32_t q = valid ? static_cast<uint32_t>(q64) : 0u;
-  const uint32_t row = q / S;
-  const uint32_t sl = q - row * S;
-  const int64_t cell = static_cast<int64_t>(sl) - 1;
-  const bool real = valid && cell >= 0 && cell < nx;
-  const int64_t rbase = static_cast<int64_t>(row) * nx;
+  const int64_t nwaves = static_cast<int64_t>(gridDim.x) * (kBlock / 64);
+  const bool owned = lane >= 2 && lane < 2 + kXOwned;
   const Gas<double> g = GasOf(a);
+  const double y_g = NearArith::inv(g.gm1inv);
   const double dt = a.dt_ptr ? *a.dt_ptr : a.dt_val;
   const double dt_dx = DivRn(dt, a.dx);
-
-  double u[NQ];
-  {
-    const int64_t off = rbase + Clamp(cell, nx);
+  const double lh = DivRn(0.5 * dt, a.dx);
+  const float crit = static_cast<float>((a.dx / dt) * (1.0 - 0x1p-20));
+  XSlotWalker walk(nx, Q, nwaves, lane);
+  auto locate = [&](int64_t c) {
+    bool valid;
+    uint32_t row, sl;
+    walk.RowSlot(c, &valid, &row, &sl);
+    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row));
+  };
+  auto load = [&](const XSlot& s, double* u) {
+    const uint32_t off = 8u * (s.rbase + static_cast<uint32_t>(Clamp(s.cell, nx)));
 #pragma unroll
-    for (int k = 0; k < NC; ++k) u[k] = a.in[k][off];
-    CompleteFromCons<D>(u, g);
-  }
-  double L[NQ];
-  ShflUpState<D>(u, L);
-  const bool face_lane = valid && lane >= 1 && sl >= 1;
-  const bool owned = lane >= 1 && lane <= kXOwned;
-  double F[NC];
-  double smax = 0.0;
-  unsigned long long it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
-  // Inline learned guess: every lane takes part in the wave's matrix-core step.
-  double inline_guess = 0.0;
-  if constexpr (LEARNED) inline_guess = mlp::LearnedGuess<D, 0>(L, u, a.tiles, a.bias);
-  if (face_lane) {
-    const int64_t f = static_cast<int64_t>(sl) - 1;
-    const double guess = LEARNED   ? inline_guess
-                         : a.guess ? a.guess[static_cast<int64_t>(row) * (nx + 1) + f]
-                                   : 0.0;
-    double speed;
-    int it, conv;
-    GodunovFace<D, 0, MIXED>(L, u, guess, LEARNED || a.guess != nullptr, a, g, F, &speed, &it,
-                             &conv);
-    if (owned) {
-      smax = speed;
-      it_sum = it;
-      it_max = it;
-      nfail = (conv & 1) ? 0 : 1;
-      nfaces = 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
+    for (int k = 0; k < NC; ++k)
+      u[k] = *reinterpret_cast<const double*>(
+          reinterpret_cast<const char*>(a.in[k] + s.wbase) + off);
+  };
+  FaceSums sums;
+  int64_t c = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) +
+              __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  walk.Place(c < nchunks ? c : 0);
+  XSlot cur = locate(c < nchunks ? c : 0);
+  double u[NC];
+  if (c < nchunks) load(cur, u);
+  for (; c < nchunks; c += nwaves) {
+    const int64_t cn = c + nwaves;
+    walk.Next(c, cn, nchunks);
+    const XSlot nxt = locate(cn < nchunks ? cn : c);
+    double un[NC];
+    if (cn < nchunks) load(nxt, un);
+    const bool real = cur.valid && cur.cell >= 0 && cur.cell < nx;
+    const bool face_lane = cur.valid && lane >= 2 && lane <= 2 + kXOwned && cur.sl >= 1;
+    CellState<D> L, R;  // states left and right of the slot's lower face
+    double ul[NC];
+    if constexpr (MUSCL) {
+      double up[NC];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        ul[k] = ShiftUp(u[k]);
+        up[k] = ShiftDown(u[k]);
+      }
+      double um[NC];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        um[k] = (a.limiter == kNoLimiter && cur.cell < 0) ? u[k] : ul[k];
+        if (a.limiter == kNoLimiter && cur.cell >= nx) up[k] = u[k];
+      }
+      ReconAnyNear<D, 0>(a.limiter, um, u, up, lh, g, y_g, R, L);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NC; ++k) R.q[k] = u[k];
+      Complete<D, false>(R, g, y_g);
+      L = R;
     }
-  } else {
 #pragma unroll
-    for (int k = 0; k < NC; ++k) F[k] = 0.0;
+    for (int k = 0; k < NQ; ++k) L.q[k] = ShiftUp(L.q[k]);
+    L.y = ShiftUp(L.y);
+    double guess = 0.0;
+    if constexpr (LEARNED) {
+      // every lane takes part in the wave's matrix-core step
+      guess = mlp::LearnedGuess<D, 0>(L.q, R.q, a.tiles, a.bias);
+    }
+    double F[NC];
+    if (face_lane) {
+      if constexpr (!LEARNED && !MUSCL) {
+        if (a.guess) {
+          const int64_t row = (cur.wbase + cur.rbase) / nx;
+          guess = a.guess[row * (nx + 1) + static_cast<int64_t>(cur.sl) - 1];
+        }
+      }
+      GodunovFace<D, 0, MIXED>(L, R, guess, LEARNED || a.guess != nullptr, a, g, F, owned, !MUSCL,
+                               sums);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NC; ++k) F[k] = 0.0;
+    }
+    double Fnext[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) Fnext[k] = ShiftDown(F[k]);
+    if (a.update && owned && real) {
+      const uint32_t off = 8u * (cur.rbase + static_cast<uint32_t>(cur.cell));
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        *reinterpret_cast<double*>(reinterpret_cast<char*>(a.out[k] + cur.wbase) + off) =
+            u[k] + dt_dx * (F[k] - Fnext[k]);
+    }
+    if constexpr (MUSCL) {
+      if (a.check) CheckFace<D, 0>(ul, u, owned && face_lane, a, g, crit, sums);
+    }
+    cur = nxt;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) u[k] = un[k];
   }
-  double Fnext[NC];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) Fnext[k] = __shfl_down(F[k], 1, 64);
-  if (a.update && owned && real) {
-    const int64_t off = rbase + cell;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) a.out[k][off] = u[k] + dt_dx * (F[k] - Fnext[k]);
-  }
-  BlockReduceGodunov<kBlock / 64>(smax, a.dx, it_sum, it_max, nfail, nfaces, a.partials + 5 * blockIdx.x);
+  BlockReduceGodunov<kBlock / 64>(sums.smax, a.dx, sums.iters, sums.max_it, sums.fails, sums.packed_faces(),
+                                  a.partials + 5 * blockIdx.x);
 }
 
-template <int D, int DIR, bool MIXED, bool LEARNED>
+// Y / Z sweep: one thread per pencil marching a segment with the cell before
+// (and, MUSCL, around) the face in registers and the next cell's load in
+// flight.  Bound by Newton's FP64 issue, like the X sweep.
+template <int D, int DIR, bool MIXED, bool LEARNED, bool MUSCL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovSweepPencil(GodunovArgs a) {
-  constexpr int NC = D + 2, NQ = D + 4;
+  constexpr int NC = D + 2;
   if (a.halt && *a.halt) return;
-  const int64_t nx = a.n[0], ny = a.n[1], nz = a.n[2];
+  const int64_t nx = a.n[0], ny = a.n[1];
   const int64_t nd = a.n[DIR];
-  const int64_t npencil = (DIR == 1) ? nx * nz : nx * ny;
+  const int64_t npencil = (DIR == 1) ? nx * a.n[2] : nx * ny;
   const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   const bool active = p0 < npencil;
   // Lanes past the last pencil repeat it (all lanes of a wave march together,
@@ -288,188 +464,196 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int64_t stride = (DIR == 1) ? nx : nx * ny;
   const int64_t base = (DIR == 1) ? (p % nx) + (p / nx) * nx * ny : p;
   // Face (x, j, z) of direction DIR in the face box (n with n[DIR] + 1).
-  const int64_t fstride = stride;
   const int64_t fbase = (DIR == 1) ? (p % nx) + (p / nx) * nx * (ny + 1) : p;
   const int64_t j0 = static_cast<int64_t>(blockIdx.y) * a.seg;
   const int64_t j1 = (j0 + a.seg < nd) ? j0 + a.seg : nd;
   const Gas<double> g = GasOf(a);
+  const double y_g = NearArith::inv(g.gm1inv);
   const double dt = a.dt_ptr ? *a.dt_ptr : a.dt_val;
   const double dt_dx = DivRn(dt, a.dx);
-  (void)nz;
+  const double lh = DivRn(0.5 * dt, a.dx);
+  const float crit = static_cast<float>((a.dx / dt) * (1.0 - 0x1p-20));
 
-  double smax = 0.0;
-  unsigned long long it_sum = 0, it_max = 0, nfail = 0, nfaces = 0;
-  {
-    auto load = [&](double* q, int64_t j) {
-      const int64_t off = base + Clamp(j, nd) * stride;
+  FaceSums sums;
+  auto load = [&](double* u, int64_t j) {
+    const int64_t off = base + Clamp(j, nd) * stride;
 #pragma unroll
-      for (int k = 0; k < NC; ++k) q[k] = a.in[k][off];
-      CompleteFromCons<D>(q, g);
-    };
-    double qm[NQ], q0[NQ];
-    load(qm, j0 - 1);
-    double Fprev[NC];
-    for (int64_t j = j0; j <= j1; ++j) {
-      load(q0, j);
-      double F[NC], speed;
-      int it, conv;
-      double guess = 0.0;
-      if constexpr (LEARNED) {
-        guess = mlp::LearnedGuess<D, DIR>(qm, q0, a.tiles, a.bias);
-      } else if (a.guess) {
-        guess = a.guess[fbase + j * fstride];
-      }
-      GodunovFace<D, DIR, MIXED>(qm, q0, guess, LEARNED || a.guess != nullptr, a, g, F, &speed,
-                                 &it, &conv);
-      if (active && (j < j1 || j1 == nd)) {
-        smax = __builtin_fmax(smax, speed);
-        it_sum += it;
-        it_max = (unsigned long long)it > it_max ? it : it_max;
-        nfail += (conv & 1) ? 0 : 1;
-        nfaces += 1 + (static_cast<unsigned long long>((conv >> 1) & 1) << 32);
-      }
-      if (a.update && active && j > j0) {
-        const int64_t off = base + (j - 1) * stride;
+    for (int k = 0; k < NC; ++k) u[k] = a.in[k][off];
+  };
+  double Um[NC], U0[NC], Unext[NC], Fprev[NC];
+  load(Um, j0 - 1);
+  load(U0, j0);
+  load(Unext, j0 + 1);
+  CellState<D> L;
+  if constexpr (MUSCL) {
+    // Half-step state of cell j0 - 1 (a ghost at j0 = 0, whose clamped
+    // neighbours give it no slope).
+    double Umm[NC];
+    load(Umm, j0 - 2);
+    CellState<D> unused;
+    if (j0 == 0)
+      ReconNear<D, DIR, kNoGradient>(Um, Um, Um, lh, g, y_g, unused, L);
+    else
+      ReconAnyNear<D, DIR>(a.limiter, Umm, Um, U0, lh, g, y_g, unused, L);
+  } else {
 #pragma unroll
-        for (int k = 0; k < NC; ++k) a.out[k][off] = qm[k] + dt_dx * (Fprev[k] - F[k]);
-      }
+    for (int k = 0; k < NC; ++k) L.q[k] = Um[k];
+    Complete<D, false>(L, g, y_g);
+  }
+  for (int64_t j = j0; j <= j1; ++j) {
+    double Up[NC];
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) qm[k] = q0[k];
+    for (int k = 0; k < NC; ++k) Up[k] = Unext[k];
+    if (j + 1 < nd && j < j1) load(Unext, j + 2);
+    CellState<D> R, Lnext;
+    if constexpr (MUSCL) {
+      if (j < nd)
+        ReconAnyNear<D, DIR>(a.limiter, Um, U0, Up, lh, g, y_g, R, Lnext);
+      else
+        ReconNear<D, DIR, kNoGradient>(U0, U0, U0, lh, g, y_g, R, Lnext);
+    } else {
 #pragma unroll
-      for (int k = 0; k < NC; ++k) Fprev[k] = F[k];
+      for (int k = 0; k < NC; ++k) R.q[k] = U0[k];
+      Complete<D, false>(R, g, y_g);
+      Lnext = R;
+    }
+    double F[NC];
+    double guess = 0.0;
+    if constexpr (LEARNED) {
+      guess = mlp::LearnedGuess<D, DIR>(L.q, R.q, a.tiles, a.bias);
+    } else if constexpr (!MUSCL) {
+      if (a.guess) guess = a.guess[fbase + j * stride];
+    }
+    const bool mine = active && (j < j1 || j1 == nd);
+    GodunovFace<D, DIR, MIXED>(L, R, guess, LEARNED || a.guess != nullptr, a, g, F, mine, !MUSCL,
+                               sums);
+    if (a.update && active && j > j0) {
+      const int64_t off = base + (j - 1) * stride;
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        __builtin_nontemporal_store(Um[k] + dt_dx * (Fprev[k] - F[k]), &a.out[k][off]);
+    }
+    if constexpr (MUSCL) {
+      if (a.check) CheckFace<D, DIR>(Um, U0, mine, a, g, crit, sums);
+    }
+    L = Lnext;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      Um[k] = U0[k];
+      U0[k] = Up[k];
+      Fprev[k] = F[k];
     }
   }
-  BlockReduceGodunov<kBlock / 64>(smax, a.dx, it_sum, it_max, nfail, nfaces,
-                     a.partials + 5 * (blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x));
+  BlockReduceGodunov<kBlock / 64>(sums.smax, a.dx, sums.iters, sums.max_it, sums.fails, sums.packed_faces(),
+                                  a.partials + 5 * (blockIdx.x + static_cast<int64_t>(blockIdx.y) * gridDim.x));
 }
 
 // Reduction of the per-workgroup Godunov partials: out[0] = min dt,
 // stats[0..3] = total iterations, max iterations, non-converged, faces.
+// One workgroup per direction (partials of direction d at p + 5 n d, its
+// minimum to out[d]); with `check` the value is also the split step's CFL
+// check against ctl->split_dt.
 constexpr int kRedBlock = 1024;
 __global__ __launch_bounds__(kRedBlock) void GodunovFinalize(const unsigned long long* p,
                                                              int64_t n, double* out,
-                                                             unsigned long long* stats,
-                                                             Ctl* ctl) {
+                                                             unsigned long long* stats, Ctl* ctl,
+                                                             int check) {
   if (ctl && ctl->halt) return;
+  p += 5 * n * blockIdx.x;
   __shared__ unsigned long long s[5][kRedBlock / 64];
-  unsigned long long r[5] = {kInfKey, 0, 0, 0, 0};
+  unsigned long long key = kInfKey, iters = 0, max_it = 0, fails = 0, faces = 0;
   for (int64_t i = threadIdx.x; i < n; i += kRedBlock) {
-    r[0] = KMin(r[0], p[5 * i]);
-    r[1] += p[5 * i + 1];
-    r[2] = p[5 * i + 2] > r[2] ? p[5 * i + 2] : r[2];
-    r[3] += p[5 * i + 3];
-    r[4] += p[5 * i + 4];
+    key = KMin(key, p[5 * i]);
+    iters += p[5 * i + 1];
+    max_it = p[5 * i + 2] > max_it ? p[5 * i + 2] : max_it;
+    fails += p[5 * i + 3];
+    faces += p[5 * i + 4];
   }
-  r[0] = WaveMinKey(r[0]);
-  r[1] = WaveSum(r[1]);
-  r[2] = WaveMaxU(r[2]);
-  r[3] = WaveSum(r[3]);
-  r[4] = WaveSum(r[4]);
+  key = WaveMinKey(key);
+  iters = WaveSum(iters);
+  max_it = WaveMaxU(max_it);
+  fails = WaveSum(fails);
+  faces = WaveSum(faces);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0)
-    for (int i = 0; i < 5; ++i) s[i][wave] = r[i];
+  if (lane == 0) {
+    s[0][wave] = key;
+    s[1][wave] = iters;
+    s[2][wave] = max_it;
+    s[3][wave] = fails;
+    s[4][wave] = faces;
+  }
   __syncthreads();
   if (threadIdx.x != 0) return;
   for (int w = 1; w < kRedBlock / 64; ++w) {
-    r[0] = KMin(r[0], s[0][w]);
-    r[1] += s[1][w];
-    r[2] = s[2][w] > r[2] ? s[2][w] : r[2];
-    r[3] += s[3][w];
-    r[4] += s[4][w];
+    key = KMin(key, s[0][w]);
+    iters += s[1][w];
+    max_it = s[2][w] > max_it ? s[2][w] : max_it;
+    fails += s[3][w];
+    faces += s[4][w];
   }
-  r[0] = s[0][0] < r[0] ? s[0][0] : r[0];
-  const double v = __longlong_as_double(static_cast<long long>(r[0]));
-  if (out) *out = v;
+  const double v = __longlong_as_double(static_cast<long long>(key));
+  if (out) out[blockIdx.x] = v;
   if (stats) {
-    // r[4] packs faces (low 32 bits per face) and fallbacks (high bits).
-    stats[0] += r[1];
-    stats[1] = r[2] > stats[1] ? r[2] : stats[1];
-    stats[2] += r[3];
-    stats[3] += r[4] & 0xffffffffull;
-    stats[4] += r[4] >> 32;
+    // faces packs the faces (low 32 bits) and the fallbacks (high bits)
+    atomicAdd(&stats[0], iters);
+    atomicMax(&stats[1], max_it);
+    atomicAdd(&stats[2], fails);
+    atomicAdd(&stats[3], faces & 0xffffffffull);
+    atomicAdd(&stats[4], faces >> 32);
+  }
+  if (check && v < ctl->split_dt) {
+    // TimeStepTooLarge{level_dt} (DimensionalSplitLevelIntegrator.hpp:243-245)
+    ctl->halt = 1;
+    ctl->failure_dt = v;
   }
 }
 
 // Per-face Godunov flux on strided views (FluxMethod seq driver): first
 // order, or MUSCL-Hancock with the sequential (scalar) CompleteFromCons.
-template <int D, int DIR, int LIM>
-__device__ __forceinline__ void ReconScalarKE(const double* um, const double* u0,
-                                              const double* up, double lh,
-                                              const Gas<double>& g, double* recL,
-                                              double* recR) {
-  constexpr int NC = D + 2, NQ = D + 4;
-  double qL[NQ], qR[NQ];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    const double s = LimitedSlope<LIM>(um[k], u0[k], up[k]);
-    qL[k] = u0[k] - 0.5 * s;
-    qR[k] = u0[k] + 0.5 * s;
-  }
-  CompleteFromConsScalar<D>(qL, g);
-  CompleteFromConsScalar<D>(qR, g);
-  double fL[NC], fR[NC];
-  PhysFlux<D, DIR>(fL, qL);
-  PhysFlux<D, DIR>(fR, qR);
-#pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    const double dq = lh * (fL[k] - fR[k]);
-    recR[k] = qR[k] + dq;
-    recL[k] = qL[k] + dq;
-  }
-  CompleteFromConsScalar<D>(recR, g);
-  CompleteFromConsScalar<D>(recL, g);
-}
-
 template <int D, int DIR>
 __global__ __launch_bounds__(kBlock) void GodunovViewFlux(DevView fl, DevView st, double dt,
                                                           double dx, Gas<double> g, int limiter,
                                                           int muscl, double tol, int max_it,
                                                           unsigned long long* nfail) {
+  using I = Idx<D>;
   constexpr int NC = D + 2, NQ = D + 4;
   const int64_t q = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (q >= fl.count()) return;
   int64_t f[3];
   fl.index(q, f);
-  double L[NQ], R[NQ];
-  auto loadc = [&](int64_t off, double* out) {
+  CellState<D> L, R;
+  auto loadc = [&](int64_t off, double* out, int n) {
     int64_t c[3] = {f[0], f[1], f[2]};
     c[DIR] += off;
-    for (int k = 0; k < NQ; ++k) out[k] = *st.at(c, k);
+    for (int k = 0; k < n; ++k) out[k] = *st.at(c, k);
   };
   if (muscl) {
-    double u[4][NQ];
-    for (int s = 0; s < 4; ++s) loadc(s - 2, u[s]);
+    const double y_g = NearArith::inv(g.gm1inv);
+    double u[4][NC];
+    for (int s = 0; s < 4; ++s) loadc(s - 2, u[s], NC);
     const double lh = 0.5 * dt / dx;
-    double dummy[NQ];
-    switch (limiter) {
-    case kMinMod:
-      ReconScalarKE<D, DIR, kMinMod>(u[0], u[1], u[2], lh, g, dummy, L);
-      ReconScalarKE<D, DIR, kMinMod>(u[1], u[2], u[3], lh, g, R, dummy);
-      break;
-    case kVanLeer:
-      ReconScalarKE<D, DIR, kVanLeer>(u[0], u[1], u[2], lh, g, dummy, L);
-      ReconScalarKE<D, DIR, kVanLeer>(u[1], u[2], u[3], lh, g, R, dummy);
-      break;
-    case kNoLimiter:
-      ReconScalarKE<D, DIR, kNoLimiter>(u[0], u[1], u[2], lh, g, dummy, L);
-      ReconScalarKE<D, DIR, kNoLimiter>(u[1], u[2], u[3], lh, g, R, dummy);
-      break;
-    default:
-      ReconScalarKE<D, DIR, kNoGradient>(u[0], u[1], u[2], lh, g, dummy, L);
-      ReconScalarKE<D, DIR, kNoGradient>(u[1], u[2], u[3], lh, g, R, dummy);
-      break;
-    }
+    CellState<D> unused;
+    ReconAnyNear<D, DIR>(limiter, u[0], u[1], u[2], lh, g, y_g, unused, L);
+    ReconAnyNear<D, DIR>(limiter, u[1], u[2], u[3], lh, g, y_g, R, unused);
   } else {
-    loadc(-1, L);
-    loadc(0, R);
+    loadc(-1, L.q, NQ);
+    loadc(0, R.q, NQ);
+    L.y = NearArith::inv(L.q[0]);
+    R.y = NearArith::inv(R.q[0]);
   }
   NewtonParams np;
   np.tol = tol;
   np.max_it = max_it;
-  const MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, 0.5 * (L[D + 2] + R[D + 2]));
+  const double uL = NearArith::div(L.q[1 + DIR], L.q[0], L.y);
+  const double uR = NearArith::div(R.q[1 + DIR], R.q[0], R.y);
+  const MiddleState ms =
+      SolveMiddleState(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA], g,
+                       np, 0.5 * (L.q[I::kP] + R.q[I::kP]));
   if (!ms.converged) atomicAdd(nfail, 1ull);
-  double F[NC], speed;
-  FaceFluxSpeed<D, DIR, false>(L, R, ms, g, F, &speed);
+  double F[NC], wL, wR;
+  GodunovSpeed(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA], ms, &wL,
+               &wR);
+  GodunovFlux<D, DIR, false>(F, L.q, L.y, R.q, R.y, ms, wL, wR, g);
   for (int k = 0; k < NC; ++k) *fl.at(f, k) = F[k];
 }
 
@@ -491,11 +675,7 @@ __global__ __launch_bounds__(kBlock) void GodunovViewStableDt(DevView st, DevVie
     for (int k = 0; k < NQ; ++k) L[k] = *st.at(c, k);
     c[DIR] += 1;
     for (int k = 0; k < NQ; ++k) R[k] = *st.at(c, k);
-    NewtonParams np;
-    np.tol = tol;
-    np.max_it = max_it;
-    const MiddleState ms = ComputeMiddleState<D, DIR>(L, R, g, np, 0.5 * (L[D + 2] + R[D + 2]));
-    key = SpeedKey(dx, FaceSpeed<D, DIR>(L, R, ms));
+    key = SpeedKey(dx, CellFaceSpeed<D>(L, L[1 + DIR], R, R[1 + DIR], g, tol, max_it, nullptr));
   }
   __shared__ unsigned long long s[kBlock / 64];
   key = WaveMinKey(key);
@@ -543,6 +723,8 @@ struct GodunovCflArgs {
   int* halt;
   const double* floor;  // speed floor per direction (nullable: none)
   int* hit;
+  int count_fails;  // faces that hit the iteration cap count as failures (first
+                    // order, where the sweeps solve the same faces)
 };
 
 // The face of direction d between the cells at off_l and off_r: its largest
@@ -551,7 +733,6 @@ template <int D>
 __device__ __forceinline__ double CflFace(const GodunovCflArgs& a, const Gas<double>& g, int d,
                                           int64_t off_l, int64_t off_r,
                                           unsigned long long* acc) {
-  using I = Idx<D>;
   double L[D + 4], R[D + 4];
 #pragma unroll
   for (int k = 0; k < D + 2; ++k) {
@@ -562,18 +743,7 @@ __device__ __forceinline__ double CflFace(const GodunovCflArgs& a, const Gas<dou
   CompleteFromCons<D>(R, g);
   const double mL = d == 0 ? L[1] : (D == 2 || d == 1) ? L[2] : L[D];
   const double mR = d == 0 ? R[1] : (D == 2 || d == 1) ? R[2] : R[D];
-  const double uL = NearArith::quot(mL, L[0]), uR = NearArith::quot(mR, R[0]);
-  NewtonParams np;
-  np.tol = a.tol;
-  np.max_it = a.max_it;
-  const MiddleState ms = SolveMiddleState(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP],
-                                          R[I::kA], g, np, 0.5 * (L[I::kP] + R[I::kP]));
-  const unsigned long long it = static_cast<unsigned long long>(ms.iterations);
-  acc[0] += it;
-  acc[1] = it > acc[1] ? it : acc[1];
-  acc[2] += ms.converged ? 0 : 1;
-  double wL, wR;
-  return GodunovSpeed(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP], R[I::kA], ms, &wL, &wR);
+  return CellFaceSpeed<D>(L, mL, R, mR, g, a.tol, a.max_it, acc);
 }
 
 template <int D> __device__ __forceinline__ SpeedCell<D> ShiftUpCell(const SpeedCell<D>& c) {
@@ -720,7 +890,7 @@ __global__ __launch_bounds__(64 * kCflRows) __attribute__((amdgpu_waves_per_eu(4
   for (int d = 0; d < D; ++d) {
     const bool first_dir = d == 0;
     BlockReduceGodunov<kCflRows>(smax[d], a.dx[d], first_dir ? acc[0] : 0, first_dir ? acc[1] : 0,
-                                 first_dir ? acc[2] : 0, faces[d],
+                                 first_dir && a.count_fails ? acc[2] : 0, faces[d],
                                  a.partials + 5 * (d * nblocks + blockIdx.x));
     const bool hit = a.floor && a.floor[d] > 0.0 && smax[d] >= a.floor[d];
     if (__syncthreads_or(hit ? 1 : 0) && threadIdx.x == 0 && a.hit) a.hit[d] = 1;
@@ -827,15 +997,16 @@ int LaunchMiddleState(int dim, hipStream_t s, const double* L, const double* R, 
   return FVS_OK;
 }
 
-int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3], int seg) {
-  const int64_t nz = dim == 3 ? n[2] : 1;
-  if (dir == 0) {
-    const int64_t slots = (n[0] + 2) * n[1] * nz;
-    const int64_t waves = (slots + kXOwned - 1) / kXOwned;
-    return (waves + kBlock / 64 - 1) / (kBlock / 64);
-  }
-  const int64_t npencil = (dir == 1) ? n[0] * nz : n[0] * n[1];
-  return ((npencil + kBlock - 1) / kBlock) * ((n[dir] + seg - 1) / seg);
+// Segment of a pencil sweep: PencilSeg, longer where the grid's second
+// dimension (65,535) would not hold its segments.
+static int GodunovSeg(int dim, int dir, const int64_t n[3]) {
+  int64_t seg = PencilSeg(dim, dir, n);
+  while ((n[dir] + seg - 1) / seg > 65535) seg *= 2;
+  return static_cast<int>(seg);
+}
+
+int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3]) {
+  return SweepBlocks(dim, dir, n, GodunovSeg(dim, dir, n));
 }
 
 static int64_t GodunovCflItems(int dim, const int64_t n[3]) {
@@ -855,7 +1026,7 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
                        const double* const* in, double* const* out, const int64_t n[3],
                        double dx, const double* dt_ptr, double dt_val, const double* guess,
                        unsigned long long* partials, int* halt, int update,
-                       const fvs_mlp* net) {
+                       const fvs_mlp* net, int check) {
   GodunovArgs a;
   std::memset(&a, 0, sizeof a);
   const int D = desc.dim;
@@ -875,23 +1046,34 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
   if (net) MlpOperands(net, &a.tiles, &a.bias);
   a.partials = partials;
   a.halt = halt;
-  a.seg = PencilSeg(D, dir, a.n);
+  a.seg = GodunovSeg(D, dir, a.n);
   a.update = update;
+  const bool muscl = desc.reconstruction == FVS_RECON_MUSCL_HANCOCK;
+  a.limiter = desc.limiter;
+  a.check = check;
+  a.bound = MakeSpeedBound(desc.gamma, desc.newton_tolerance, desc.max_newton_iterations);
   const bool mixed = desc.precision == FVS_FP32_FLUX;
   const bool learned = a.tiles != nullptr;
-  const int64_t blocks = GodunovSweepBlocks(D, dir, a.n, a.seg);
+  if (muscl && (learned || guess)) {
+    SetError("MUSCL-Hancock sweeps take no guess");
+    return FVS_BAD_ARGUMENT;
+  }
+  const int64_t blocks = GodunovSweepBlocks(D, dir, a.n);
   if (blocks <= 0) return FVS_BAD_ARGUMENT;
   if (dir == 0) {
-    if ((a.n[0] + 2) * a.n[1] * a.n[2] >= (int64_t(1) << 32) || blocks > 0x7fffffff) {
+    if ((a.n[0] + 2) * a.n[1] * a.n[2] >= (int64_t(1) << 32)) {
       SetError("Godunov X sweep: patch too large for 32-bit slot indices");
       return FVS_BAD_ARGUMENT;
     }
     using K = void (*)(GodunovArgs);
-    const K ks[2][2][2] = {{{GodunovSweepX<2, false, false>, GodunovSweepX<2, false, true>},
-                            {GodunovSweepX<2, true, false>, GodunovSweepX<2, true, true>}},
-                           {{GodunovSweepX<3, false, false>, GodunovSweepX<3, false, true>},
-                            {GodunovSweepX<3, true, false>, GodunovSweepX<3, true, true>}}};
-    hipLaunchKernelGGL(ks[D == 3][mixed][learned], dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+    const K ks[2][2][2] = {
+        {{GodunovSweepX<2, false, false, false>, GodunovSweepX<2, false, true, false>},
+         {GodunovSweepX<2, true, false, false>, GodunovSweepX<2, true, true, false>}},
+        {{GodunovSweepX<3, false, false, false>, GodunovSweepX<3, false, true, false>},
+         {GodunovSweepX<3, true, false, false>, GodunovSweepX<3, true, true, false>}}};
+    const K km[2] = {GodunovSweepX<2, false, false, true>, GodunovSweepX<3, false, false, true>};
+    hipLaunchKernelGGL(muscl ? km[D == 3] : ks[D == 3][mixed][learned], dim3(unsigned(blocks)),
+                       dim3(kBlock), 0, s, a);
   } else {
     const int64_t npencil = (dir == 1) ? a.n[0] * a.n[2] : a.n[0] * a.n[1];
     const int64_t bx = (npencil + kBlock - 1) / kBlock;
@@ -899,24 +1081,27 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
     if (bx > 0x7fffffff || nseg > 65535) return FVS_BAD_ARGUMENT;
     const dim3 grid{static_cast<unsigned>(bx), static_cast<unsigned>(nseg), 1u};
     using K = void (*)(GodunovArgs);
-    const K ks[3][2][2] = {
-        {{GodunovSweepPencil<2, 1, false, false>, GodunovSweepPencil<2, 1, false, true>},
-         {GodunovSweepPencil<2, 1, true, false>, GodunovSweepPencil<2, 1, true, true>}},
-        {{GodunovSweepPencil<3, 1, false, false>, GodunovSweepPencil<3, 1, false, true>},
-         {GodunovSweepPencil<3, 1, true, false>, GodunovSweepPencil<3, 1, true, true>}},
-        {{GodunovSweepPencil<3, 2, false, false>, GodunovSweepPencil<3, 2, false, true>},
-         {GodunovSweepPencil<3, 2, true, false>, GodunovSweepPencil<3, 2, true, true>}}};
+#define FVS_GP(D_, R_)                                                                          \
+  {                                                                                             \
+    {GodunovSweepPencil<D_, R_, false, false, false>, GodunovSweepPencil<D_, R_, false, true, false>}, \
+    {GodunovSweepPencil<D_, R_, true, false, false>, GodunovSweepPencil<D_, R_, true, true, false>} \
+  }
+    const K ks[3][2][2] = {FVS_GP(2, 1), FVS_GP(3, 1), FVS_GP(3, 2)};
+#undef FVS_GP
+    const K km[3] = {GodunovSweepPencil<2, 1, false, false, true>,
+                     GodunovSweepPencil<3, 1, false, false, true>,
+                     GodunovSweepPencil<3, 2, false, false, true>};
     const int which = D == 2 ? 0 : (dir == 1 ? 1 : 2);
-    hipLaunchKernelGGL(ks[which][mixed][learned], grid, dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(muscl ? km[which] : ks[which][mixed][learned], grid, dim3(kBlock), 0, s, a);
   }
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }
 
 int LaunchGodunovFinalize(hipStream_t s, const unsigned long long* partials, int64_t nblocks,
-                          double* out, unsigned long long* stats, Ctl* ctl) {
-  hipLaunchKernelGGL(GodunovFinalize, dim3(1), dim3(kRedBlock), 0, s, partials, nblocks, out,
-                     stats, ctl);
+                          int ndir, double* out, unsigned long long* stats, Ctl* ctl, int check) {
+  hipLaunchKernelGGL(GodunovFinalize, dim3(ndir), dim3(kRedBlock), 0, s, partials, nblocks, out,
+                     stats, ctl, check);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }
@@ -940,6 +1125,7 @@ int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* c
   a.max_it = desc.max_newton_iterations;
   a.bound = MakeSpeedBound(desc.gamma, desc.newton_tolerance, desc.max_newton_iterations);
   a.items = GodunovCflItems(D, a.n);
+  a.count_fails = desc.reconstruction == FVS_RECON_NONE;
   a.partials = partials;
   a.halt = halt;
   const dim3 grid(static_cast<unsigned>(GodunovCflBlocks(D, a.n)));

@@ -163,15 +163,18 @@ int LaunchPatchCfl(const fvs_method_desc& desc, hipStream_t stream,
                    double* out, Ctl* ctl, int* halt, int first_dir, int strang);
 // Exact-Godunov flux method (fvs_godunov.hip).  Partials hold 5 keys per
 // workgroup: min dt, iteration sum, iteration max, non-converged, faces.
-int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3], int seg);
+int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3]);
 int64_t GodunovCflBlocks(int dim, const int64_t n[3]);
 int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
                        const double* const* in, double* const* out, const int64_t n[3],
                        double dx, const double* dt_ptr, double dt_val, const double* guess,
                        unsigned long long* partials, int* halt, int update,
-                       const fvs_mlp* net = nullptr);
+                       const fvs_mlp* net = nullptr, int check = 0);
+// Reduces the partials of ndir directions (nblocks each) into out[0 .. ndir)
+// and the Newton counters; check: out[0] is the split step's CFL check.
 int LaunchGodunovFinalize(hipStream_t s, const unsigned long long* partials, int64_t nblocks,
-                          double* out, unsigned long long* stats, Ctl* ctl = nullptr);
+                          int ndir, double* out, unsigned long long* stats, Ctl* ctl = nullptr,
+                          int check = 0);
 // With floor_ctl (the level driver) and an iteration cap of at least
 // kGodunovFloorCap, the faces that a certified speed bound keeps below
 // ctl->cfl_floor skip their Newton solve.
@@ -203,7 +206,6 @@ int LaunchStepEnd(hipStream_t s, Ctl* ctl);
 // with a speed floor) the floor is validated and renewed (dx: cell widths).
 int LaunchStepDt(hipStream_t s, Ctl* ctl, int dim, int first_dir, int strang,
                  const double* dx = nullptr, int use_floor = 0);
-int LaunchCheckValue(hipStream_t s, Ctl* ctl, const double* value);
 int LaunchKeysToDt(hipStream_t s, unsigned long long* keys, int n, double* out);
 int LaunchResetKeys(hipStream_t s, unsigned long long* keys, int n,
                     unsigned int* counters, int nc);

@@ -1,7 +1,5 @@
 // Single-patch level integrator for the flux methods that have no fused
-// sweep: MUSCL-Hancock over the exact-Godunov base (the reference's default
-// MusclHancockMethod, include/fub/flux_method/MusclHancockMethod.hpp:277-285),
-// the HLL base, MusclHancockPrim and MusclHancockCharacteristic.
+// sweep: the HLL base, MusclHancockPrim and MusclHancockCharacteristic.
 //
 // The step is the reference's DimensionalSplitLevelIntegrator sequence
 // (include/fub/solver/DimensionalSplitLevelIntegrator.hpp:221-276) composed
@@ -20,7 +18,7 @@
 //     CompleteFromCons.
 // Each check reads one double back to the host, so this path synchronises
 // a few times per step; the fused level kernels serve the HLLEM and
-// first-order exact-Godunov methods.
+// exact-Godunov methods.
 #include "fvs_internal.hpp"
 
 #include <algorithm>
@@ -109,14 +107,6 @@ int DirStableDt(CL* C, int dir, double* dt) {
   return FVS_OK;
 }
 
-// Newton iterations that hit the cap so far (exact-Godunov base).
-int NewtonCapHits(CL* C, uint64_t* hits) {
-  uint64_t st[5];
-  if (int rc = fvs_newton_stats(C->h, st, 0)) return rc;
-  *hits = st[2];
-  return FVS_OK;
-}
-
 // One split step in dir with the split dt; *level_dt receives the
 // direction's stable dt.  With known_dt > 0 the ghosts of dir are filled and
 // known_dt is that stable dt already (the step-start value of the first
@@ -149,20 +139,7 @@ int SplitStep(CL* C, int dir, double split_dt, double known_dt, double* level_dt
   slo[dir] -= C->gw;
   shi[dir] += C->gw;
   const fvs_view sv = ScratchView(C, slo, shi, D + 4);
-  const bool godunov = C->h->desc.base == FVS_BASE_GODUNOV_EXACT;
-  uint64_t caps0 = 0, caps1 = 0;
-  if (godunov) {
-    if (int rc = NewtonCapHits(C, &caps0)) return rc;
-  }
   if (int rc = fvs_numeric_fluxes(C->h, &fv, &sv, split_dt, C->patch.dx[dir], dir)) return rc;
-  if (godunov) {
-    if (int rc = NewtonCapHits(C, &caps1)) return rc;
-    if (caps1 != caps0) {
-      SetError("Newton iteration hit its cap in %llu faces",
-               static_cast<unsigned long long>(caps1 - caps0));
-      return FVS_NEWTON_NOT_CONVERGED;
-    }
-  }
   int64_t ilo[3], ihi[3];
   Interior(C, ilo, ihi);
   const fvs_view cons = ScratchView(C, ilo, ihi, D + 2);
@@ -209,8 +186,7 @@ int CopyInterior(CL* C, const double* const* comps, double* const* out) {
 } // namespace
 
 bool ComposedLevelNeeded(const fvs_method_desc& d) {
-  return (d.base == FVS_BASE_GODUNOV_EXACT && d.reconstruction != FVS_RECON_NONE) ||
-         d.base == FVS_BASE_HLL_EINFELDT || d.reconstruction >= FVS_RECON_MUSCL_HANCOCK_PRIM;
+  return d.base == FVS_BASE_HLL_EINFELDT || d.reconstruction >= FVS_RECON_MUSCL_HANCOCK_PRIM;
 }
 
 int ComposedCreate(fvs_handle* h, const fvs_patch_desc* patch, fvs_composed_level** out) {

@@ -970,17 +970,6 @@ __global__ void StepDtKernel(Ctl* ctl, int dim, int first_dir, int strang, doubl
   }
 }
 
-// CFL check of a split step whose stable dt was reduced into ctl->last_check.
-__global__ void CheckValueKernel(Ctl* ctl, const double* value) {
-  if (ctl->halt) return;
-  const double v = *value;
-  ctl->last_check = v;
-  if (v < ctl->split_dt) {
-    ctl->halt = 1;
-    ctl->failure_dt = v;
-  }
-}
-
 __device__ __forceinline__ void EndStep(Ctl* ctl) {
   const int64_t slot = ctl->cycle - ctl->dt_log_base;
   if (ctl->dt_log && slot >= 0 && slot < ctl->dt_log_len) ctl->dt_log[slot] = ctl->dt;
@@ -1266,12 +1255,6 @@ int LaunchStepDt(hipStream_t s, Ctl* ctl, int dim, int first_dir, int strang, co
   const double f0 = dx ? dx[0] : 1.0, f1 = dx ? dx[1] : 1.0, f2 = dx ? dx[2] : 1.0;
   hipLaunchKernelGGL(StepDtKernel, dim3(1), dim3(1), 0, s, ctl, dim, first_dir, strang, f0, f1,
                      f2, (dx && use_floor) ? 1 : 0);
-  FVS_LAUNCH_CHECK();
-  return FVS_OK;
-}
-
-int LaunchCheckValue(hipStream_t s, Ctl* ctl, const double* value) {
-  hipLaunchKernelGGL(CheckValueKernel, dim3(1), dim3(1), 0, s, ctl, value);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }

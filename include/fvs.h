@@ -249,10 +249,10 @@ typedef struct fvs_patch_desc {
 typedef struct fvs_level fvs_level;
 
 /* Allocates the level's three state buffers and its device control block and
- * uploads nothing.  The state starts zeroed.  HLLEM (with MUSCL-Hancock or
- * first order) and first-order exact Godunov run the fused sweep kernels.
- * The other methods (MUSCL-Hancock over exact Godunov, the reference's
- * default MusclHancockMethod; the HLL base; MusclHancockPrim;
+ * uploads nothing.  The state starts zeroed.  HLLEM and exact Godunov, first
+ * order or with MUSCL-Hancock (over exact Godunov the reference's default
+ * MusclHancockMethod, in FP64 whatever the precision field says), run the
+ * fused sweep kernels.  The other methods (the HLL base; MusclHancockPrim;
  * MusclHancockCharacteristic) get a level composed from the patch operators
  * above on one ghosted scratch of complete states, in the same sequence and
  * with the same results as the reference's level integrator; it synchronises
@@ -263,7 +263,8 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch,
                      fvs_level** out);
 int fvs_level_destroy(fvs_level* level);
 /* Device pointer of component c of the current state (valid until the next
- * advance call); NULL for a composed level. */
+ * advance call); NULL for a composed level and for MUSCL-Hancock over exact
+ * Godunov (fvs_level_get_state serves both). */
 double* fvs_level_state(fvs_level* level, int c);
 /* Copies D+2 component arrays (device memory, ncell each) into the current
  * state; resets time and cycle count to (t0, 0). */

@@ -9,8 +9,8 @@
 // v_mfma_f32_16x16x16_bf16.  Activations are kept transposed (hidden units x
 // faces) so that a layer's 16x16 accumulator tile has exactly the lane and
 // element layout of the next layer's B operand (no data movement between
-// layers).  Training (forward, backward, Adam) is FP32 on the VALU; labels
-// come from the FP64 Newton iteration itself.  The Newton iteration that
+// layers).  Training (forward, backward, Adam) is FP32 throughout, its
+// products on the matrix cores' FP32 instruction; labels come from the FP64 Newton iteration itself.  The Newton iteration that
 // refines the guess is unchanged (include/fub/NewtonIteration.hpp:28-52).
 #include "fvs_internal.hpp"
 #include "fvs_mlp_infer.hpp"
@@ -207,12 +207,9 @@ __global__ __launch_bounds__(kBlock) void MlpSampleKernel(int64_t n, uint64_t se
   target[i] = static_cast<float>(log(ms.pM) - 0.5 * (log(pL) + log(pR)));
 }
 
-// FP32 forward of one sample per thread; stores activations for backward.
-// x: 6 x n, h1/h2: 64 x n, y: n.
+// FP32 forward of one sample per thread.  x: 6 x n, y: n.
 __global__ __launch_bounds__(kBlock) void MlpForwardKernel(const float* __restrict__ p,
                                                            const float* __restrict__ x, int64_t n,
-                                                           float* __restrict__ h1,
-                                                           float* __restrict__ h2,
                                                            float* __restrict__ y) {
   __shared__ float sp[kNParams];
   for (int k = threadIdx.x; k < kNParams; k += kBlock) sp[k] = p[k];
@@ -226,123 +223,239 @@ __global__ __launch_bounds__(kBlock) void MlpForwardKernel(const float* __restri
     float s = sp[kOffB1 + o];
     for (int k = 0; k < kIn; ++k) s += sp[kOffW1 + o * kInPad + k] * xi[k];
     a1[o] = fmaxf(s, 0.0f);
-    if (h1) h1[o * n + i] = a1[o];
   }
   float out = sp[kOffB3];
   for (int o = 0; o < kH; ++o) {
     float s = sp[kOffB2 + o];
     for (int k = 0; k < kH; ++k) s += sp[kOffW2 + o * kH + k] * a1[k];
     const float a2 = fmaxf(s, 0.0f);
-    if (h2) h2[o * n + i] = a2;
     out += sp[kOffW3 + o] * a2;
   }
   y[i] = out;
 }
 
-// Backward part 1 (per sample): loss e^2 (or the Huber form 2 h |e| - h^2
-// beyond |e| > h when huber h > 0) over valid samples, e = y - t;
-// dy = 2 clamp(e, -h, h) / N (mask 0 otherwise), dh2 = dy W3 [h2 > 0],
-// dh1 = W2^T dh2 [h1 > 0] (ReLU derivative).
-// dh2 / dh1 overwrite h2 / h1's storage in separate arrays.
-__global__ __launch_bounds__(kBlock) void MlpBackwardSamples(
-    const float* __restrict__ p, const float* __restrict__ y, const float* __restrict__ t,
-    const int* __restrict__ flag, int64_t n, float inv_count, float huber,
-    const float* __restrict__ h1,
-    const float* __restrict__ h2, float* __restrict__ dy, float* __restrict__ dh1,
-    float* __restrict__ dh2, float* __restrict__ loss) {
-  __shared__ float sp[kNParams];
-  __shared__ float sl[kBlock / 64];
-  for (int k = threadIdx.x; k < kNParams; k += kBlock) sp[k] = p[k];
-  __syncthreads();
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  float li = 0.0f;
-  if (i < n) {
-    const bool ok = flag[i] == 0;
-    const float e = ok ? (y[i] - t[i]) : 0.0f;
-    const float ae = fabsf(e);
-    const bool quad = !(huber > 0.0f) || ae <= huber;
-    li = (quad ? e * e : 2.0f * huber * ae - huber * huber) * inv_count;
-    const float ec = quad ? e : copysignf(huber, e);
-    const float d = 2.0f * ec * inv_count;
-    dy[i] = d;
-    float g2[kH];
-    for (int o = 0; o < kH; ++o) {
-      const float a = h2[o * n + i];
-      g2[o] = a > 0.0f ? d * sp[kOffW3 + o] : 0.0f;
-      dh2[o * n + i] = g2[o];
+// Loss and parameter gradients of a batch on the matrix cores, in FP32
+// (v_mfma_f32_16x16x4_f32: FP32 operands, products and sums).
+//
+// A workgroup takes tiles of 16 samples, its four waves 16 hidden units each:
+//   H1 = relu(W1 X + b1), H2 = relu(W2 H1 + b2), y = W3 H2 + b3,
+//   loss e^2 (or the Huber form 2 h |e| - h^2 beyond |e| > h when huber h > 0)
+//   over samples with flag 0, e = y - t, dy = 2 clamp(e, -h, h) inv_count,
+//   dH2 = W3 dy [H2 > 0], dH1 = W2^T dH2 [H1 > 0],
+//   gradients dW2 = dH2 H1^T, dW1 = dH1 X^T, biases and dW3 the row sums.
+// The parameters sit in LDS and activations pass between the waves through
+// it; the gradient tiles stay in accumulators over the workgroup's tiles and
+// leave as one partial vector (part[block][kNParams]) that MlpReduceKernel
+// sums in a fixed order, so training is deterministic.
+//
+// Operand layouts of the 16x16x4 product: A[i][k] and B[k][j] one value a
+// lane (i or j = lane % 16, k = lane / 16), D[i][j] in lane j + 16 (i / 4),
+// element i % 4.  The order of the summation index is free: step s of a
+// 64-long sum takes index 16 k + s, so that LDS rows of 17 (and 65) floats are
+// read without bank conflicts.
+//
+// A batch of 1,024 is 64 workgroups of 13 MFLOP together: latency bound.
+// Three kernels of one sample (or one parameter) a thread, four and sixteen
+// workgroups, took 41 + 87 + 145 us here; this one and the reduction take
+// 11 + 3 us, and an epoch over 2^17 pairs 35.2 -> 2.6 ms with its data
+// generation.
+constexpr int kTile = 16;         // samples per tile
+constexpr int kActStride = 17;    // LDS floats per activation row
+constexpr int kW2Stride = 65;
+constexpr int kGradBlocks = 512;  // most workgroups (partial vectors)
+
+__device__ __forceinline__ floatx4_t MfmaF32(float a, float b, floatx4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float RowSum16(float v) {  // over the 16 lanes of a row
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+__global__ __launch_bounds__(kBlock) void MlpGradKernel(
+    const float* __restrict__ p, const float* __restrict__ x, const float* __restrict__ t,
+    const int* __restrict__ flag, int64_t n, const uint32_t* __restrict__ idx, int64_t nb,
+    float inv_count, float huber, float* __restrict__ part, float* __restrict__ loss_part) {
+  __shared__ float s_w1[kH * 9], s_w2[kH * kW2Stride], s_b1[kH], s_b2[kH], s_w3[kH];
+  __shared__ float s_x[kInPad][kActStride];
+  __shared__ float s_h1[kH][kActStride], s_d2[kH][kActStride], s_d1[kH][kActStride];
+  __shared__ float s_y[4][kTile], s_dy[kTile], s_t[kTile];
+  __shared__ int s_ok[kTile];
+  for (int k = threadIdx.x; k < kH * kInPad; k += kBlock)
+    s_w1[(k / kInPad) * 9 + k % kInPad] = p[kOffW1 + k];
+  for (int k = threadIdx.x; k < kH * kH; k += kBlock)
+    s_w2[(k / kH) * kW2Stride + k % kH] = p[kOffW2 + k];
+  if (threadIdx.x < kH) {
+    s_b1[threadIdx.x] = p[kOffB1 + threadIdx.x];
+    s_b2[threadIdx.x] = p[kOffB2 + threadIdx.x];
+    s_w3[threadIdx.x] = p[kOffW3 + threadIdx.x];
+  }
+  const float b3 = p[kOffB3];
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;  // this wave's hidden units 16 w .. 16 w + 15
+  const int q = lane >> 4, j = lane & 15;
+  const int row = 16 * w + 4 * q;  // accumulator rows row .. row + 3, column j
+  floatx4_t g_w2[4] = {}, g_w1 = {};
+  float g_b2[4] = {}, g_w3[4] = {}, loss = 0.0f, g_b3 = 0.0f;
+  const int64_t tiles = (nb + kTile - 1) / kTile;
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    __syncthreads();  // parameters staged; the last tile's readers are done
+    if (threadIdx.x < kTile * kInPad) {
+      // features 0..5, then a row of ones (its products are the bias sums)
+      const int k = threadIdx.x / kTile, c = threadIdx.x % kTile;
+      const int64_t i = tile * kTile + c;
+      float v = 0.0f;
+      if (i < nb) {
+        const int64_t at = idx ? static_cast<int64_t>(idx[i]) : i;
+        v = k < kIn ? x[k * n + at] : (k == kIn ? 1.0f : 0.0f);
+        if (k == 0) {
+          s_t[c] = t[at];
+          s_ok[c] = flag[at] == 0;
+        }
+      } else if (k == 0) {
+        s_ok[c] = 0;  // no sample
+      }
+      s_x[k][c] = v;
     }
-    for (int k = 0; k < kH; ++k) {
-      float s = 0.0f;
-      for (int o = 0; o < kH; ++o) s += sp[kOffW2 + o * kH + k] * g2[o];
-      const float a = h1[k * n + i];
-      dh1[k * n + i] = a > 0.0f ? s : 0.0f;
+    __syncthreads();
+    // H1: two steps of the 8 inputs (row 6 of X is not an input: W1's padding
+    // columns are zero)
+    floatx4_t h1 = {s_b1[row], s_b1[row + 1], s_b1[row + 2], s_b1[row + 3]};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = 2 * q + s;
+      h1 = MfmaF32(s_w1[(16 * w + j) * 9 + k], s_x[k][j], h1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      h1[r] = Relu(h1[r]);
+      s_h1[row + r][j] = h1[r];
+    }
+    __syncthreads();
+    floatx4_t h2 = {s_b2[row], s_b2[row + 1], s_b2[row + 2], s_b2[row + 3]};
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      h2 = MfmaF32(s_w2[(16 * w + j) * kW2Stride + 16 * q + s], s_h1[16 * q + s][j], h2);
+    float out = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      h2[r] = Relu(h2[r]);
+      out += s_w3[row + r] * h2[r];
+    }
+    out += __shfl_xor(out, 16, 64);
+    out += __shfl_xor(out, 32, 64);
+    if (q == 0) s_y[w][j] = out;
+    __syncthreads();
+    if (threadIdx.x < kTile) {
+      const float y = ((s_y[0][threadIdx.x] + s_y[1][threadIdx.x]) +
+                       (s_y[2][threadIdx.x] + s_y[3][threadIdx.x])) + b3;
+      const float e = s_ok[threadIdx.x] ? y - s_t[threadIdx.x] : 0.0f;
+      const float ae = fabsf(e);
+      const bool quad = !(huber > 0.0f) || ae <= huber;
+      loss += (quad ? e * e : 2.0f * huber * ae - huber * huber) * inv_count;
+      const float d = 2.0f * (quad ? e : copysignf(huber, e)) * inv_count;
+      s_dy[threadIdx.x] = d;
+      g_b3 += d;
+    }
+    __syncthreads();
+    const float dy = s_dy[j];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float d2 = h2[r] > 0.0f ? dy * s_w3[row + r] : 0.0f;
+      s_d2[row + r][j] = d2;
+      g_b2[r] += d2;
+      g_w3[r] += dy * h2[r];
+    }
+    __syncthreads();
+    floatx4_t d1 = {};
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      d1 = MfmaF32(s_w2[(16 * q + s) * kW2Stride + 16 * w + j], s_d2[16 * q + s][j], d1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s_d1[row + r][j] = h1[r] > 0.0f ? d1[r] : 0.0f;
+    // sums over the tile's samples (index 4 s + q)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float a2 = s_d2[16 * w + j][4 * s + q];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) g_w2[m] = MfmaF32(a2, s_h1[16 * m + j][4 * s + q], g_w2[m]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // this wave's own rows of dH1
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      g_w1 = MfmaF32(s_d1[16 * w + j][4 * s + q], s_x[j & 7][4 * s + q], g_w1);
+  }
+  float* out = part + static_cast<int64_t>(blockIdx.x) * kNParams;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (j < kInPad) {
+      const float v = g_w1[r];
+      out[kOffW1 + (row + r) * kInPad + j] = j < kIn ? v : 0.0f;
+      if (j == kIn) out[kOffB1 + row + r] = v;
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) out[kOffW2 + (row + r) * kH + 16 * m + j] = g_w2[m][r];
+    const float b2 = RowSum16(g_b2[r]), w3 = RowSum16(g_w3[r]);
+    if (j == 0) {
+      out[kOffB2 + row + r] = b2;
+      out[kOffW3 + row + r] = w3;
     }
   }
-  for (int off = 32; off > 0; off >>= 1) li += __shfl_xor(li, off, 64);
-  if ((threadIdx.x & 63) == 0) sl[threadIdx.x >> 6] = li;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, sl[0] + sl[1] + sl[2] + sl[3]);
-}
-
-// Backward part 2: parameter gradients as reductions over the samples of a
-// chunk; one workgroup per chunk adds its partial sums to grad (FP32).
-// Thread t handles parameters t, t + 256, ...
-__global__ __launch_bounds__(kBlock) void MlpWeightGrads(
-    const float* __restrict__ x, const float* __restrict__ h1, const float* __restrict__ h2,
-    const float* __restrict__ dy, const float* __restrict__ dh1, const float* __restrict__ dh2,
-    int64_t n, int64_t chunk, float* __restrict__ grad) {
-  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;
-  const int64_t b1 = (b0 + chunk < n) ? b0 + chunk : n;
-  for (int k = threadIdx.x; k < kNParams; k += kBlock) {
-    float s = 0.0f;
-    if (k < kOffB1) {
-      const int o = k / kInPad, in = k % kInPad;
-      if (in < kIn)
-        for (int64_t b = b0; b < b1; ++b) s += dh1[o * n + b] * x[in * n + b];
-    } else if (k < kOffW2) {
-      const int o = k - kOffB1;
-      for (int64_t b = b0; b < b1; ++b) s += dh1[o * n + b];
-    } else if (k < kOffB2) {
-      const int o = (k - kOffW2) / kH, in = (k - kOffW2) % kH;
-      for (int64_t b = b0; b < b1; ++b) s += dh2[o * n + b] * h1[in * n + b];
-    } else if (k < kOffW3) {
-      const int o = k - kOffB2;
-      for (int64_t b = b0; b < b1; ++b) s += dh2[o * n + b];
-    } else if (k < kOffB3) {
-      const int o = k - kOffW3;
-      for (int64_t b = b0; b < b1; ++b) s += dy[b] * h2[o * n + b];
-    } else {
-      for (int64_t b = b0; b < b1; ++b) s += dy[b];
+  if (w == 0) {
+    loss = RowSum16(loss);
+    g_b3 = RowSum16(g_b3);
+    if (lane == 0) {
+      out[kOffB3] = g_b3;
+      loss_part[blockIdx.x] = loss;
     }
-    atomicAdd(&grad[k], s);
   }
 }
 
-__global__ void MlpAdamKernel(float* __restrict__ p, const float* __restrict__ grad,
-                              float* __restrict__ m, float* __restrict__ v, float lr, float b1,
-                              float b2, float eps, float bc1, float bc2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= kNParams) return;
-  if (k < kOffB1 && (k % kInPad) >= kIn) return;  // padding columns stay zero
-  const float gk = grad[k];
-  m[k] = b1 * m[k] + (1.0f - b1) * gk;
-  v[k] = b2 * v[k] + (1.0f - b2) * gk * gk;
-  const float mh = m[k] / bc1, vh = v[k] / bc2;
-  p[k] -= lr * mh / (sqrtf(vh) + eps);
-}
+// Adam's update (p null: none).
+struct AdamStep {
+  float lr, b1, b2, eps, bc1, bc2;
+  float *p, *m, *v;
+};
 
-// Gathers a minibatch (indices idx) of features / targets / flags.
-__global__ void MlpGatherKernel(const float* __restrict__ x, const float* __restrict__ t,
-                                const int* __restrict__ flag, int64_t n,
-                                const int64_t* __restrict__ idx, int64_t nb,
-                                float* __restrict__ xb, float* __restrict__ tb,
-                                int* __restrict__ fb) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  const int64_t j = idx[i];
-  for (int k = 0; k < kIn; ++k) xb[k * nb + i] = x[k * n + j];
-  tb[i] = t[j];
-  fb[i] = flag[j];
+// Sums the workgroups' partial gradients (and losses) in block order: 64
+// parameters a workgroup, each wave a quarter of the blocks; writes grad
+// (nullable) and the loss, and takes the Adam step (p nullable).
+__global__ __launch_bounds__(kBlock) void MlpReduceKernel(const float* __restrict__ part,
+                                                          const float* __restrict__ loss_part,
+                                                          int nblocks, float* grad, float* loss,
+                                                          AdamStep a) {
+  __shared__ float s_g[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
+  float g = 0.0f;
+  if (k < kNParams) {
+#pragma unroll 8
+    for (int b = w; b < nblocks; b += 4) g += part[static_cast<int64_t>(b) * kNParams + k];
+  }
+  s_g[w][lane] = g;
+  __syncthreads();
+  if (w == 0 && k < kNParams) {
+    g = (s_g[0][lane] + s_g[1][lane]) + (s_g[2][lane] + s_g[3][lane]);
+    if (grad) grad[k] = g;
+    // padding columns of W1 stay zero
+    if (a.p && !(k < kOffB1 && (k % kInPad) >= kIn)) {
+      const float m = a.b1 * a.m[k] + (1.0f - a.b1) * g;
+      const float v = a.b2 * a.v[k] + (1.0f - a.b2) * g * g;
+      a.m[k] = m;
+      a.v[k] = v;
+      const float mh = m / a.bc1, vh = v / a.bc2;
+      a.p[k] -= a.lr * mh / (sqrtf(vh) + a.eps);
+    }
+  }
+  if (blockIdx.x == 0 && w == 1) {
+    float l = 0.0f;
+    for (int b = lane; b < nblocks; b += 64) l += loss_part[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
+    if (lane == 0) *loss = l;
+  }
 }
 
 } // namespace
@@ -369,11 +482,8 @@ struct fvs_mlp {
   float* target;
   int* flag;
   int* iters;
-  // scratch for a minibatch
-  int64_t cap;
-  float *xb, *tb, *yb, *h1, *h2, *dy, *dh1, *dh2;
-  int* fb;
-  int64_t* idx;
+  float* part;       // partial gradients, kGradBlocks x kNParams
+  float* loss_part;  // kGradBlocks
 };
 
 namespace {
@@ -393,55 +503,18 @@ int Pack(fvs_mlp* m) {
   return FVS_OK;
 }
 
-void FreeBatch(fvs_mlp* m) {
-  void* ps[] = {m->xb, m->tb, m->yb, m->h1, m->h2, m->dy, m->dh1, m->dh2, m->fb, m->idx};
-  for (void* p : ps)
-    if (p) (void)hipFree(p);
-  m->xb = m->tb = m->yb = m->h1 = m->h2 = m->dy = m->dh1 = m->dh2 = nullptr;
-  m->fb = nullptr;
-  m->idx = nullptr;
-  m->cap = 0;
-}
-
-int EnsureBatch(fvs_mlp* m, int64_t nb) {
-  if (nb <= m->cap) return FVS_OK;
-  FVS_HIP_CHECK(hipStreamSynchronize(m->stream));
-  FreeBatch(m);
-  const size_t f = sizeof(float);
-  if (Alloc((void**)&m->xb, nb * kIn * f) || Alloc((void**)&m->tb, nb * f) ||
-      Alloc((void**)&m->yb, nb * f) || Alloc((void**)&m->h1, nb * kH * f) ||
-      Alloc((void**)&m->h2, nb * kH * f) || Alloc((void**)&m->dy, nb * f) ||
-      Alloc((void**)&m->dh1, nb * kH * f) || Alloc((void**)&m->dh2, nb * kH * f) ||
-      Alloc((void**)&m->fb, nb * sizeof(int)) || Alloc((void**)&m->idx, nb * sizeof(int64_t)))
-    return FVS_HIP_ERROR;
-  m->cap = nb;
-  return FVS_OK;
-}
-
-// Forward pass of one minibatch already gathered into xb/tb/fb (activations
-// kept for Backward); zeroes the gradient and loss accumulators.
-int Forward(fvs_mlp* m, int64_t nb) {
-  hipStream_t s = m->stream;
-  const unsigned blocks = unsigned((nb + kBlock - 1) / kBlock);
-  FVS_HIP_CHECK(hipMemsetAsync(m->grad, 0, kNParams * sizeof(float), s));
-  FVS_HIP_CHECK(hipMemsetAsync(m->loss, 0, sizeof(float), s));
-  hipLaunchKernelGGL(MlpForwardKernel, dim3(blocks), dim3(kBlock), 0, s, m->params, m->xb, nb,
-                     m->h1, m->h2, m->yb);
+// Partial gradients of a batch (idx nullable: samples 0 .. nb - 1) and their
+// reduction.  grad (nullable) and loss: device memory.
+int BatchGradients(fvs_mlp* m, const float* x, const float* t, const int* flag, int64_t n,
+                   const uint32_t* idx, int64_t nb, float inv_count, float huber, float* grad,
+                   float* loss, const AdamStep& adam) {
+  const int64_t tiles = (nb + kTile - 1) / kTile;
+  const int blocks = static_cast<int>(tiles < kGradBlocks ? tiles : kGradBlocks);
+  hipLaunchKernelGGL(MlpGradKernel, dim3(blocks), dim3(kBlock), 0, m->stream, m->params, x, t,
+                     flag, n, idx, nb, inv_count, huber, m->part, m->loss_part);
   FVS_LAUNCH_CHECK();
-  return FVS_OK;
-}
-
-int Backward(fvs_mlp* m, int64_t nb, float inv_count, float huber) {
-  hipStream_t s = m->stream;
-  const unsigned blocks = unsigned((nb + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(MlpBackwardSamples, dim3(blocks), dim3(kBlock), 0, s, m->params, m->yb,
-                     m->tb, m->fb, nb, inv_count, huber, m->h1, m->h2, m->dy, m->dh1, m->dh2,
-                     m->loss);
-  FVS_LAUNCH_CHECK();
-  const int64_t chunk = 64;
-  const unsigned gb = unsigned((nb + chunk - 1) / chunk);
-  hipLaunchKernelGGL(MlpWeightGrads, dim3(gb), dim3(kBlock), 0, s, m->xb, m->h1, m->h2, m->dy,
-                     m->dh1, m->dh2, nb, chunk, m->grad);
+  hipLaunchKernelGGL(MlpReduceKernel, dim3((kNParams + 63) / 64), dim3(kBlock), 0, m->stream,
+                     m->part, m->loss_part, blocks, grad, loss, adam);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }
@@ -507,6 +580,8 @@ int fvs_mlp_create(void* hip_stream, uint64_t seed, fvs_mlp** out) {
   if (Alloc((void**)&m->params, pb) || Alloc((void**)&m->adam_m, pb) ||
       Alloc((void**)&m->adam_v, pb) || Alloc((void**)&m->grad, pb) ||
       Alloc((void**)&m->loss, sizeof(float)) ||
+      Alloc((void**)&m->part, kGradBlocks * pb) ||
+      Alloc((void**)&m->loss_part, kGradBlocks * sizeof(float)) ||
       Alloc((void**)&m->tiles, kNTiles * kTileShorts * sizeof(short)) ||
       Alloc((void**)&m->bias, (2 * kH + 1) * sizeof(float))) {
     delete m;
@@ -537,8 +612,8 @@ int fvs_mlp_create(void* hip_stream, uint64_t seed, fvs_mlp** out) {
 int fvs_mlp_destroy(fvs_mlp* m) {
   if (!m) return FVS_OK;
   (void)hipStreamSynchronize(m->stream);
-  FreeBatch(m);
   void* ps[] = {m->params, m->adam_m, m->adam_v, m->grad, m->loss, m->tiles, m->bias,
+                m->part, m->loss_part,
                 m->prim, m->x, m->target, m->flag, m->iters};
   for (void* p : ps)
     if (p) (void)hipFree(p);
@@ -635,7 +710,7 @@ int fvs_mlp_forward(fvs_mlp* m, const float* x, int64_t n, float* y) {
     return FVS_BAD_ARGUMENT;
   }
   hipLaunchKernelGGL(MlpForwardKernel, dim3(unsigned((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     m->stream, m->params, x, n, nullptr, nullptr, y);
+                     m->stream, m->params, x, n, y);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }
@@ -649,17 +724,15 @@ int fvs_mlp_gradients(fvs_mlp* m, const float* x, const float* target, const int
     SetError("bad argument");
     return FVS_BAD_ARGUMENT;
   }
-  if (int rc = EnsureBatch(m, n)) return rc;
-  FVS_HIP_CHECK(hipMemcpyAsync(m->xb, x, n * kIn * sizeof(float), hipMemcpyDeviceToDevice, m->stream));
-  FVS_HIP_CHECK(hipMemcpyAsync(m->tb, target, n * sizeof(float), hipMemcpyDeviceToDevice, m->stream));
-  FVS_HIP_CHECK(hipMemcpyAsync(m->fb, flag, n * sizeof(int), hipMemcpyDeviceToDevice, m->stream));
   std::vector<int> f(n);
   FVS_HIP_CHECK(hipMemcpyAsync(f.data(), flag, n * sizeof(int), hipMemcpyDeviceToHost, m->stream));
   FVS_HIP_CHECK(hipStreamSynchronize(m->stream));
   int64_t valid = 0;
   for (int64_t i = 0; i < n; ++i) valid += (f[i] == 0);
-  if (int rc = Forward(m, n)) return rc;
-  if (int rc = Backward(m, n, valid > 0 ? 1.0f / float(valid) : 0.0f, huber)) return rc;
+  if (int rc = BatchGradients(m, x, target, flag, n, nullptr, n,
+                              valid > 0 ? 1.0f / float(valid) : 0.0f, huber, m->grad, m->loss,
+                              AdamStep{}))
+    return rc;
   if (grad_host)
     FVS_HIP_CHECK(hipMemcpyAsync(grad_host, m->grad, kNParams * sizeof(float),
                                  hipMemcpyDeviceToHost, m->stream));
@@ -680,84 +753,109 @@ int fvs_mlp_train(fvs_mlp* m, int epochs, int64_t batch, float lr, float huber, 
     SetError("bad argument (dataset generated?)");
     return FVS_BAD_ARGUMENT;
   }
-  if (int rc = EnsureBatch(m, batch)) return rc;
   const int64_t n = m->n;
   std::vector<int> flags(n);
   FVS_HIP_CHECK(hipMemcpyAsync(flags.data(), m->flag, n * sizeof(int), hipMemcpyDeviceToHost,
                                m->stream));
   FVS_HIP_CHECK(hipStreamSynchronize(m->stream));
-  std::vector<int64_t> valid;
+  // Sample indices fit 32 bits: 2^32 samples (84 bytes each) exceed the card.
+  std::vector<uint32_t> valid;
   valid.reserve(n);
   for (int64_t i = 0; i < n; ++i)
-    if (flags[i] == 0) valid.push_back(i);
+    if (flags[i] == 0) valid.push_back(static_cast<uint32_t>(i));
   const int64_t nv = static_cast<int64_t>(valid.size());
   if (nv < batch) {
     SetError("dataset has %lld valid samples, fewer than one batch", (long long)nv);
     return FVS_BAD_ARGUMENT;
   }
-  int64_t* perm = nullptr;
-  if (Alloc((void**)&perm, nv * sizeof(int64_t))) return FVS_HIP_ERROR;
-  uint64_t st = seed;
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const int64_t nbatches = nv / batch;
+  // Device: two epochs' permutations (the next one is shuffled and uploaded
+  // while an epoch runs) and the loss of every step; host: pinned staging.
+  uint32_t* perm = nullptr;
+  float* losses = nullptr;
+  uint32_t* stage = nullptr;
+  hipEvent_t uploaded[2] = {nullptr, nullptr};
+  const size_t pbytes = nv * sizeof(uint32_t);
+  const size_t nloss = static_cast<size_t>(epochs > 0 ? epochs : 1) * nbatches;
+  const int nbuf = epochs > 1 ? 2 : 1;
+  int rc = FVS_OK;
+  if (Alloc((void**)&perm, nbuf * pbytes) || Alloc((void**)&losses, nloss * sizeof(float)))
+    rc = FVS_HIP_ERROR;
+  if (rc == FVS_OK && epochs > 1) {
+    if (hipHostMalloc(&stage, nbuf * pbytes, hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&uploaded[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&uploaded[1], hipEventDisableTiming) != hipSuccess) {
+      SetError("training buffers failed");
+      rc = FVS_HIP_ERROR;
+    }
+  }
+  uint64_t st = seed;
+  AdamStep adam{};
+  adam.b1 = 0.9f;
+  adam.b2 = 0.999f;
+  adam.eps = 1e-8f;
+  adam.p = m->params;
+  adam.m = m->adam_m;
+  adam.v = m->adam_v;
   const double total = static_cast<double>(epochs) * static_cast<double>(nbatches);
   int64_t step = 0;
-  int rc = FVS_OK;
   for (int e = 0; e < epochs && rc == FVS_OK; ++e) {
     for (int64_t i = nv - 1; i > 0; --i) {
       const int64_t j = static_cast<int64_t>(HostSplitMix(st) % static_cast<uint64_t>(i + 1));
       std::swap(valid[i], valid[j]);
     }
-    // one upload of the epoch's permutation, complete before the host
-    // reshuffles (the previous epoch's gathers are done after the sync)
-    if (hipStreamSynchronize(m->stream) != hipSuccess ||
-        hipMemcpyAsync(perm, valid.data(), nv * sizeof(int64_t), hipMemcpyHostToDevice,
-                       m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess) {
+    const int buf = e % nbuf;
+    uint32_t* dst = perm + buf * nv;
+    const uint32_t* src = valid.data();
+    if (stage) {
+      // the staging buffer's upload of two epochs ago has left it
+      if (e >= 2 && hipEventSynchronize(uploaded[buf]) != hipSuccess) rc = FVS_HIP_ERROR;
+      std::memcpy(stage + buf * nv, valid.data(), pbytes);
+      src = stage + buf * nv;
+    }
+    if (rc != FVS_OK ||
+        hipMemcpyAsync(dst, src, pbytes, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+        (stage ? hipEventRecord(uploaded[buf], m->stream) : hipStreamSynchronize(m->stream)) !=
+            hipSuccess) {
       SetError("permutation upload failed");
       rc = FVS_HIP_ERROR;
       break;
     }
-    double loss_sum = 0.0;
-    for (int64_t b = 0; b < nbatches; ++b) {
-      hipLaunchKernelGGL(MlpGatherKernel, dim3(unsigned((batch + kBlock - 1) / kBlock)),
-                         dim3(kBlock), 0, m->stream, m->x, m->target, m->flag, n,
-                         perm + b * batch, batch, m->xb, m->tb, m->fb);
-      if (hipGetLastError() != hipSuccess) {
-        SetError("gather launch failed");
-        rc = FVS_HIP_ERROR;
-        break;
-      }
-      if ((rc = Forward(m, batch)) != FVS_OK) break;
-      if ((rc = Backward(m, batch, 1.0f / float(batch), huber)) != FVS_OK) break;
+    for (int64_t b = 0; b < nbatches && rc == FVS_OK; ++b) {
       m->adam_t += 1;
       step += 1;
-      const float bc1 = 1.0f - std::pow(b1, float(m->adam_t));
-      const float bc2 = 1.0f - std::pow(b2, float(m->adam_t));
-      const float lr_t =
+      adam.bc1 = 1.0f - std::pow(adam.b1, float(m->adam_t));
+      adam.bc2 = 1.0f - std::pow(adam.b2, float(m->adam_t));
+      adam.lr =
           static_cast<float>(lr * 0.5 * (1.0 + std::cos(3.141592653589793 * step / total)));
-      hipLaunchKernelGGL(MlpAdamKernel, dim3((kNParams + 255) / 256), dim3(256), 0, m->stream,
-                         m->params, m->grad, m->adam_m, m->adam_v, lr_t, b1, b2, eps, bc1, bc2);
-      if (hipGetLastError() != hipSuccess) {
-        SetError("adam launch failed");
-        rc = FVS_HIP_ERROR;
-        break;
-      }
-      if (loss_history && (b % 64 == 0 || b == nbatches - 1)) {
-        float l = 0.0f;
-        if (hipMemcpyAsync(&l, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream) !=
-                hipSuccess ||
-            hipStreamSynchronize(m->stream) != hipSuccess) {
-          rc = FVS_HIP_ERROR;
-          break;
-        }
-        loss_sum = (b == 0) ? l : 0.9 * loss_sum + 0.1 * l;
-      }
+      rc = BatchGradients(m, m->x, m->target, m->flag, n, dst + b * batch, batch,
+                          1.0f / float(batch), huber, nullptr, losses + e * nbatches + b, adam);
     }
-    if (loss_history) loss_history[e] = static_cast<float>(loss_sum);
+  }
+  if (rc == FVS_OK && loss_history && epochs > 0) {
+    std::vector<float> l(nloss);
+    if (hipMemcpyAsync(l.data(), losses, nloss * sizeof(float), hipMemcpyDeviceToHost,
+                       m->stream) != hipSuccess ||
+        hipStreamSynchronize(m->stream) != hipSuccess) {
+      SetError("loss readback failed");
+      rc = FVS_HIP_ERROR;
+    }
+    for (int e = 0; e < epochs && rc == FVS_OK; ++e) {
+      double smooth = 0.0;
+      for (int64_t b = 0; b < nbatches; ++b) {
+        if (b % 64 != 0 && b != nbatches - 1) continue;
+        const float v = l[e * nbatches + b];
+        smooth = (b == 0) ? v : 0.9 * smooth + 0.1 * v;
+      }
+      loss_history[e] = static_cast<float>(smooth);
+    }
   }
   (void)hipStreamSynchronize(m->stream);
-  (void)hipFree(perm);
+  if (perm) (void)hipFree(perm);
+  if (losses) (void)hipFree(losses);
+  if (stage) (void)hipHostFree(stage);
+  for (hipEvent_t ev : uploaded)
+    if (ev) (void)hipEventDestroy(ev);
   if (rc != FVS_OK) return rc;
   if (int rc = Pack(m)) return rc;
   FVS_HIP_CHECK(hipStreamSynchronize(m->stream));

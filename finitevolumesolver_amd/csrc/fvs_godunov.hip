@@ -558,16 +558,30 @@ __global__ __launch_bounds__(kRedBlock) void GodunovFinalize(const unsigned long
                                                              int64_t n, double* out,
                                                              unsigned long long* stats, Ctl* ctl,
                                                              int check) {
-  if (ctl && ctl->halt) return;
+  const int halt = ctl ? ctl->halt : 0;
+  const double split_dt = check ? ctl->split_dt : 0.0;
+  if (halt) return;
   p += 5 * n * blockIdx.x;
   __shared__ unsigned long long s[5][kRedBlock / 64];
   unsigned long long key = kInfKey, iters = 0, max_it = 0, fails = 0, faces = 0;
-  for (int64_t i = threadIdx.x; i < n; i += kRedBlock) {
-    key = KMin(key, p[5 * i]);
-    iters += p[5 * i + 1];
-    max_it = p[5 * i + 2] > max_it ? p[5 * i + 2] : max_it;
-    fails += p[5 * i + 3];
-    faces += p[5 * i + 4];
+  // two blocks' partials a thread and round, loaded unconditionally
+  for (int64_t i = threadIdx.x; i < n; i += 2 * kRedBlock) {
+    const int64_t i2 = i + kRedBlock < n ? i + kRedBlock : i;
+    unsigned long long v[2][5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      v[0][k] = p[5 * i + k];
+      v[1][k] = p[5 * i2 + k];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (u == 1 && i2 == i) break;
+      key = KMin(key, v[u][0]);
+      iters += v[u][1];
+      max_it = v[u][2] > max_it ? v[u][2] : max_it;
+      fails += v[u][3];
+      faces += v[u][4];
+    }
   }
   key = WaveMinKey(key);
   iters = WaveSum(iters);
@@ -601,7 +615,7 @@ __global__ __launch_bounds__(kRedBlock) void GodunovFinalize(const unsigned long
     atomicAdd(&stats[3], faces & 0xffffffffull);
     atomicAdd(&stats[4], faces >> 32);
   }
-  if (check && v < ctl->split_dt) {
+  if (check && v < split_dt) {
     // TimeStepTooLarge{level_dt} (DimensionalSplitLevelIntegrator.hpp:243-245)
     ctl->halt = 1;
     ctl->failure_dt = v;

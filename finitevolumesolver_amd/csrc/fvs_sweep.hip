@@ -787,26 +787,19 @@ __device__ __forceinline__ double KeyToDt(unsigned long long k) {
   return __longlong_as_double(static_cast<long long>(k));
 }
 
-__device__ unsigned long long ReduceKeys(const unsigned long long* p, int64_t n) {
-  __shared__ unsigned long long s[kRedBlock / 64];
-  unsigned long long k = kInfKey;
-  for (int64_t i = threadIdx.x; i < n; i += kRedBlock) k = KMin(k, p[i]);
-  k = WaveMinKey(k);
-  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = k;
-  __syncthreads();
-  unsigned long long r = s[0];
-  for (int w = 1; w < kRedBlock / 64; ++w) r = KMin(r, s[w]);
-  __syncthreads();
-  return r;
-}
-
 // Minima of up to N key arrays (array r: p[r * stride .. + n[r]]) in one
-// pass, every thread's loads of all arrays in flight together; out[r] for
-// r < count.  Every thread of the block must call it.
+// pass; out[r] for r < count.  Every thread of the block must call it.  A
+// thread's loads of a round (four per array) are unconditional, with the index
+// clamped instead of a branch around the load, so they are all in flight
+// together: the kernel is a chain of memory latencies and nothing else, and a
+// branch per load had made that chain ten loads long (16 to 20 us for the
+// checks of a step, 6 to 9 now).
 template <int N>
-__device__ void ReduceKeysMulti(const unsigned long long* p, int64_t stride, const int64_t* n,
-                                int count, unsigned long long* out) {
+__device__ __forceinline__ void ReduceKeysMulti(const unsigned long long* p, int64_t stride,
+                                                const int64_t* n, int count,
+                                                unsigned long long* out) {
   __shared__ unsigned long long s[N][kRedBlock / 64];
+  constexpr int kUnroll = 4;
   unsigned long long k[N];
   int64_t nmax = 0;
 #pragma unroll
@@ -814,11 +807,24 @@ __device__ void ReduceKeysMulti(const unsigned long long* p, int64_t stride, con
     k[r] = kInfKey;
     if (r < count && n[r] > nmax) nmax = n[r];
   }
-#pragma unroll 4
-  for (int64_t i = threadIdx.x; i < nmax; i += kRedBlock) {
+  for (int64_t i = threadIdx.x; i < nmax; i += kUnroll * kRedBlock) {
+    unsigned long long v[N][kUnroll];
 #pragma unroll
-    for (int r = 0; r < N; ++r)
-      if (r < count && i < n[r]) k[r] = KMin(k[r], p[r * stride + i]);
+    for (int r = 0; r < N; ++r) {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const int64_t at = i + u * kRedBlock;
+        v[r][u] = p[(r < count && at < n[r]) ? r * stride + at : 0];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const bool valid = r < count && i + u * kRedBlock < n[r];
+        k[r] = KMin(k[r], valid ? v[r][u] : kInfKey);
+      }
+    }
   }
 #pragma unroll
   for (int r = 0; r < N; ++r) {
@@ -832,18 +838,22 @@ __device__ void ReduceKeysMulti(const unsigned long long* p, int64_t stride, con
     for (int w = 1; w < kRedBlock / 64; ++w) m = KMin(m, s[r][w]);
     out[r] = m;
   }
-  __syncthreads();
 }
 
 __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
     const unsigned long long* partials, int64_t n, double* out, Ctl* ctl) {
-  if (ctl && ctl->halt) return;
-  const double v = KeyToDt(ReduceKeys(partials, n));
+  // control words read ahead of the reduction, not after it
+  const int halt = ctl ? ctl->halt : 0;
+  const double split_dt = ctl ? ctl->split_dt : 0.0;
+  if (halt) return;
+  unsigned long long key;
+  ReduceKeysMulti<1>(partials, 0, &n, 1, &key);
+  const double v = KeyToDt(key);
   if (threadIdx.x == 0) {
     if (out) *out = v;
     if (ctl) {
       ctl->last_check = v;
-      if (v < ctl->split_dt) {
+      if (v < split_dt) {
         // TimeStepTooLarge{level_dt} (DimensionalSplitLevelIntegrator.hpp:243-245)
         ctl->halt = 1;
         ctl->failure_dt = v;
@@ -857,14 +867,16 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
 // a floor (halt 3) and the margin quadruples; otherwise the next floor is
 // this pass's largest speed per direction (dx / dt) less a margin that
 // follows how fast that speed falls.  Returns false after setting halt 3.
-__device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, int dim) {
+__device__ __forceinline__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, int dim) {
   bool floor_ok = true;
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (ctl->cfl_floor[d] > 0.0 && !ctl->floor_hit[d]) floor_ok = false;
     ctl->floor_hit[d] = 0;
   }
   const double old_margin = ctl->floor_margin > 0.0 ? ctl->floor_margin : kFloorMarginFirst;
   if (!floor_ok) {
+#pragma unroll
     for (int d = 0; d < 3; ++d) ctl->cfl_floor[d] = 0.0;
     ctl->floor_margin = fmin(4.0 * old_margin, kFloorMarginMax);
     // the last pass's floor: the next one comes from the cells; that too: none
@@ -874,7 +886,9 @@ __device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, in
   }
   ctl->floor_known = 1;
   double speed[3] = {0.0, 0.0, 0.0}, drop = 0.0;
-  for (int d = 0; d < dim; ++d) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= dim) break;
     speed[d] = fdx[d] / v[d];
     if (ctl->floor_speed[d] > 0.0 && speed[d] > 0.0)
       drop = fmax(drop, (ctl->floor_speed[d] - speed[d]) / speed[d]);
@@ -882,6 +896,7 @@ __device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, in
   const double margin =
       fmin(kFloorMarginMax, fmax(fmax(kFloorMarginMin, 4.0 * drop), 0.5 * old_margin));
   ctl->floor_margin = margin;
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
     const double f = speed[d] * (1.0 - margin);
     const bool finite = d < dim && f > 0.0 && f < 1.7976931348623157e308;
@@ -891,35 +906,19 @@ __device__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, in
   return true;
 }
 
-// With use_floor (the level's 3D pass, fdx the cell widths), the floor of
-// the pass is validated first and the next step's floor set from this pass's
-// largest speeds.
-__global__ __launch_bounds__(kRedBlock) void FinalizeCflKernel(
-    const unsigned long long* partials, int64_t n, int dim, double* out, Ctl* ctl,
-    int first_dir, int strang, double fdx0, double fdx1, double fdx2, int use_floor) {
-  if (ctl && ctl->halt) return;
-  double v[3];
-  {
-    const int64_t ns[3] = {n, n, n};
-    unsigned long long keys[3];
-    ReduceKeysMulti<3>(partials, n, ns, dim, keys);
-    for (int d = 0; d < dim; ++d) v[d] = KeyToDt(keys[d]);
-  }
-  if (threadIdx.x != 0) return;
-  if (out) {
-    for (int d = 0; d < dim; ++d) out[d] = v[d];
-  }
-  if (!ctl) return;
-  if (use_floor) {
-    const double fdx[3] = {fdx0, fdx1, fdx2};
-    if (!RenewSpeedFloor(ctl, v, fdx, dim)) return;
-  }
+// The step's dt and split dt from the directions' stable dts, with the first
+// split step's CFL check.
+__device__ __forceinline__ void SetStepDt(Ctl* ctl, const double* v, int dim, int first_dir,
+                                          int strang) {
   // DimensionalSplitLevelIntegrator::ComputeStableDt (:204-219) starts from
   // DBL_MAX; RunSimulation's limited_dt (RunSimulation.hpp:121-131).
-  double stable = 1.7976931348623157e308;
-  for (int d = 0; d < dim; ++d) {
+  double stable = 1.7976931348623157e308, first = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= dim) break;
     ctl->dt_dir[d] = v[d];
     stable = (v[d] < stable) ? v[d] : stable;
+    if (d == first_dir) first = v[d];
   }
   if (!(ctl->t + ctl->eps < ctl->final_time)) {
     ctl->halt = 2;
@@ -933,7 +932,6 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCflKernel(
   ctl->split_dt = strang ? 0.5 * dt : dt;
   // The first sweep's CFL check is the step-start stable dt of its
   // direction: the same faces of the same state.
-  const double first = v[first_dir];
   ctl->last_check = first;
   if (first < ctl->split_dt) {
     ctl->halt = 1;
@@ -941,33 +939,57 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCflKernel(
   }
 }
 
+// With use_floor (the level's 3D pass, fdx the cell widths), the floor of
+// the pass is validated first and the next step's floor set from this pass's
+// largest speeds.
+__global__ __launch_bounds__(kRedBlock) void FinalizeCflKernel(
+    const unsigned long long* partials, int64_t n, int dim, double* out, Ctl* ctl,
+    int first_dir, int strang, double fdx0, double fdx1, double fdx2, int use_floor) {
+  // A copy of the control block, read ahead of the reduction.
+  Ctl c;
+  if (ctl) c = *ctl;
+  if (ctl && c.halt) return;
+  double v[3];
+  {
+    const int64_t ns[3] = {n, n, n};
+    unsigned long long keys[3];
+    ReduceKeysMulti<3>(partials, n, ns, dim, keys);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) v[d] = KeyToDt(keys[d]);
+  }
+  if (threadIdx.x != 0) return;
+  if (out) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (d < dim) out[d] = v[d];
+  }
+  if (!ctl) return;
+  if (use_floor) {
+    const double fdx[3] = {fdx0, fdx1, fdx2};
+    if (!RenewSpeedFloor(&c, v, fdx, dim)) {
+      *ctl = c;
+      return;
+    }
+  }
+  SetStepDt(&c, v, dim, first_dir, strang);
+  *ctl = c;
+}
+
 // Step dt from per-direction stable dts already in ctl->dt_dir (used by
 // methods whose CFL pass reduces into ctl->dt_dir itself).
 __global__ void StepDtKernel(Ctl* ctl, int dim, int first_dir, int strang, double fdx0,
                              double fdx1, double fdx2, int use_floor) {
-  if (ctl->halt) return;
+  Ctl c = *ctl;
+  if (c.halt) return;
   if (use_floor) {
     const double fdx[3] = {fdx0, fdx1, fdx2};
-    if (!RenewSpeedFloor(ctl, ctl->dt_dir, fdx, dim)) return;
+    if (!RenewSpeedFloor(&c, c.dt_dir, fdx, dim)) {
+      *ctl = c;
+      return;
+    }
   }
-  double stable = 1.7976931348623157e308;
-  for (int d = 0; d < dim; ++d) stable = (ctl->dt_dir[d] < stable) ? ctl->dt_dir[d] : stable;
-  if (!(ctl->t + ctl->eps < ctl->final_time)) {
-    ctl->halt = 2;
-    return;
-  }
-  const double sdt = ctl->have_failure ? ctl->failure_dt : stable;
-  const double rem = ctl->final_time - ctl->t;
-  const double cdt = ctl->cfl * sdt;
-  const double dt = (cdt < rem) ? cdt : rem;
-  ctl->dt = dt;
-  ctl->split_dt = strang ? 0.5 * dt : dt;
-  const double first = ctl->dt_dir[first_dir];
-  ctl->last_check = first;
-  if (first < ctl->split_dt) {
-    ctl->halt = 1;
-    ctl->failure_dt = first;
-  }
+  SetStepDt(&c, c.dt_dir, dim, first_dir, strang);
+  *ctl = c;
 }
 
 __device__ __forceinline__ void EndStep(Ctl* ctl) {
@@ -990,23 +1012,37 @@ __global__ void StepEndKernel(Ctl* ctl) {
 // and a step-end kernel.
 __global__ __launch_bounds__(kRedBlock) void FinalizeStepKernel(
     const unsigned long long* partials, CheckList cl, Ctl* ctl) {
-  if (ctl->halt) return;
+  // control words read ahead of the reduction, not after it
+  const int halt = ctl->halt;
+  const double split_dt = ctl->split_dt, dt = ctl->dt, t = ctl->t;
+  const int64_t cycle = ctl->cycle, log_base = ctl->dt_log_base, log_len = ctl->dt_log_len;
+  double* log = ctl->dt_log;
+  if (halt) return;
   unsigned long long keys[kMaxChecks];
   ReduceKeysMulti<kMaxChecks>(partials, cl.stride, cl.n, cl.count, keys);
-  for (int r = 0; r < cl.count; ++r) {
+  if (threadIdx.x != 0) return;
+  double last = 0.0;
+  bool fail = false;
+#pragma unroll
+  for (int r = 0; r < kMaxChecks; ++r) {
     const double v = KeyToDt(keys[r]);
-    const bool fail = v < ctl->split_dt;
-    if (threadIdx.x == 0) {
-      ctl->last_check = v;
-      if (fail) {
-        // TimeStepTooLarge{level_dt} (DimensionalSplitLevelIntegrator.hpp:243-245)
-        ctl->halt = 1;
-        ctl->failure_dt = v;
-      }
+    if (r < cl.count && !fail) {
+      last = v;
+      fail = v < split_dt;
     }
-    if (fail) return;
   }
-  if (threadIdx.x == 0) EndStep(ctl);
+  if (cl.count > 0) ctl->last_check = last;
+  if (fail) {
+    // TimeStepTooLarge{level_dt} (DimensionalSplitLevelIntegrator.hpp:243-245)
+    ctl->halt = 1;
+    ctl->failure_dt = last;
+    return;
+  }
+  const int64_t slot = cycle - log_base;
+  if (log && slot >= 0 && slot < log_len) log[slot] = dt;
+  ctl->t = t + dt;
+  ctl->cycle = cycle + 1;
+  ctl->have_failure = 0;
 }
 
 __global__ void KeysToDtKernel(unsigned long long* keys, int n, double* out) {

@@ -33,6 +33,8 @@
 #include "fvs_physics.hpp"
 #include "fvs_xslots.hpp"
 
+#include <type_traits>
+
 namespace fvs {
 
 namespace {
@@ -257,11 +259,12 @@ template <class T> __device__ __forceinline__ Gas<T> MakeGas(const SweepArgs& a)
 // flight behind its FP64 work; no LDS, no barrier until the final CFL
 // reduction.
 template <int D, bool LARR, class T, bool FAST>
-__global__ __launch_bounds__(kBlock) void SweepXKernel(SweepArgs a) {
+__global__ __launch_bounds__(kBlock, FAST ? 1 : 3) void SweepXKernel(SweepArgs a) {
   using TA = typename Policies<T, FAST>::TA;
   using DA = typename Policies<T, FAST>::DA;
   constexpr int NC = D + 2;
   constexpr int NQ = D + 4;
+  constexpr bool kIeee = !FAST && std::is_same<T, double>::value;
   if (a.halt && *a.halt) return;
   const int64_t nx = a.n[0];
   const uint32_t S = static_cast<uint32_t>(nx + 2);
@@ -338,9 +341,14 @@ __global__ __launch_bounds__(kBlock) void SweepXKernel(SweepArgs a) {
       }
     }
 
-    T recL[NQ], recR[NQ];
-    typename TA::Inv irL, irR;
-    {
+    // Face sl - 1 (left face of the slot's cell) for slots 1 .. nx + 1.
+    const bool face_lane = cur.valid && lane >= 2 && lane <= 2 + kXOwned && cur.sl >= 1;
+    T F[NC];
+    // Half-step states and face flux in arithmetic P, by the whole wave.
+    auto flux = [&](auto policy) {
+      using P = decltype(policy);
+      T recL[NQ], recR[NQ], recRprev[NQ];
+      typename P::Inv irL, irR, irRprev;
       T tm[NC], t0[NC], tp[NC];
 #pragma unroll
       for (int k = 0; k < NC; ++k) {
@@ -348,26 +356,31 @@ __global__ __launch_bounds__(kBlock) void SweepXKernel(SweepArgs a) {
         t0[k] = static_cast<T>(u[k]);
         tp[k] = static_cast<T>(up[k]);
       }
-      ReconAny<D, 0, T, TA>(tm, t0, tp, lh, g, a.limiter, a.muscl, recL, recR, irL, irR);
-    }
-    T recRprev[NQ];
+      ReconAny<D, 0, T, P>(tm, t0, tp, lh, g, a.limiter, a.muscl, recL, recR, irL, irR);
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) recRprev[k] = ShiftUp(recR[k]);
-    typename TA::Inv irRprev;
-    if constexpr (TA::kFast) {
-      irRprev.y = ShiftUp(irR.y);
-    } else {
-      irRprev = TA::inv(recRprev[0]);
-    }
-
-    // Face sl - 1 (left face of the slot's cell) for slots 1 .. nx + 1.
-    const bool face_lane = cur.valid && lane >= 2 && lane <= 2 + kXOwned && cur.sl >= 1;
-    T F[NC];
-    if (face_lane) {
-      FaceFlux<D, 0, LARR, T, TA>(F, recRprev, irRprev, recL, irL, g, a.quirk3d);
-    } else {
+      for (int k = 0; k < NQ; ++k) recRprev[k] = ShiftUp(recR[k]);
+      if constexpr (std::is_same<P, IeeeArith<T>>::value) {
+        irRprev = P::inv(recRprev[0]);
+      } else {
+        if constexpr (!P::kFast) irRprev.b = recRprev[0];
+        irRprev.y = ShiftUp(irR.y);
+      }
+      if (face_lane) {
+        FaceFlux<D, 0, LARR, T, P>(F, recRprev, irRprev, recL, irL, g, a.quirk3d);
+      } else {
 #pragma unroll
-      for (int k = 0; k < NC; ++k) F[k] = T(0);
+        for (int k = 0; k < NC; ++k) F[k] = T(0);
+      }
+    };
+    if constexpr (kIeee) {
+      // The wave votes: regular cells take the shared reciprocals.
+      if (__builtin_expect(RegularStep(lh) && __all(RegularCell<D>(u)), 1)) {
+        flux(RegularArith<T>{});
+      } else {
+        flux(IeeeArith<T>{});
+      }
+    } else {
+      flux(TA{});
     }
     T Fnext[NC];
 #pragma unroll
@@ -411,6 +424,7 @@ __global__ __launch_bounds__(kBlock) void SweepPencilKernel(SweepArgs a) {
   using DA = typename Policies<T, FAST>::DA;
   constexpr int NC = D + 2;
   constexpr int NQ = D + 4;
+  constexpr bool kIeee = !FAST && std::is_same<T, double>::value;
   if (a.halt && *a.halt) return;
   const int64_t nx = a.n[0], ny = a.n[1];
   const int64_t nd = a.n[DIR];
@@ -443,12 +457,25 @@ __global__ __launch_bounds__(kBlock) void SweepPencilKernel(SweepArgs a) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) u[c] = LdOff(a.in[c] + uoff, toff);
     };
-    load(Um, j0 - 1);
-    load(U0, j0);
-    load(Unext, j0 + 1);
+    // Cell j0 - 1 (the ghost cell at the lower end) is only reconstructed: by
+    // a round of the loop in the IEEE kernels, whose code then exists once
+    // (the Y sweep of a 256^2 patch, one wave per SIMD, waits for instructions:
+    // 13.7 us with a copy ahead of the loop, 11.8 without), ahead of the loop
+    // in the others (Y sweep of 256^3: 327 us, as a round 351).
+    const int64_t jfirst = kIeee ? j0 - 1 : j0;
+    load(Um, jfirst - 1);
+    load(U0, jfirst);
+    load(Unext, jfirst + 1);
+    // Which cells of the window the wave's pencils all have regular (kIeee).
+    bool reg_mm = RegularStep(lh), reg_m = true, reg_0 = true;
+    if constexpr (kIeee) {
+      reg_m = __all(RegularCell<D>(Um));
+      reg_0 = __all(RegularCell<D>(U0));
+    }
     T recRprev[NQ];
     typename TA::Inv irRprev;
-    {
+    T yprev;  // reciprocal of recRprev's density (kIeee)
+    if constexpr (!kIeee) {
       T t0[NC];
       if (j0 == 0) {
 #pragma unroll
@@ -472,32 +499,69 @@ __global__ __launch_bounds__(kBlock) void SweepPencilKernel(SweepArgs a) {
     BoundCell<D> bprev;
     if (a.check && a.bound_check) bprev = MakeBoundCell<D>(Um, gd);
     T Fprev[NC];
-    for (int64_t j = j0; j <= j1; ++j) {
+    for (int64_t j = jfirst; j <= j1; ++j) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) Up[c] = Unext[c];
       if (j + 1 < nd) load(Unext, j + 2);
-      T recL[NQ], recR[NQ];
-      typename TA::Inv irL, irR;
-      if (j < nd) {
-        T tm[NC], t0[NC], tp[NC];
+      T recR[NQ], F[NC];
+      typename TA::Inv irR;
+      if constexpr (kIeee) {
+        // Half-step states of cell j and the flux of its lower face in
+        // arithmetic P.
+        auto flux = [&](auto policy) {
+          using P = decltype(policy);
+          T recL[NQ];
+          typename P::Inv irL, irRp, irPrev;
+          if (j >= 0 && j < nd) {
+            ReconAny<D, DIR, T, P>(Um, U0, Up, lh, g, a.limiter, a.muscl, recL, recR, irL, irRp);
+          } else {
+            irL = irRp = GhostRec<D, T, P>(U0, g, recL);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          tm[c] = static_cast<T>(Um[c]);
-          t0[c] = static_cast<T>(U0[c]);
-          tp[c] = static_cast<T>(Up[c]);
+            for (int k = 0; k < NQ; ++k) recR[k] = recL[k];
+          }
+          if constexpr (std::is_same<P, TA>::value) {
+            irPrev = P::inv(recRprev[0]);
+            yprev = RegularArith<T>::inv(recR[0]).y;
+          } else {
+            irPrev = typename P::Inv{recRprev[0], yprev};
+            yprev = irRp.y;
+          }
+          if (j >= j0) FaceFlux<D, DIR, LARR, T, P>(F, recRprev, irPrev, recL, irL, g, a.quirk3d);
+        };
+        // The wave votes: where the cells of both half-step states are
+        // regular it takes the shared reciprocals.
+        const bool reg_p = __all(RegularCell<D>(Up));
+        if (__builtin_expect(reg_mm && reg_m && reg_0 && reg_p, 1)) {
+          flux(RegularArith<T>{});
+        } else {
+          flux(TA{});
         }
-        ReconAny<D, DIR, T, TA>(tm, t0, tp, lh, g, a.limiter, a.muscl, recL, recR, irL, irR);
+        reg_mm = reg_m && RegularStep(lh);
+        reg_m = reg_0;
+        reg_0 = reg_p;
       } else {
-        T t0[NC];
+        T recL[NQ];
+        typename TA::Inv irL;
+        if (j < nd) {
+          T tm[NC], t0[NC], tp[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) t0[c] = static_cast<T>(U0[c]);
-        irL = GhostRec<D, T, TA>(t0, g, recL);
-        irR = irL;
+          for (int c = 0; c < NC; ++c) {
+            tm[c] = static_cast<T>(Um[c]);
+            t0[c] = static_cast<T>(U0[c]);
+            tp[c] = static_cast<T>(Up[c]);
+          }
+          ReconAny<D, DIR, T, TA>(tm, t0, tp, lh, g, a.limiter, a.muscl, recL, recR, irL, irR);
+        } else {
+          T t0[NC];
 #pragma unroll
-        for (int k = 0; k < NQ; ++k) recR[k] = recL[k];
+          for (int c = 0; c < NC; ++c) t0[c] = static_cast<T>(U0[c]);
+          irL = GhostRec<D, T, TA>(t0, g, recL);
+          irR = irL;
+#pragma unroll
+          for (int k = 0; k < NQ; ++k) recR[k] = recL[k];
+        }
+        FaceFlux<D, DIR, LARR, T, TA>(F, recRprev, irRprev, recL, irL, g, a.quirk3d);
       }
-      T F[NC];
-      FaceFlux<D, DIR, LARR, T, TA>(F, recRprev, irRprev, recL, irL, g, a.quirk3d);
       if (j > j0) {
         const int64_t uoff = ubase + (j - 1) * stride;
 #pragma unroll
@@ -509,10 +573,10 @@ __global__ __launch_bounds__(kBlock) void SweepPencilKernel(SweepArgs a) {
       if (a.check && (j < j1 || j1 == nd)) {
         // The face index is uniform over the workgroup, so the vote covers
         // one face per active pencil.
-        bool exact = true;
+        bool exact = !kIeee || j >= j0;
         if (a.bound_check) {
           const BoundCell<D> b0 = MakeBoundCell<D>(U0, gd);
-          exact = !__all(BoundPasses<D, DIR>(bprev, b0, s_crit, kbound));
+          if (exact) exact = !__all(BoundPasses<D, DIR>(bprev, b0, s_crit, kbound));
           bprev = b0;
         }
         if (exact) {

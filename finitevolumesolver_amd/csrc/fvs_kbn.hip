@@ -24,6 +24,7 @@
 #include "fvs_lanes.hpp"
 #include "fvs_physics.hpp"
 #include "fvs_riemann.hpp"
+#include "fvs_speeds.hpp"
 #include "fvs_views.hpp"
 
 #include <algorithm>
@@ -360,15 +361,14 @@ __global__ __launch_bounds__(kBlock) void BoundaryFluxKernel(DevView bflux, DevV
 
 // PerfectGas::CompleteFromCons, masked array form: the zero state unless
 // the lane is valid with positive density.  T / A: the arithmetic of the
-// reconstruction (double IEEE, or float for the FP32-flux form).
+// reconstruction (double IEEE, or float for the FP32-flux form).  Returns the
+// density's reciprocal.
 template <int D, class T = double, class A = IeeeArith<T>>
-__device__ __forceinline__ void CompleteMasked(T* q, bool mask, const Gas<T>& g) {
-  if (mask && q[0] > T(0)) {
-    CompleteFromCons<D, T, A>(q, g);
-  } else {
+__device__ __forceinline__ typename A::Inv CompleteMasked(T* q, bool mask, const Gas<T>& g) {
+  if (mask && q[0] > T(0)) return CompleteFromCons<D, T, A>(q, g);
 #pragma unroll
-    for (int k = 0; k < D + 4; ++k) q[k] = T(0);
-  }
+  for (int k = 0; k < D + 4; ++k) q[k] = T(0);
+  return A::inv(T(0));
 }
 
 // Masked PerfectGas::Flux: zero for the zero state (density 1 stands in
@@ -388,14 +388,16 @@ __device__ __forceinline__ void FluxMasked(T* f, const T* q) {
 template <int D, int DIR, int LIM, class T = double, class A = IeeeArith<T>>
 __device__ __forceinline__ void MaskedRecon(const T* um, const T* u0, const T* up,
                                             bool slope_mask, T lh, const Gas<T>& g,
-                                            T* recL, T* recR) {
+                                            T* recL, T* recR, typename A::Inv& irL,
+                                            typename A::Inv& irR) {
   constexpr int NC = D + 2, NQ = D + 4;
   T qL[NQ], qR[NQ];
 #pragma unroll
   for (int k = 0; k < NC; ++k) {
     const T s = slope_mask ? LimitedSlope<LIM, T, A>(um[k], u0[k], up[k]) : T(0);
-    qL[k] = u0[k] - T(0.5) * s;
-    qR[k] = u0[k] + T(0.5) * s;
+    const T hs = A::half(s);
+    qL[k] = u0[k] - hs;
+    qR[k] = u0[k] + hs;
   }
   CompleteMasked<D, T, A>(qL, true, g);
   CompleteMasked<D, T, A>(qR, true, g);
@@ -408,8 +410,8 @@ __device__ __forceinline__ void MaskedRecon(const T* um, const T* u0, const T* u
     recR[k] = qR[k] + dq;
     recL[k] = qL[k] + dq;
   }
-  CompleteMasked<D, T, A>(recR, true, g);
-  CompleteMasked<D, T, A>(recL, true, g);
+  irR = CompleteMasked<D, T, A>(recR, true, g);
+  irL = CompleteMasked<D, T, A>(recL, true, g);
 }
 
 struct FluxParams {
@@ -433,6 +435,7 @@ __global__ __launch_bounds__(kBlock) void RegularFluxKernel(DevView fl, DevView 
   } else {
     double L[NQ], R[NQ];
     if (fp.muscl) {
+      IeeeArith<double>::Inv ir;
       double u[4][NQ];
       double a[4];
 #pragma unroll
@@ -448,20 +451,20 @@ __global__ __launch_bounds__(kBlock) void RegularFluxKernel(DevView fl, DevView 
       double dummy[NQ];
       switch (fp.limiter) {
       case kMinMod:
-        MaskedRecon<D, DIR, kMinMod>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L);
-        MaskedRecon<D, DIR, kMinMod>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy);
+        MaskedRecon<D, DIR, kMinMod>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L, ir, ir);
+        MaskedRecon<D, DIR, kMinMod>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy, ir, ir);
         break;
       case kVanLeer:
-        MaskedRecon<D, DIR, kVanLeer>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L);
-        MaskedRecon<D, DIR, kVanLeer>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy);
+        MaskedRecon<D, DIR, kVanLeer>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L, ir, ir);
+        MaskedRecon<D, DIR, kVanLeer>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy, ir, ir);
         break;
       case kNoLimiter:
-        MaskedRecon<D, DIR, kNoLimiter>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L);
-        MaskedRecon<D, DIR, kNoLimiter>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy);
+        MaskedRecon<D, DIR, kNoLimiter>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L, ir, ir);
+        MaskedRecon<D, DIR, kNoLimiter>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy, ir, ir);
         break;
       default:
-        MaskedRecon<D, DIR, kNoGradient>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L);
-        MaskedRecon<D, DIR, kNoGradient>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy);
+        MaskedRecon<D, DIR, kNoGradient>(u[0], u[1], u[2], mL, lh, fp.g, dummy, L, ir, ir);
+        MaskedRecon<D, DIR, kNoGradient>(u[1], u[2], u[3], mR, lh, fp.g, R, dummy, ir, ir);
         break;
       }
     } else {
@@ -1248,6 +1251,11 @@ __device__ __forceinline__ unsigned long long BlockMinKey(unsigned long long k) 
   return m;
 }
 
+// Key of the smallest face dt of a lane whose largest face speed is s.
+__device__ __forceinline__ unsigned long long SpeedKey(double dx, double s) {
+  return s > 0.0 ? DtKey(DivRn(dx, s)) : 0x7ff0000000000000ull;
+}
+
 // Complete state of interior cell c with the volume mask.
 __device__ __forceinline__ void CellComplete(const LevelState& st, const LevelGeom& g, int64_t c,
                                              const Gas<double>& gas, double* q) {
@@ -1291,15 +1299,22 @@ __global__ __launch_bounds__(kBlock) void LevelDtKernel(LevelState st, LevelGeom
   if (threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
-// Step-start masked HLLEM CFL of both directions in one pass: a workgroup
-// is a tile of 256 columns (column x0 - 1 + t; threads 1..255 own theirs)
-// marching kDt2Seg rows, each thread completing its cell once per row; the
-// x face to its left pairs it with the left neighbour through LDS, the y
-// face below with the previous row kept in registers.  Face values are
-// those of LevelDtKernel (DBL_MAX where beta is zero); the per-direction
-// minima go to partials[b] (x) and partials[nblocks + b] (y); blocks beyond
-// the tiles write +inf.
+// Step-start masked HLLEM CFL of both directions in one pass: a wave is a tile
+// of 64 columns (column x0 - 1 + lane; lanes 1..63 own theirs) marching kDt2Seg
+// rows, each lane forming its cell's ingredients (DtCell) once per row while
+// the next row loads; the x face to its left takes the left neighbour's by
+// DPP, the y face below the previous row's from registers.  Face values are
+// those of LevelDtKernel (DBL_MAX where beta is zero); the smallest face dt is
+// the quotient by the largest speed, taken once per lane.  The per-direction
+// minima go to partials[b] (x) and partials[nblocks + b] (y).  2048 x 1024
+// cells take 32 us (84 MB: near the memory rate); with complete states through
+// LDS, one dt per face and IEEE sequences throughout they took 58.
 constexpr int kDt2Seg = 8;
+constexpr int kDt2Own = 63;
+
+__host__ __device__ inline int64_t Dt2Waves(int64_t nx, int64_t ny) {
+  return ((nx + 1 + kDt2Own - 1) / kDt2Own) * ((ny + 1 + kDt2Seg - 1) / kDt2Seg);
+}
 
 __global__ __launch_bounds__(kBlock) void LevelDt2Kernel(LevelState st, LevelGeom g, int64_t nx,
                                                          int64_t ny, double dx0, double dx1,
@@ -1307,62 +1322,66 @@ __global__ __launch_bounds__(kBlock) void LevelDt2Kernel(LevelState st, LevelGeo
                                                          unsigned long long* partials,
                                                          int64_t nblocks, const int* halt) {
   if (*halt) return;
-  constexpr int kOwn = kBlock - 1;
-  const int64_t tiles_x = (nx + 1 + kOwn - 1) / kOwn;
-  const int64_t segs = (ny + 1 + kDt2Seg - 1) / kDt2Seg;
-  const int64_t b = blockIdx.x;
+  const int64_t tiles_x = (nx + 1 + kDt2Own - 1) / kDt2Own;
+  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
   unsigned long long kx = 0x7ff0000000000000ull, ky = 0x7ff0000000000000ull;
-  if (b < tiles_x * segs) {
-    __shared__ double s_q[6][kBlock];
-    const int t = threadIdx.x;
-    const int64_t i = (b % tiles_x) * kOwn - 1 + t;   // column, -1 .. nx (+ tile padding)
-    const int64_t j0 = (b / tiles_x) * kDt2Seg;        // first face row of the segment
+  if (wave < Dt2Waves(nx, ny)) {
+    const int lane = threadIdx.x & 63;
+    const int64_t i = (wave % tiles_x) * kDt2Own - 1 + lane;  // column, -1 .. nx (+ tile padding)
+    const int64_t j0 = (wave / tiles_x) * kDt2Seg;             // first face row of the segment
     const int64_t j1 = j0 + kDt2Seg < ny + 1 ? j0 + kDt2Seg : ny + 1;
-    const bool col_ok = i <= nx;
-    const int64_t ic = col_ok ? i : nx;
+    const int64_t ic = i <= nx ? i : nx;
+    const bool own_x = lane >= 1 && i >= 0 && i <= nx, own_y = lane >= 1 && i >= 0 && i < nx;
     // The cell words carry the volume mask (bit 0 of either direction's)
     // and the fractions of the cell's lower x and y faces.
-    double prev[6];
-    {
-      LoadCons(st, g.state_cell(ic, j0 - 1), prev);
-      CompleteMasked<2>(prev, CellCode::Pos(g.code[0][g.cell(ic, j0 - 1)]), gas);
-    }
-    for (int64_t j = j0; j < j1; ++j) {
+    struct Row {
+      double u[4];
+      int32_t cx, cy;
+    };
+    auto load = [&](Row& r, int64_t j) {
       const int64_t c = g.cell(ic, j);
-      const int32_t cx = g.code[0][c], cy = g.code[1][c];
-      double cur[6];
-      LoadCons(st, g.state_cell(ic, j), cur);
-      CompleteMasked<2>(cur, CellCode::Pos(cx), gas);
+      r.cx = g.code[0][c];
+      r.cy = g.code[1][c];
+      LoadCons(st, g.state_cell(ic, j), r.u);
+    };
+    Row next;
+    load(next, j0 - 1);
+    DtCell<2> prev;
+    double sx = 0.0, sy = 0.0;
+    bool bare_x = false, bare_y = false;  // met a face without a flux
+    for (int64_t j = j0 - 1; j < j1; ++j) {
+      const Row r = next;
+      if (j + 1 < j1) load(next, j + 1);
+      double q[4];
+      const bool keep = CellCode::Pos(r.cx) && r.u[0] > 0.0;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) s_q[k][t] = cur[k];
-      __syncthreads();
-      if (t >= 1 && col_ok) {
-        // x face i between cells i - 1 and i (rows 0 .. ny - 1, faces 0 .. nx)
-        if (j < ny && i >= 0 && CellCode::Face(cx)) {
-          double L[6];
-#pragma unroll
-          for (int k = 0; k < 6; ++k) L[k] = s_q[k][t - 1];
-          kx = KeyMin(kx, DtKey(HllemStableDt<2, 0>(L, cur, dx0, gas)));
-        } else if (j < ny && i >= 0) {
-          kx = KeyMin(kx, DtKey(DBL_MAX));
-        }
-        // y face j between cells (i, j - 1) and (i, j) (columns 0 .. nx - 1)
-        if (i >= 0 && i < nx) {
-          const double v = CellCode::Face(cy) ? HllemStableDt<2, 1>(prev, cur, dx1, gas) : DBL_MAX;
-          ky = KeyMin(ky, DtKey(v));
-        }
+      for (int k = 0; k < 4; ++k) q[k] = keep ? r.u[k] : 0.0;
+      const bool face_x = own_x && j >= j0 && j < ny, face_y = own_y && j >= j0;
+      bare_x |= face_x && !CellCode::Face(r.cx);
+      bare_y |= face_y && !CellCode::Face(r.cy);
+      auto speeds = [&](auto policy) {
+        using P = decltype(policy);
+        const DtCell<2> dc = MakeDtCell<2, P>(q, gas);
+        const DtCell<2> dl = ShflUp<2>(dc);
+        if (face_x && CellCode::Face(r.cx)) sx = SMax(sx, FaceSpeed<2, 0, P>(dl, dc, gas.gm1));
+        if (face_y && CellCode::Face(r.cy)) sy = SMax(sy, FaceSpeed<2, 1, P>(prev, dc, gas.gm1));
+        prev = dc;
+      };
+      if (__builtin_expect(__all(!keep || RegularCell<2>(q)), 1)) {
+        speeds(RegularArith<double>{});
+      } else {
+        speeds(IeeeArith<double>{});
       }
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < 6; ++k) prev[k] = cur[k];
     }
+    kx = KeyMin(SpeedKey(dx0, sx), bare_x ? DtKey(DBL_MAX) : kx);
+    ky = KeyMin(SpeedKey(dx1, sy), bare_y ? DtKey(DBL_MAX) : ky);
   }
   const unsigned long long mx = BlockMinKey(kx);
   __syncthreads();  // BlockMinKey's shared slots are reused
   const unsigned long long my = BlockMinKey(ky);
   if (threadIdx.x == 0) {
-    partials[b] = mx;
-    partials[nblocks + b] = my;
+    partials[blockIdx.x] = mx;
+    partials[nblocks + blockIdx.x] = my;
   }
 }
 
@@ -1565,6 +1584,88 @@ template <class T> __device__ __forceinline__ Gas<T> GasAs(const Gas<double>& g)
   return r;
 }
 
+// Fluxes of the lower faces of a wave's cells (one cell a lane, consecutive
+// along DIR; face: the lane's face carries a regular flux) from the masked
+// half-step states in arithmetic P: the state q (conservative, masked), its
+// neighbours' and their masks one lane away.  Called by the whole wave.
+template <int DIR, int LIM, bool LARR, class T, class P>
+__device__ __forceinline__ void KbnWaveFluxes(const double* qm, const double* q, const double* qp,
+                                              bool mask, bool face, T lh, const Gas<T>& gas,
+                                              double* F) {
+  T tm[4], t0[4], tp[4], recL[6], recR[6], recRm[6];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    tm[k] = static_cast<T>(qm[k]);
+    t0[k] = static_cast<T>(q[k]);
+    tp[k] = static_cast<T>(qp[k]);
+  }
+  typename P::Inv irL, irR, irRm;
+  MaskedRecon<2, DIR, LIM, T, P>(tm, t0, tp, mask, lh, gas, recL, recR, irL, irR);
+#pragma unroll
+  for (int k = 0; k < 6; ++k) recRm[k] = ShiftUp(recR[k]);
+  if constexpr (std::is_same<P, IeeeArith<T>>::value) {
+    irRm = P::inv(recRm[0]);
+  } else {
+    if constexpr (!P::kFast) irRm.b = recRm[0];
+    irRm.y = ShiftUp(irR.y);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) F[k] = 0.0;
+  if (face) {
+    T Ft[4];
+    HllemFlux<2, DIR, LARR, false, T, P>(Ft, recRm, irRm, recL, irL, gas);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) F[k] = static_cast<double>(Ft[k]);
+  }
+}
+
+// One wave's lane-parallel step along DIR: fluxes F of the lanes' lower faces
+// (as KbnWaveFluxes), and the largest signal speed of the checked faces in
+// smax.  u: the lane's conservative state, code its cell word.  The check only
+// has to tell whether a face's stable dt is below dt, so waves whose faces
+// all pass the bound (BoundPasses) evaluate no speed, and a step's first sweep
+// has no check.  2048 x 1024 cells: X 60, Y 66 us; with a speed for every face
+// and IEEE sequences throughout 92 and 99.
+template <int DIR, int LIM, bool LARR, class T, bool FAST>
+__device__ __forceinline__ void KbnWaveStep(const double* u, int32_t code, bool face, bool check,
+                                            double lh, double s_crit, const Gas<double>& gas,
+                                            const Gas<T>& gasT, double* F, double& smax) {
+  double q[4], qm[4], qp[4];
+  const bool keep = CellCode::Pos(code) && u[0] > 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) q[k] = keep ? u[k] : 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    qm[k] = ShiftUp(q[k]);
+    qp[k] = ShiftDown(q[k]);
+  }
+  // Every lane must take part in a DPP shift (an inactive source lane yields
+  // the reader's own value): shift first, combine without short-circuit.
+  const int code_m = DppUp(code), code_p = DppDown(code);
+  const bool mask = CellCode::Pos(code_m) & CellCode::Pos(code) & CellCode::Pos(code_p);
+  face = face && CellCode::Face(code);
+  if constexpr (!FAST) {
+    // zero states meet no division
+    if (__builtin_expect(RegularStep(lh) && __all(!keep || RegularCell<2>(q)), 1)) {
+      KbnWaveFluxes<DIR, LIM, LARR, T, RegularArith<T>>(qm, q, qp, mask, face, lh, gasT, F);
+    } else {
+      KbnWaveFluxes<DIR, LIM, LARR, T, IeeeArith<T>>(qm, q, qp, mask, face, lh, gasT, F);
+    }
+  } else {
+    KbnWaveFluxes<DIR, LIM, LARR, T, FastArith<T>>(qm, q, qp, mask, face, static_cast<T>(lh),
+                                                   gasT, F);
+  }
+  if (check) {
+    const BoundCell<2> bc = MakeBoundCell<2>(q, gas);
+    const BoundCell<2> bm = ShflUp<2>(bc);
+    if (!__all(!face || BoundPasses<2, DIR>(bm, bc, s_crit, 0.125 * gas.gm1))) {
+      const DtCell<2> dc = MakeDtCell<2, IeeeArith<double>>(q, gas);
+      const DtCell<2> dm = ShflUp<2>(dc);
+      if (face) smax = SMax(smax, FaceSpeed<2, DIR, IeeeArith<double>>(dm, dc, gas.gm1));
+    }
+  }
+}
+
 template <int LIM, bool LARR, class T, bool FAST>
 __global__ __launch_bounds__(kBlock) void KbnSweepXKernel(LevelState in, LevelState out,
                                                           LevelGeom g, int64_t nx, int64_t ny,
@@ -1572,7 +1673,6 @@ __global__ __launch_bounds__(kBlock) void KbnSweepXKernel(LevelState in, LevelSt
                                                           Gas<double> gas,
                                                           unsigned long long* partials,
                                                           const int* halt) {
-  using TA = typename Policies<T, FAST>::TA;
   if (*halt) return;
   const Gas<T> gasT = GasAs<T>(gas);
   const int lane = threadIdx.x & 63;
@@ -1585,58 +1685,27 @@ __global__ __launch_bounds__(kBlock) void KbnSweepXKernel(LevelState in, LevelSt
   const int64_t ic = i < nx + 1 ? i : nx + 1;            // stay inside the ghost ring
   const int64_t c = g.cell(ic, j);
   const int32_t code = g.code[0][c];
-  double q[6];
-  LoadCons(in, g.state_cell(ic, j), q);
-  CompleteMasked<2>(q, CellCode::Pos(code), gas);
-  double qm[6], qp[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    qm[k] = ShiftUp(q[k]);
-    qp[k] = ShiftDown(q[k]);
-  }
-  // Every lane must take part in a DPP shift (an inactive source lane yields
-  // the reader's own value): shift first, combine without short-circuit.
-  const int code_m = DppUp(code), code_p = DppDown(code);
-  const bool mask = CellCode::Pos(code_m) & CellCode::Pos(code) & CellCode::Pos(code_p);
+  double u[4];
+  LoadCons(in, g.state_cell(ic, j), u);
   const double dt = *dt_ptr;
   const double lh = DivRn(0.5 * dt, dx);
-  T recL[6], recR[6];
-  {
-    T tm[4], t0[4], tp[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      tm[k] = static_cast<T>(qm[k]);
-      t0[k] = static_cast<T>(q[k]);
-      tp[k] = static_cast<T>(qp[k]);
-    }
-    MaskedRecon<2, 0, LIM, T, TA>(tm, t0, tp, mask, static_cast<T>(lh), gasT, recL, recR);
-  }
-  T recRm[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) recRm[k] = ShiftUp(recR[k]);
   // left face of the lane's cell: faces 0 .. nx, lanes 2 .. 62
   const bool face_lane = wave_ok && lane >= 2 && lane <= 2 + kKbnOwned && i >= 0 && i <= nx;
-  double F[4] = {0.0, 0.0, 0.0, 0.0};
-  unsigned long long key = 0x7ff0000000000000ull;
-  if (face_lane && CellCode::Face(code)) {
-    T Ft[4];
-    HllemFlux<2, 0, LARR, false, T, TA>(Ft, recRm, recL, gasT);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) F[k] = static_cast<double>(Ft[k]);
-    key = DtKey(HllemStableDt<2, 0>(qm, q, dx, gas));
-  }
+  double F[4], smax = 0.0;
+  KbnWaveStep<0, LIM, LARR, T, FAST>(u, code, face_lane, partials != nullptr, lh,
+                                     BoundSpeedLimit(dx, dt), gas, gasT, F, smax);
   double Fr[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) Fr[k] = ShiftDown(F[k]);
   if (wave_ok && lane >= 2 && lane < 2 + kKbnOwned && i >= 0 && i < nx) {
-    double u[4], res[4];
-    LoadCons(in, c, u);
+    double res[4];  // an interior cell's u is its own state
     if (KbnSweepUpdate<0>(g, code, u, F, Fr, DivRn(dt, dx), res)) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) out.u[k][c] = res[k];
     }
   }
-  const unsigned long long m = BlockMinKey(key);
+  if (!partials) return;
+  const unsigned long long m = BlockMinKey(SpeedKey(dx, smax));
   if (threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
@@ -1658,7 +1727,6 @@ __global__ __launch_bounds__(kBlock) void KbnSweepYKernel(LevelState in, LevelSt
                                                           Gas<double> gas,
                                                           unsigned long long* partials,
                                                           const int* halt) {
-  using TA = typename Policies<T, FAST>::TA;
   __shared__ double s_u[4][kYtCols][kYtPitch];
   __shared__ int32_t s_code[kYtCols][kYtPitch];
   if (*halt) return;
@@ -1690,46 +1758,18 @@ __global__ __launch_bounds__(kBlock) void KbnSweepYKernel(LevelState in, LevelSt
   const double dt_over_dx = DivRn(dt, dx);
   const bool face_row = lane >= 2 && lane <= 2 + kKbnOwned && j >= 0 && j <= ny;
   const bool own_row = lane >= 2 && lane < 2 + kKbnOwned && j < ny;
-  unsigned long long key = 0x7ff0000000000000ull;
+  const double s_crit = BoundSpeedLimit(dx, dt);
+  double smax = 0.0;
 #pragma unroll 1
   for (int cc = threadIdx.x >> 6; cc < kYtCols; cc += kBlock / 64) {
     const bool col_ok = i0 + cc < nx;
     const int32_t code = s_code[cc][lane];
-    double u[4], q[6];
+    double u[4], F[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) q[k] = u[k] = s_u[k][cc][lane];
-    CompleteMasked<2>(q, CellCode::Pos(code), gas);
-    double qm[6], qp[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      qm[k] = ShiftUp(q[k]);
-      qp[k] = ShiftDown(q[k]);
-    }
-    const int code_m = DppUp(code), code_p = DppDown(code);
-    const bool mask = CellCode::Pos(code_m) & CellCode::Pos(code) & CellCode::Pos(code_p);
-    T recL[6], recR[6];
-    {
-      T tm[4], t0[4], tp[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        tm[k] = static_cast<T>(qm[k]);
-        t0[k] = static_cast<T>(q[k]);
-        tp[k] = static_cast<T>(qp[k]);
-      }
-      MaskedRecon<2, 1, LIM, T, TA>(tm, t0, tp, mask, static_cast<T>(lh), gasT, recL, recR);
-    }
-    T recRm[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) recRm[k] = ShiftUp(recR[k]);
+    for (int k = 0; k < 4; ++k) u[k] = s_u[k][cc][lane];
     // lower face of the lane's cell: faces 0 .. ny, lanes 2 .. 62
-    double F[4] = {0.0, 0.0, 0.0, 0.0};
-    if (face_row && CellCode::Face(code)) {
-      T Ft[4];
-      HllemFlux<2, 1, LARR, false, T, TA>(Ft, recRm, recL, gasT);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) F[k] = static_cast<double>(Ft[k]);
-      if (col_ok) key = KeyMin(key, DtKey(HllemStableDt<2, 1>(qm, q, dx, gas)));
-    }
+    KbnWaveStep<1, LIM, LARR, T, FAST>(u, code, face_row && col_ok, partials != nullptr, lh, s_crit,
+                                       gas, gasT, F, smax);
     double Fr[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) Fr[k] = ShiftDown(F[k]);
@@ -1754,7 +1794,8 @@ __global__ __launch_bounds__(kBlock) void KbnSweepYKernel(LevelState in, LevelSt
 #pragma unroll
     for (int k = 0; k < 4; ++k) out.u[k][c] = s_u[k][cc][r];
   }
-  const unsigned long long m = BlockMinKey(key);
+  if (!partials) return;
+  const unsigned long long m = BlockMinKey(SpeedKey(dx, smax));
   if (threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
@@ -2147,13 +2188,14 @@ static int KbnSweep(fvs_kbn_level* L, int dir, int src, int dst, bool check) {
   const int64_t nb = KbnSweepBlocks(dir, L->nx, L->ny);
   const dim3 grid(static_cast<unsigned>(nb));
   const bool fp32 = h->desc.precision == FVS_FP32_FLUX;
+  unsigned long long* partials = check ? L->partials : nullptr;  // none: no check
 #define FVS_KS(K, LM, LA)                                                                     \
   if (fp32)                                                                                   \
     hipLaunchKernelGGL((K<LM, LA, float, true>), grid, dim3(kBlock), 0, s, in, out, L->lg,    \
-                       L->nx, L->ny, dx, dtp, gas, L->partials, halt);                        \
+                       L->nx, L->ny, dx, dtp, gas, partials, halt);                           \
   else                                                                                        \
     hipLaunchKernelGGL((K<LM, LA, double, false>), grid, dim3(kBlock), 0, s, in, out, L->lg,  \
-                       L->nx, L->ny, dx, dtp, gas, L->partials, halt)
+                       L->nx, L->ny, dx, dtp, gas, partials, halt)
 #define FVS_KS_LIM(K, LA)                                  \
   switch (h->desc.limiter) {                               \
   case kMinMod: FVS_KS(K, kMinMod, LA); break;             \
@@ -2239,15 +2281,18 @@ int fvs_kbn_level_advance(fvs_kbn_level* L, int max_steps, double final_time, in
       }
       // step-start CFL of both directions
       const LevelState st0 = StateOf(L, cur);
-      const int64_t dt2_tiles = ((L->nx + 1 + kBlock - 2) / (kBlock - 1)) *
-                                ((L->ny + 1 + kDt2Seg - 1) / kDt2Seg);
+      const int64_t dt2_tiles =
+          (Dt2Waves(L->nx, L->ny) + kBlock / 64 - 1) / (kBlock / 64);
       int64_t npart = L->nblocks;  // partial minima per direction
       if (dt2_tiles <= L->nblocks) {
         npart = dt2_tiles;
         hipLaunchKernelGGL(LevelDt2Kernel, dim3(unsigned(dt2_tiles)), dim3(kBlock), 0, s, st0,
                            L->lg, L->nx, L->ny, L->patch.dx[0], L->patch.dx[1], gas, L->partials,
                            dt2_tiles, halt);
-      } else {  // very thin levels: one pass per direction
+      } else {
+        // Fewer than about eight columns: a wave tile would leave most lanes
+        // idle (a step of 8 x 32768 cells: 127 us with one pass per direction,
+        // 134 with the tiles; of 16 x 16384: 100 and 97).
         hipLaunchKernelGGL(LevelDtKernel<0>, dim3(unsigned(L->nblocks)), dim3(kBlock), 0, s, st0,
                            L->lg, L->nx, L->ny, L->patch.dx[0], gas, L->partials, halt);
         hipLaunchKernelGGL(LevelDtKernel<1>, dim3(unsigned(L->nblocks)), dim3(kBlock), 0, s, st0,

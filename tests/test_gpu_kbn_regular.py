@@ -1,0 +1,45 @@
+"""Cut-cell level sweeps where a wave leaves the common path: momenta that the
+shared-reciprocal arithmetic refuses, and CFL checks that the bound cannot
+settle or that fail; and a level thin enough for one CFL pass per direction.
+Bit-exact with the oracle's level driver."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+import finitevolumesolver_amd as fvs
+from finitevolumesolver_amd import cutcell as K
+from finitevolumesolver_amd.geometry import channel_geometry
+from finitevolumesolver_amd.initial_data import shock_channel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("limiter", ["MinMod", "VanLeer"])
+@pytest.mark.parametrize("kind,cfl", [("tiny", 0.8), ("shock", 0.95), ("shock", 1.0)])
+@pytest.mark.parametrize("shape", [(65, 61), (130, 24), (6, 200)])
+def test_level(cuda, shape, kind, cfl, limiter):
+    import torch
+    (nx, ny), steps = shape, 10
+    geom = channel_geometry(nx, ny, perturb=True)
+    cons, dx = shock_channel(nx, ny, x_shock=-0.4)
+    cons = np.ascontiguousarray(cons)
+    if kind == "tiny":
+        rng = np.random.default_rng(nx)
+        m = cons[1:3]
+        m += np.ldexp(rng.standard_normal(m.shape), -rng.integers(150, 700, m.shape))
+    fm = fvs.FluxMethod(fvs.PerfectGas(dim=2), base="HLLEM", reconstruction="MusclHancock",
+                        limiter=limiter, boundary_solver="hllem")
+    g = K.CutCellData.from_geometry2d(geom, cuda)
+    lvl = K.CutCellLevel(fm, (nx, ny), (dx, dx), g, cfl=cfl)
+    lvl.set_state(torch.from_numpy(cons).to(cuda))
+    done, fails, dts = lvl.advance(steps, batch=4, return_dts=True)
+    got = lvl.get_state().cpu().numpy()
+    ref, ref_dts, ref_fails = O.kbn_level_run(fm._h.desc, geom, cons, (dx, dx), steps, cfl=cfl)
+    assert (done, fails) == (steps, ref_fails)
+    if nx > 6:
+        assert fails > 0 if cfl == 1.0 else fails == 0
+    assert np.array_equal(np.array(dts), ref_dts)
+    assert np.array_equal(got, ref.reshape(got.shape))

@@ -973,10 +973,7 @@ int fvs_amr_stable_dt(fvs_amr* A, double* dt_host) {
   A->s = A->h->stream;
   for (int l = 0; l < A->nlevels; ++l) {
     if (int rc = FillGhosts(A, l, 0)) return rc;
-    if (int rc = SetDt(A, l, 0.0)) return rc;
-    // sweeps into the scratch pool 1 for their CFL minima only
-    for (int d = 0; d < 2; ++d)
-      if (int rc = batch::Sweep(A->lv[l], A->s, d, 0, A->cfl + base + 2 * l + d)) return rc;
+    if (int rc = batch::StableDts(A->lv[l], A->s, A->cfl + base + 2 * l)) return rc;
   }
   std::vector<double> v(2 * A->nlevels);
   FVS_HIP_CHECK(hipMemcpyAsync(v.data(), A->cfl + base, v.size() * sizeof(double),

@@ -5,12 +5,12 @@
 // FluxMethod::ComputeNumericFluxes and HyperbolicPatchIntegrator::
 // UpdateConservatively, include/fub/flux_method/FluxMethod.hpp:246-293,
 // src/HyperbolicPatchIntegrator.cpp:35-154).  Here every patch of uneven
-// size is cut into tiles of one shape, and a persistent grid walks the tile
-// list: each tile reconstructs its cells once (MUSCL-Hancock half-step
-// states into LDS), computes its faces' HLLEM fluxes into LDS and updates
-// its owned cells, all in registers/LDS; the CFL minimum of the faces is
-// reduced per workgroup.  The tile shape per direction is picked by a
-// timing autotuner; the level's sweep sequence (ghost fill, X sweep, ghost
+// size is cut into tiles of one shape, and the waves of a persistent grid walk
+// the tile list, a wave per tile: each lane reconstructs its cell
+// (MUSCL-Hancock half-step states), takes its neighbour's half-step state and
+// hands its face flux on by lane shifts, and updates its cell; the CFL minimum
+// of the faces is reduced per workgroup.  The tile shape per direction is
+// picked by a timing autotuner; the level's sweep sequence (ghost fill, X sweep, ghost
 // fill, Y sweep) is captured once into a hipGraph and replayed.
 //
 // Reconstruction and flux arithmetic run in T (double, or float for the
@@ -23,6 +23,8 @@
 // compiles the kernels of the tolerance-checked modes with multiply-add
 // contraction.
 #include "fvs_batch_internal.hpp"
+#include "fvs_lanes.hpp"
+#include "fvs_speeds.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -36,6 +38,8 @@ using batch::PatchInfo;
 using batch::kG;
 
 namespace {
+
+constexpr int kSweepBlock = 256;  // a workgroup's four waves share only the final reduction
 
 template <class T>
 __device__ __forceinline__ Gas<T> GasT(const Gas<double>& g) {
@@ -58,132 +62,213 @@ __device__ __forceinline__ unsigned long long WaveMinK(unsigned long long k) {
   return k;
 }
 
-// Tile = TX x TY threads; along the sweep direction the T_d threads hold
-// cells start-1 .. start+T_d-2, of which start .. start+T_d-3 are owned.
-template <int DIR, int LIM, class T, int TX, int TY, bool FAST>
-__global__ __launch_bounds__(TX * TY) void BatchSweepKernel(BatchArgs a) {
+// A wave's tile: W lanes along the sweep direction hold cells start - 1 ..
+// start + W - 2, of which start .. start + W - 3 are owned, in 64 / W rows
+// across it.  Neighbouring half-step states and fluxes pass between lanes by
+// DPP shifts; the shifts across a row's ends carry values no lane uses.
+// Loads across the sweep are short where W is large in Y, which the caches
+// absorb: the kernel is bound by its FP64 instructions.  A level of a million
+// cells: X 32 to 33 us, Y 37 to 44; with states and fluxes staged in LDS by
+// workgroup tiles (three barriers a tile, IEEE sequences) 42 and 48.  Every lane loads (clamped into the patch's
+// ghost ring) and computes, and the stores and minima are masked.
+template <int W> struct WaveTile {
+  PatchInfo P;
+  int c, r, w, nd, nt, td;
+  int64_t ldx, cs, step, at;
+  bool row_ok, row_inner;
+};
+
+template <int DIR, int W>
+__device__ __forceinline__ WaveTile<W> MakeWaveTile(const BatchArgs& a, int tile) {
+  WaveTile<W> t;
+  const int lane = threadIdx.x & 63;
+  const int4 q = a.tiles[tile];
+  t.P = a.patches[q.x];
+  t.nd = DIR == 0 ? t.P.nx : t.P.ny;
+  t.nt = DIR == 0 ? t.P.ny : t.P.nx;
+  t.td = lane % W;
+  t.c = q.y - 1 + t.td;
+  t.r = q.z + lane / W;
+  t.w = q.w;
+  t.ldx = t.P.nx + 2 * kG;
+  t.cs = t.ldx * (t.P.ny + 2 * kG);
+  t.step = DIR == 0 ? 1 : t.ldx;
+  t.row_ok = t.r < t.nt + t.w;  // rows start at -w
+  t.row_inner = t.r >= 0 && t.r < t.nt;
+  const int cc = t.c <= t.nd ? t.c : t.nd, rr = t.row_ok ? t.r : t.nt + t.w - 1;
+  const int i = DIR == 0 ? cc : rr, j = DIR == 0 ? rr : cc;
+  t.at = t.P.offset + (int64_t(j) + kG) * t.ldx + (int64_t(i) + kG);
+  return t;
+}
+
+// Fluxes f of the lanes' lower faces along DIR from the half-step states in
+// arithmetic P (of cells um, u0, up: the lane's and its neighbours').  The
+// lane below holds the lower cell's.
+template <int DIR, int LIM, class T, class P>
+__device__ __forceinline__ void BatchWaveFluxes(const double* um, const double* u0,
+                                                const double* up, T lh, const Gas<T>& g, T* f) {
+  constexpr int NQ = 6, NC = 4;
+  T m[NC], z[NC], p[NC], rl[NQ], rr[NQ], rm[NQ];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    m[k] = static_cast<T>(um[k]);
+    z[k] = static_cast<T>(u0[k]);
+    p[k] = static_cast<T>(up[k]);
+  }
+  typename P::Inv irL, irR, irM;
+  ReconstructCell<2, DIR, LIM, T, P>(m, z, p, lh, g, rl, rr, irL, irR);
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) rm[k] = ShiftUp(rr[k]);
+  if constexpr (std::is_same<P, IeeeArith<T>>::value) {
+    irM = P::inv(rm[0]);
+  } else {
+    if constexpr (!P::kFast) irM.b = rm[0];
+    irM.y = ShiftUp(irR.y);
+  }
+  HllemFlux<2, DIR, true, false, T, P>(f, rm, irM, rl, irL, g);
+}
+
+template <int DIR, int LIM, class T, int W, bool FAST>
+__global__ __launch_bounds__(kSweepBlock) void BatchSweepKernel(BatchArgs a) {
   using TA = typename Policies<T, FAST>::TA;
   using DA = typename Policies<T, FAST>::DA;
-  constexpr int NQ = 6, NC = 4;
-  constexpr int TD = DIR == 0 ? TX : TY;
-  __shared__ T recL[NQ][TY][TX];
-  __shared__ T recR[NQ][TY][TX];
-  __shared__ T flx[NC][TY][TX];
-  __shared__ unsigned long long red[(TX * TY + 63) / 64];
-  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-  const int td = DIR == 0 ? tx : ty;   // index along the sweep
-  const int tt = DIR == 0 ? ty : tx;   // index across
+  constexpr int NC = 4;
+  constexpr int kWaves = kSweepBlock / 64;
+  __shared__ unsigned long long red[kWaves];
   const Gas<T> gT = GasT<T>(a.g);
   const double dt = *a.dt;
   const double kbound = 0.125 * a.g.gm1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   unsigned long long kmin = 0x7ff0000000000000ull;
-  for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
-    const int4 t = a.tiles[tile];
-    const PatchInfo P = a.patches[t.x];
-    const int nd = DIR == 0 ? P.nx : P.ny;
-    const int nt = DIR == 0 ? P.ny : P.nx;
-    const int c = t.y - 1 + td;   // cell along the sweep
-    const int r = t.z + tt;       // index across (ghost rows when grown)
-    const int64_t ldx = P.nx + 2 * kG;
-    const int64_t cs = ldx * (P.ny + 2 * kG);
-    const int64_t step = DIR == 0 ? 1 : ldx;
-    const bool row_ok = r >= -t.w && r < nt + t.w;
-    const bool row_inner = r >= 0 && r < nt;
-    const bool recon_ok = row_ok && c >= -1 && c <= nd && c <= t.y + TD - 2;
-    const double s_crit = BoundSpeedLimit(P.dx, dt);
-    int64_t at = 0;
-    if (row_ok) {
-      const int i = DIR == 0 ? c : r, j = DIR == 0 ? r : c;
-      at = P.offset + (int64_t(j) + kG) * ldx + (int64_t(i) + kG);
+  for (int tile = blockIdx.x * kWaves + wave; tile < a.ntiles; tile += gridDim.x * kWaves) {
+    const WaveTile<W> t = MakeWaveTile<DIR, W>(a, tile);
+    double um[NC], u0[NC], up[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      um[k] = a.in[t.at + k * t.cs - t.step];
+      u0[k] = a.in[t.at + k * t.cs];
+      up[k] = a.in[t.at + k * t.cs + t.step];
     }
-    double u0[NC];
-    if (recon_ok) {
-      double um[NC], up[NC];
-#pragma unroll
-      for (int k = 0; k < NC; ++k) {
-        um[k] = a.in[at + k * cs - step];
-        u0[k] = a.in[at + k * cs];
-        up[k] = a.in[at + k * cs + step];
-      }
-      // CFL of face c (cells c - 1, c), FP64, interior rows.  With a time
-      // step set (dt > 0) the sweep's minimum only has to decide the check
-      // dt <= stable dt exactly: a wave whose faces all pass the certified
-      // speed bound (BoundPasses: stable dt above dt) reports dt for them
-      // instead of evaluating the exact speeds.  The reported minimum is then
-      // the exact one whenever it lies below dt (the check fails, and the
-      // slowest face's bound fails too, so its wave evaluates exactly), and
-      // a value of at least dt otherwise.  dt = 0 (a stable-dt pass)
-      // evaluates every face.
-      const bool face = row_inner && c >= 0 && c <= nd && td >= 1;
-      bool exact = true;
-      if (dt > 0.0) {
-        const BoundCell<2> bl = MakeBoundCell<2>(um, a.g), br = MakeBoundCell<2>(u0, a.g);
-        exact = !__all(!face || BoundPasses<2, DIR>(bl, br, s_crit, kbound));
-        if (!exact && face) kmin = KMinKey(kmin, DtKey(dt));
-      }
-      if (exact && face) {
-        double L[NQ], R[NQ];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-          L[k] = um[k];
-          R[k] = u0[k];
-        }
-        CompleteFromCons<2, double, DA>(L, a.g);
-        CompleteFromCons<2, double, DA>(R, a.g);
-        const double sdt = HllemStableDt<2, DIR, double, DA>(L, R, P.dx, a.g);
-        kmin = KMinKey(kmin, DtKey(sdt));
-      }
-      T m[NQ], z[NQ], p[NQ], rl[NQ], rr[NQ];
-#pragma unroll
-      for (int k = 0; k < NC; ++k) {
-        m[k] = static_cast<T>(um[k]);
-        z[k] = static_cast<T>(u0[k]);
-        p[k] = static_cast<T>(up[k]);
-      }
-      const T lh = static_cast<T>(DivRn(0.5 * dt, P.dx));
-      ReconstructCell<2, DIR, LIM, T, TA>(m, z, p, lh, gT, rl, rr);
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        recL[k][ty][tx] = rl[k];
-        recR[k][ty][tx] = rr[k];
-      }
+    const double dt_dx = DivRn(dt, t.P.dx);
+    // halving is exact above the subnormal range
+    const double lh = dt_dx >= 0x1p-1000 ? 0.5 * dt_dx : DivRn(0.5 * dt, t.P.dx);
+    // CFL of face c (cells c - 1, c), FP64, interior rows.  With a time
+    // step set (dt > 0) the sweep's minimum only has to decide the check
+    // dt <= stable dt exactly: a wave whose faces all pass the certified
+    // speed bound (BoundPasses: stable dt above dt) reports dt for them
+    // instead of evaluating the exact speeds.  The reported minimum is then
+    // the exact one whenever it lies below dt (the check fails, and the
+    // slowest face's bound fails too, so its wave evaluates exactly), and
+    // a value of at least dt otherwise.  dt = 0 (a stable-dt pass)
+    // evaluates every face.
+    const bool face = t.row_inner && t.c >= 0 && t.c <= t.nd && t.td >= 1;
+    bool exact = true;
+    if (dt > 0.0) {
+      // the refined reciprocal's error is far inside the bound's margin
+      const double s_crit = FastArith<double>::inv(dt_dx).y * (1.0 - 0x1p-20);
+      const BoundCell<2> br = MakeBoundCell<2>(u0, a.g);
+      const BoundCell<2> bl = ShflUp<2>(br);
+      exact = !__all(!face || BoundPasses<2, DIR>(bl, br, s_crit, kbound));
+      if (!exact && face) kmin = KMinKey(kmin, DtKey(dt));
     }
-    __syncthreads();
-    // face c between cells c - 1 (thread td - 1) and c (thread td)
-    if (recon_ok && td >= 1 && c >= 0) {
-      T L[NQ], R[NQ], f[NC];
-      const int ptx = DIR == 0 ? tx - 1 : tx, pty = DIR == 0 ? ty : ty - 1;
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        L[k] = recR[k][pty][ptx];
-        R[k] = recL[k][ty][tx];
-      }
-      HllemFlux<2, DIR, true, false, T, TA>(f, L, R, gT);
-#pragma unroll
-      for (int k = 0; k < NC; ++k) flx[k][ty][tx] = f[k];
+    if (exact) {
+      const DtCell<2> dc = MakeDtCell<2, DA>(u0, a.g);
+      const DtCell<2> dl = ShflUp<2>(dc);
+      if (face)
+        kmin = KMinKey(kmin, DtKey(DA::quot(t.P.dx, FaceSpeed<2, DIR, DA>(dl, dc, a.g.gm1))));
     }
-    __syncthreads();
-    // update of owned cell c from faces c (this thread) and c + 1 (next)
-    if (recon_ok && td >= 1 && td <= TD - 2 && c >= 0 && c < nd) {
-      const double dt_dx = DivRn(dt, P.dx);
-      const int ntx = DIR == 0 ? tx + 1 : tx, nty = DIR == 0 ? ty : ty + 1;
+    T f[NC];
+    if constexpr (!FAST) {
+      double edge[NC];  // the rows' end lanes read a cell that no lane holds
 #pragma unroll
-      for (int k = 0; k < NC; ++k) {
-        const double fl = static_cast<double>(flx[k][ty][tx]);
-        const double fr = static_cast<double>(flx[k][nty][ntx]);
-        a.out[at + k * cs] = u0[k] + dt_dx * (fl - fr);
-      }
+      for (int k = 0; k < NC; ++k) edge[k] = t.td == 0 ? um[k] : up[k];
+      if (__builtin_expect(RegularStep(lh) && __all(RegularCell<2>(u0) && RegularCell<2>(edge)), 1))
+        BatchWaveFluxes<DIR, LIM, T, RegularArith<T>>(um, u0, up, lh, gT, f);
+      else
+        BatchWaveFluxes<DIR, LIM, T, TA>(um, u0, up, lh, gT, f);
+    } else {
+      BatchWaveFluxes<DIR, LIM, T, TA>(um, u0, up, static_cast<T>(lh), gT, f);
     }
-    __syncthreads();
+    // update of owned cell c from faces c (this lane) and c + 1 (the next)
+    T fn[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) fn[k] = ShiftDown(f[k]);
+    if (t.row_ok && t.td >= 1 && t.td <= W - 2 && t.c < t.nd) {
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        a.out[t.at + k * t.cs] =
+            u0[k] + dt_dx * (static_cast<double>(f[k]) - static_cast<double>(fn[k]));
+    }
   }
   kmin = WaveMinK(kmin);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) red[w] = kmin;
+  if ((threadIdx.x & 63) == 0) red[wave] = kmin;
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long m = red[0];
-    for (int i = 1; i < (TX * TY + 63) / 64; ++i) m = red[i] < m ? red[i] : m;
+    for (int i = 1; i < kWaves; ++i) m = red[i] < m ? red[i] : m;
     a.partials[blockIdx.x] = m;
+  }
+}
+
+// The smallest HLLEM stable dt of a level's faces in both directions (X in
+// partials[b], Y in partials[gridDim.x + b]) over the X sweep's tiles, without
+// the sweeps' reconstruction and fluxes: each lane forms its cell's speed
+// ingredients and those of the cell below, and takes the left cell's by DPP.
+// A level of a million cells: 24 us; two sweeps with a zero time step took 109.
+template <int W, bool FAST>
+__global__ __launch_bounds__(kSweepBlock) void BatchCflKernel(BatchArgs a) {
+  using DA = typename Policies<double, FAST>::DA;
+  constexpr int NC = 4;
+  constexpr int kWaves = kSweepBlock / 64;
+  __shared__ unsigned long long red[2][kWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  unsigned long long kmin[2] = {0x7ff0000000000000ull, 0x7ff0000000000000ull};
+  for (int tile = blockIdx.x * kWaves + wave; tile < a.ntiles; tile += gridDim.x * kWaves) {
+    const WaveTile<W> t = MakeWaveTile<0, W>(a, tile);
+    double u[NC], ub[NC], ut[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      u[k] = a.in[t.at + k * t.cs];
+      ub[k] = a.in[t.at + k * t.cs - t.ldx];
+      ut[k] = a.in[t.at + k * t.cs + t.ldx];
+    }
+    const bool face_x = t.row_inner && t.td >= 1 && t.c >= 0 && t.c <= t.nd;
+    const bool face_y = t.row_inner && t.td >= 1 && t.c >= 0 && t.c < t.nd;
+    const bool top = face_y && t.r == t.nt - 1;  // also the face above
+    auto speeds = [&](auto policy) {
+      using P = decltype(policy);
+      const DtCell<2> dc = MakeDtCell<2, P>(u, a.g), db = MakeDtCell<2, P>(ub, a.g);
+      const DtCell<2> dl = ShflUp<2>(dc);
+      double sx = 0.0, sy = 0.0;
+      if (face_x) sx = FaceSpeed<2, 0, P>(dl, dc, a.g.gm1);
+      if (face_y) sy = FaceSpeed<2, 1, P>(db, dc, a.g.gm1);
+      if (top) {
+        const DtCell<2> dt = MakeDtCell<2, P>(ut, a.g);
+        sy = SMax(sy, FaceSpeed<2, 1, P>(dc, dt, a.g.gm1));
+      }
+      // a tile's cells share dx: its largest speed gives its smallest dt
+      sx = WaveMaxSpeed(sx);
+      sy = WaveMaxSpeed(sy);
+      if (sx > 0.0) kmin[0] = KMinKey(kmin[0], DtKey(DA::quot(t.P.dx, sx)));
+      if (sy > 0.0) kmin[1] = KMinKey(kmin[1], DtKey(DA::quot(t.P.dx, sy)));
+    };
+    if constexpr (!FAST) {
+      if (__builtin_expect(__all(RegularCell<2>(u) && RegularCell<2>(ub) && RegularCell<2>(ut)), 1))
+        speeds(RegularArith<double>{});
+      else
+        speeds(DA{});
+    } else {
+      speeds(DA{});
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+    if ((threadIdx.x & 63) == 0) red[d][wave] = kmin[d];
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned long long m = red[threadIdx.x][0];
+    for (int i = 1; i < kWaves; ++i) m = KMinKey(m, red[threadIdx.x][i]);
+    a.partials[static_cast<int64_t>(threadIdx.x) * gridDim.x + blockIdx.x] = m;
   }
 }
 
@@ -219,26 +304,19 @@ __global__ void BatchGhostKernel(const PatchInfo* patches, int npatch, double* p
 struct Shape {
   int tx, ty;
 };
-// Candidate tile shapes (threads along x, along y) per sweep direction.
-constexpr Shape kShapesX[] = {{64, 4}, {32, 8}, {128, 2}, {64, 2}};
-constexpr Shape kShapesY[] = {{16, 16}, {32, 8}, {64, 4}, {8, 32}};
+// Candidate tile shapes (cells along x, along y) per sweep direction.
+constexpr Shape kShapesX[] = {{64, 1}, {32, 2}, {16, 4}, {8, 8}};
+constexpr Shape kShapesY[] = {{4, 16}, {8, 8}, {2, 32}, {1, 64}};
 constexpr int kNumShapes = 4;
 
-template <int DIR, class T, int TX, int TY, bool FAST>
+template <int DIR, class T, int W, bool FAST>
 void LaunchShape(hipStream_t s, const BatchArgs& a, int limiter, unsigned grid) {
+  const dim3 g(grid), b(kSweepBlock);
   switch (limiter) {
-  case kMinMod:
-    hipLaunchKernelGGL((BatchSweepKernel<DIR, kMinMod, T, TX, TY, FAST>), dim3(grid), dim3(TX * TY), 0, s, a);
-    break;
-  case kVanLeer:
-    hipLaunchKernelGGL((BatchSweepKernel<DIR, kVanLeer, T, TX, TY, FAST>), dim3(grid), dim3(TX * TY), 0, s, a);
-    break;
-  case kNoLimiter:
-    hipLaunchKernelGGL((BatchSweepKernel<DIR, kNoLimiter, T, TX, TY, FAST>), dim3(grid), dim3(TX * TY), 0, s, a);
-    break;
-  default:
-    hipLaunchKernelGGL((BatchSweepKernel<DIR, kNoGradient, T, TX, TY, FAST>), dim3(grid), dim3(TX * TY), 0, s, a);
-    break;
+  case kMinMod: hipLaunchKernelGGL((BatchSweepKernel<DIR, kMinMod, T, W, FAST>), g, b, 0, s, a); break;
+  case kVanLeer: hipLaunchKernelGGL((BatchSweepKernel<DIR, kVanLeer, T, W, FAST>), g, b, 0, s, a); break;
+  case kNoLimiter: hipLaunchKernelGGL((BatchSweepKernel<DIR, kNoLimiter, T, W, FAST>), g, b, 0, s, a); break;
+  default: hipLaunchKernelGGL((BatchSweepKernel<DIR, kNoGradient, T, W, FAST>), g, b, 0, s, a); break;
   }
 }
 
@@ -247,31 +325,67 @@ void LaunchSweepShape(hipStream_t s, int dir, int shape, const BatchArgs& a, int
                       unsigned grid) {
   if (dir == 0) {
     switch (shape) {
-    case 0: LaunchShape<0, T, 64, 4, FAST>(s, a, limiter, grid); break;
-    case 1: LaunchShape<0, T, 32, 8, FAST>(s, a, limiter, grid); break;
-    case 2: LaunchShape<0, T, 128, 2, FAST>(s, a, limiter, grid); break;
-    default: LaunchShape<0, T, 64, 2, FAST>(s, a, limiter, grid); break;
+    case 0: LaunchShape<0, T, 64, FAST>(s, a, limiter, grid); break;
+    case 1: LaunchShape<0, T, 32, FAST>(s, a, limiter, grid); break;
+    case 2: LaunchShape<0, T, 16, FAST>(s, a, limiter, grid); break;
+    default: LaunchShape<0, T, 8, FAST>(s, a, limiter, grid); break;
     }
   } else {
     switch (shape) {
-    case 0: LaunchShape<1, T, 16, 16, FAST>(s, a, limiter, grid); break;
-    case 1: LaunchShape<1, T, 32, 8, FAST>(s, a, limiter, grid); break;
-    case 2: LaunchShape<1, T, 64, 4, FAST>(s, a, limiter, grid); break;
-    default: LaunchShape<1, T, 8, 32, FAST>(s, a, limiter, grid); break;
+    case 0: LaunchShape<1, T, 16, FAST>(s, a, limiter, grid); break;
+    case 1: LaunchShape<1, T, 8, FAST>(s, a, limiter, grid); break;
+    case 2: LaunchShape<1, T, 32, FAST>(s, a, limiter, grid); break;
+    default: LaunchShape<1, T, 64, FAST>(s, a, limiter, grid); break;
     }
   }
 }
 
+template <bool FAST>
+void LaunchCflShape(hipStream_t s, int shape, const BatchArgs& a, unsigned grid) {
+  const dim3 g(grid), b(kSweepBlock);
+  switch (shape) {
+  case 0: hipLaunchKernelGGL((BatchCflKernel<64, FAST>), g, b, 0, s, a); break;
+  case 1: hipLaunchKernelGGL((BatchCflKernel<32, FAST>), g, b, 0, s, a); break;
+  case 2: hipLaunchKernelGGL((BatchCflKernel<16, FAST>), g, b, 0, s, a); break;
+  default: hipLaunchKernelGGL((BatchCflKernel<8, FAST>), g, b, 0, s, a); break;
+  }
+}
 
-// Flux-register contributions: one thread per register entry, the entry's
-// faces in order (the fine faces along the coarse face, or the coarse face),
-// each face flux computed exactly as BatchSweepKernel computes it (the two
-// adjacent cells' MUSCL-Hancock half-step states, then HLLEM) from the same
-// pool and time step, so the register holds the fluxes the sweeps applied.
+// Flux-register contributions: G lanes per register entry, one per face of
+// the entry (the fine faces along the coarse face, or the coarse face; a
+// single lane walks the faces of ratios other than 1, 2 and 4), each face flux
+// computed exactly as BatchSweepKernel computes it (the two adjacent cells'
+// MUSCL-Hancock half-step states, then HLLEM) from the same pool and time
+// step, so the register holds the fluxes the sweeps applied.  The entry's
+// first lane adds them in the faces' order.  A launch has some tens of
+// workgroups and lasts as long as one lane's chain: 6.1 to 7.1 us; two faces
+// in a row with IEEE sequences took 7.6 to 8.9.
+template <int DIR, int LIM, class T, class P>
+__device__ __forceinline__ void RegFaceFlux(const double (*s)[4], T lh, const Gas<T>& g, T* f) {
+  constexpr int NQ = 6, NC = 4;
+  T t[4][NC], rlA[NQ], rrA[NQ], rlB[NQ], rrB[NQ];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int k = 0; k < NC; ++k) t[c][k] = static_cast<T>(s[c][k]);
+  typename P::Inv irA, irB, ir;
+  ReconstructCell<2, DIR, LIM, T, P>(t[0], t[1], t[2], lh, g, rlA, rrA, ir, irA);
+  ReconstructCell<2, DIR, LIM, T, P>(t[1], t[2], t[3], lh, g, rlB, rrB, irB, ir);
+  HllemFlux<2, DIR, true, false, T, P>(f, rrA, irA, rlB, irB, g);
+}
+
+// Lanes per entry.
+__host__ __device__ constexpr int RegLanes(int ratio) {
+  return (ratio == 2 || ratio == 4) ? ratio : 1;
+}
+
 template <int DIR, int LIM, class T, bool FAST>
 __device__ __forceinline__ void RegFluxEntry(const batch::RegArgs& a, int q0) {
   using TA = typename Policies<T, FAST>::TA;
-  constexpr int NQ = 6, NC = 4;
+  constexpr int NC = 4;
+  const int lanes = RegLanes(a.ratio);
+  const int sub = q0 % lanes;
+  q0 /= lanes;
   if (q0 >= a.count) return;
   const int q = a.first + q0;
   const batch::RegFace F = a.faces[q];
@@ -280,29 +394,41 @@ __device__ __forceinline__ void RegFluxEntry(const batch::RegArgs& a, int q0) {
   const int64_t ldx = P.nx + 2 * kG, cs = ldx * (P.ny + 2 * kG);
   const int64_t step = DIR == 0 ? 1 : ldx, across = DIR == 0 ? ldx : 1;
   const double dt = *a.dt;
-  const T lh = static_cast<T>(DivRn(0.5 * dt, P.dx));
+  const double lh = DivRn(0.5 * dt, P.dx);
   const double w = P.dx * dt;
   const Gas<T> gT = GasT<T>(a.g);
   double acc[NC];
 #pragma unroll
   for (int k = 0; k < NC; ++k) acc[k] = a.reg[k * a.nfaces + q];
-  for (int m = 0; m < a.ratio; ++m) {
+  for (int m = sub; m < a.ratio; m += lanes) {
     const int64_t b = P.offset + (int64_t(j) + kG) * ldx + (int64_t(i) + kG) + m * across;
-    T s0[NQ], s1[NQ], s2[NQ], s3[NQ];
+    double s[4][NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-      s0[k] = static_cast<T>(a.pool[b - 2 * step + k * cs]);
-      s1[k] = static_cast<T>(a.pool[b - step + k * cs]);
-      s2[k] = static_cast<T>(a.pool[b + k * cs]);
-      s3[k] = static_cast<T>(a.pool[b + step + k * cs]);
+      s[0][k] = a.pool[b - 2 * step + k * cs];
+      s[1][k] = a.pool[b - step + k * cs];
+      s[2][k] = a.pool[b + k * cs];
+      s[3][k] = a.pool[b + step + k * cs];
     }
-    T rlA[NQ], rrA[NQ], rlB[NQ], rrB[NQ], f[NC];
-    ReconstructCell<2, DIR, LIM, T, TA>(s0, s1, s2, lh, gT, rlA, rrA);
-    ReconstructCell<2, DIR, LIM, T, TA>(s1, s2, s3, lh, gT, rlB, rrB);
-    HllemFlux<2, DIR, true, false, T, TA>(f, rrA, rlB, gT);
+    T f[NC];
+    if constexpr (!FAST) {
+      if (RegularStep(lh) && __all(RegularCell<2>(s[0]) && RegularCell<2>(s[1]) &&
+                                   RegularCell<2>(s[2]) && RegularCell<2>(s[3])))
+        RegFaceFlux<DIR, LIM, T, RegularArith<T>>(s, lh, gT, f);
+      else
+        RegFaceFlux<DIR, LIM, T, TA>(s, lh, gT, f);
+    } else {
+      RegFaceFlux<DIR, LIM, T, TA>(s, static_cast<T>(lh), gT, f);
+    }
+    for (int l = 0; l < lanes; ++l) {
 #pragma unroll
-    for (int k = 0; k < NC; ++k) acc[k] = acc[k] + a.sign * (w * static_cast<double>(f[k]));
+      for (int k = 0; k < NC; ++k) {
+        const T v = lanes == 1 ? f[k] : __shfl(f[k], (threadIdx.x & 63) - sub + l, 64);
+        acc[k] = acc[k] + a.sign * (w * static_cast<double>(v));
+      }
+    }
   }
+  if (sub > 0) return;
 #pragma unroll
   for (int k = 0; k < NC; ++k) a.reg[k * a.nfaces + q] = acc[k];
 }
@@ -322,7 +448,8 @@ __global__ __launch_bounds__(256) void RegFluxKernel(batch::RegArgs a0, batch::R
 
 template <int DIR, class T, bool FAST>
 void LaunchRegFluxT(hipStream_t s, const batch::RegArgs& a0, const batch::RegArgs& a1) {
-  const int nb0 = (a0.count + 255) / 256, nb1 = (a1.count + 255) / 256;
+  const int nb0 = (a0.count * RegLanes(a0.ratio) + 255) / 256;
+  const int nb1 = (a1.count * RegLanes(a1.ratio) + 255) / 256;
   const dim3 grid(nb0 + nb1);
   switch (a0.count > 0 ? a0.limiter : a1.limiter) {
   case kMinMod: hipLaunchKernelGGL((RegFluxKernel<DIR, kMinMod, T, FAST>), grid, dim3(256), 0, s, a0, a1, nb0); break;
@@ -351,6 +478,10 @@ void batch::LaunchSweepFast(hipStream_t s, int dir, int shape, const BatchArgs& 
     LaunchSweepShape<float, true>(s, dir, shape, a, a.limiter, grid);
   else
     LaunchSweepShape<double, true>(s, dir, shape, a, a.limiter, grid);
+}
+
+void batch::LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid) {
+  LaunchCflShape<true>(s, shape, a, grid);
 }
 
 } // namespace fvs
@@ -401,9 +532,9 @@ int UploadTiles(fvs_batch* b, const std::vector<int4>& tiles, int4** dst, int* n
   FVS_HIP_CHECK(hipMalloc(dst, std::max<size_t>(tiles.size(), 1) * sizeof(int4)));
   FVS_HIP_CHECK(hipMemcpy(*dst, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
   *n = static_cast<int>(tiles.size());
-  // persistent grid: a few workgroups per CU, never more than tiles
-  const unsigned want = static_cast<unsigned>(b->cus * 8);
-  *grid = std::max(1u, std::min<unsigned>(want, static_cast<unsigned>(tiles.size())));
+  // persistent grid: a few workgroups per CU, a wave per tile at most
+  const unsigned want = static_cast<unsigned>(b->cus * 8), per = kSweepBlock / 64;
+  *grid = std::max(1u, std::min<unsigned>(want, static_cast<unsigned>((tiles.size() + per - 1) / per)));
   return FVS_OK;
 }
 
@@ -421,15 +552,12 @@ int Upload(fvs_batch* b, int dir, int shape_idx) {
   return FVS_OK;
 }
 
-// The sweep kernel alone, its per-workgroup minima written to `partials`
-// (b->grid[dir] entries).
-int LaunchSweepOnly(fvs_batch* b, hipStream_t s, int dir, int src, unsigned long long* partials,
-                    int precision, bool grown = false) {
+BatchArgs SweepArgsOf(const fvs_batch* b, int dir, int src, unsigned long long* partials,
+                      bool grown) {
   BatchArgs a;
   a.patches = b->patches;
   a.tiles = grown ? b->tiles_grown[dir] : b->tiles[dir];
   a.ntiles = grown ? b->ntiles_grown[dir] : b->ntiles[dir];
-  const unsigned grid = grown ? b->grid_grown[dir] : b->grid[dir];
   a.in = b->pool[src];
   a.out = b->pool[1 - src];
   a.dt = b->dts;
@@ -438,6 +566,15 @@ int LaunchSweepOnly(fvs_batch* b, hipStream_t s, int dir, int src, unsigned long
   a.g.gm1 = b->h->desc.gamma - 1.0;
   a.limiter = b->h->desc.limiter;
   a.partials = partials;
+  return a;
+}
+
+// The sweep kernel alone, its per-workgroup minima written to `partials`
+// (b->grid[dir] entries).
+int LaunchSweepOnly(fvs_batch* b, hipStream_t s, int dir, int src, unsigned long long* partials,
+                    int precision, bool grown = false) {
+  const BatchArgs a = SweepArgsOf(b, dir, src, partials, grown);
+  const unsigned grid = grown ? b->grid_grown[dir] : b->grid[dir];
   if (precision != FVS_FP64)
     batch::LaunchSweepFast(s, dir, b->shape[dir], a, grid, precision);
   else
@@ -452,10 +589,6 @@ int Launch(fvs_batch* b, hipStream_t s, int dir, int src, double* dt_out, int pr
 }
 
 } // namespace
-
-int fvs::batch::Sweep(fvs_batch* b, hipStream_t s, int dir, int src, double* dt_out) {
-  return Launch(b, s, dir, src, dt_out, b->h->desc.precision);
-}
 
 namespace {
 
@@ -498,6 +631,17 @@ int fvs::batch::LaunchSlotMin(hipStream_t s, unsigned long long* partials, int n
   }
   FVS_LAUNCH_CHECK();
   return FVS_OK;
+}
+
+int fvs::batch::StableDts(fvs_batch* b, hipStream_t s, double* out2) {
+  // the grids of X tiles hold at most half of the partials buffer
+  const BatchArgs a = SweepArgsOf(b, 0, 0, b->partials, false);
+  if (b->h->desc.precision != FVS_FP64)
+    batch::LaunchCflFast(s, b->shape[0], a, b->grid[0]);
+  else
+    LaunchCflShape<false>(s, b->shape[0], a, b->grid[0]);
+  FVS_LAUNCH_CHECK();
+  return LaunchSlotMin(s, b->partials, 2, static_cast<int>(b->grid[0]), out2, false);
 }
 
 int fvs::batch::SweepPartials(fvs_batch* b, hipStream_t s, int dir, int src,

@@ -36,6 +36,9 @@ struct BatchArgs {
 void LaunchSweepFast(hipStream_t s, int dir, int shape, const BatchArgs& a, unsigned grid,
                      int precision);
 
+// The level's CFL pass of the same modes over the X tiles of `shape`.
+void LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid);
+
 // One coarse face of a coarse-fine interface (a flux-register entry): the
 // fine patch's `ratio` faces along it and the coarse face itself.  (fi, fj)
 // is the fine patch's cell right of / above the first fine face, (ci, cj)
@@ -100,10 +103,10 @@ struct fvs_batch {
 
 namespace fvs {
 namespace batch {
+// The smallest stable dt of pool 0's faces in x (out2[0]) and y (out2[1]).
+int StableDts(fvs_batch* b, hipStream_t s, double* out2);
 // One batched sweep of direction dir from pool src into pool 1 - src on
-// stream s; the minimum stable dt of its faces goes to *dt_out (nullable).
-int Sweep(fvs_batch* b, hipStream_t s, int dir, int src, double* dt_out);
-// The same sweep without its reduction: the per-workgroup minima (keys, at
+// stream s without its reduction: the per-workgroup minima (keys, at
 // most 8 per CU) go to `partials`.  grown: the sweep also updates the kG
 // ghost rows (dir 0) / columns (dir 1) on each side across the direction,
 // reading the ghost layers along it; its CFL minimum covers the interior

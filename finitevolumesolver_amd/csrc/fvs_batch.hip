@@ -68,7 +68,7 @@ __device__ __forceinline__ unsigned long long WaveMinK(unsigned long long k) {
 // DPP shifts; the shifts across a row's ends carry values no lane uses.
 // Loads across the sweep are short where W is large in Y, which the caches
 // absorb: the kernel is bound by its FP64 instructions.  A level of a million
-// cells: X 32 to 33 us, Y 37 to 44; with states and fluxes staged in LDS by
+// cells: X 32, Y 33 us (about 22 of instruction issue); with states and fluxes staged in LDS by
 // workgroup tiles (three barriers a tile, IEEE sequences) 42 and 48.  Every lane loads (clamped into the patch's
 // ghost ring) and computes, and the stores and minima are masked.
 template <int W> struct WaveTile {
@@ -230,11 +230,15 @@ __global__ __launch_bounds__(kSweepBlock) void BatchCflKernel(BatchArgs a) {
     for (int k = 0; k < NC; ++k) {
       u[k] = a.in[t.at + k * t.cs];
       ub[k] = a.in[t.at + k * t.cs - t.ldx];
-      ut[k] = a.in[t.at + k * t.cs + t.ldx];
+      ut[k] = ub[k];
     }
     const bool face_x = t.row_inner && t.td >= 1 && t.c >= 0 && t.c <= t.nd;
     const bool face_y = t.row_inner && t.td >= 1 && t.c >= 0 && t.c < t.nd;
     const bool top = face_y && t.r == t.nt - 1;  // also the face above
+    if (top) {
+#pragma unroll
+      for (int k = 0; k < NC; ++k) ut[k] = a.in[t.at + k * t.cs + t.ldx];
+    }
     auto speeds = [&](auto policy) {
       using P = decltype(policy);
       const DtCell<2> dc = MakeDtCell<2, P>(u, a.g), db = MakeDtCell<2, P>(ub, a.g);
@@ -518,8 +522,16 @@ void BuildTiles(const std::vector<PatchInfo>& ps, int dir, Shape sh, int grow,
   for (size_t p = 0; p < ps.size(); ++p) {
     const int nd = dir == 0 ? ps[p].nx : ps[p].ny;
     const int nt = dir == 0 ? ps[p].ny : ps[p].nx;
-    for (int r = -grow; r < nt + grow; r += tt)
-      for (int s = 0; s < nd; s += own) out.push_back(make_int4(int(p), s, r, grow));
+    // x fastest: a Y tile is a few columns wide, and its neighbours in x,
+    // which share its cache lines, belong to the same workgroup (level of a
+    // million cells: Y sweep 33 us, with y fastest 37 to 44)
+    if (dir == 0) {
+      for (int r = -grow; r < nt + grow; r += tt)
+        for (int s = 0; s < nd; s += own) out.push_back(make_int4(int(p), s, r, grow));
+    } else {
+      for (int s = 0; s < nd; s += own)
+        for (int r = -grow; r < nt + grow; r += tt) out.push_back(make_int4(int(p), s, r, grow));
+    }
   }
 }
 

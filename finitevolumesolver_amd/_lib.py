@@ -188,6 +188,8 @@ SIGNATURES = {
     "fvs_amr_advance": (_I, [_P, _D]),
     "fvs_amr_level_cfl": (_I, [_P, _P]),
     "fvs_amr_stable_dt": (_I, [_P, _PD]),
+    "fvs_amr_begin_step": (_I, [_P, _PD]),
+    "fvs_amr_restore": (_I, [_P]),
     "fvs_amr_set_graphs": (_I, [_P, _I]),
     "fvs_amr_set_sequencing": (_I, [_P, _I]),
     "fvs_amr_cycle": (_I, [_P, C.POINTER(C.c_int64)]),

@@ -269,8 +269,9 @@ class AmrHierarchy:
                 break
             if regrid_every > 0 and step > 0 and step % regrid_every == 0:
                 self._adopt(self.regrid_all(0, tol_rho, tol_p))
-            dt = limited(cfl * self.stable_dt())
-            saved = [b.download(0) for b in self.levels]
+            stable = C.c_double()
+            L.check(self._lib.fvs_amr_begin_step(self.a, C.byref(stable)))
+            dt = limited(cfl * stable.value)
             cycle, time = self.cycle, self.time
             for attempt in range(max_restarts + 1):
                 self.advance(dt)
@@ -278,8 +279,7 @@ class AmrHierarchy:
                 limit = min(got[l] * self.ratio ** l for l in range(self.nlevels))
                 if all(got[l] >= dt / self.ratio ** l for l in range(self.nlevels)):
                     break
-                for b, pool in zip(self.levels, saved):
-                    b.upload(pool, 0)
+                L.check(self._lib.fvs_amr_restore(self.a))
                 self.cycle, self.time = cycle, time
                 dt = limited(cfl * limit)
             else:

@@ -231,6 +231,10 @@ struct fvs_amr {
   double* dtc = nullptr;  // device: the coarse time step of the current advance
   unsigned long long* slot_partials = nullptr;  // per sweep of a step: pcap minima
   int pcap = 0;
+  double* host = nullptr;  // pinned, ncfl values read back
+  // the levels' states kept by fvs_amr_begin_step (allocated by its first call)
+  std::vector<double*> kept;
+  bool has_kept = false;
   hipStream_t s = nullptr;  // stream the operations are enqueued on
   // whole coarse steps captured per cycle parity (the split order flips)
   int use_graphs = 1;
@@ -519,6 +523,7 @@ int Build(fvs_amr* A, const int32_t* lo) {
   FVS_HIP_CHECK(hipMalloc(&A->dtc, sizeof(double)));
   A->pcap = A->lv[0]->cus * 8;  // the batched sweeps' largest grid
   FVS_HIP_CHECK(hipMalloc(&A->slot_partials, sizeof(unsigned long long) * A->pcap * slot));
+  FVS_HIP_CHECK(hipHostMalloc(&A->host, A->ncfl * sizeof(double), hipHostMallocDefault));
   FVS_HIP_CHECK(hipStreamCreateWithFlags(&A->cap, hipStreamNonBlocking));
   return FVS_OK;
 }
@@ -737,6 +742,9 @@ int fvs_amr_destroy(fvs_amr* A) {
       if (p) (void)hipFree(p);
   }
   if (A->cfl) (void)hipFree(A->cfl);
+  if (A->host) (void)hipHostFree(A->host);
+  for (double* p : A->kept)
+    if (p) (void)hipFree(p);
   delete A;
   return FVS_OK;
 }
@@ -950,8 +958,8 @@ int fvs_amr_level_cfl(fvs_amr* A, double* host) {
     SetError("bad argument");
     return FVS_BAD_ARGUMENT;
   }
-  std::vector<double> v(A->ncfl);
-  FVS_HIP_CHECK(hipMemcpyAsync(v.data(), A->cfl, A->ncfl * sizeof(double),
+  const double* v = A->host;
+  FVS_HIP_CHECK(hipMemcpyAsync(A->host, A->cfl, A->ncfl * sizeof(double),
                                hipMemcpyDeviceToHost, A->h->stream));
   FVS_HIP_CHECK(hipStreamSynchronize(A->h->stream));
   for (int l = 0; l < A->nlevels; ++l) {
@@ -964,28 +972,83 @@ int fvs_amr_level_cfl(fvs_amr* A, double* host) {
   return FVS_OK;
 }
 
+// Ghost fill and the CFL pass of every level, one reduction for all (the
+// slots are the sweeps', of which every level has at least two), and the copy
+// of the minima to the host; not synchronised.
+static int EnqueueStableDt(fvs_amr* A) {
+  const int base = A->ncfl - 2 * A->nlevels;
+  A->s = A->h->stream;
+  for (int l = 0; l < A->nlevels; ++l) {
+    if (int rc = FillGhosts(A, l, 0)) return rc;
+    if (int rc = batch::StableDtPartials(
+            A->lv[l], A->s, A->slot_partials + static_cast<int64_t>(2 * l) * A->pcap, A->pcap))
+      return rc;
+  }
+  if (int rc = batch::LaunchSlotMin(A->s, A->slot_partials, 2 * A->nlevels, A->pcap, A->cfl + base,
+                                    false))
+    return rc;
+  FVS_HIP_CHECK(hipMemcpyAsync(A->host, A->cfl + base, 2 * A->nlevels * sizeof(double),
+                               hipMemcpyDeviceToHost, A->s));
+  return FVS_OK;
+}
+
+// The coarse step's stable dt from the minima on the host.
+static double CoarseStableDt(const fvs_amr* A) {
+  double m = __builtin_huge_val();
+  double scale = 1.0;
+  for (int l = 0; l < A->nlevels; ++l) {
+    m = std::min(m, scale * std::min(A->host[2 * l], A->host[2 * l + 1]));
+    scale *= A->ratio;
+  }
+  return m;
+}
+
 int fvs_amr_stable_dt(fvs_amr* A, double* dt_host) {
   if (!A || !dt_host) {
     SetError("bad argument");
     return FVS_BAD_ARGUMENT;
   }
-  const int base = A->ncfl - 2 * A->nlevels;
-  A->s = A->h->stream;
-  for (int l = 0; l < A->nlevels; ++l) {
-    if (int rc = FillGhosts(A, l, 0)) return rc;
-    if (int rc = batch::StableDts(A->lv[l], A->s, A->cfl + base + 2 * l)) return rc;
-  }
-  std::vector<double> v(2 * A->nlevels);
-  FVS_HIP_CHECK(hipMemcpyAsync(v.data(), A->cfl + base, v.size() * sizeof(double),
-                               hipMemcpyDeviceToHost, A->h->stream));
+  if (int rc = EnqueueStableDt(A)) return rc;
   FVS_HIP_CHECK(hipStreamSynchronize(A->h->stream));
-  double m = __builtin_huge_val();
-  double scale = 1.0;
-  for (int l = 0; l < A->nlevels; ++l) {
-    m = std::min(m, scale * std::min(v[2 * l], v[2 * l + 1]));
-    scale *= A->ratio;
+  *dt_host = CoarseStableDt(A);
+  return FVS_OK;
+}
+
+int fvs_amr_begin_step(fvs_amr* A, double* dt_host) {
+  if (!A || !dt_host) {
+    SetError("bad argument");
+    return FVS_BAD_ARGUMENT;
   }
-  *dt_host = m;
+  A->kept.resize(A->nlevels, nullptr);
+  for (int l = 0; l < A->nlevels; ++l)
+    if (!A->kept[l])
+      FVS_HIP_CHECK(hipMalloc(&A->kept[l], A->lv[l]->pool_size * sizeof(double)));
+  A->has_kept = false;
+  if (int rc = EnqueueStableDt(A)) return rc;
+  // the copies run while the host waits for the minima and forms dt
+  hipEvent_t ready;
+  FVS_HIP_CHECK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
+  hipError_t e = hipEventRecord(ready, A->s);
+  for (int l = 0; l < A->nlevels && e == hipSuccess; ++l)
+    e = hipMemcpyAsync(A->kept[l], A->lv[l]->pool[0], A->lv[l]->pool_size * sizeof(double),
+                       hipMemcpyDeviceToDevice, A->s);
+  if (e == hipSuccess) e = hipEventSynchronize(ready);
+  (void)hipEventDestroy(ready);
+  FVS_HIP_CHECK(e);
+  A->has_kept = true;
+  *dt_host = CoarseStableDt(A);
+  return FVS_OK;
+}
+
+int fvs_amr_restore(fvs_amr* A) {
+  if (!A || !A->has_kept) {
+    SetError(A ? "no kept state" : "bad argument");
+    return FVS_BAD_ARGUMENT;
+  }
+  for (int l = 0; l < A->nlevels; ++l)
+    FVS_HIP_CHECK(hipMemcpyAsync(A->lv[l]->pool[0], A->kept[l],
+                                 A->lv[l]->pool_size * sizeof(double), hipMemcpyDeviceToDevice,
+                                 A->h->stream));
   return FVS_OK;
 }
 

@@ -68,9 +68,10 @@ __device__ __forceinline__ unsigned long long WaveMinK(unsigned long long k) {
 // DPP shifts; the shifts across a row's ends carry values no lane uses.
 // Loads across the sweep are short where W is large in Y, which the caches
 // absorb: the kernel is bound by its FP64 instructions.  A level of a million
-// cells: X 32, Y 33 us (about 22 of instruction issue); with states and fluxes staged in LDS by
-// workgroup tiles (three barriers a tile, IEEE sequences) 42 and 48.  Every lane loads (clamped into the patch's
-// ghost ring) and computes, and the stores and minima are masked.
+// cells: X 32, Y 33 us (about 22 of instruction issue); with states and fluxes
+// staged in LDS by workgroup tiles (three barriers a tile, IEEE sequences) 42
+// and 48.  Every lane loads (clamped into the patch's ghost ring) and computes,
+// and the stores and minima are masked.
 template <int W> struct WaveTile {
   PatchInfo P;
   int c, r, w, nd, nt, td;
@@ -211,12 +212,13 @@ __global__ __launch_bounds__(kSweepBlock) void BatchSweepKernel(BatchArgs a) {
 }
 
 // The smallest HLLEM stable dt of a level's faces in both directions (X in
-// partials[b], Y in partials[gridDim.x + b]) over the X sweep's tiles, without
+// partials[b], Y in partials[cap + b], +inf in the rest of the two slots of cap
+// entries) over the X sweep's tiles, without
 // the sweeps' reconstruction and fluxes: each lane forms its cell's speed
 // ingredients and those of the cell below, and takes the left cell's by DPP.
 // A level of a million cells: 24 us; two sweeps with a zero time step took 109.
 template <int W, bool FAST>
-__global__ __launch_bounds__(kSweepBlock) void BatchCflKernel(BatchArgs a) {
+__global__ __launch_bounds__(kSweepBlock) void BatchCflKernel(BatchArgs a, int cap) {
   using DA = typename Policies<double, FAST>::DA;
   constexpr int NC = 4;
   constexpr int kWaves = kSweepBlock / 64;
@@ -272,7 +274,9 @@ __global__ __launch_bounds__(kSweepBlock) void BatchCflKernel(BatchArgs a) {
   if (threadIdx.x < 2) {
     unsigned long long m = red[threadIdx.x][0];
     for (int i = 1; i < kWaves; ++i) m = KMinKey(m, red[threadIdx.x][i]);
-    a.partials[static_cast<int64_t>(threadIdx.x) * gridDim.x + blockIdx.x] = m;
+    unsigned long long* slot = a.partials + static_cast<int64_t>(threadIdx.x) * cap;
+    slot[blockIdx.x] = m;
+    for (int i = blockIdx.x + gridDim.x; i < cap; i += gridDim.x) slot[i] = 0x7ff0000000000000ull;
   }
 }
 
@@ -345,13 +349,13 @@ void LaunchSweepShape(hipStream_t s, int dir, int shape, const BatchArgs& a, int
 }
 
 template <bool FAST>
-void LaunchCflShape(hipStream_t s, int shape, const BatchArgs& a, unsigned grid) {
+void LaunchCflShape(hipStream_t s, int shape, const BatchArgs& a, unsigned grid, int cap) {
   const dim3 g(grid), b(kSweepBlock);
   switch (shape) {
-  case 0: hipLaunchKernelGGL((BatchCflKernel<64, FAST>), g, b, 0, s, a); break;
-  case 1: hipLaunchKernelGGL((BatchCflKernel<32, FAST>), g, b, 0, s, a); break;
-  case 2: hipLaunchKernelGGL((BatchCflKernel<16, FAST>), g, b, 0, s, a); break;
-  default: hipLaunchKernelGGL((BatchCflKernel<8, FAST>), g, b, 0, s, a); break;
+  case 0: hipLaunchKernelGGL((BatchCflKernel<64, FAST>), g, b, 0, s, a, cap); break;
+  case 1: hipLaunchKernelGGL((BatchCflKernel<32, FAST>), g, b, 0, s, a, cap); break;
+  case 2: hipLaunchKernelGGL((BatchCflKernel<16, FAST>), g, b, 0, s, a, cap); break;
+  default: hipLaunchKernelGGL((BatchCflKernel<8, FAST>), g, b, 0, s, a, cap); break;
   }
 }
 
@@ -484,8 +488,8 @@ void batch::LaunchSweepFast(hipStream_t s, int dir, int shape, const BatchArgs& 
     LaunchSweepShape<double, true>(s, dir, shape, a, a.limiter, grid);
 }
 
-void batch::LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid) {
-  LaunchCflShape<true>(s, shape, a, grid);
+void batch::LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid, int cap) {
+  LaunchCflShape<true>(s, shape, a, grid, cap);
 }
 
 } // namespace fvs
@@ -645,15 +649,19 @@ int fvs::batch::LaunchSlotMin(hipStream_t s, unsigned long long* partials, int n
   return FVS_OK;
 }
 
-int fvs::batch::StableDts(fvs_batch* b, hipStream_t s, double* out2) {
-  // the grids of X tiles hold at most half of the partials buffer
-  const BatchArgs a = SweepArgsOf(b, 0, 0, b->partials, false);
+int fvs::batch::StableDtPartials(fvs_batch* b, hipStream_t s, unsigned long long* partials,
+                                 int cap) {
+  if (b->grid[0] > static_cast<unsigned>(cap)) {
+    SetError("batch: more workgroups than partial minima");
+    return FVS_BAD_ARGUMENT;
+  }
+  const BatchArgs a = SweepArgsOf(b, 0, 0, partials, false);
   if (b->h->desc.precision != FVS_FP64)
-    batch::LaunchCflFast(s, b->shape[0], a, b->grid[0]);
+    batch::LaunchCflFast(s, b->shape[0], a, b->grid[0], cap);
   else
-    LaunchCflShape<false>(s, b->shape[0], a, b->grid[0]);
+    LaunchCflShape<false>(s, b->shape[0], a, b->grid[0], cap);
   FVS_LAUNCH_CHECK();
-  return LaunchSlotMin(s, b->partials, 2, static_cast<int>(b->grid[0]), out2, false);
+  return FVS_OK;
 }
 
 int fvs::batch::SweepPartials(fvs_batch* b, hipStream_t s, int dir, int src,

@@ -37,7 +37,7 @@ void LaunchSweepFast(hipStream_t s, int dir, int shape, const BatchArgs& a, unsi
                      int precision);
 
 // The level's CFL pass of the same modes over the X tiles of `shape`.
-void LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid);
+void LaunchCflFast(hipStream_t s, int shape, const BatchArgs& a, unsigned grid, int cap);
 
 // One coarse face of a coarse-fine interface (a flux-register entry): the
 // fine patch's `ratio` faces along it and the coarse face itself.  (fi, fj)
@@ -103,8 +103,9 @@ struct fvs_batch {
 
 namespace fvs {
 namespace batch {
-// The smallest stable dt of pool 0's faces in x (out2[0]) and y (out2[1]).
-int StableDts(fvs_batch* b, hipStream_t s, double* out2);
+// Partial minima of the stable dts of pool 0's faces: x in partials[0, cap), y
+// in partials[cap, 2 cap) (keys, to be reduced by LaunchSlotMin).
+int StableDtPartials(fvs_batch* b, hipStream_t s, unsigned long long* partials, int cap);
 // One batched sweep of direction dir from pool src into pool 1 - src on
 // stream s without its reduction: the per-workgroup minima (keys, at
 // most 8 per CU) go to `partials`.  grown: the sweep also updates the kG

@@ -638,8 +638,14 @@ int fvs_amr_level_cfl(fvs_amr* amr, double* host);
 /* Stable coarse dt of the current state: min over levels of ratio^l times
  * the level's minimum HLLEM stable dt over both directions
  * (SubcycleFineFirstSolver::ComputeStableDt, :101-112), without the CFL
- * factor.  Uses pool 1 of each level as scratch; synchronises. */
+ * factor.  Fills the ghost layers of pool 0; synchronises. */
 int fvs_amr_stable_dt(fvs_amr* amr, double* dt_host);
+/* fvs_amr_stable_dt that also keeps the state (pool 0 of every level, ghost
+ * layers included, in device memory of the hierarchy) for fvs_amr_restore,
+ * which puts it back any number of times: the reference's data / scratch pair.
+ * Waits for the dt only. */
+int fvs_amr_begin_step(fvs_amr* amr, double* dt_host);
+int fvs_amr_restore(fvs_amr* amr);
 /* Coarse-step count of the hierarchy (it selects the split order of the
  * next step, MakeSplitDirections).  A caller that undoes a step by
  * restoring the levels' states restores the count with it, as the

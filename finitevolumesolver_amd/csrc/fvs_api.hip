@@ -661,7 +661,7 @@ int fvs_split_sweep(fvs_handle* h, const double* const* cons_in, double* const* 
   }
   a.dt_val = dt;
   a.check = stable_dt_device != nullptr;
-  const int64_t nb = SweepBlocks(h->desc.dim, dir, a.n, a.seg);
+  const int64_t nb = HllemSweepBlocks(h->desc.dim, dir, a.n, a.seg, h->desc.precision == FVS_FP64);
   if (a.check) {
     if (int rc = EnsurePartials(h, nb)) return rc;
     a.partials = h->partials;
@@ -1038,7 +1038,9 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch, fvs_level** out
   int64_t np = D * CflBlocks(D, n);
   int64_t sweep_blocks = 0;
   for (int d = 0; d < D; ++d)
-    sweep_blocks = std::max<int64_t>(sweep_blocks, SweepBlocks(D, d, n, PencilSeg(D, d, n)));
+    sweep_blocks = std::max<int64_t>(
+        sweep_blocks,
+        HllemSweepBlocks(D, d, n, PencilSeg(D, d, n), h->desc.precision == FVS_FP64));
   // the checked sweeps of a step keep their partial minima side by side
   // (at most 2D - 1 of them, Strang)
   np = std::max<int64_t>(np, (2 * D - 1) * sweep_blocks);
@@ -1274,8 +1276,10 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
   int src = b0, dst = b1;
   CheckList checks{};
   checks.stride = 0;
+  const bool ieee = h->desc.precision == FVS_FP64;
   for (int d = 0; d < D; ++d)
-    checks.stride = std::max<int64_t>(checks.stride, SweepBlocks(D, d, L->n, PencilSeg(D, d, L->n)));
+    checks.stride = std::max<int64_t>(
+        checks.stride, HllemSweepBlocks(D, d, L->n, PencilSeg(D, d, L->n), ieee));
   for (int w = 0; w < ns; ++w) {
     SweepArgs a;
     double* outp[5];
@@ -1307,7 +1311,7 @@ static int LaunchLevelStep(fvs_level* L, hipStream_t s, int cur, int64_t cyc,
     if (a.check) {
       if (checks.count >= kMaxChecks) return FVS_BAD_ARGUMENT;
       a.partials = L->partials + checks.count * checks.stride;
-      checks.n[checks.count++] = SweepBlocks(D, seq[w], L->n, a.seg);
+      checks.n[checks.count++] = HllemSweepBlocks(D, seq[w], L->n, a.seg, ieee);
     }
     rc = Timed(L, s, FVS_TIMER_SWEEP_X + seq[w], [&] { return LaunchSweep(h->desc, s, seq[w], a); });
     if (rc) break;

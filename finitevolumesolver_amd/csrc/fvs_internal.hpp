@@ -125,6 +125,9 @@ struct Ctl {
 
 // Number of workgroups (= partial minima) of a sweep / of the CFL pass.
 int64_t SweepBlocks(int dim, int dir, const int64_t n[3], int seg);
+// The same of LaunchSweep, whose small 2D Y sweeps in IEEE arithmetic take
+// another kernel.
+int64_t HllemSweepBlocks(int dim, int dir, const int64_t n[3], int seg, bool ieee);
 int64_t CflBlocks(int dim, const int64_t n[3]);
 // Cells per thread of a Y/Z pencil sweep: 32, fewer when the patch is too
 // small to give the device about 1,024 workgroups (down to 1).

@@ -118,7 +118,7 @@ template <class T> struct IeeeArith {
 // rounded reciprocal is correctly rounded (Markstein, IBM J. Res. Dev. 34,
 // 1990).  The square root is the compiler's iteration (Goldschmidt, two
 // residual steps) without its scaling.  A split step of a 160^3 patch took
-// 561 us with IeeeArith alone and takes 460, one of a 256^2 patch 66.7 and 61.5.
+// 561 us with IeeeArith alone and takes 460.
 //
 // Regular cells (RegularCell) and a dt / dx within 2^100 of 1 (RegularStep)
 // keep every operand of a fused sweep far from the exponents that would need

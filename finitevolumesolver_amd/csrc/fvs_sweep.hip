@@ -523,6 +523,83 @@ __global__ __launch_bounds__(kBlock) void SweepPencilKernel(SweepArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// IEEE Y sweep of a 2D patch too small for long pencils (YLanes): a wave's
+// lanes are 16 rows of 4 columns, rows 1 .. 14 owned, with each lane
+// reconstructing one cell and half-step states and fluxes passing by DPP, as in
+// the X sweep; a pencil of S rows reconstructs S + 2 cells one after the other.
+// A workgroup covers 16 columns, one 128-byte line a row.
+constexpr int kYRows = 16, kYOwned = kYRows - 2, kYCols = 64 / kYRows * (kBlock / 64);
+
+template <bool LARR, class P>
+__device__ __forceinline__ void LaneFluxes(const double* um, const double* u, const double* up,
+                                           double lh, const Gas<double>& g, const SweepArgs& a,
+                                           double* F) {
+  constexpr int D = 2, NQ = D + 4;
+  double recL[NQ], recR[NQ], recRprev[NQ];
+  typename P::Inv irL, irR, irRprev;
+  ReconAny<D, 1, double, P>(um, u, up, lh, g, a.limiter, a.muscl, recL, recR, irL, irR);
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) recRprev[k] = ShiftUp(recR[k]);
+  irRprev.b = recRprev[0];
+  if constexpr (!std::is_same<P, IeeeArith<double>>::value) irRprev.y = ShiftUp(irR.y);
+  FaceFlux<D, 1, LARR, double, P>(F, recRprev, irRprev, recL, irL, g, 0);
+}
+
+template <bool LARR>
+__global__ __launch_bounds__(kBlock) void SweepYLanesKernel(SweepArgs a) {
+  using A = IeeeArith<double>;
+  constexpr int D = 2, NC = D + 2;
+  if (a.halt && *a.halt) return;
+  const int64_t nx = a.n[0], ny = a.n[1];
+  const int64_t ncols = (nx + kYCols - 1) / kYCols;
+  const int lane = threadIdx.x & 63, row = lane % kYRows;
+  const int64_t x = (blockIdx.x % ncols) * kYCols + threadIdx.x / kYRows;
+  const int64_t j = (blockIdx.x / ncols) * kYOwned - 1 + row;  // -1 .. ny (+ tile padding)
+  const int64_t xc = x < nx ? x : nx - 1;
+  const bool face = x < nx && row >= 1 && j <= ny;
+  double um[NC], u[NC], up[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    um[k] = a.in[k][xc + Clamp(j - 1, ny) * nx];
+    u[k] = a.in[k][xc + Clamp(j, ny) * nx];
+    up[k] = a.in[k][xc + Clamp(j + 1, ny) * nx];
+  }
+  const double dt = a.dt_ptr ? *a.dt_ptr : a.dt_val;
+  const double lh = DivRn(0.5 * dt, a.dx);
+  const double dt_dx = DivRn(dt, a.dx);
+  const Gas<double> g = MakeGas<double>(a);
+  double F[NC], Fnext[NC];
+  double edge[NC];  // a column's end lanes read a cell that no lane holds
+#pragma unroll
+  for (int k = 0; k < NC; ++k) edge[k] = row == 0 ? um[k] : up[k];
+  if (__builtin_expect(RegularStep(lh) && __all(RegularCell<D>(u) && RegularCell<D>(edge)), 1))
+    LaneFluxes<LARR, RegularArith<double>>(um, u, up, lh, g, a, F);
+  else
+    LaneFluxes<LARR, A>(um, u, up, lh, g, a, F);
+#pragma unroll
+  for (int k = 0; k < NC; ++k) Fnext[k] = ShiftDown(F[k]);
+  if (face && row <= kYOwned && j < ny) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) a.out[k][x + j * nx] = u[k] + dt_dx * (F[k] - Fnext[k]);
+  }
+  if (a.check) {
+    double smax = 0.0;
+    bool exact = true;
+    if (a.bound_check) {
+      const BoundCell<D> b0 = MakeBoundCell<D>(u, g);
+      const BoundCell<D> bm = ShflUp<D>(b0);
+      exact = !__all(!face || BoundPasses<D, 1>(bm, b0, BoundSpeedLimit(a.dx, dt), 0.125 * g.gm1));
+    }
+    if (exact) {
+      const DtCell<D> d0 = MakeDtCell<D, A>(u, g);
+      const DtCell<D> dm = ShflUp<D>(d0);
+      if (face) smax = FaceSpeed<D, 1, A>(dm, d0, g.gm1);
+    }
+    BlockSpeedToPartials<1, kBlock / 64, A>(&smax, &a.dx, a.partials + blockIdx.x, 0);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // 2D step-start CFL: stable dt of both directions in one pass.  A workgroup
 // is a 256-cell x tile marching along y over a segment; x neighbours come
 // through LDS and the y neighbour is kept in registers.  Boundary faces pair
@@ -1044,9 +1121,22 @@ __global__ void ResetKeysKernel(unsigned long long* keys, int n, unsigned int* c
   if (i < nc) counters[i] = 0u;
 }
 
+// Whether a Y sweep takes SweepYLanesKernel: 2D IEEE sweeps whose pencils
+// reconstruct more than twice per useful cell, that is (S + 2) / S cells over
+// the fraction of the pencils' lanes in use.  Lanes and pencils measured, us:
+// 256^2 7.3, 8.0; 512^2 13.4, 18.2 (S = 1); 768^2 24.3, 22.6 (S = 3);
+// 100 x 5000 18.9, 27.3 (S = 5, two fifths of the lanes in use).  The lanes'
+// short rows cost the faster modes what they save (512^2, FP32 12.0, 9.3).
+bool YLanes(int dim, int dir, const int64_t n[3], int seg, bool ieee) {
+  if (!ieee || dim != 2 || dir != 1) return false;
+  const int64_t lanes = (n[0] + kBlock - 1) / kBlock * kBlock;
+  return (seg + 2) * lanes > 2 * seg * n[0];
+}
+
 template <int D, bool LARR, class T, bool FAST>
 int LaunchTyped(hipStream_t s, int dir, const SweepArgs& a) {
-  const int64_t blocks = SweepBlocks(D, dir, a.n, a.seg);
+  constexpr bool kIeee = !FAST && std::is_same<T, double>::value;
+  const int64_t blocks = HllemSweepBlocks(D, dir, a.n, a.seg, kIeee);
   if (blocks <= 0) return FVS_BAD_ARGUMENT;
   // Per-thread byte offsets from the uniform base are 32-bit: a Z sweep spans
   // one x-y plane, a Y sweep 256 / nx + 2 planes.
@@ -1072,6 +1162,15 @@ int LaunchTyped(hipStream_t s, int dir, const SweepArgs& a) {
     const int64_t bx = (npencil + kBlock - 1) / kBlock;
     const int64_t nseg = (a.n[dir] + a.seg - 1) / a.seg;
     if (bx > 0x7fffffff || nseg > 65535) return FVS_BAD_ARGUMENT;
+    if constexpr (D == 2 && kIeee) {
+      if (YLanes(D, dir, a.n, a.seg, kIeee)) {
+        if (blocks > 0x7fffffff) return FVS_BAD_ARGUMENT;
+        hipLaunchKernelGGL((SweepYLanesKernel<LARR>), dim3(static_cast<unsigned>(blocks)),
+                           dim3(kBlock), 0, s, a);
+        FVS_LAUNCH_CHECK();
+        return FVS_OK;
+      }
+    }
     if (dir == 1) {
       hipLaunchKernelGGL((SweepPencilKernel<D, 1, LARR, T, FAST>),
                          dim3(static_cast<unsigned>(bx), static_cast<unsigned>(nseg)),
@@ -1156,6 +1255,11 @@ int LaunchPatchCflFast(int dim, unsigned gx, unsigned gy, hipStream_t s,
 }
 
 #else // FVS_SWEEP_FAST_TU
+
+int64_t HllemSweepBlocks(int dim, int dir, const int64_t n[3], int seg, bool ieee) {
+  if (!YLanes(dim, dir, n, seg, ieee)) return SweepBlocks(dim, dir, n, seg);
+  return ((n[0] + kYCols - 1) / kYCols) * ((n[1] + kYOwned - 1) / kYOwned);
+}
 
 int64_t SweepBlocks(int dim, int dir, const int64_t n[3], int seg) {
   const int64_t nz = dim == 3 ? n[2] : 1;

@@ -320,9 +320,7 @@ def bench_level(state, dx, n, steps, precision, torch, fvs) -> dict:
 
 def bench_composed(state, dx, n, steps, torch, fvs) -> dict:
     """The reference's default method, MUSCL-Hancock over the exact Godunov
-    flux (FP64 Newton), on the same 3D field: a level composed from the patch
-    operators (ghost fill, stable dt, face fluxes, conservative update and
-    completion per split step), with no fused sweep."""
+    flux (FP64 Newton), on the same 3D field, by its fused sweeps."""
     if state is None:
         from finitevolumesolver_amd.initial_data import fourier_modes_3d_device
         state, dx = fourier_modes_3d_device(n, seed0=1)
@@ -340,7 +338,7 @@ def bench_composed(state, dx, n, steps, torch, fvs) -> dict:
     ms = ev0.elapsed_time(ev1)
     del lvl
     return {"workload": f"3D {n}^3, MUSCL-Hancock(MinMod) + exact Godunov (FP64 Newton), "
-                        "Godunov split, CFL 0.8, composed from the patch operators",
+                        "Godunov split, CFL 0.8, fused sweeps",
             "value": round(n ** 3 * 3 * done / (ms * 1e-3) / 1e9, 4), "unit": "Gcell-updates/s",
             "steps": done, "cfl_restarts": fails, "ms_per_step": round(ms / max(done, 1), 4),
             "dtype": "f64"}
@@ -715,7 +713,7 @@ def main() -> int:
                 continue
             log(f"[bench] variant: {prec}")
             variants[f"{prec}_{n}"] = bench_level(t_cons, dx, n, args.steps, prec, torch, fvs)
-        log("[bench] variant: MUSCL-Hancock + exact Godunov, composed level")
+        log("[bench] variant: MUSCL-Hancock + exact Godunov")
         torch.cuda.empty_cache()
         variants["muscl_godunov_composed"] = bench_composed(t_cons, dx, n, 3, torch, fvs)
         del t_cons

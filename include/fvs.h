@@ -296,7 +296,9 @@ int fvs_level_time(fvs_level* level, double* t, int64_t* cycles);
  * signal speed less a margin (four times its last relative drop, between
  * 2^-10 and 1/4), and confirms that some evaluated face did reach it.  When
  * none did, the step is repeated with every face evaluated (and the margin
- * quadruples), so the floor never changes a result.
+ * quadruples), so the floor never changes a result.  An exact-Godunov level
+ * that has no floor yet (a new state's first step) takes one from its cells'
+ * |u| + a.
  * fvs_level_hint_max_speed sets the floor for the current state
  * (speed[d] >= 0; 0: none; ignored by other levels); fvs_level_cfl_redos
  * reports how many steps were repeated. */

@@ -357,10 +357,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     bool valid;
     uint32_t row, sl;
     walk.RowSlot(c, &valid, &row, &sl);
-    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row));
+    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row),
+                     __builtin_amdgcn_readfirstlane(sl));
   };
   auto load = [&](const XSlot& s, double* u) {
-    const uint32_t off = 8u * (s.rbase + static_cast<uint32_t>(Clamp(s.cell, nx)));
+    const uint32_t off = s.Bytes(Clamp(s.cell, nx));
 #pragma unroll
     for (int k = 0; k < NC; ++k)
       u[k] = *reinterpret_cast<const double*>(
@@ -415,8 +416,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     if (face_lane) {
       if constexpr (!LEARNED && !MUSCL) {
         if (a.guess) {
-          const int64_t row = (cur.wbase + cur.rbase) / nx;
-          guess = a.guess[row * (nx + 1) + static_cast<int64_t>(cur.sl) - 1];
+          guess = a.guess[static_cast<int64_t>(cur.row) * (nx + 1) + cur.cell];
         }
       }
       GodunovFace<D, 0, MIXED>(L, R, guess, LEARNED || a.guess != nullptr, a, g, F, owned, !MUSCL,
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
     for (int k = 0; k < NC; ++k) Fnext[k] = ShiftDown(F[k]);
     if (a.update && owned && real) {
-      const uint32_t off = 8u * (cur.rbase + static_cast<uint32_t>(cur.cell));
+      const uint32_t off = cur.Bytes(cur.cell);
 #pragma unroll
       for (int k = 0; k < NC; ++k)
         *reinterpret_cast<double*>(reinterpret_cast<char*>(a.out[k] + cur.wbase) + off) =

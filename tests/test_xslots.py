@@ -1,10 +1,10 @@
 """The X sweep's slot walker (finitevolumesolver_amd/csrc/fvs_xslots.hpp)
 compiled for the host: over ragged 2D and 3D row counts and row lengths
 (1 .. 256 cells, around the 60-slot chunk) and persistent wave counts from
-4 to 4,096, every lane's loads stay inside the arrays, its row never lies
-below the wave's base row (the unsigned offset cannot wrap), valid lanes sit
-on their true slot after each stride, and every cell is stored exactly
-once (tests/host_stub/xslots.cpp)."""
+4 to 4,096, every lane's loads stay inside the arrays, its byte offset from
+the wave's base does not wrap, valid lanes sit on their true slot after each
+stride, and every cell is stored exactly once; rows of 2^29 to 2^32 slots by
+their addresses (tests/host_stub/xslots.cpp)."""
 from __future__ import annotations
 
 import shutil

@@ -41,7 +41,7 @@ __global__ void MlpPackKernel(const float* __restrict__ p, short* __restrict__ t
     float v = 0.0f;
     if (t < 4) {
       const int out = t * 16 + i;
-      v = (k < kInPad) ? p[kOffW1 + out * kInPad + k] : 0.0f;
+      v = (k < kIn) ? p[kOffW1 + out * kInPad + k] : 0.0f;
     } else if (t < 20) {
       const int m = (t - 4) / 4, kb = (t - 4) % 4;
       v = p[kOffW2 + (m * 16 + i) * kH + kb * 16 + k];
@@ -283,8 +283,10 @@ __global__ __launch_bounds__(kBlock) void MlpGradKernel(
   __shared__ float s_h1[kH][kActStride], s_d2[kH][kActStride], s_d1[kH][kActStride];
   __shared__ float s_y[4][kTile], s_dy[kTile], s_t[kTile];
   __shared__ int s_ok[kTile];
+  // W1's padding columns, which a caller may have set to anything, meet the row
+  // of ones below
   for (int k = threadIdx.x; k < kH * kInPad; k += kBlock)
-    s_w1[(k / kInPad) * 9 + k % kInPad] = p[kOffW1 + k];
+    s_w1[(k / kInPad) * 9 + k % kInPad] = k % kInPad < kIn ? p[kOffW1 + k] : 0.0f;
   for (int k = threadIdx.x; k < kH * kH; k += kBlock)
     s_w2[(k / kH) * kW2Stride + k % kH] = p[kOffW2 + k];
   if (threadIdx.x < kH) {
@@ -320,8 +322,8 @@ __global__ __launch_bounds__(kBlock) void MlpGradKernel(
       s_x[k][c] = v;
     }
     __syncthreads();
-    // H1: two steps of the 8 inputs (row 6 of X is not an input: W1's padding
-    // columns are zero)
+    // H1: two steps of the 8 inputs (rows 6 and 7 of X are no inputs: W1's
+    // padding columns are staged as zeros)
     floatx4_t h1 = {s_b1[row], s_b1[row + 1], s_b1[row + 2], s_b1[row + 3]};
 #pragma unroll
     for (int s = 0; s < 2; ++s) {

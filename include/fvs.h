@@ -410,6 +410,8 @@ int fvs_mlp_create(void* hip_stream, uint64_t seed, fvs_mlp** out);
 int fvs_mlp_destroy(fvs_mlp* mlp);
 int fvs_mlp_num_params(void);
 int fvs_mlp_get_params(fvs_mlp* mlp, float* host_params);
+/* W1 has rows of 8 for 6 inputs: the two padding columns are ignored by
+ * inference and training, whatever they hold. */
 int fvs_mlp_set_params(fvs_mlp* mlp, const float* host_params);
 /* Generates n labelled pairs on the device: rho, p log-uniform in
  * [1e-3, 1e3], u uniform in [-5, 5]; label = FP64 Newton star pressure.

@@ -47,3 +47,33 @@ def test_training_is_deterministic(cuda):
         runs.append((net.get_params(), hist))
     assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1], runs[1][1])
     assert runs[0][1][-1] < runs[0][1][0]
+
+
+def test_padding_columns_of_w1_are_ignored(cuda):
+    """fvs_mlp_set_params takes any floats in the two padding columns of W1
+    (inputs 6 and 7 do not exist): forward, inference, gradients and training
+    are those of zero padding, and the columns are returned as they were set."""
+    import torch
+    rng = np.random.default_rng(3)
+    n = 200
+    x = torch.from_numpy(rng.uniform(-1.0, 1.0, (6, n)).astype(np.float32)).to(cuda)
+    t = torch.from_numpy(rng.uniform(-1.0, 1.0, n).astype(np.float32)).to(cuda)
+    flag = torch.zeros(n, dtype=torch.int32, device=cuda)
+    prim = torch.from_numpy(np.stack([rng.uniform(0.5, 2.0, n), rng.uniform(-1, 1, n), 0.1 * rng.random(n),
+                                      rng.uniform(5.0, 9.0, n), rng.uniform(0.5, 2.0, n),
+                                      rng.uniform(0.8, 1.2, n)])).to(cuda)
+    runs = []
+    for pad in ((0.0, 0.0), (0.75, -2.0), (np.inf, np.nan)):
+        net = fvs.LearnedNewtonGuess(seed=6)
+        p = net.get_params()
+        p[:512].reshape(64, 8)[:, 6:] = pad
+        net.set_params(p)
+        net.generate(4096, seed=2)
+        out = [net.forward(x).cpu().numpy(), net.infer_pairs(2, 0, prim, prim.flip(1))[0].cpu().numpy(),
+               *net.gradients(x, t, flag, 0.25), net.train(epochs=2, batch=512)]
+        w = net.get_params()
+        assert np.array_equal(w[:512].reshape(64, 8)[:, 6:], p[:512].reshape(64, 8)[:, 6:], equal_nan=True)
+        runs.append(out + [fvs.newton_guess.unpack_params(w)["W1"], w[512:]])
+    for other in runs[1:]:
+        for a, b in zip(runs[0], other):
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b)

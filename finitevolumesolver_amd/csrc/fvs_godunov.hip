@@ -25,8 +25,6 @@ namespace fvs {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kTX = 256;
-constexpr int kCflSeg = 32;
 constexpr unsigned long long kInfKey = 0x7ff0000000000000ull;
 
 __device__ __forceinline__ int64_t Clamp(int64_t i, int64_t n) {
@@ -733,6 +731,7 @@ struct GodunovCflArgs {
   int max_it;
   SpeedBound bound;
   int64_t items;                 // tiles x segments
+  int seg;                       // cells of a segment along the march
   unsigned long long* partials;  // 5 per workgroup and direction
   int* halt;
   const double* floor;  // speed floor per direction (nullable: none)
@@ -770,9 +769,13 @@ template <int D> __device__ __forceinline__ SpeedCell<D> ShiftUpCell(const Speed
   return r;
 }
 
-template <int D>
+constexpr int kCflSeg = 32;  // cells of a segment along the march, at most
+
+// SHORT: segments of a.seg cells (GodunovCflSeg), otherwise of kCflSeg.
+template <int D, bool SHORT>
 __global__ __launch_bounds__(64 * kCflRows) __attribute__((amdgpu_waves_per_eu(4))) void GodunovCflKernel(GodunovCflArgs a) {
   constexpr int NC = D + 2;
+  const int seg_cells = SHORT ? a.seg : kCflSeg;
   constexpr int M = D - 1;  // marching direction
   if (a.halt && *a.halt) return;
   Gas<double> g;
@@ -834,8 +837,8 @@ __global__ __launch_bounds__(64 * kCflRows) __attribute__((amdgpu_waves_per_eu(4
     const bool own = lane >= 1 && lane <= kCflOwnX && x < nx && (D == 2 || (row >= 1 && y < ny));
     const int64_t xs = Clamp(x, nx), ys = (D == 3) ? Clamp(y, ny) : 0;
     const int64_t col = xs + (D == 3 ? ys * nx : 0);
-    const int64_t m0 = seg * kCflSeg;
-    const int64_t m1 = (m0 + kCflSeg < nm) ? m0 + kCflSeg : nm;
+    const int64_t m0 = seg * seg_cells;
+    const int64_t m1 = (m0 + seg_cells < nm) ? m0 + seg_cells : nm;
     auto load = [&](double* u, int64_t m) {
       const int64_t off = col + Clamp(m, nm) * ms;
 #pragma unroll
@@ -1023,11 +1026,26 @@ int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3]) {
   return SweepBlocks(dim, dir, n, GodunovSeg(dim, dir, n));
 }
 
-static int64_t GodunovCflItems(int dim, const int64_t n[3]) {
+// Cells of a segment of the CFL pass: 32, halved down to 1 while the items are
+// too few to fill the chip (3D: 512 workgroups of eight waves, 2D: 1,024
+// waves).  A segment is a serial chain of loads and barriers, and a row more is
+// loaded per segment.  First-order step, us, with 32 cells always and with this
+// rule: 16^2 76, 57; 256^2 114, 62; 1000^2 227, 174; 32^3 194, 79; 64^3 285,
+// 151; 128^3 496, 405; 203 x 149 x 121 701, 641 (512 waves in 2D: 1000^2 227;
+// 1,024 workgroups in 3D: 64^3 168, 203 x 149 x 121 625).
+static int GodunovCflSeg(int64_t nm, int64_t tiles, int64_t enough) {
+  int seg = kCflSeg;
+  while (seg > 1 && tiles * ((nm + seg - 1) / seg) < enough) seg /= 2;
+  return seg;
+}
+
+static int64_t GodunovCflItems(int dim, const int64_t n[3], int* seg = nullptr) {
   const int64_t tx = (n[0] + kCflOwnX - 1) / kCflOwnX;
   const int64_t ty = dim == 3 ? (n[1] + kCflRows - 2) / (kCflRows - 1) : 1;
   const int64_t nm = dim == 3 ? n[2] : n[1];
-  return tx * ty * ((nm + kCflSeg - 1) / kCflSeg);
+  const int s = GodunovCflSeg(nm, tx * ty, dim == 3 ? 512 : 1024);
+  if (seg) *seg = s;
+  return tx * ty * ((nm + s - 1) / s);
 }
 
 int64_t GodunovCflBlocks(int dim, const int64_t n[3]) {
@@ -1138,7 +1156,7 @@ int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* c
   a.tol = desc.newton_tolerance;
   a.max_it = desc.max_newton_iterations;
   a.bound = MakeSpeedBound(desc.gamma, desc.newton_tolerance, desc.max_newton_iterations);
-  a.items = GodunovCflItems(D, a.n);
+  a.items = GodunovCflItems(D, a.n, &a.seg);
   a.count_fails = desc.reconstruction == FVS_RECON_NONE;
   a.partials = partials;
   a.halt = halt;
@@ -1155,10 +1173,10 @@ int LaunchGodunovCfl(const fvs_method_desc& desc, hipStream_t s, const double* c
       hipLaunchKernelGGL(GodunovFloorKernel<2>, fgrid, dim3(kBlock), 0, s, a, ncell, floor_ctl);
     FVS_LAUNCH_CHECK();
   }
-  if (D == 3)
-    hipLaunchKernelGGL(GodunovCflKernel<3>, grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL(GodunovCflKernel<2>, grid, block, 0, s, a);
+  using K = void (*)(GodunovCflArgs);
+  const K ks[2][2] = {{GodunovCflKernel<2, false>, GodunovCflKernel<2, true>},
+                      {GodunovCflKernel<3, false>, GodunovCflKernel<3, true>}};
+  hipLaunchKernelGGL(ks[D == 3][a.seg < kCflSeg], grid, block, 0, s, a);
   FVS_LAUNCH_CHECK();
   return FVS_OK;
 }

@@ -2,7 +2,7 @@
 (GodunovSweepX / GodunovSweepPencil with half-step states) against the
 oracle's level driver: patches narrower than a stencil, widths around the X
 sweep's 60-slot chunks and 64-lane waves, lengths around the pencils'
-segments, every limiter, both splittings, strong waves (whose CFL checks need
+segments and the CFL pass's (one to four cells here), every limiter, both splittings, strong waves (whose CFL checks need
 solved faces) and restarts; graphs and eager launches give the same bits.
 Bar: 1e-12 per cell and 1e-13 for dt (tolerances.py), the exact solver's."""
 from __future__ import annotations
@@ -41,6 +41,8 @@ def _run(cuda, cons, shape, limiter, split, cfl, steps, graphs=True):
     ((58, 33), "NoLimiter", "Godunov", 0.4),
     ((63, 31), "NoGradient", "Strang", 0.8),
     ((129, 64), "MinMod", "Strang", 0.8),
+    ((70, 1501), "MinMod", "Godunov", 0.8),
+    ((310, 1203), "VanLeer", "Godunov", 0.8),
     ((3, 1, 2), "MinMod", "Godunov", 0.8),
     ((31, 17, 5), "VanLeer", "Strang", 0.8),
     ((61, 6, 35), "NoLimiter", "Godunov", 0.4),

@@ -1452,8 +1452,9 @@ __device__ __forceinline__ FaceFrac Fractions(double bl, double bm, double br) {
 }
 
 // A regular cell away from the boundary: both faces are unshielded
-// (fractions 1, 0, 0), no boundary flux enters, and the general formula of
-// KbnUpdateCell reduces to the plain update with the same result bits.
+// (fractions 1, 0, 0), neither it nor a neighbour along the sweep is a cut
+// cell, so no boundary flux enters, and the general formula of KbnUpdateCell
+// reduces to the plain update with the same result bits.
 // u: the cell's conservative state.
 __device__ __forceinline__ void KbnRegularUpdate(const double* u, const double* Fl,
                                                  const double* Fr, double dt_over_dx,
@@ -1493,9 +1494,12 @@ __device__ __forceinline__ bool KbnSweepUpdate(const LevelGeom& g, int32_t code,
 
 // h-box update (TimeIntegrator, or TimeIntegrator2 when `second`) of the
 // uncovered interior cell (i, j) from the regular fluxes Fl / Fr of its two
-// faces in DIR; the boundary fluxes fb are read only where a shielded
-// fraction or unequal face fractions need them.  Returns the masked result
-// (the zero state unless the density is positive).
+// faces in DIR.  The boundary fluxes fb of the cell and its two neighbours
+// (zero away from cut cells) enter whatever their weights are, as in the
+// reference: a cut cell that is no gas any more (its wall problem has no
+// solution) has a NaN there, which the reference's zero weights hand on to its
+// neighbours.  Returns the masked result (the zero state unless the density is
+// positive).
 template <int DIR>
 __device__ __forceinline__ void KbnUpdateCell(const LevelState& in, const LevelGeom& g,
                                               const double* fb, int64_t i, int64_t j,
@@ -1508,12 +1512,6 @@ __device__ __forceinline__ void KbnUpdateCell(const LevelState& in, const LevelG
   const double bL = g.beta_at(DIR, i, j);
   const double bR = g.beta_at(DIR, i + di, j + dj);
   const double bRR = g.beta_at(DIR, i + 2 * di, j + 2 * dj);
-  if (alpha == 1.0 && bLL == 1.0 && bL == 1.0 && bR == 1.0 && bRR == 1.0) {
-    double u[4];
-    LoadCons(in, c, u);
-    KbnRegularUpdate(u, Fl, Fr, dt_over_dx, res);
-    return;
-  }
   const FaceFrac fl = Fractions(bLL, bL, bR);
   const FaceFrac fr = Fractions(bL, bR, bRR);
   const int64_t plane = g.ngx * g.ngy;
@@ -1528,9 +1526,9 @@ __device__ __forceinline__ void KbnUpdateCell(const LevelState& in, const LevelG
   const double dR_r = affR ? Clamp01(0.5 + xc[cr]) : 0.5;
   const double center = xc[c];
   for (int k = 0; k < 4; ++k) {
-    const double fbl = affL ? fb[k * plane + cl] : 0.0;
-    const double fbc = (affL || affR || bL != bR) ? fb[k * plane + c] : 0.0;
-    const double fbr = affR ? fb[k * plane + cr] : 0.0;
+    const double fbl = fb[k * plane + cl];
+    const double fbc = fb[k * plane + c];
+    const double fbr = fb[k * plane + cr];
     // stabilised fluxes and the shielded ones of both faces
     const double sL_l = dL_l * Fl[k] + (1.0 - dL_l) * fbl;
     const double sR_l = dR_l * Fl[k] + (1.0 - dR_l) * fbc;
@@ -1978,6 +1976,28 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
   L->lg.centroids = gc;
   L->lg.ngx = ngx;
   L->lg.ngy = ngy;
+  // flags of the interior cut cells
+  int32_t* flags = nullptr;
+  if (hipMalloc(&flags, nx * ny * sizeof(int32_t)) != hipSuccess) return fail(FVS_HIP_ERROR);
+  {
+    GeomViews gv;
+    if (GeomOf(geom, 2, &gv)) {
+      (void)hipFree(flags);
+      return fail(FVS_BAD_ARGUMENT);
+    }
+    const int64_t ilo[3] = {0, 0, 0}, ihi[3] = {nx - 1, ny - 1, 0};
+    const DevView box = BoxView(ilo, ihi);
+    hipLaunchKernelGGL(IsCutCellKernel<2>, dim3(Blocks(box.count())), dim3(kBlock), 0, s, gv, box,
+                       flags);
+  }
+  std::vector<int32_t> hflags(nx * ny);
+  if (hipMemcpyAsync(hflags.data(), flags, nx * ny * sizeof(int32_t), hipMemcpyDeviceToHost, s) !=
+          hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess) {
+    (void)hipFree(flags);
+    return fail(FVS_HIP_ERROR);
+  }
+  (void)hipFree(flags);
   // geometry words of every cell (CellCode) and the irregular cells per
   // direction
   {
@@ -1995,6 +2015,10 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
       auto beta = [&](int64_t ci, int64_t cj) {
         return d == 0 ? hbx[cj * (ngx + 1) + ci] : hby[cj * ngx + ci];
       };
+      auto is_cut = [&](int64_t ci, int64_t cj) {
+        const int64_t i = ci - kG, j = cj - kG;
+        return i >= 0 && i < nx && j >= 0 && j < ny && hflags[j * nx + i] != 0;
+      };
       std::vector<int32_t> code(ncg), cells;
       for (int64_t cj = 0; cj < ngy; ++cj)
         for (int64_t ci = 0; ci < ngx; ++ci) {
@@ -2003,10 +2027,13 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
           int32_t kind = CellCode::kCovered;
           const bool interior = ci >= kG && ci < nx + kG && cj >= kG && cj < ny + kG;
           if (interior && a != 0.0) {
-            // face fractions at faces i - 1 .. i + 2 (or j - 1 .. j + 2)
+            // face fractions at faces i - 1 .. i + 2 (or j - 1 .. j + 2), and
+            // no wall flux in the cells i - 1 .. i + 1
             bool regular = a == 1.0;
             for (int64_t f = -1; f <= 2 && regular; ++f)
               regular = (d == 0 ? beta(ci + f, cj) : beta(ci, cj + f)) == 1.0;
+            for (int64_t f = -1; f <= 1 && regular; ++f)
+              regular = d == 0 ? !is_cut(ci + f, cj) : !is_cut(ci, cj + f);
             if (regular) {
               kind = CellCode::kRegular;
             } else {
@@ -2034,27 +2061,6 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
     }
   }
   // list of the interior cut cells
-  int32_t* flags = nullptr;
-  if (hipMalloc(&flags, nx * ny * sizeof(int32_t)) != hipSuccess) return fail(FVS_HIP_ERROR);
-  {
-    GeomViews gv;
-    if (GeomOf(geom, 2, &gv)) {
-      (void)hipFree(flags);
-      return fail(FVS_BAD_ARGUMENT);
-    }
-    const int64_t ilo[3] = {0, 0, 0}, ihi[3] = {nx - 1, ny - 1, 0};
-    const DevView box = BoxView(ilo, ihi);
-    hipLaunchKernelGGL(IsCutCellKernel<2>, dim3(Blocks(box.count())), dim3(kBlock), 0, s, gv, box,
-                       flags);
-  }
-  std::vector<int32_t> hflags(nx * ny);
-  if (hipMemcpyAsync(hflags.data(), flags, nx * ny * sizeof(int32_t), hipMemcpyDeviceToHost, s) !=
-          hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess) {
-    (void)hipFree(flags);
-    return fail(FVS_HIP_ERROR);
-  }
-  (void)hipFree(flags);
   std::vector<int32_t> cut;
   for (int64_t j = 0; j < ny; ++j)
     for (int64_t i = 0; i < nx; ++i)

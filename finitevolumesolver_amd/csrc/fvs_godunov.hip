@@ -1027,12 +1027,13 @@ int64_t GodunovSweepBlocks(int dim, int dir, const int64_t n[3]) {
 }
 
 // Cells of a segment of the CFL pass: 32, halved down to 1 while the items are
-// too few to fill the chip (3D: 512 workgroups of eight waves, 2D: 1,024
+// too few to fill the chip (3D: 256 workgroups of eight waves, 2D: 1,024
 // waves).  A segment is a serial chain of loads and barriers, and a row more is
 // loaded per segment.  First-order step, us, with 32 cells always and with this
 // rule: 16^2 76, 57; 256^2 114, 62; 1000^2 227, 174; 32^3 194, 79; 64^3 285,
-// 151; 128^3 496, 405; 203 x 149 x 121 701, 641 (512 waves in 2D: 1000^2 227;
-// 1,024 workgroups in 3D: 64^3 168, 203 x 149 x 121 625).
+// 142; 96^3 362, 239; 128^3 490, 419 (512 waves in 2D: 1000^2 227; 512
+// workgroups in 3D: 64^3 151, 128^3 404, and 203 x 149 x 121 in strong waves,
+// 352 workgroups of whole segments, 4.23 -> 4.32 ms for four steps).
 static int GodunovCflSeg(int64_t nm, int64_t tiles, int64_t enough) {
   int seg = kCflSeg;
   while (seg > 1 && tiles * ((nm + seg - 1) / seg) < enough) seg /= 2;
@@ -1043,7 +1044,7 @@ static int64_t GodunovCflItems(int dim, const int64_t n[3], int* seg = nullptr) 
   const int64_t tx = (n[0] + kCflOwnX - 1) / kCflOwnX;
   const int64_t ty = dim == 3 ? (n[1] + kCflRows - 2) / (kCflRows - 1) : 1;
   const int64_t nm = dim == 3 ? n[2] : n[1];
-  const int s = GodunovCflSeg(nm, tx * ty, dim == 3 ? 512 : 1024);
+  const int s = GodunovCflSeg(nm, tx * ty, dim == 3 ? 256 : 1024);
   if (seg) *seg = s;
   return tx * ty * ((nm + s - 1) / s);
 }

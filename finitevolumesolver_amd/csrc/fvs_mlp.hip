@@ -262,6 +262,7 @@ __global__ __launch_bounds__(kBlock) void MlpForwardKernel(const float* __restri
 constexpr int kTile = 16;         // samples per tile
 constexpr int kActStride = 17;    // LDS floats per activation row
 constexpr int kW2Stride = 65;
+static_assert(kBlock % kInPad == 0, "a thread stages one column of W1");
 constexpr int kGradBlocks = 512;  // most workgroups (partial vectors)
 
 __device__ __forceinline__ floatx4_t MfmaF32(float a, float b, floatx4_t c) {
@@ -285,8 +286,11 @@ __global__ __launch_bounds__(kBlock) void MlpGradKernel(
   __shared__ int s_ok[kTile];
   // W1's padding columns, which a caller may have set to anything, meet the row
   // of ones below
-  for (int k = threadIdx.x; k < kH * kInPad; k += kBlock)
-    s_w1[(k / kInPad) * 9 + k % kInPad] = k % kInPad < kIn ? p[kOffW1 + k] : 0.0f;
+  const bool input = threadIdx.x % kInPad < kIn;
+  for (int k = threadIdx.x; k < kH * kInPad; k += kBlock) {
+    const float v = p[kOffW1 + k];
+    s_w1[(k / kInPad) * 9 + k % kInPad] = input ? v : 0.0f;
+  }
   for (int k = threadIdx.x; k < kH * kH; k += kBlock)
     s_w2[(k / kH) * kW2Stride + k % kH] = p[kOffW2 + k];
   if (threadIdx.x < kH) {

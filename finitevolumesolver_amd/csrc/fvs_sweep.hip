@@ -202,19 +202,18 @@ __global__ __launch_bounds__(kBlock, FAST ? 1 : 3) void SweepXKernel(SweepArgs a
   const double s_crit = BoundSpeedLimit(a.dx, dt);
   const double kbound = 0.125 * gd.gm1;
 
-  // Slot of this lane in chunk c (fvs_xslots.hpp): the base is lane 0's cell,
-  // read across the wave.
+  // Slot of this lane in chunk c (fvs_xslots.hpp): the row base is lane 0's
+  // row, read across the wave.
   XSlotWalker walk(nx, Q, nwaves, lane);
   using Slot = XSlot;
   auto locate = [&](int64_t c) {
     bool valid;
     uint32_t row, sl;
     walk.RowSlot(c, &valid, &row, &sl);
-    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row),
-                     __builtin_amdgcn_readfirstlane(sl));
+    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row));
   };
   auto load = [&](const Slot& s, double* u) {
-    const uint32_t off = s.Bytes(Clamp(s.cell, nx));
+    const uint32_t off = 8u * (s.rbase + static_cast<uint32_t>(Clamp(s.cell, nx)));
 #pragma unroll
     for (int k = 0; k < NC; ++k) u[k] = LdOff(a.in[k] + s.wbase, off);
   };
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(kBlock, FAST ? 1 : 3) void SweepXKernel(SweepArgs a
     for (int k = 0; k < NC; ++k) Fnext[k] = ShiftDown(F[k]);
 
     if (owned && real) {
-      const uint32_t off = cur.Bytes(cur.cell);
+      const uint32_t off = 8u * (cur.rbase + static_cast<uint32_t>(cur.cell));
 #pragma unroll
       for (int k = 0; k < NC; ++k) {
         StOff(a.out[k] + cur.wbase, off,

@@ -8,13 +8,11 @@
 // chunks c, c + nwaves, c + 2 nwaves, ...; the (row, slot) of its lane
 // advances by the constant stride without a division per chunk.
 //
-// Addresses are a wave-uniform base (the cell of lane 0) plus a 32-bit lane
-// offset in bytes relative to it, at most 64 cells whatever the length of a
-// row (relative to the start of lane 0's row it would wrap in rows of 2^29
-// cells).  The offset is unsigned, so no lane's cell may lie below lane 0's:
-// lanes whose slot falls outside the sequence take its nearest end (slot 0
-// before it, slot Q - 1 after it), which keeps cells non-decreasing in the
-// lane index.  The same holds after a stride only if
+// Addresses are a wave-uniform base (the row of lane 0) plus a 32-bit lane
+// offset relative to it.  The offset is unsigned, so no lane's row may lie
+// below lane 0's: lanes whose slot falls outside the sequence take its
+// nearest end (slot 0 before it, slot Q - 1 after it), which keeps rows
+// non-decreasing in the lane index.  The same holds after a stride only if
 // the lane's slot in the previous chunk was its true slot: lanes 0 and 1 of
 // a wave's first chunk sit on the clamped slot 0, and advancing them from
 // there can put lane 0 a row beyond lanes 2 .. 63, whose offsets then wrap
@@ -38,16 +36,9 @@ constexpr int kXWavesPerCu = 16;  // persistent waves per CU
 struct XSlot {
   bool valid;      // the lane's slot lies in the sequence
   uint32_t sl;     // slot within its row (0 .. nx + 1)
-  uint32_t row;
   int64_t cell;    // sl - 1: -1 and nx are the ghost slots
-  uint32_t rbase;  // start of the row relative to wbase (modulo 2^32)
-  int64_t wbase;   // cell of lane 0 (wave-uniform)
-
-  // Byte offset from wbase of cell i of the slot's row (the slot's own, or
-  // the end of the row next to a ghost slot).
-  __host__ __device__ uint32_t Bytes(int64_t i) const {
-    return 8u * (rbase + static_cast<uint32_t>(i));
-  }
+  uint32_t rbase;  // (row - row of lane 0) * nx
+  int64_t wbase;   // row of lane 0 * nx (wave-uniform)
 };
 
 struct XSlotWalker {
@@ -91,30 +82,25 @@ struct XSlotWalker {
     }
   }
 
-  // The slot record given lane 0's row and slot (read across the wave).
-  __host__ __device__ XSlot Make(bool valid, uint32_t row, uint32_t sl, uint32_t row0,
-                                 uint32_t sl0) const {
-    // lane 0's cell, a ghost's inner neighbour
-    const uint32_t last = S - 3u;  // nx - 1
-    const uint32_t inner = sl0 > 0u ? sl0 - 1u : 0u;
-    const uint32_t cell0 = inner < last ? inner : last;
+  // The slot record given lane 0's row (row0, read across the wave).
+  __host__ __device__ XSlot Make(bool valid, uint32_t row, uint32_t sl, uint32_t row0) const {
     XSlot s;
     s.valid = valid;
     s.sl = sl;
-    s.row = row;
     s.cell = static_cast<int64_t>(sl) - 1;
-    s.rbase = (row - row0) * static_cast<uint32_t>(nx) - cell0;
-    s.wbase = static_cast<int64_t>(row0) * nx + cell0;
+    s.rbase = (row - row0) * static_cast<uint32_t>(nx);
+    s.wbase = static_cast<int64_t>(row0) * nx;
     return s;
   }
 
-  // Moves the position by the stride, with one compare (S - step_sl > 0: no
-  // sum of two slots, which may pass 2^32).
+  // Moves the position by the stride, with one compare.
   __host__ __device__ void Advance() {
-    const uint32_t room = S - step_sl;
-    const bool wraps = q_sl >= room;
-    q_sl = wraps ? q_sl - room : q_sl + step_sl;
-    q_row += step_rows + (wraps ? 1u : 0u);
+    q_sl += step_sl;
+    q_row += step_rows;
+    if (q_sl >= S) {
+      q_sl -= S;
+      q_row += 1;
+    }
   }
 
   // Position of the next chunk cn = c + nwaves: advanced from chunk c unless

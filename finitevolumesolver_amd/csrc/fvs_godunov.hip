@@ -334,7 +334,8 @@ __device__ __forceinline__ void CheckFace(const double* uL, const double* uR, bo
 // 384^3 strong-wave blocks: 3.9 -> 2.9 ms a sweep against one wave per 62
 // slots with LDS shuffles; MUSCL over 256^3: 8.6 -> 2.8 ms a step against the
 // patch operators' passes (fluxes, stable dt, update, completion).
-template <int D, bool MIXED, bool LEARNED, bool MUSCL>
+// LONG: rows of kXLongRow cells or more, whose offsets take 64 bits.
+template <int D, bool MIXED, bool LEARNED, bool MUSCL, bool LONG>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovSweepX(GodunovArgs a) {
   constexpr int NC = D + 2, NQ = D + 4;
   if (a.halt && *a.halt) return;
@@ -355,15 +356,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     bool valid;
     uint32_t row, sl;
     walk.RowSlot(c, &valid, &row, &sl);
-    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row),
-                     __builtin_amdgcn_readfirstlane(sl));
+    return walk.Make(valid, row, sl, __builtin_amdgcn_readfirstlane(row));
   };
   auto load = [&](const XSlot& s, double* u) {
-    const uint32_t off = s.Bytes(Clamp(s.cell, nx));
+    if constexpr (LONG) {
 #pragma unroll
-    for (int k = 0; k < NC; ++k)
-      u[k] = *reinterpret_cast<const double*>(
-          reinterpret_cast<const char*>(a.in[k] + s.wbase) + off);
+      for (int k = 0; k < NC; ++k) u[k] = a.in[k][s.wbase + s.rbase + Clamp(s.cell, nx)];
+    } else {
+      const uint32_t off = 8u * (s.rbase + static_cast<uint32_t>(Clamp(s.cell, nx)));
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        u[k] = *reinterpret_cast<const double*>(
+            reinterpret_cast<const char*>(a.in[k] + s.wbase) + off);
+    }
   };
   FaceSums sums;
   int64_t c = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) +
@@ -374,7 +379,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   if (c < nchunks) load(cur, u);
   for (; c < nchunks; c += nwaves) {
     const int64_t cn = c + nwaves;
-    walk.Next(c, cn, nchunks);
+    walk.Next<LONG>(c, cn, nchunks);
     const XSlot nxt = locate(cn < nchunks ? cn : c);
     double un[NC];
     if (cn < nchunks) load(nxt, un);
@@ -414,7 +419,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     if (face_lane) {
       if constexpr (!LEARNED && !MUSCL) {
         if (a.guess) {
-          guess = a.guess[static_cast<int64_t>(cur.row) * (nx + 1) + cur.cell];
+          const int64_t row = (cur.wbase + cur.rbase) / nx;
+          guess = a.guess[row * (nx + 1) + static_cast<int64_t>(cur.sl) - 1];
         }
       }
       GodunovFace<D, 0, MIXED>(L, R, guess, LEARNED || a.guess != nullptr, a, g, F, owned, !MUSCL,
@@ -427,11 +433,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
     for (int k = 0; k < NC; ++k) Fnext[k] = ShiftDown(F[k]);
     if (a.update && owned && real) {
-      const uint32_t off = cur.Bytes(cur.cell);
+      if constexpr (LONG) {
 #pragma unroll
-      for (int k = 0; k < NC; ++k)
-        *reinterpret_cast<double*>(reinterpret_cast<char*>(a.out[k] + cur.wbase) + off) =
-            u[k] + dt_dx * (F[k] - Fnext[k]);
+        for (int k = 0; k < NC; ++k)
+          a.out[k][cur.wbase + cur.rbase + cur.cell] = u[k] + dt_dx * (F[k] - Fnext[k]);
+      } else {
+        const uint32_t off = 8u * (cur.rbase + static_cast<uint32_t>(cur.cell));
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+          *reinterpret_cast<double*>(reinterpret_cast<char*>(a.out[k] + cur.wbase) + off) =
+              u[k] + dt_dx * (F[k] - Fnext[k]);
+      }
     }
     if constexpr (MUSCL) {
       if (a.check) CheckFace<D, 0>(ul, u, owned && face_lane, a, g, crit, sums);
@@ -1099,14 +1111,19 @@ int LaunchGodunovSweep(const fvs_method_desc& desc, hipStream_t s, int dir,
       return FVS_BAD_ARGUMENT;
     }
     using K = void (*)(GodunovArgs);
-    const K ks[2][2][2] = {
-        {{GodunovSweepX<2, false, false, false>, GodunovSweepX<2, false, true, false>},
-         {GodunovSweepX<2, true, false, false>, GodunovSweepX<2, true, true, false>}},
-        {{GodunovSweepX<3, false, false, false>, GodunovSweepX<3, false, true, false>},
-         {GodunovSweepX<3, true, false, false>, GodunovSweepX<3, true, true, false>}}};
-    const K km[2] = {GodunovSweepX<2, false, false, true>, GodunovSweepX<3, false, false, true>};
-    hipLaunchKernelGGL(muscl ? km[D == 3] : ks[D == 3][mixed][learned], dim3(unsigned(blocks)),
-                       dim3(kBlock), 0, s, a);
+#define FVS_GX(D_, LONG_)                                                                          \
+  {                                                                                                \
+    {GodunovSweepX<D_, false, false, false, LONG_>, GodunovSweepX<D_, false, true, false, LONG_>}, \
+    {GodunovSweepX<D_, true, false, false, LONG_>, GodunovSweepX<D_, true, true, false, LONG_>}    \
+  }
+    const K ks[2][2][2][2] = {{FVS_GX(2, false), FVS_GX(3, false)}, {FVS_GX(2, true), FVS_GX(3, true)}};
+#undef FVS_GX
+    const K km[2][2] = {
+        {GodunovSweepX<2, false, false, true, false>, GodunovSweepX<3, false, false, true, false>},
+        {GodunovSweepX<2, false, false, true, true>, GodunovSweepX<3, false, false, true, true>}};
+    const int lr = a.n[0] >= kXLongRow;
+    hipLaunchKernelGGL(muscl ? km[lr][D == 3] : ks[lr][D == 3][mixed][learned],
+                       dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
   } else {
     const int64_t npencil = (dir == 1) ? a.n[0] * a.n[2] : a.n[0] * a.n[1];
     const int64_t bx = (npencil + kBlock - 1) / kBlock;

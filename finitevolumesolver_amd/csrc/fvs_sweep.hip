@@ -1155,6 +1155,11 @@ int LaunchTyped(hipStream_t s, int dir, const SweepArgs& a) {
       SetError("X sweep: %lld slots exceed the 32-bit slot index", static_cast<long long>(slots));
       return FVS_BAD_ARGUMENT;
     }
+    if (a.n[0] >= kXLongRow) {
+      SetError("X sweep: a row of %lld cells exceeds the 32-bit offset range",
+               static_cast<long long>(a.n[0]));
+      return FVS_BAD_ARGUMENT;
+    }
     hipLaunchKernelGGL((SweepXKernel<D, LARR, T, FAST>), dim3(static_cast<unsigned>(blocks)),
                        dim3(kBlock), 0, s, a);
   } else {

@@ -19,6 +19,10 @@
 // to about 2^32 and send their loads outside the arrays.  Such lanes are
 // placed anew (Next).
 //
+// The lane offset in bytes stays below 2^32 in rows shorter than kXLongRow
+// cells (64 slots reach at most 62 cells into the next row).  Longer rows need
+// 64-bit offsets, and the LONG form of Next, whose slots may pass 2^32.
+//
 // The header compiles for the device and, with tests/host_stub, for the
 // host, where tests/test_xslots.py walks every lane of every wave over
 // ragged shapes and checks that each load and store stays inside the
@@ -32,6 +36,7 @@ namespace fvs {
 
 constexpr int kXOwned = 60;      // slots owned per chunk (lanes 2 .. 61)
 constexpr int kXWavesPerCu = 16;  // persistent waves per CU
+constexpr int64_t kXLongRow = (int64_t(1) << 29) - 64;
 
 struct XSlot {
   bool valid;      // the lane's slot lies in the sequence
@@ -94,7 +99,14 @@ struct XSlotWalker {
   }
 
   // Moves the position by the stride, with one compare.
-  __host__ __device__ void Advance() {
+  template <bool LONG> __host__ __device__ void Advance() {
+    if (LONG) {  // no sum of two slots
+      const uint32_t room = S - step_sl;
+      const bool wraps = q_sl >= room;
+      q_sl = wraps ? q_sl - room : q_sl + step_sl;
+      q_row += step_rows + (wraps ? 1u : 0u);
+      return;
+    }
     q_sl += step_sl;
     q_row += step_rows;
     if (q_sl >= S) {
@@ -108,9 +120,10 @@ struct XSlotWalker {
   // anew).  A lane past the end in c is past it in cn as well, where
   // RowSlot ignores the position.  Past the last chunk the position stays at
   // c.
+  template <bool LONG = false>
   __host__ __device__ void Next(int64_t c, int64_t cn, int64_t nchunks) {
     if (cn < nchunks && Slot(c) >= 0) {
-      Advance();
+      Advance<LONG>();
     } else {
       Place(cn < nchunks ? cn : c);
     }

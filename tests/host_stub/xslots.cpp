@@ -1,12 +1,13 @@
 // The X sweep's slot walker (fvs_xslots.hpp) on the host: every lane of
 // every persistent wave walks its chunks exactly as SweepXKernel does (one
-// Place for the first chunk, Next per stride, lane 0's cell as the wave base).
+// Place for the first chunk, Next per stride, lane 0's row as the wave base).
 // Checked for each (nx, rows, waves): a valid lane sits on its true slot,
 // every load address lies inside the nx * rows cells, the owned real slots
 // write each cell exactly once, and no offset wraps.  Rows of up to 2^32
 // slots, which no array here could hold, are checked at chunks around their
 // ends and around the cells whose byte offsets within the row pass 2^32: every
-// lane's address is its cell's.  Prints the number of violations (0 expected).
+// lane's address is its cell's, with 64-bit offsets from kXLongRow cells on.
+// Prints the number of violations (0 expected).
 #include "fvs_xslots.hpp"
 
 #include <cstdio>
@@ -16,8 +17,9 @@ using fvs::XSlot;
 using fvs::XSlotWalker;
 
 // Byte address of cell i of the slot's row, as the kernels form it.
-static int64_t Address(const XSlot& s, int64_t i) {
-  return 8 * s.wbase + static_cast<int64_t>(s.Bytes(i));
+static int64_t Address(const XSlot& s, int64_t nx, int64_t i) {
+  if (nx >= fvs::kXLongRow) return 8 * (s.wbase + s.rbase + i);
+  return 8 * s.wbase + static_cast<int64_t>(8u * (s.rbase + static_cast<uint32_t>(i)));
 }
 
 static long Check(int64_t nx, int64_t rows, int64_t nwaves) {
@@ -37,14 +39,14 @@ static long Check(int64_t nx, int64_t rows, int64_t nwaves) {
       uint32_t row[64], sl[64];
       for (int l = 0; l < 64; ++l) lanes[l].RowSlot(c, &valid[l], &row[l], &sl[l]);
       for (int l = 0; l < 64; ++l) {
-        const XSlot s = lanes[l].Make(valid[l], row[l], sl[l], row[0], sl[0]);
+        const XSlot s = lanes[l].Make(valid[l], row[l], sl[l], row[0]);
         if (valid[l] && static_cast<int64_t>(row[l]) * S + sl[l] != lanes[l].Slot(c)) ++bad;
         const int64_t cl = s.cell < 0 ? 0 : (s.cell >= nx ? nx - 1 : s.cell);
-        if (Address(s, cl) != 8 * (row[l] * nx + cl) || row[l] * nx + cl >= ncell) ++bad;
+        if (Address(s, nx, cl) != 8 * (row[l] * nx + cl) || row[l] * nx + cl >= ncell) ++bad;
         const bool owned = l >= 2 && l < 2 + fvs::kXOwned;
         const bool real = s.valid && s.cell >= 0 && s.cell < nx;
         if (owned && real) {
-          const int64_t st = Address(s, s.cell);
+          const int64_t st = Address(s, nx, s.cell);
           if (st < 0 || st >= 8 * ncell || st % 8 != 0) ++bad;
           else ++written[st / 8];
         }
@@ -74,14 +76,19 @@ static long CheckLong(int64_t nx, int64_t rows, int64_t nwaves) {
         for (int l = 0; l < 64; ++l) {
           lanes.emplace_back(nx, Q, nwaves, l);
           lanes[l].Place(c >= nwaves ? c - nwaves : c);
-          if (c >= nwaves) lanes[l].Next(c - nwaves, c, nchunks);
+          if (c >= nwaves) {
+            if (nx >= fvs::kXLongRow)
+              lanes[l].Next<true>(c - nwaves, c, nchunks);
+            else
+              lanes[l].Next(c - nwaves, c, nchunks);
+          }
           lanes[l].RowSlot(c, &valid[l], &row[l], &sl[l]);
         }
         for (int l = 0; l < 64; ++l) {
-          const XSlot s = lanes[l].Make(valid[l], row[l], sl[l], row[0], sl[0]);
+          const XSlot s = lanes[l].Make(valid[l], row[l], sl[l], row[0]);
           if (valid[l] && row[l] * S + sl[l] != lanes[l].Slot(c)) ++bad;
           const int64_t cl = s.cell < 0 ? 0 : (s.cell >= nx ? nx - 1 : s.cell);
-          if (Address(s, cl) != 8 * (row[l] * nx + cl)) ++bad;
+          if (Address(s, nx, cl) != 8 * (row[l] * nx + cl)) ++bad;
         }
       }
   return bad;
@@ -106,7 +113,7 @@ int main() {
         ++cases;
       }
     }
-  const int64_t lengths[] = {(int64_t(1) << 29) - 1, (int64_t(1) << 29) + 5, (int64_t(1) << 30) + 61,
+  const int64_t lengths[] = {fvs::kXLongRow - 1, fvs::kXLongRow, (int64_t(1) << 29) + 5, (int64_t(1) << 30) + 61,
                              (int64_t(1) << 31) + 3, (int64_t(1) << 32) - 4};
   for (int64_t nx : lengths)
     for (int64_t nwaves : {4, 4096}) {

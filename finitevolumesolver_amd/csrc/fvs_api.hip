@@ -891,6 +891,15 @@ int fvs_newton_stats(fvs_handle* h, uint64_t stats[5], int reset) {
 
 // ---- level driver ----------------------------------------------------------
 
+// Steps per chained graph (the step sequence depends only on the start
+// buffer and the cycle parity, so a chain is captured once per pair).  Also the
+// steps a level takes before it captures anything: a capture costs as much host
+// time as the eager steps it replaces, so a level that runs a few steps and no
+// more is faster without, and in a longer run the captures overlap the steps
+// already enqueued.  First two steps of a MUSCL-Hancock level over exact
+// Godunov, 64^2: 230 us; with all twelve graphs captured ahead 1,075.
+static constexpr int kChainSteps = 8;
+
 struct fvs_level {
   fvs_handle* h;
   fvs_patch_desc patch;
@@ -927,11 +936,9 @@ struct fvs_level {
     hipGraphExec_t exec;
   };
   std::vector<StepGraph> graphs;
+  // Steps still to be launched eagerly before the first capture.
+  int eager_left = kChainSteps;
 };
-
-// Steps per chained graph (the step sequence depends only on the start
-// buffer and the cycle parity, so a chain is captured once per pair).
-constexpr int kChainSteps = 8;
 
 namespace {
 
@@ -1098,6 +1105,7 @@ int fvs_level_set_graphs(fvs_level* L, int on) {
     return FVS_BAD_ARGUMENT;
   }
   L->use_graphs = on ? 1 : 0;
+  L->eager_left = 0;  // asked for: from the next step on
   return FVS_OK;
 }
 
@@ -1370,18 +1378,6 @@ static int CaptureLevelSteps(fvs_level* L, int cur, int parity, const fvs_mlp* n
   return FVS_OK;
 }
 
-// Every single-step and chained graph of the level for this network (six
-// start states: three buffers, two cycle parities), captured before the
-// first replay so that no capture falls inside a run of steps.
-static int EnsureLevelGraphs(fvs_level* L, const fvs_mlp* net) {
-  const fvs_level::StepGraph* g = nullptr;
-  for (int cur = 0; cur < 3; ++cur)
-    for (int parity = 0; parity < 2; ++parity)
-      for (int nsteps : {1, kChainSteps})
-        if (int rc = CaptureLevelSteps(L, cur, parity, net, nsteps, &g)) return rc;
-  return FVS_OK;
-}
-
 // Launches nsteps (1 or kChainSteps) steps from buffer cur as one replayed
 // graph; curs receives the start buffer of each step and, last, the result's.
 static int LaunchLevelStepGraph(fvs_level* L, int cur, int64_t cyc, const fvs_mlp* net,
@@ -1435,24 +1431,19 @@ int fvs_level_advance(fvs_level* L, int max_steps, double final_time, int batch,
                                  hipMemcpyDeviceToHost, s));
     FVS_HIP_CHECK(hipStreamSynchronize(s));
   }
-  if (!L->timing && L->use_graphs && max_steps > 0) {
-    if (int rc2 = EnsureLevelGraphs(L, net)) {
-      if (dlog) (void)hipFree(dlog);
-      return rc2;
-    }
-  }
-  while (cycle - cycle0 < max_steps) {
+  while (rc == FVS_OK && cycle - cycle0 < max_steps) {
     const int k = static_cast<int>(std::min<int64_t>(batch, max_steps - (cycle - cycle0)));
     start_buf.assign(k + 1, 0);
     int cur = L->cur;
     std::vector<int> curs;
     for (int sidx = 0; sidx < k && rc == FVS_OK;) {
       const int64_t cyc = cycle + sidx;
-      if (L->timing || !L->use_graphs) {
-        start_buf[sidx] = cur;
+      start_buf[sidx] = cur;
+      if (L->timing || !L->use_graphs || L->eager_left > 0) {
         int next = cur;
         rc = LaunchLevelStep(L, s, cur, cyc, net, &next);
         if (rc) break;
+        if (L->eager_left > 0) --L->eager_left;
         cur = next;
         ++sidx;
         continue;
@@ -1464,7 +1455,7 @@ int fvs_level_advance(fvs_level* L, int max_steps, double final_time, int batch,
       cur = curs[nsteps];
       sidx += nsteps;
     }
-    if (rc) break;
+    // After a failed launch or capture (rc) the steps enqueued before it count.
     FVS_HIP_CHECK(hipMemcpyAsync(&c, L->ctl, sizeof c, hipMemcpyDeviceToHost, s));
     if (godunov)
       FVS_HIP_CHECK(hipMemcpyAsync(newton1, h->newton_stats, sizeof newton1,
@@ -1491,8 +1482,9 @@ int fvs_level_advance(fvs_level* L, int max_steps, double final_time, int batch,
     cycle = c.cycle;
     if (c.halt == 2) break;
     if (c.halt == 3) {
-      // The CFL pass's speed floor (already cleared) was not reached: the
-      // step runs again with every face evaluated.  Not a CFL failure.
+      // The CFL pass's speed floor was not reached: the step runs again with
+      // the floor that RenewSpeedFloor left (an exact-Godunov level's from its
+      // cells, or none, with every face evaluated).  Not a CFL failure.
       ++L->cfl_redos;
       c.halt = 0;
       FVS_HIP_CHECK(hipMemcpyAsync(L->ctl, &c, sizeof c, hipMemcpyHostToDevice, s));

@@ -323,11 +323,12 @@ int fvs_level_set_timing(fvs_level* level, int on);
 int fvs_level_kernel_times(fvs_level* level, double* ms, int64_t* count);
 
 /* Replay the level's time steps from HIP graphs (on by default; the timing
- * mode launches eagerly): on the first advance with graphs on, every
- * distinct step (per start buffer, cycle parity and attached network) is
- * captured once as a single-step graph and as an 8-step chain, and runs of
- * eight steps are replayed as one graph launch.  No counterpart in the
- * reference, whose steps are host loops; results are identical either way. */
+ * mode launches eagerly).  A level launches its first eight steps eagerly
+ * (none after a call of this function with on = 1); after them a step of a
+ * new kind (start buffer, cycle parity, attached network) is captured where it
+ * is met, as a single step or, in runs of eight and more, as a chain of eight
+ * that one graph launch replays.  No counterpart in the reference, whose steps
+ * are host loops; results are identical either way. */
 int fvs_level_set_graphs(fvs_level* level, int on);
 
 /* One fused split sweep (flux + update + completion + CFL check of the

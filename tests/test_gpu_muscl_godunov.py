@@ -60,3 +60,22 @@ def test_fused_level_matches_oracle(cuda, shape, limiter, split, cfl):
     assert tolerance_ratio(got, ref) <= 1.0
     eager = _run(cuda, cons, shape, limiter, split, cfl, 5, graphs=False)
     assert np.array_equal(eager[3], got) and list(eager[2]) == list(dts)
+
+
+@pytest.mark.parametrize("base,recon", [("Godunov", "MusclHancock"), ("Godunov", "None"), ("HLLEM", "MusclHancock")])
+def test_captures_within_a_run(cuda, base, recon):
+    """By default a level launches its first eight steps and captures the later
+    ones where it meets them, inside a run: same bits as eager launches."""
+    import torch
+    cons = rough_field((1, 40, 50), seed=8)
+    runs = []
+    for eager in (False, True):
+        fm = fvs.FluxMethod(fvs.PerfectGas(dim=2), base=base, reconstruction=recon)
+        lvl = fvs.SinglePatchLevel(fm, (50, 40), (0.02, 0.02), cfl=0.8)
+        if eager:
+            lvl.set_graphs(False)
+        lvl.set_state(torch.from_numpy(cons).to(cuda))
+        runs.append([lvl.advance(n, batch=b, return_dts=True) + (lvl.get_state().cpu().numpy(),)
+                     for n, b in ((3, 3), (11, 11), (37, 37), (5, 2))])
+    for a, b in zip(*runs):
+        assert a[:2] == b[:2] and a[2] == b[2] and np.array_equal(a[3], b[3])

@@ -16,6 +16,7 @@
 #include "fvs_mlp_infer.hpp"
 #include "fvs_riemann.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -776,25 +777,37 @@ int fvs_mlp_train(fvs_mlp* m, int epochs, int64_t batch, float lr, float huber, 
   }
   const int64_t nbatches = nv / batch;
   // Device: two epochs' permutations (the next one is shuffled and uploaded
-  // while an epoch runs) and the loss of every step; host: pinned staging.
+  // while an epoch runs) and their steps' losses; host: pinned staging of both.
+  // A single epoch stages in pageable memory.
   uint32_t* perm = nullptr;
   float* losses = nullptr;
-  uint32_t* stage = nullptr;
-  hipEvent_t uploaded[2] = {nullptr, nullptr};
-  const size_t pbytes = nv * sizeof(uint32_t);
-  const size_t nloss = static_cast<size_t>(epochs > 0 ? epochs : 1) * nbatches;
+  char* stage = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr};  // an epoch's steps and loss copy
+  const size_t pbytes = nv * sizeof(uint32_t), lbytes = nbatches * sizeof(float);
   const int nbuf = epochs > 1 ? 2 : 1;
+  std::vector<float> one(nbuf == 1 ? nbatches : 0);
   int rc = FVS_OK;
-  if (Alloc((void**)&perm, nbuf * pbytes) || Alloc((void**)&losses, nloss * sizeof(float)))
+  if (Alloc((void**)&perm, nbuf * pbytes) || Alloc((void**)&losses, nbuf * lbytes))
     rc = FVS_HIP_ERROR;
-  if (rc == FVS_OK && epochs > 1) {
-    if (hipHostMalloc(&stage, nbuf * pbytes, hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&uploaded[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&uploaded[1], hipEventDisableTiming) != hipSuccess) {
+  if (rc == FVS_OK && nbuf > 1) {
+    if (hipHostMalloc(&stage, nbuf * (pbytes + lbytes), hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&done[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&done[1], hipEventDisableTiming) != hipSuccess) {
       SetError("training buffers failed");
       rc = FVS_HIP_ERROR;
     }
   }
+  float* host_losses = stage ? reinterpret_cast<float*>(stage + nbuf * pbytes) : one.data();
+  // The smoothed loss of epoch e, whose losses have arrived.
+  auto record = [&](int e) {
+    const float* l = host_losses + (e % nbuf) * nbatches;
+    double smooth = 0.0;
+    for (int64_t b = 0; b < nbatches; ++b) {
+      if (b % 64 != 0 && b != nbatches - 1) continue;
+      smooth = (b == 0) ? l[b] : 0.9 * smooth + 0.1 * l[b];
+    }
+    loss_history[e] = static_cast<float>(smooth);
+  };
   uint64_t st = seed;
   AdamStep adam{};
   adam.b1 = 0.9f;
@@ -812,17 +825,18 @@ int fvs_mlp_train(fvs_mlp* m, int epochs, int64_t batch, float lr, float huber, 
     }
     const int buf = e % nbuf;
     uint32_t* dst = perm + buf * nv;
-    const uint32_t* src = valid.data();
+    const void* src = valid.data();
     if (stage) {
-      // the staging buffer's upload of two epochs ago has left it
-      if (e >= 2 && hipEventSynchronize(uploaded[buf]) != hipSuccess) rc = FVS_HIP_ERROR;
-      std::memcpy(stage + buf * nv, valid.data(), pbytes);
-      src = stage + buf * nv;
+      // the epoch before last has left its buffers
+      if (e >= 2) {
+        if (hipEventSynchronize(done[buf]) != hipSuccess) rc = FVS_HIP_ERROR;
+        if (rc == FVS_OK && loss_history) record(e - 2);
+      }
+      src = std::memcpy(stage + buf * pbytes, valid.data(), pbytes);
     }
     if (rc != FVS_OK ||
         hipMemcpyAsync(dst, src, pbytes, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-        (stage ? hipEventRecord(uploaded[buf], m->stream) : hipStreamSynchronize(m->stream)) !=
-            hipSuccess) {
+        (!stage && hipStreamSynchronize(m->stream) != hipSuccess)) {
       SetError("permutation upload failed");
       rc = FVS_HIP_ERROR;
       break;
@@ -835,32 +849,27 @@ int fvs_mlp_train(fvs_mlp* m, int epochs, int64_t batch, float lr, float huber, 
       adam.lr =
           static_cast<float>(lr * 0.5 * (1.0 + std::cos(3.141592653589793 * step / total)));
       rc = BatchGradients(m, m->x, m->target, m->flag, n, dst + b * batch, batch,
-                          1.0f / float(batch), huber, nullptr, losses + e * nbatches + b, adam);
+                          1.0f / float(batch), huber, nullptr, losses + buf * nbatches + b, adam);
     }
-  }
-  if (rc == FVS_OK && loss_history && epochs > 0) {
-    std::vector<float> l(nloss);
-    if (hipMemcpyAsync(l.data(), losses, nloss * sizeof(float), hipMemcpyDeviceToHost,
-                       m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess) {
+    if (rc != FVS_OK) break;
+    if ((loss_history &&
+         hipMemcpyAsync(host_losses + buf * nbatches, losses + buf * nbatches, lbytes,
+                        hipMemcpyDeviceToHost, m->stream) != hipSuccess) ||
+        (stage && hipEventRecord(done[buf], m->stream) != hipSuccess)) {
       SetError("loss readback failed");
       rc = FVS_HIP_ERROR;
     }
-    for (int e = 0; e < epochs && rc == FVS_OK; ++e) {
-      double smooth = 0.0;
-      for (int64_t b = 0; b < nbatches; ++b) {
-        if (b % 64 != 0 && b != nbatches - 1) continue;
-        const float v = l[e * nbatches + b];
-        smooth = (b == 0) ? v : 0.9 * smooth + 0.1 * v;
-      }
-      loss_history[e] = static_cast<float>(smooth);
-    }
   }
-  (void)hipStreamSynchronize(m->stream);
+  if (hipStreamSynchronize(m->stream) != hipSuccess && rc == FVS_OK) {
+    SetError("training failed");
+    rc = FVS_HIP_ERROR;
+  }
+  if (rc == FVS_OK && loss_history)
+    for (int e = std::max(0, epochs - nbuf); e < epochs; ++e) record(e);
   if (perm) (void)hipFree(perm);
   if (losses) (void)hipFree(losses);
   if (stage) (void)hipHostFree(stage);
-  for (hipEvent_t ev : uploaded)
+  for (hipEvent_t ev : done)
     if (ev) (void)hipEventDestroy(ev);
   if (rc != FVS_OK) return rc;
   if (int rc = Pack(m)) return rc;

@@ -171,7 +171,9 @@ __device__ __forceinline__ double CellFaceSpeed(const double* L, double mL, cons
                                                 double mR, const Gas<double>& g, double tol,
                                                 int max_it, unsigned long long* acc) {
   using I = Idx<D>;
-  const double uL = NearArith::quot(mL, L[0]), uR = NearArith::quot(mR, R[0]);
+  double uL, uR;
+  FaceVelocities(mL, L[0], NearArith::inv(L[0]), L[I::kA], mR, R[0], NearArith::inv(R[0]),
+                 R[I::kA], &uL, &uR);
   NewtonParams np;
   np.tol = tol;
   np.max_it = max_it;
@@ -184,25 +186,40 @@ __device__ __forceinline__ double CellFaceSpeed(const double* L, double mL, cons
     acc[2] += ms.converged ? 0 : 1;
   }
   double wL, wR;
-  return GodunovSpeed(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP], R[I::kA], ms, &wL, &wR);
+  return GodunovSpeed(L[0], uL, L[I::kP], L[I::kA], R[0], uR, R[I::kP], R[I::kA], ms, g.gamma, &wL,
+                      &wR);
+}
+
+// A quotient by NearArith, with special results where FIX.
+template <bool FIX> __device__ __forceinline__ double Quot(double a, double b, double y) {
+  const double q = NearArith::div(a, b, y);
+  return FIX ? NearArith::fix(q, a, b) : q;
 }
 
 // Pressure and speed of sound of a conservative state; SCALAR: kinetic energy
-// in the order of the scalar path (fvs_riemann.hpp).  y_g = inv(gm1inv).
-template <int D, bool SCALAR>
-__device__ __forceinline__ void Complete(CellState<D>& c, const Gas<double>& g, double y_g) {
+// in the order of the scalar path (fvs_riemann.hpp).  y_g = inv(gm1inv).  A
+// state that is no gas (IsGas) is completed with FIX.
+template <int D, bool SCALAR, bool FIX>
+__device__ __forceinline__ void CompleteNear(CellState<D>& c, const Gas<double>& g, double y_g) {
   using I = Idx<D>;
   c.y = NearArith::inv(c.q[0]);
   const double sq = SCALAR ? SqNormScalar<D>(c.q + 1) : SqNormArray<D>(c.q + 1);
-  const double e_int = c.q[I::kE] - NearArith::div(0.5 * sq, c.q[0], c.y);
-  c.q[I::kP] = NearArith::div(e_int, g.gm1inv, y_g);
-  c.q[I::kA] = NearArith::sqrt(NearArith::div(g.gamma * c.q[I::kP], c.q[0], c.y));
+  const double e_int = c.q[I::kE] - Quot<FIX>(0.5 * sq, c.q[0], c.y);
+  c.q[I::kP] = Quot<FIX>(e_int, g.gm1inv, y_g);
+  c.q[I::kA] = NearArith::sqrt(Quot<FIX>(g.gamma * c.q[I::kP], c.q[0], c.y));
+}
+
+// A first-order cell.
+template <int D>
+__device__ __forceinline__ void Complete(CellState<D>& c, const Gas<double>& g, double y_g) {
+  CompleteNear<D, false, false>(c, g, y_g);
+  if (__builtin_expect(!IsGas(c.q[Idx<D>::kA]), 0)) CompleteNear<D, false, true>(c, g, y_g);
 }
 
 // MUSCL-Hancock half-step states of one cell at its left and right face
 // (MusclHancockMethod.hpp:419-485) in the sequential driver's arithmetic.
-template <int D, int DIR, int LIM>
-__device__ __forceinline__ void ReconNear(const double* um, const double* u0, const double* up,
+template <int D, int DIR, int LIM, bool FIX>
+__device__ __forceinline__ void HalfStep(const double* um, const double* u0, const double* up,
                                           double lh, const Gas<double>& g, double y_g,
                                           CellState<D>& recL, CellState<D>& recR) {
   using I = Idx<D>;
@@ -218,9 +235,9 @@ __device__ __forceinline__ void ReconNear(const double* um, const double* u0, co
   for (int side = 0; side < 2; ++side) {
     const double* q = side == 0 ? recL.q : recR.q;
     const double y = NearArith::inv(q[0]);
-    const double e_kin = NearArith::div(0.5 * SqNormScalar<D>(q + 1), q[0], y);
-    const double p = NearArith::div(q[I::kE] - e_kin, g.gm1inv, y_g);
-    const double v = NearArith::div(q[1 + DIR], q[0], y);
+    const double e_kin = Quot<FIX>(0.5 * SqNormScalar<D>(q + 1), q[0], y);
+    const double p = Quot<FIX>(q[I::kE] - e_kin, g.gm1inv, y_g);
+    const double v = Quot<FIX>(q[1 + DIR], q[0], y);
     f[side][0] = q[1 + DIR];
 #pragma unroll
     for (int d = 0; d < D; ++d) f[side][1 + d] = v * q[1 + d];
@@ -233,19 +250,36 @@ __device__ __forceinline__ void ReconNear(const double* um, const double* u0, co
     recR.q[k] += dq;
     recL.q[k] += dq;
   }
-  Complete<D, true>(recR, g, y_g);
-  Complete<D, true>(recL, g, y_g);
+  CompleteNear<D, true, FIX>(recR, g, y_g);
+  CompleteNear<D, true, FIX>(recL, g, y_g);
 }
 
-template <int D, int DIR>
-__device__ __forceinline__ void ReconAnyNear(int limiter, const double* um, const double* u0,
-                                             const double* up, double lh, const Gas<double>& g,
-                                             double y_g, CellState<D>& recL, CellState<D>& recR) {
+// Which states of a cell a caller reads.
+constexpr int kLeftState = 1, kRightState = 2, kBothStates = 3;
+
+// Any cell.  A special quotient of one state's flux makes neither state a gas,
+// so the states that are read tell (the other one's are never computed).
+template <int D, int DIR, int LIM, int USE>
+__device__ __forceinline__ void Recon(const double* um, const double* u0, const double* up,
+                                      double lh, const Gas<double>& g, double y_g,
+                                      CellState<D>& recL, CellState<D>& recR) {
+  using I = Idx<D>;
+  HalfStep<D, DIR, LIM, false>(um, u0, up, lh, g, y_g, recL, recR);
+  const bool gas = (!(USE & kLeftState) || IsGas(recL.q[I::kA])) &&
+                   (!(USE & kRightState) || IsGas(recR.q[I::kA]));
+  if (__builtin_expect(!gas, 0))
+    HalfStep<D, DIR, LIM, true>(um, u0, up, lh, g, y_g, recL, recR);
+}
+
+template <int D, int DIR, int USE = kBothStates>
+__device__ __forceinline__ void ReconAny(int limiter, const double* um, const double* u0,
+                                         const double* up, double lh, const Gas<double>& g,
+                                         double y_g, CellState<D>& recL, CellState<D>& recR) {
   switch (limiter) {
-  case kMinMod: ReconNear<D, DIR, kMinMod>(um, u0, up, lh, g, y_g, recL, recR); break;
-  case kVanLeer: ReconNear<D, DIR, kVanLeer>(um, u0, up, lh, g, y_g, recL, recR); break;
-  case kNoLimiter: ReconNear<D, DIR, kNoLimiter>(um, u0, up, lh, g, y_g, recL, recR); break;
-  default: ReconNear<D, DIR, kNoGradient>(um, u0, up, lh, g, y_g, recL, recR); break;
+  case kMinMod: Recon<D, DIR, kMinMod, USE>(um, u0, up, lh, g, y_g, recL, recR); break;
+  case kVanLeer: Recon<D, DIR, kVanLeer, USE>(um, u0, up, lh, g, y_g, recL, recR); break;
+  case kNoLimiter: Recon<D, DIR, kNoLimiter, USE>(um, u0, up, lh, g, y_g, recL, recR); break;
+  default: Recon<D, DIR, kNoGradient, USE>(um, u0, up, lh, g, y_g, recL, recR); break;
   }
 }
 
@@ -271,15 +305,16 @@ __device__ __forceinline__ void GodunovFace(const CellState<D>& L, const CellSta
   NewtonParams np;
   np.tol = a.tol;
   np.max_it = a.max_it;
-  const double uL = NearArith::div(L.q[1 + DIR], L.q[0], L.y);
-  const double uR = NearArith::div(R.q[1 + DIR], R.q[0], R.y);
+  double uL, uR;
+  FaceVelocities(L.q[1 + DIR], L.q[0], L.y, L.q[I::kA], R.q[1 + DIR], R.q[0], R.y, R.q[I::kA], &uL,
+                 &uR);
   const double mean = 0.5 * (L.q[I::kP] + R.q[I::kP]);
   int it, fallback;
   const MiddleState ms = SeededMiddleState<D>(L, uL, R, uR, g, np, has_guess, guess, mean, &it,
                                               &fallback);
   double wL, wR;
   const double speed = GodunovSpeed(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP],
-                                    R.q[I::kA], ms, &wL, &wR);
+                                    R.q[I::kA], ms, g.gamma, &wL, &wR);
   GodunovFlux<D, DIR, MIXED>(F, L.q, L.y, R.q, R.y, ms, wL, wR, g);
   if (count) {
     const unsigned n = static_cast<unsigned>(it);
@@ -400,11 +435,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         um[k] = (a.limiter == kNoLimiter && cur.cell < 0) ? u[k] : ul[k];
         if (a.limiter == kNoLimiter && cur.cell >= nx) up[k] = u[k];
       }
-      ReconAnyNear<D, 0>(a.limiter, um, u, up, lh, g, y_g, R, L);
+      ReconAny<D, 0>(a.limiter, um, u, up, lh, g, y_g, R, L);
     } else {
 #pragma unroll
       for (int k = 0; k < NC; ++k) R.q[k] = u[k];
-      Complete<D, false>(R, g, y_g);
+      Complete<D>(R, g, y_g);
       L = R;
     }
 #pragma unroll
@@ -502,13 +537,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     load(Umm, j0 - 2);
     CellState<D> unused;
     if (j0 == 0)
-      ReconNear<D, DIR, kNoGradient>(Um, Um, Um, lh, g, y_g, unused, L);
+      Recon<D, DIR, kNoGradient, kRightState>(Um, Um, Um, lh, g, y_g, unused, L);
     else
-      ReconAnyNear<D, DIR>(a.limiter, Umm, Um, U0, lh, g, y_g, unused, L);
+      ReconAny<D, DIR, kRightState>(a.limiter, Umm, Um, U0, lh, g, y_g, unused, L);
   } else {
 #pragma unroll
     for (int k = 0; k < NC; ++k) L.q[k] = Um[k];
-    Complete<D, false>(L, g, y_g);
+    Complete<D>(L, g, y_g);
   }
   for (int64_t j = j0; j <= j1; ++j) {
     double Up[NC];
@@ -518,13 +553,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     CellState<D> R, Lnext;
     if constexpr (MUSCL) {
       if (j < nd)
-        ReconAnyNear<D, DIR>(a.limiter, Um, U0, Up, lh, g, y_g, R, Lnext);
+        ReconAny<D, DIR>(a.limiter, Um, U0, Up, lh, g, y_g, R, Lnext);
       else
-        ReconNear<D, DIR, kNoGradient>(U0, U0, U0, lh, g, y_g, R, Lnext);
+        Recon<D, DIR, kNoGradient, kLeftState>(U0, U0, U0, lh, g, y_g, R, Lnext);
     } else {
 #pragma unroll
       for (int k = 0; k < NC; ++k) R.q[k] = U0[k];
-      Complete<D, false>(R, g, y_g);
+      Complete<D>(R, g, y_g);
       Lnext = R;
     }
     double F[NC];
@@ -657,8 +692,8 @@ __global__ __launch_bounds__(kBlock) void GodunovViewFlux(DevView fl, DevView st
     for (int s = 0; s < 4; ++s) loadc(s - 2, u[s], NC);
     const double lh = 0.5 * dt / dx;
     CellState<D> unused;
-    ReconAnyNear<D, DIR>(limiter, u[0], u[1], u[2], lh, g, y_g, unused, L);
-    ReconAnyNear<D, DIR>(limiter, u[1], u[2], u[3], lh, g, y_g, R, unused);
+    ReconAny<D, DIR, kRightState>(limiter, u[0], u[1], u[2], lh, g, y_g, unused, L);
+    ReconAny<D, DIR, kLeftState>(limiter, u[1], u[2], u[3], lh, g, y_g, R, unused);
   } else {
     loadc(-1, L.q, NQ);
     loadc(0, R.q, NQ);
@@ -668,15 +703,16 @@ __global__ __launch_bounds__(kBlock) void GodunovViewFlux(DevView fl, DevView st
   NewtonParams np;
   np.tol = tol;
   np.max_it = max_it;
-  const double uL = NearArith::div(L.q[1 + DIR], L.q[0], L.y);
-  const double uR = NearArith::div(R.q[1 + DIR], R.q[0], R.y);
+  double uL, uR;
+  FaceVelocities(L.q[1 + DIR], L.q[0], L.y, L.q[I::kA], R.q[1 + DIR], R.q[0], R.y, R.q[I::kA], &uL,
+                 &uR);
   const MiddleState ms =
       SolveMiddleState(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA], g,
                        np, 0.5 * (L.q[I::kP] + R.q[I::kP]));
   if (!ms.converged) atomicAdd(nfail, 1ull);
   double F[NC], wL, wR;
-  GodunovSpeed(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA], ms, &wL,
-               &wR);
+  GodunovSpeed(L.q[0], uL, L.q[I::kP], L.q[I::kA], R.q[0], uR, R.q[I::kP], R.q[I::kA], ms,
+               g.gamma, &wL, &wR);
   GodunovFlux<D, DIR, false>(F, L.q, L.y, R.q, R.y, ms, wL, wR, g);
   for (int k = 0; k < NC; ++k) *fl.at(f, k) = F[k];
 }
@@ -753,22 +789,40 @@ struct GodunovCflArgs {
 };
 
 // The face of direction d between the cells at off_l and off_r: its largest
-// signal speed, from Newton.
+// signal speed, from Newton.  Out of line: inlined, the solver's registers are
+// the marching loop's spills (the pass at 384^3 on strong waves: 1103 us, out
+// of line 1035).
+struct CflFaceResult {
+  double speed;
+  int iterations, converged;
+};
 template <int D>
-__device__ __forceinline__ double CflFace(const GodunovCflArgs& a, const Gas<double>& g, int d,
-                                          int64_t off_l, int64_t off_r,
-                                          unsigned long long* acc) {
+__device__ __attribute__((noinline)) CflFaceResult CflFace(const double* u0, const double* u1,
+                                                           const double* u2, const double* u3,
+                                                           const double* u4, double gamma,
+                                                           double gm1inv, double tol, int max_it,
+                                                           int d, int64_t off_l, int64_t off_r) {
+  const double* in[5] = {u0, u1, u2, u3, u4};
+  Gas<double> g;
+  g.gamma = gamma;
+  g.gm1inv = gm1inv;
+  g.gm1 = gamma - 1.0;
   double L[D + 4], R[D + 4];
 #pragma unroll
   for (int k = 0; k < D + 2; ++k) {
-    L[k] = a.in[k][off_l];
-    R[k] = a.in[k][off_r];
+    L[k] = in[k][off_l];
+    R[k] = in[k][off_r];
   }
   CompleteFromCons<D>(L, g);
   CompleteFromCons<D>(R, g);
   const double mL = d == 0 ? L[1] : (D == 2 || d == 1) ? L[2] : L[D];
   const double mR = d == 0 ? R[1] : (D == 2 || d == 1) ? R[2] : R[D];
-  return CellFaceSpeed<D>(L, mL, R, mR, g, a.tol, a.max_it, acc);
+  unsigned long long acc[3] = {0, 0, 0};
+  CflFaceResult r;
+  r.speed = CellFaceSpeed<D>(L, mL, R, mR, g, tol, max_it, acc);
+  r.iterations = static_cast<int>(acc[0]);
+  r.converged = acc[2] == 0;
+  return r;
 }
 
 template <int D> __device__ __forceinline__ SpeedCell<D> ShiftUpCell(const SpeedCell<D>& c) {
@@ -826,7 +880,14 @@ __global__ __launch_bounds__(64 * kCflRows) __attribute__((amdgpu_waves_per_eu(4
       const int d = static_cast<int>(entry & 3);
       const int64_t off = entry >> 3;
       const int64_t back = d == 0 ? 1 : d == M ? ms : nx;
-      const double v = CflFace<D>(a, g, d, (entry & 4) ? off : off - back, off, acc);
+      const CflFaceResult r =
+          CflFace<D>(a.in[0], a.in[1], a.in[2], a.in[3], a.in[4], a.gamma, a.gm1inv, a.tol,
+                     a.max_it, d, (entry & 4) ? off : off - back, off);
+      const double v = r.speed;
+      const unsigned long long it = static_cast<unsigned long long>(r.iterations);
+      acc[0] += it;
+      acc[1] = it > acc[1] ? it : acc[1];
+      acc[2] += r.converged ? 0 : 1;
       faces[0] += d == 0;
       faces[1] += d == 1;
       faces[2] += d == 2;

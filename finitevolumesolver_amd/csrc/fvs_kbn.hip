@@ -297,7 +297,7 @@ __device__ void WallProblem(double* sol, double* state, const double* normal,
   } else if (0.0 < reflected[0] && 0.0 < state[0]) {
     const MiddleState ms = ComputeMiddleState<D, 0>(reflected, state, bp.g, bp.np,
                                                     0.5 * (reflected[D + 2] + state[D + 2]));
-    SampleRiemann<D, 0>(sol, reflected, state, ms, bp.g);
+    SampleRiemann<D, 0>(sol, reflected, state, ms.pM, ms.uM, bp.g);
   }
   RotateMomentum<D>(sol + 1, unit, normal);
 }

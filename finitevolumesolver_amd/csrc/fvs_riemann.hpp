@@ -21,6 +21,13 @@
 // fluxes and stable dt of a 131 x 97 x 75 patch: 221 -> 131 us; the error of
 // the states against 64-bit arithmetic stays at 1e-16 to 3e-16.
 //
+// States that are no gas (no or negative pressure, no density, infinities and
+// NaNs) keep the numbers, infinities and NaNs of the reference's formulas:
+// their sound speed is not positive and finite (IsGas), where the special
+// results of the quotients are set (NearArith::fix; in every quotient it would
+// cost 3% of a step).  Not kept are the results for densities and pressures
+// beyond 1e150 or below 1e-150, whose products leave the range.
+//
 // Mixed form (MIXED = true): the same FP64 iteration; the sampled star
 // density takes its power from the single-precision estimates,
 // x^e = exp2(e log2 x).
@@ -35,7 +42,8 @@ namespace fvs {
 // one Newton step, and one residual correction of the result, whose error
 // beyond the final rounding is about 2^-45 units in the last place.  9
 // instructions a quotient, 3 for each further one by the same denominator.
-// A zero or non-finite denominator yields NaN.
+// A zero, infinite, subnormal or huge (above 2^1022) operand yields NaN; fix
+// and sqrt set the results of zero and infinite ones.
 struct NearArith {
   static __device__ __forceinline__ double inv(double b) {
     const double y = __builtin_amdgcn_rcp(b);
@@ -47,6 +55,11 @@ struct NearArith {
     return __builtin_fma(__builtin_fma(-q, b, a), y, q);
   }
   static __device__ __forceinline__ double quot(double a, double b) { return div(a, b, inv(b)); }
+  // q, the quotient div(a, b, y), with the results of zero, infinite and NaN
+  // operands set
+  static __device__ __forceinline__ double fix(double q, double a, double b) {
+    return __builtin_amdgcn_div_fixup(q, b, a);
+  }
   static __device__ __forceinline__ double sqrt(double x) {
     const double r = __builtin_amdgcn_rsq(x);
     double s = x * r;
@@ -55,7 +68,7 @@ struct NearArith {
     s = __builtin_fma(s, e, s);
     h = __builtin_fma(h, e, h);
     s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
-    return (x == 0.0) ? x : s;
+    return __builtin_amdgcn_class(x, 0x260) ? x : s;  // zeros, +infinity
   }
   // x^(-1/2) to about one unit in the last place: the estimate with one
   // third-order step, 1 / sqrt(1 - e) = 1 + e (1/2 + 3/8 e) + O(e^3).
@@ -133,11 +146,15 @@ __device__ __forceinline__ double PowPos(double x, double e) {
   return __builtin_ldexp(h + w, static_cast<int>(n));
 }
 
-// x^e, e > 0, for any x as pow returns it for a non-integer e: 0 and inf stay,
-// negative x and NaN give NaN.
+// x^e, e > 0, for any x as pow returns it: 0, infinity and NaN stay, and a
+// negative x has a power where e is a whole number (the fans of gamma = 5 / 3
+// and 2 have such exponents) or x is infinite.
 __device__ __forceinline__ double PowState(double x, double e) {
-  const double r = PowPos(x, e);
-  return (x > 0.0 && x <= 1.7976931348623157e308) ? r : (x < 0.0 ? __builtin_nan("") : x);
+  const double a = rabs(x);
+  const double r = (a > 0.0 && a <= 1.7976931348623157e308) ? PowPos(a, e) : a;
+  if (__builtin_expect(!(x < 0.0), 1)) return r;
+  if (__builtin_rint(e) == e) return __builtin_rint(0.5 * e) == 0.5 * e ? r : -r;
+  return a <= 1.7976931348623157e308 ? __builtin_nan("") : r;
 }
 
 // x^e of the sampled star density (x a ratio of pressures).
@@ -291,15 +308,39 @@ __device__ __forceinline__ MiddleState ComputeMiddleState(const double* L, const
                           x0);
 }
 
+// Whether a speed of sound is one: positive and finite.
+__device__ __forceinline__ bool IsGas(double a) { return __builtin_amdgcn_class(a, 0x180); }
+
+// Normal velocities of a face's sides from their momenta; y: refined reciprocals
+// of their densities.
+__device__ __forceinline__ void FaceVelocities(double mL, double rhoL, double yL, double aL,
+                                               double mR, double rhoR, double yR, double aR,
+                                               double* uL, double* uR) {
+  *uL = NearArith::div(mL, rhoL, yL);
+  *uR = NearArith::div(mR, rhoR, yR);
+  if (__builtin_expect(!(IsGas(aL) && IsGas(aR)), 0)) {
+    *uL = NearArith::fix(*uL, mL, rhoL);
+    *uR = NearArith::fix(*uR, mR, rhoR);
+  }
+}
+
 // Largest signal speed of a face (ComputeSignals): uL less and uR plus the
 // side's wave speed, a sqrt((gamma + 1) / (2 gamma) (pM / p - 1) + 1) for a
 // shock, which is 1 / (rho r) with the side's r, and a for a rarefaction.
 // The face's stable dt is dx / speed.
 __device__ __forceinline__ double GodunovSpeed(double rhoL, double uL, double pL, double aL,
                                                double rhoR, double uR, double pR, double aR,
-                                               const MiddleState& ms, double* wL, double* wR) {
+                                               const MiddleState& ms, double g, double* wL,
+                                               double* wR) {
   *wL = ms.pM > pL ? NearArith::quot(1.0, rhoL * ms.auxL) : aL;
   *wR = ms.pM > pR ? NearArith::quot(1.0, rhoR * ms.auxR) : aR;
+  if (__builtin_expect(!(IsGas(aL) && IsGas(aR)), 0)) {
+    auto wave = [&](double p, double a) {
+      return ms.pM > p ? a * rsqrt_ieee(((g + 1.0) * (ms.pM / p) + (g - 1.0)) / (2.0 * g)) : a;
+    };
+    *wL = wave(pL, aL);
+    *wR = wave(pR, aR);
+  }
   double s_max = 0.0;
   s_max = rmax(s_max, rabs(uL - *wL));
   s_max = rmax(s_max, rabs(uR + *wR));
@@ -308,40 +349,41 @@ __device__ __forceinline__ double GodunovSpeed(double rhoL, double uL, double pL
 
 // SolveRiemannProblem: the complete state at x/t = 0 given the middle state
 // (the cut cells' wall problems).
-template <int D, int DIR, class T>
-__device__ __forceinline__ void SampleRiemannT(T* state, const T* left, const T* right, T pM,
-                                               T uM, const Gas<T>& eq) {
+template <int D, int DIR>
+__device__ __forceinline__ void SampleRiemann(double* state, const double* left,
+                                              const double* right, double pM, double uM,
+                                              const Gas<double>& eq) {
   using I = Idx<D>;
   constexpr int NQ = I::kComp;
   constexpr int M = I::kMom;
-  auto set_momentum = [&](T momentum, const T* side) {
+  auto set_momentum = [&](double momentum, const double* side) {
 #pragma unroll
     for (int d = 0; d < D; ++d) state[M + d] = state[I::kRho] * (side[M + d] / side[I::kRho]);
     state[M + DIR] = momentum;
   };
   auto from_prim = [&]() {
-    const T rhoE_kin = T(0.5) * SqNormScalar<D>(state + M) / state[I::kRho];
-    const T rhoE_internal = state[I::kP] * eq.gm1inv;
+    const double rhoE_kin = 0.5 * SqNormScalar<D>(state + M) / state[I::kRho];
+    const double rhoE_internal = state[I::kP] * eq.gm1inv;
     state[I::kE] = rhoE_internal + rhoE_kin;
     state[I::kA] = rsqrt_ieee(eq.gamma * state[I::kP] / state[I::kRho]);
   };
-  auto copy = [&](const T* s) {
+  auto copy = [&](const double* s) {
 #pragma unroll
     for (int k = 0; k < NQ; ++k) state[k] = s[k];
   };
-  const T g = eq.gamma;
-  const T gp1 = g + T(1.0);
-  const T gm1 = g - T(1.0);
-  if (T(0.0) <= uM) {
-    const T uL = left[M + DIR] / left[I::kRho];
-    const T aL = left[I::kA];
-    const T pL = left[I::kP];
-    const T p_ratio = pM / pL;
-    const T g_ratio = gm1 / gp1;
+  const double g = eq.gamma;
+  const double gp1 = g + 1.0;
+  const double gm1 = g - 1.0;
+  if (0.0 <= uM) {
+    const double uL = left[M + DIR] / left[I::kRho];
+    const double aL = left[I::kA];
+    const double pL = left[I::kP];
+    const double p_ratio = pM / pL;
+    const double g_ratio = gm1 / gp1;
     if (pM > pL) {
-      const T shock_speed = uL - aL * rsqrt_ieee((gp1 * p_ratio + gm1) / (T(2.0) * g));
-      if (shock_speed < T(0.0)) {
-        state[I::kRho] = left[I::kRho] * (p_ratio + g_ratio) / (g_ratio * p_ratio + T(1.0));
+      const double shock_speed = uL - aL * rsqrt_ieee((gp1 * p_ratio + gm1) / (2.0 * g));
+      if (shock_speed < 0.0) {
+        state[I::kRho] = left[I::kRho] * (p_ratio + g_ratio) / (g_ratio * p_ratio + 1.0);
         set_momentum(state[I::kRho] * uM, left);
         state[I::kP] = pM;
         from_prim();
@@ -349,34 +391,34 @@ __device__ __forceinline__ void SampleRiemannT(T* state, const T* left, const T*
         copy(left);
       }
     } else {
-      const T aM = aL * PowState(p_ratio, gm1 / (T(2.0) * g));
-      const T shock_speed_TL = uM - aM;
-      const T shock_speed_HL = uL - aL;
-      if (T(0.0) < shock_speed_HL) {
+      const double aM = aL * PowState(p_ratio, gm1 / (2.0 * g));
+      const double shock_speed_TL = uM - aM;
+      const double shock_speed_HL = uL - aL;
+      if (0.0 < shock_speed_HL) {
         copy(left);
-      } else if (shock_speed_TL < T(0.0)) {
-        state[I::kRho] = left[I::kRho] * PowState(p_ratio, T(1) / g);
+      } else if (shock_speed_TL < 0.0) {
+        state[I::kRho] = left[I::kRho] * PowState(p_ratio, 1.0 / g);
         set_momentum(state[I::kRho] * uM, left);
         state[I::kP] = pM;
         from_prim();
       } else {
-        state[I::kRho] = left[I::kRho] * PowState(T(2.0) / gp1 + g_ratio * uL / aL, T(2.0) / gm1);
-        const T u = T(2.0) / gp1 * (aL + T(0.5) * gm1 * uL);
+        state[I::kRho] = left[I::kRho] * PowState(2.0 / gp1 + g_ratio * uL / aL, 2.0 / gm1);
+        const double u = 2.0 / gp1 * (aL + 0.5 * gm1 * uL);
         set_momentum(state[I::kRho] * u, left);
-        state[I::kP] = pL * PowState(T(2.0) / gp1 + g_ratio * uL / aL, T(2.0) * g / gm1);
+        state[I::kP] = pL * PowState(2.0 / gp1 + g_ratio * uL / aL, 2.0 * g / gm1);
         from_prim();
       }
     }
   } else {
-    const T uR = right[M + DIR] / right[I::kRho];
-    const T aR = right[I::kA];
-    const T pR = right[I::kP];
-    const T p_ratio = pM / pR;
-    const T g_ratio = gm1 / gp1;
+    const double uR = right[M + DIR] / right[I::kRho];
+    const double aR = right[I::kA];
+    const double pR = right[I::kP];
+    const double p_ratio = pM / pR;
+    const double g_ratio = gm1 / gp1;
     if (pM > pR) {
-      const T shock_speed = uR + aR * rsqrt_ieee((gp1 * p_ratio + gm1) / (T(2.0) * g));
-      if (T(0.0) < shock_speed) {
-        state[I::kRho] = right[I::kRho] * (p_ratio + g_ratio) / (g_ratio * p_ratio + T(1.0));
+      const double shock_speed = uR + aR * rsqrt_ieee((gp1 * p_ratio + gm1) / (2.0 * g));
+      if (0.0 < shock_speed) {
+        state[I::kRho] = right[I::kRho] * (p_ratio + g_ratio) / (g_ratio * p_ratio + 1.0);
         set_momentum(state[I::kRho] * uM, right);
         state[I::kP] = pM;
         from_prim();
@@ -384,32 +426,25 @@ __device__ __forceinline__ void SampleRiemannT(T* state, const T* left, const T*
         copy(right);
       }
     } else {
-      const T aM = aR * PowState(p_ratio, gm1 / (T(2.0) * g));
-      const T shock_speed_TR = uM + aM;
-      const T shock_speed_HR = uR + aR;
-      if (shock_speed_HR <= T(0.0)) {
+      const double aM = aR * PowState(p_ratio, gm1 / (2.0 * g));
+      const double shock_speed_TR = uM + aM;
+      const double shock_speed_HR = uR + aR;
+      if (shock_speed_HR <= 0.0) {
         copy(right);
-      } else if (shock_speed_TR >= T(0.0)) {
-        state[I::kRho] = right[I::kRho] * PowState(p_ratio, T(1) / g);
+      } else if (shock_speed_TR >= 0.0) {
+        state[I::kRho] = right[I::kRho] * PowState(p_ratio, 1.0 / g);
         set_momentum(state[I::kRho] * uM, right);
         state[I::kP] = pM;
         from_prim();
       } else {
-        state[I::kRho] = right[I::kRho] * PowState(T(2.0) / gp1 - g_ratio * uR / aR, T(2.0) / gm1);
-        const T u = T(2.0) / gp1 * (-aR + T(0.5) * gm1 * uR);
+        state[I::kRho] = right[I::kRho] * PowState(2.0 / gp1 - g_ratio * uR / aR, 2.0 / gm1);
+        const double u = 2.0 / gp1 * (-aR + 0.5 * gm1 * uR);
         set_momentum(state[I::kRho] * u, right);
-        state[I::kP] = pR * PowState(T(2.0) / gp1 - g_ratio * uR / aR, T(2.0) * g / gm1);
+        state[I::kP] = pR * PowState(2.0 / gp1 - g_ratio * uR / aR, 2.0 * g / gm1);
         from_prim();
       }
     }
   }
-}
-
-template <int D, int DIR>
-__device__ __forceinline__ void SampleRiemann(double* state, const double* left,
-                                              const double* right, const MiddleState& ms,
-                                              const Gas<double>& eq) {
-  SampleRiemannT<D, DIR, double>(state, left, right, ms.pM, ms.uM, eq);
 }
 
 // Godunov<PerfectGas<D>, ExactRiemannSolver> numeric flux between complete
@@ -438,11 +473,16 @@ __device__ __forceinline__ void GodunovFlux(double* flux, const double* L, doubl
   double vel[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) vel[d] = NearArith::div(q[M + d], rho, y);
+  if (__builtin_expect(!IsGas(a), 0)) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) vel[d] = NearArith::fix(vel[d], q[M + d], rho);
+  }
   const double u = sign * vel[DIR];
   const double um = sign * ms.uM;
   const bool shock = ms.pM > p;
-  // head of the wave left of x/t = 0: the side's own state
-  const bool own = shock ? !(u - w < 0.0) : 0.0 < u - a;
+  // head of the wave left of x/t = 0: the side's own state (a head that stands
+  // still counts for the right side only)
+  const bool own = shock ? !(u - w < 0.0) : (left ? 0.0 < u - a : 0.0 <= u - a);
   const bool star = shock ? !own : (!own && um - a * aux < 0.0);
   const double t = NearArith::quot(ms.pM, p);
   double r0 = rho, p0 = p, u0 = u;

@@ -8,6 +8,8 @@
 #include <random>
 #undef __builtin_amdgcn_rcp
 #undef __builtin_amdgcn_rsq
+#undef __builtin_amdgcn_div_fixup
+#undef __builtin_amdgcn_class
 static std::mt19937_64 rng(11);
 static double Off() { return 1.0 + std::uniform_real_distribution<double>(-0x1p-24, 0x1p-24)(rng); }
 static double Rcp(double b) { return (1.0 / b) * Off(); }

@@ -44,6 +44,10 @@ int main() {
   bad += fvs::PowState(0.0, e) != 0.0;
   bad += !std::isinf(fvs::PowState(HUGE_VAL, e));
   bad += !std::isnan(fvs::PowState(-1.0, e)) + !std::isnan(fvs::PowState(NAN, e));
+  // negative numbers have whole powers only (and infinite ones any)
+  bad += fvs::PowState(-2.0, 3.0) != -8.0 || fvs::PowState(-2.0, 4.0) != 16.0;
+  bad += !std::isnan(fvs::PowState(-2.0, 5.000000000000001));
+  bad += fvs::PowState(-HUGE_VAL, 3.0) != -HUGE_VAL || fvs::PowState(-HUGE_VAL, 5.5) != HUGE_VAL;
   std::printf("%.3f %.3f %d\n", worst[0], worst[1], bad);
   return 0;
 }

@@ -1998,9 +1998,22 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
     return fail(FVS_HIP_ERROR);
   }
   (void)hipFree(flags);
+  // list of the interior cut cells
+  std::vector<int32_t> cut;
+  for (int64_t j = 0; j < ny; ++j)
+    for (int64_t i = 0; i < nx; ++i)
+      if (hflags[j * nx + i]) cut.push_back(static_cast<int32_t>((j + kG) * ngx + (i + kG)));
   // geometry words of every cell (CellCode) and the irregular cells per
   // direction
   {
+    // bit d: a wall flux in the cell or a neighbour of it along d
+    std::vector<uint8_t> wall(ncg, 0);
+    for (const int64_t c : cut) {
+      for (int64_t f = -1; f <= 1; ++f) {
+        wall[c + f] |= 1;
+        wall[c + f * ngx] |= 2;
+      }
+    }
     std::vector<double> ha(ncg), hbx(nbx), hby(nby);
     if (hipMemcpyAsync(ha.data(), ga, ncg * sizeof(double), hipMemcpyDeviceToHost, s) !=
             hipSuccess ||
@@ -2015,10 +2028,6 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
       auto beta = [&](int64_t ci, int64_t cj) {
         return d == 0 ? hbx[cj * (ngx + 1) + ci] : hby[cj * ngx + ci];
       };
-      auto is_cut = [&](int64_t ci, int64_t cj) {
-        const int64_t i = ci - kG, j = cj - kG;
-        return i >= 0 && i < nx && j >= 0 && j < ny && hflags[j * nx + i] != 0;
-      };
       std::vector<int32_t> code(ncg), cells;
       for (int64_t cj = 0; cj < ngy; ++cj)
         for (int64_t ci = 0; ci < ngx; ++ci) {
@@ -2029,11 +2038,9 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
           if (interior && a != 0.0) {
             // face fractions at faces i - 1 .. i + 2 (or j - 1 .. j + 2), and
             // no wall flux in the cells i - 1 .. i + 1
-            bool regular = a == 1.0;
+            bool regular = a == 1.0 && !(wall[c] & (1 << d));
             for (int64_t f = -1; f <= 2 && regular; ++f)
               regular = (d == 0 ? beta(ci + f, cj) : beta(ci, cj + f)) == 1.0;
-            for (int64_t f = -1; f <= 1 && regular; ++f)
-              regular = d == 0 ? !is_cut(ci + f, cj) : !is_cut(ci, cj + f);
             if (regular) {
               kind = CellCode::kRegular;
             } else {
@@ -2060,11 +2067,6 @@ int fvs_kbn_level_create(fvs_handle* h, const fvs_patch_desc* patch,
       L->lg.irr_flux[d] = L->irr_flux[d];
     }
   }
-  // list of the interior cut cells
-  std::vector<int32_t> cut;
-  for (int64_t j = 0; j < ny; ++j)
-    for (int64_t i = 0; i < nx; ++i)
-      if (hflags[j * nx + i]) cut.push_back(static_cast<int32_t>((j + kG) * ngx + (i + kG)));
   L->ncut = static_cast<int>(cut.size());
   const int nc = L->ncut > 0 ? L->ncut : 1;
   if (hipMalloc(&L->cut, nc * sizeof(int32_t)) != hipSuccess ||

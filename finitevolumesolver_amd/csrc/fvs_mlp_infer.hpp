@@ -161,13 +161,13 @@ __device__ __forceinline__ bool WeakPair(double rhoL, double uL, double pL, doub
   return ep < kWeakPair * sp && eu < kWeakPair * sp;
 }
 
-
 // Waves run the network only when at least this many of their 64 faces are
 // non-weak.  A wave's Newton loop runs until its slowest face converges, so
 // a few strong faces among weak ones gain little from the guess while the
-// whole wave pays for the inference.  40 against 48 saves another 3% of the
-// strong field's iterations at equal step time.
-constexpr int kWaveStrongLanes = 40;
+// whole wave pays for the inference.  First-order step on strong waves,
+// 203 x 149 x 121 and 256^3: 960 and 3565 us with 40, 938 and 3480 us with 48
+// (a smooth field: equal).
+constexpr int kWaveStrongLanes = 48;
 
 // The learned initial guess of one face per lane; every lane of the wave
 // must call it (the matrix-core step is wave-wide).  Weak pairs, and every

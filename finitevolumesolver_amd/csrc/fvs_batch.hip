@@ -68,7 +68,7 @@ __device__ __forceinline__ unsigned long long WaveMinK(unsigned long long k) {
 // DPP shifts; the shifts across a row's ends carry values no lane uses.
 // Loads across the sweep are short where W is large in Y, which the caches
 // absorb: the kernel is bound by its FP64 instructions.  A level of a million
-// cells: X 32, Y 33 us (about 22 of instruction issue); with states and fluxes
+// cells: X 32, Y 33 us (19 to 22 of instruction issue, VALU busy 53 to 64%); with states and fluxes
 // staged in LDS by workgroup tiles (three barriers a tile, IEEE sequences) 42
 // and 48.  Every lane loads (clamped into the patch's ghost ring) and computes,
 // and the stores and minima are masked.

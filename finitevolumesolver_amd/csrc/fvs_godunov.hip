@@ -364,11 +364,13 @@ __device__ __forceinline__ void CheckFace(const double* uL, const double* uR, bo
 // matrix-core code or its registers.  MUSCL: half-step states (FP64, mean
 // guess) and, with a.check, the cells' CFL check; a ghost slot's slopes vanish
 // (its clamped value equals its inner neighbour's; NoLimiter's outer neighbour
-// is replaced).  Bound by Newton's FP64 issue at two waves per SIMD (180 to 230
+// is replaced).  Bound by Newton's FP64 instructions (1560 a cell at 256^3,
+// smooth and strong waves; VALU busy 76%) at two waves per SIMD (180 to 250
 // registers; held to 168 or 128 it spills and runs 1.5 to 3 times slower).
-// 384^3 strong-wave blocks: 3.9 -> 2.9 ms a sweep against one wave per 62
-// slots with LDS shuffles; MUSCL over 256^3: 8.6 -> 2.8 ms a step against the
-// patch operators' passes (fluxes, stable dt, update, completion).
+// 384^3 strong-wave blocks, faces seeded by the CFL pass: 3.9 -> 2.9 ms a sweep
+// against one wave per 62 slots with LDS shuffles (3.9 ms from the mean guess,
+// as now); MUSCL over 256^3: 8.6 -> 2.8 ms a step against the patch operators'
+// passes (fluxes, stable dt, update, completion).
 // LONG: rows of kXLongRow cells or more, whose offsets take 64 bits.
 template <int D, bool MIXED, bool LEARNED, bool MUSCL, bool LONG>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovSweepX(GodunovArgs a) {
@@ -493,7 +495,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 
 // Y / Z sweep: one thread per pencil marching a segment with the cell before
 // (and, MUSCL, around) the face in registers and the next cell's load in
-// flight.  Bound by Newton's FP64 issue, like the X sweep.
+// flight.  Bound by Newton's FP64 instructions, like the X sweep (1080 a cell,
+// VALU busy 74%).
 template <int D, int DIR, bool MIXED, bool LEARNED, bool MUSCL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void GodunovSweepPencil(GodunovArgs a) {
   constexpr int NC = D + 2;
@@ -753,16 +756,18 @@ __global__ __launch_bounds__(kBlock) void GodunovViewStableDt(DevView st, DevVie
 //
 // With a speed floor (floor[d] > 0, a lower bound of direction d's largest
 // speed) a face is solved only when its certified bounds (QuickSpeedBelow for
-// every face, SpeedBelow for those it leaves) reach the floor; blocks whose solved faces reach it set hit[d], which proves that
-// the skipped ones are slower than the maximum.  Without a floor every face is
+// every face, SpeedBelow for those it leaves) reach the floor; blocks whose
+// solved faces reach it set hit[d], which proves that the skipped ones are
+// slower than the maximum.  Without a floor every face is
 // solved, by the same instructions, so dt does not depend on the floor.
 //
 // 3D: a workgroup's eight waves are eight x rows of 64 cells marching along
 // z; lanes 1..62 own their cells and lane 0 and row 0 are halos.  2D: each
 // wave marches along y by itself.  A cell's six floats reach the x neighbour
 // by DPP, the y neighbour through LDS (3D), the marching neighbour in
-// registers; faces to be solved reload their cells.  Bound by instruction
-// issue (about 350 a cell) next to one read of the state.  The kernel it
+// registers; faces to be solved reload their cells.  Bound by the serial march
+// (a step's loads and barriers) and 318 (smooth) to 380 (strong waves)
+// instructions a cell, VALU busy 47%, next to one read of the state.  The kernel it
 // replaces solved every face of the first sweep's direction, for that sweep's
 // reuse, and every face outside a narrow class; solving them in the sweep
 // alone costs less.  First-order step, 384^3 strong-wave blocks: 19.7 -> 11.0

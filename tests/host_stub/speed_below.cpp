@@ -2,7 +2,7 @@
 // conservative states (rho, m0, m1, E each side) and a speed a pair, doubles
 // in component-major order, from the file argv[1]; prints how many pairs each
 // test certifies to stay below their own speed, and below 1.05 and 2 times it.
-// argv[2]: Newton iteration cap.
+// argv[2]: Newton iteration cap, argv[3]: gamma.
 #include <cmath>
 #define __builtin_amdgcn_rsqf(x) (1.0f / std::sqrt(x))
 #include "fvs_godunov_bound.hpp"
@@ -18,8 +18,9 @@ int main(int argc, char** argv) {
   std::rewind(f);
   std::vector<double> v(9 * n);
   if (std::fread(v.data(), 72, n, f) != static_cast<size_t>(n)) return 1;
-  const fvs::SpeedBound b = fvs::MakeSpeedBound(1.4, 1e-7, std::atoi(argv[2]));
-  const fvs::Gas<double> g{1.4, 1.0 / (1.4 - 1.0), 1.4 - 1.0};
+  const double gamma = std::atof(argv[3]);
+  const fvs::SpeedBound b = fvs::MakeSpeedBound(gamma, 1e-7, std::atoi(argv[2]));
+  const fvs::Gas<double> g{gamma, 1.0 / (gamma - 1.0), gamma - 1.0};
   long count[2][3] = {};
   const double scale[3] = {1.0 - 0x1p-20, 1.05, 2.0};
   for (long i = 0; i < n; ++i) {

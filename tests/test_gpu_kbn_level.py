@@ -25,18 +25,18 @@ def _note(msg):
 
 
 def _one_pass_cfl(nx, ny):
-    """The level's choice of step-start CFL kernel: the one-pass kernel
-    (255 owned columns by 8-row segments per workgroup) when its tiles fit
-    the level's workgroup count (one per 256 faces of the larger direction),
-    else one pass per direction."""
-    tiles = -(-(nx + 1) // 255) * -(-(ny + 1) // 8)
+    """The level's choice of step-start CFL kernel: the one-pass kernel (waves
+    of 63 owned columns by 8-row segments, four a workgroup) when its
+    workgroups fit the level's count (one per 256 faces of the larger
+    direction), else one pass per direction."""
+    tiles = -(-(-(-(nx + 1) // 63) * -(-(ny + 1) // 8)) // 4)
     nblocks = -(-max((nx + 1) * ny, nx * (ny + 1)) // 256)
     return tiles <= nblocks
 
 
 def test_cfl_kernel_choice_covers_both_paths():
     assert _one_pass_cfl(160, 80) and _one_pass_cfl(121, 61)
-    assert not _one_pass_cfl(16, 512)
+    assert _one_pass_cfl(16, 512) and not _one_pass_cfl(7, 512)
 
 
 @pytest.mark.parametrize("solver,integrator,splitting,shape", [
@@ -47,8 +47,9 @@ def test_cfl_kernel_choice_covers_both_paths():
     # ragged: the last 60-cell row segment holds one cell, the last
     # 16-row column segment 13 rows
     ("hllem", "TimeIntegrator", "Godunov", (121, 61)),
-    # narrow: too few cells per workgroup for the one-pass step-start CFL
-    # kernel, so the two per-direction passes run
+    # narrow: waves of the one-pass step-start CFL kernel with 17 of 63
+    # columns (a level of seven columns takes the per-direction passes:
+    # test_gpu_kbn_regular.py)
     ("hllem", "TimeIntegrator", "Godunov", (16, 512)),
 ])
 def test_cutcell_level_matches_oracle(cuda, solver, integrator, splitting, shape):

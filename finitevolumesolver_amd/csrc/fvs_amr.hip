@@ -554,12 +554,6 @@ int FillPhysical(fvs_amr* A, int l, int which, int d) {
   return FVS_OK;
 }
 
-int SetDt(fvs_amr* A, int l, double dt) {
-  hipLaunchKernelGGL(FillKernel, dim3(1), dim3(64), 0, A->s, A->lv[l]->dts, int64_t(1), dt);
-  FVS_LAUNCH_CHECK();
-  return FVS_OK;
-}
-
 // Arguments of the register contributions of register f (between level f
 // and level f - 1) from a sweep in dir of the fine (fine = 1) or the coarse
 // level reading pool src; count 0 when the register has no such entries.

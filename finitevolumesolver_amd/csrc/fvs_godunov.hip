@@ -337,7 +337,6 @@ template <int D, int DIR>
 __device__ __forceinline__ void CheckFace(const double* uL, const double* uR, bool face,
                                           const GodunovArgs& a, const Gas<double>& g, float crit,
                                           FaceSums& sums) {
-  using I = Idx<D>;
   const SpeedCell<D> l = MakeSpeedCell<D>(uL, g), r = MakeSpeedCell<D>(uR, g);
   bool pass = !face || QuickSpeedBelow<D>(l, l.u[DIR], r, r.u[DIR], a.bound, crit);
   if (__builtin_expect(__any(!pass), 0)) {

@@ -100,11 +100,12 @@ struct Ctl {
   int have_failure;   // use failure_dt for the next step
   int halt;           // 0 running, 1 TimeStepTooLarge, 2 final time reached,
                       // 3 the speed floor of the step-start CFL pass was wrong
-                      // (the host repeats the step without it)
+                      // (the host repeats the step; floor_known says with
+                      // which floor)
   int64_t cycle;
   double dt_dir[3];   // step-start stable dt per direction (decoded)
   double last_check;
-  // 3D step-start CFL pass: a speed floor per direction (0: none), the
+  // Step-start CFL pass (3D HLLEM, exact Godunov): a speed floor per direction (0: none), the
   // previous pass's largest signal speed less floor_margin.  The pass
   // evaluates the exact speed only of faces whose cheap upper bound reaches
   // it; floor_hit[d] records that some evaluated face did reach it, which

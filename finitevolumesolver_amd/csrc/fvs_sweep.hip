@@ -903,7 +903,7 @@ __device__ __forceinline__ void ReduceKeysMulti(const unsigned long long* p, int
 
 __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
     const unsigned long long* partials, int64_t n, double* out, Ctl* ctl) {
-  // control words read ahead of the reduction, not after it
+  // control words read ahead of the reduction, not after it (hence not EndStep)
   const int halt = ctl ? ctl->halt : 0;
   const double split_dt = ctl ? ctl->split_dt : 0.0;
   if (halt) return;
@@ -924,8 +924,9 @@ __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
 }
 
 // The CFL pass's speed floor after a pass: a floor that no evaluated face
-// reached may have hidden the fastest face, so the step is repeated without
-// a floor (halt 3) and the margin quadruples; otherwise the next floor is
+// reached may have hidden the fastest face, so the step is repeated (halt 3)
+// without that floor (exact Godunov: first with the cells', floor_known) and
+// the margin quadruples; otherwise the next floor is
 // this pass's largest speed per direction (dx / dt) less a margin that
 // follows how fast that speed falls.  Returns false after setting halt 3.
 __device__ __forceinline__ bool RenewSpeedFloor(Ctl* ctl, const double* v, const double* fdx, int dim) {
@@ -1073,7 +1074,7 @@ __global__ void StepEndKernel(Ctl* ctl) {
 // and a step-end kernel.
 __global__ __launch_bounds__(kRedBlock) void FinalizeStepKernel(
     const unsigned long long* partials, CheckList cl, Ctl* ctl) {
-  // control words read ahead of the reduction, not after it
+  // control words read ahead of the reduction, not after it (hence not EndStep)
   const int halt = ctl->halt;
   const double split_dt = ctl->split_dt, dt = ctl->dt, t = ctl->t;
   const int64_t cycle = ctl->cycle, log_base = ctl->dt_log_base, log_len = ctl->dt_log_len;

@@ -295,13 +295,15 @@ int fvs_level_time(fvs_level* level, double* t, int64_t* cycles);
  * whose certified upper bound reaches a floor, the previous pass's largest
  * signal speed less a margin (four times its last relative drop, between
  * 2^-10 and 1/4), and confirms that some evaluated face did reach it.  When
- * none did, the step is repeated with every face evaluated (and the margin
- * quadruples), so the floor never changes a result.  An exact-Godunov level
- * that has no floor yet (a new state's first step) takes one from its cells'
- * |u| + a.
+ * none did, the step is repeated (and the margin quadruples), so the floor
+ * never changes a result: on an HLLEM level with every face evaluated, on an
+ * exact-Godunov level first with a floor from its cells' |u| + a, and with
+ * every face evaluated if that one is not reached either.  An exact-Godunov
+ * level that has no floor yet (a new state's first step) takes the cells'.
  * fvs_level_hint_max_speed sets the floor for the current state
  * (speed[d] >= 0; 0: none; ignored by other levels); fvs_level_cfl_redos
- * reports how many steps were repeated. */
+ * reports how many repeats there were (a step can have two on an exact-Godunov
+ * level). */
 int fvs_level_hint_max_speed(fvs_level* level, const double speed[3]);
 int fvs_level_cfl_redos(fvs_level* level, int64_t* redos);
 
@@ -448,8 +450,8 @@ int fvs_mlp_infer_pairs(fvs_mlp* mlp, int dim, int dir, const double* left,
 int fvs_mlp_face_guess(fvs_mlp* mlp, int dim, double gamma, const double* const* cons,
                        const int64_t n[3], int dir, double* guess);
 /* Attaches a network to a first-order exact-Godunov handle: the level
- * driver then seeds every Newton iteration (fluxes and CFL) with it.
- * NULL detaches.  The handle does not own the network. */
+ * driver's sweeps then seed their Newton iterations with it (the step-start
+ * CFL pass starts from the mean pressure).  NULL detaches.  The handle does not own the network. */
 int fvs_set_mlp(fvs_handle* h, fvs_mlp* mlp);
 
 /* ---- KBN h-box cut-cell method (KbnCutCellMethod) ---------------------- */
@@ -648,6 +650,8 @@ int fvs_amr_stable_dt(fvs_amr* amr, double* dt_host);
 /* fvs_amr_stable_dt that also keeps the state (pool 0 of every level, ghost
  * layers included, in device memory of the hierarchy) for fvs_amr_restore,
  * which puts it back any number of times: the reference's data / scratch pair.
+ * The first call allocates one more pool per level, kept until the hierarchy is
+ * destroyed.
  * Waits for the dt only. */
 int fvs_amr_begin_step(fvs_amr* amr, double* dt_host);
 int fvs_amr_restore(fvs_amr* amr);

@@ -903,7 +903,7 @@ __device__ __forceinline__ void ReduceKeysMulti(const unsigned long long* p, int
 
 __global__ __launch_bounds__(kRedBlock) void FinalizeCheckKernel(
     const unsigned long long* partials, int64_t n, double* out, Ctl* ctl) {
-  // control words read ahead of the reduction, not after it (hence not EndStep)
+  // control words read ahead of the reduction, not after it
   const int halt = ctl ? ctl->halt : 0;
   const double split_dt = ctl ? ctl->split_dt : 0.0;
   if (halt) return;

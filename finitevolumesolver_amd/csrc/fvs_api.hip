@@ -1073,6 +1073,14 @@ int fvs_level_create(fvs_handle* h, const fvs_patch_desc* patch, fvs_level** out
     SetError("level initialisation failed");
     return FVS_HIP_ERROR;
   }
+  // The capture stream, while nothing runs: created between steps in flight it
+  // waits for all of them, and the first one of a process takes milliseconds
+  // (256^3, a process's first 50 steps: 57 to 63 ms with it made at the first
+  // capture, 57 with it made here).  A failure shows at the first capture.
+  if (hipStreamCreateWithFlags(&L->cap, hipStreamNonBlocking) != hipSuccess) {
+    L->cap = nullptr;
+    (void)hipGetLastError();
+  }
   *out = L;
   return FVS_OK;
 }
